@@ -616,12 +616,31 @@ int gemm(const void* act, int64_t ldact, const void* weight, int64_t ldw, const 
 bool uqvk_fused_shape(const HstuUqvkArgs* a) {
     const int n_u = a->hidden_dim * a->heads;
     const int n_out = (2 * a->hidden_dim + 2 * a->attn_dim) * a->heads;
-    return (a->d_model == 128 || a->d_model == 256 || a->d_model == 384 || a->d_model == 512) && n_u % 128 == 0 && n_out % 128 == 0 &&
-           (a->dtype == 0 || a->dtype == 1);
+    // (SiLU is applied per 32 columns; the e4m3 copy, which the kernel makes per 64 columns of one tensor, wants whole 128s)
+    return (a->d_model == 128 || a->d_model == 256 || a->d_model == 384 || a->d_model == 512) &&
+           n_u % (a->qkv_fp8 ? 128 : 32) == 0 && n_out % 128 == 0 && (a->dtype == 0 || a->dtype == 1);
+}
+
+// Column blocks (of 128) per workgroup of the fused producer.  With two workgroups resident per CU a launch runs in rounds of
+// 512; a workgroup costs its prologue (the rows' layer norm, about 2.3 column blocks' time) plus its column blocks, and the
+// cheapest division of a row block's columns is the one with the smallest rounds x (prologue + blocks).  Few rows: 50
+// rows of d_model 512 into 2048 columns took 89 us when one workgroup walked all of W, 19 us with 16 (what the host needs
+// for the call); 8192 rows 95 -> 36 us with 8; 80000 rows (625 row blocks, 1.2 rounds) 259 -> 226 us with 2.  From two full rounds on the
+// workgroups no longer start together and the division only repeats prologues: 136226 rows 407 us undivided, 426 us with 2.
+int uqvk_chunks_per_wg(long long row_blocks, int nchunks) {
+    if (row_blocks >= 2 * 512) return nchunks;
+    int best = nchunks;
+    float best_cost = 0.f;
+    for (int per = nchunks; per >= 1; --per) {
+        const long long rounds = (row_blocks * ((nchunks + per - 1) / per) + 511) / 512;
+        const float cost = (float)rounds * (2.3f + (float)per);
+        if (per == nchunks || cost < best_cost) best_cost = cost, best = per;
+    }
+    return best;
 }
 
 template <class TT, int KT>
-int launch_uqvk_fused(const hstu::UqvkFusedParams& p, hipStream_t stream) {
+int launch_uqvk_fused(hstu::UqvkFusedParams p, hipStream_t stream) {
     auto kern = hstu::hstu_uqvk_fused_kernel<TT, KT>;
     // (a function attribute belongs to the device it was set on: one flag per device)
     static bool attr_done[64];
@@ -637,7 +656,10 @@ int launch_uqvk_fused(const hstu::UqvkFusedParams& p, hipStream_t stream) {
     }
     constexpr int kRows = hstu::kUqvkWaves * hstu::kUqvkRowsPerWave;
     const long long grid = (p.rows + kRows - 1) / kRows;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(hstu::kUqvkWaves * 64), hstu::kUqvkLds, stream, p);
+    const int nchunks = p.n_out / hstu::kUqvkTileN;
+    p.chunks_per_wg = uqvk_chunks_per_wg(grid, nchunks);
+    const unsigned splits = (unsigned)((nchunks + p.chunks_per_wg - 1) / p.chunks_per_wg);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid, splits), dim3(hstu::kUqvkWaves * 64), hstu::kUqvkLds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         snprintf(g_last_error, sizeof(g_last_error), "fused uqvk kernel launch: %s", hipGetErrorString(e));

@@ -11,8 +11,8 @@
 // global_load_lds_dwordx4, and is read transposed (ds_read_b64_tr_b16) as the A operand:
 //     C^T[n, r] += W^T[n, k] . LN(x)^T[k, r]
 // so that a lane ends up with one output row and, per 32-column block, four runs of four consecutive columns -- the
-// accumulator layout of the attention kernels.  A workgroup of 4 waves owns 128 rows and walks all of W once (two
-// workgroups per CU): for each block of 128 output columns, d_model / 64 k tiles of 16 MFMAs per wave, then the
+// accumulator layout of the attention kernels.  A workgroup of 4 waves owns 128 rows and walks its share of W's columns
+// once (all of them when the row blocks alone fill the chip, see uqvk_chunks_per_wg; two workgroups per CU): for each block of 128 output columns, d_model / 64 k tiles of 16 MFMAs per wave, then the
 // epilogue (bias from LDS, SiLU for the u columns, rounding, a transposition through a per-wave LDS area so that
 // every store instruction covers whole 128-byte lines).  W (2 MB for 512 x 2048) stays in every XCD's L2.
 // Stores count in the same counter as the copies (vmcnt), so the wait after an epilogue leaves room for them.
@@ -32,7 +32,8 @@ struct UqvkFusedParams {
     char* out;         // [rows, n_out] dense
     int64_t rows;
     int n_out;   // multiple of 128
-    int n_silu;  // multiple of 128: columns [0, n_silu) go through SiLU
+    int n_silu;  // multiple of 32: columns [0, n_silu) go through SiLU
+    int chunks_per_wg;  // column blocks (of 128) a workgroup walks: the grid holds ceil(n_out / 128 / chunks_per_wg) workgroups per row block
     // Optional second output: the v | q | k columns (those from n_silu on) once more as e4m3 bytes,
     // out8[r, n - n_silu] = e4m3(rounded out[r, n] * inv_scale[t]), t = 0 (v: the next n_silu columns), 1 (q: the next
     // n_attn), 2 (k: the rest), clamped to +-448; and the largest |rounded out| of each of the three, for the scales of
@@ -70,7 +71,10 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, l32 = lane & 31;
     const int64_t row0 = ((int64_t)blockIdx.x * kUqvkWaves + wave) * kUqvkRowsPerWave;  // first row of the wave
-    const int nchunks = p.n_out / kUqvkTileN;
+    // the column blocks of this workgroup: [c_begin, c_begin + nchunks)
+    const int c_begin = blockIdx.y * p.chunks_per_wg;
+    const int left = p.n_out / kUqvkTileN - c_begin;
+    const int nchunks = left < p.chunks_per_wg ? left : p.chunks_per_wg;
     const int ntiles = nchunks * KT;
 
     // copy of tile t = (column block c, k tile kt) into slot t % 3; wave 0 adds the block's bias values with the first k tile
@@ -85,12 +89,12 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
     auto issue_copy = [&](int t) {
         const int c = t / KT, kt = t - c * KT;
         char* slot = smem + (t % 3) * kUqvkSlot;
-        const char* src = p.w + ((int64_t)kt * kUqvkTileK * p.n_out + (int64_t)c * kUqvkTileN) * 2;
+        const char* src = p.w + ((int64_t)kt * kUqvkTileK * p.n_out + (int64_t)(c_begin + c) * kUqvkTileN) * 2;
 #pragma unroll
         for (int i = 0; i < NPW; ++i) global_load_lds16_soff(src, coff[i], slot + (wave + kUqvkWaves * i) * 1024);
         // block c's bias is read after its last k tile, when at most the copies of block c + 1 have been issued
         if (kt == 0 && wave == 0 && lane < 16)
-            global_load_lds16(p.bias + (int64_t)c * kUqvkTileN * 2 + lane * 16, smem + 3 * kUqvkSlot + (c & 3) * 256);
+            global_load_lds16(p.bias + (int64_t)(c_begin + c) * kUqvkTileN * 2 + lane * 16, smem + 3 * kUqvkSlot + (c & 3) * 256);
     };
     issue_copy(0);
     if (ntiles > 1) issue_copy(1);
@@ -193,7 +197,7 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- epilogue of the column block: bias, SiLU for the u columns, rounding, transposition through LDS, stores
-        const bool silu = c * kUqvkTileN < p.n_silu;
+        const int col_block = (c_begin + c) * kUqvkTileN;
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
@@ -201,6 +205,7 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
 #pragma unroll
             for (int d2 = 0; d2 < 2; ++d2) {
                 const int dt = hf * 2 + d2;
+                const bool silu = col_block + dt * 32 < p.n_silu;
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
                     typedef __attribute__((ext_vector_type(4))) elem elem4;
@@ -217,7 +222,7 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
             }
             // 8 lanes cover one row's 128 bytes, 8 rows per instruction
             const int chunk = lane & 7, rsub = lane >> 3;
-            const int col0 = c * kUqvkTileN + hf * 64;  // first column of this half block
+            const int col0 = col_block + hf * 64;  // first column of this half block
             const bool to8 = p.out8 != nullptr && col0 >= p.n_silu;
             const int tensor = col0 < 2 * p.n_silu ? 0 : col0 < 2 * p.n_silu + p.n_attn ? 1 : 2;
 #pragma unroll

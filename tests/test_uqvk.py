@@ -199,6 +199,33 @@ def test_compute_uqvk_hand_written_gemm(pkg, dev, L, d_model, H, attn, hidden, d
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L,d_model,H,attn,hidden", [(129, 128, 1, 32, 32), (1, 256, 2, 64, 32), (300, 384, 3, 96, 32), (40, 512, 1, 64, 64)])
+def test_uqvk_fused_kernel_with_u_columns_that_end_inside_a_block(pkg, dev, L, d_model, H, attn, hidden):
+    """The fused kernel's blocks of 128 columns may hold the end of the u columns (a multiple of 32)."""
+    print(f"[case] uqvk u columns {L} {d_model} {H} {attn} {hidden}", flush=True)
+    x, nw, nb, w, b = _inputs(L + 7, L, d_model, H, attn, hidden, torch.bfloat16)
+    got = pkg.hstu_compute_uqvk(x.to(dev), nw.to(dev), nb.to(dev), 1e-6, H, attn, hidden, w.to(dev), b.to(dev), path=2)
+    torch.cuda.synchronize()
+    for name, g_, ref in zip("uqkv", got, U.compute_uqvk(x, nw, nb, 1e-6, H, attn, hidden, w, b)):
+        _close(g_, ref, name)
+
+
+@pytest.mark.gpu
+def test_uqvk_columns_divided_over_workgroups_give_the_same_bits(pkg, dev):
+    """A row's result does not depend on how many workgroups share its row block's columns (16 blocks of 128: one
+    workgroup for 131073 rows, several below, sixteen for a few)."""
+    d_model, H, D = 128, 4, 128
+    x, nw, nb, w, b = [t.to(dev) for t in _inputs(3, 131073, d_model, H, D, D, torch.bfloat16)]
+    whole = pkg.hstu_compute_uqvk(x, nw, nb, 1e-6, H, D, D, w, b, path=2)
+    for L in (1, 128, 129, 4097, 20000, 70000):
+        print(f"[case] uqvk divided columns {L}", flush=True)
+        part = pkg.hstu_compute_uqvk(x[:L], nw, nb, 1e-6, H, D, D, w, b, path=2)
+        torch.cuda.synchronize()
+        for g_, w_ in zip(part, whole):
+            assert torch.equal(g_, w_[:L])
+
+
+@pytest.mark.gpu
 def test_uqvk_with_a_total_length_that_changes_from_batch_to_batch(pkg, dev):
     """The hipBLASLt path keeps one plan per size class of the row count, not per row count: lengths of one class
     (1100, 1101, 1279), of others (640, 5000), and the first again, each against the oracle."""
