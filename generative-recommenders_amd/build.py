@@ -1,15 +1,17 @@
 """Compile ``csrc/`` into ``csrc/libhstu_hip.so`` and ``csrc/libhstu_linear.so`` with hipcc for gfx950 (cross-compiles
-without a GPU)."""
+without a GPU), and ``csrc/hstu_native.so``, the operators' native front, with the host compiler."""
 
 import os
 import shutil
 import subprocess
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(_HERE), "include")
 LIB_PATH = os.path.join(CSRC, "libhstu_hip.so")
 LINEAR_LIB_PATH = os.path.join(CSRC, "libhstu_linear.so")  # separate: it links hipBLASLt, the attention library does not
+NATIVE_PATH = os.path.join(CSRC, "hstu_native.so")  # links the two above and libtorch; finds them beside itself
 
 # -packed-fp32-ops off: hipcc must not fuse scalar float code into v_pk_*_f32 on this hardware pool.
 HIPCC_FLAGS = [
@@ -33,9 +35,29 @@ def _run(cmd, verbose):
         print(" ".join(cmd))
 
 
+def _native_commands():
+    """Compile and link commands of the native front (host code only: the linking needs the two libraries)."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    obj = os.path.join(CSRC, "hstu_native.o")
+    cxx = shutil.which("g++") or "c++"
+    includes = [f"-I{INCLUDE}"]
+    for path in (os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include",
+                 sysconfig.get_paths()["include"]):
+        includes += ["-isystem", path]
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    compile_ = [cxx, "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+                "-DTORCH_EXTENSION_NAME=hstu_native", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *includes, "-c", os.path.join(CSRC, "hstu_native.cpp"), "-o", obj]
+    link = [cxx, "-shared", obj, "-o", NATIVE_PATH, f"-L{CSRC}", "-l:libhstu_hip.so", "-l:libhstu_linear.so", "-L" + os.path.join(root, "lib"),
+            "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    return compile_, link, obj
+
+
 def build_library(verbose: bool = False) -> str:
     """Always recompiles; returns the path of the attention library.  The translation units compile side by side
-    (forward, backward, dense steps), then libhstu_hip.so is linked from the first two."""
+    (forward, backward, dense steps, native front), then libhstu_hip.so is linked from the first two and the front against
+    both libraries."""
     from concurrent.futures import ThreadPoolExecutor
 
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -46,9 +68,12 @@ def build_library(verbose: bool = False) -> str:
         common + ["-c", os.path.join(CSRC, "hstu_bwd_api.hip"), "-o", objs[1]],
         common + ["-shared", os.path.join(CSRC, "hstu_linear.hip"), "-o", LINEAR_LIB_PATH, "-lhipblaslt"],
     ]
-    with ThreadPoolExecutor(max_workers=3) as pool:
+    native_compile, native_link, native_obj = _native_commands()
+    jobs.append(native_compile)
+    with ThreadPoolExecutor(max_workers=4) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB_PATH], verbose)
-    for o in objs:
+    _run(native_link, verbose)
+    for o in objs + [native_obj]:
         os.remove(o)
     return LIB_PATH

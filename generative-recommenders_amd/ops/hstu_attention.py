@@ -25,7 +25,7 @@ from typing import Optional
 import torch
 
 from ..common import HammerKernel, switch_to_contiguous_if_needed
-from . import hip_backend
+from . import hip_backend, native
 
 
 def _kernel_layout(x: torch.Tensor) -> torch.Tensor:
@@ -123,7 +123,6 @@ def _profiled(name: str):
     return decorate
 
 
-@_profiled("hstu_mha")
 def hstu_mha(
     max_seq_len: int,
     alpha: float,
@@ -164,6 +163,25 @@ def hstu_mha(
     ``hip_backend.mha_bwd_workspace_bytes`` bytes, kept by the caller across steps) selects the faster form that stores
     dS there; the choice never depends on how much device memory is free.
     """
+    if causal and dropout_pr < 1e-6 and attn_scale is None:
+        out = native.front.hstu_mha(
+            max_seq_len, alpha, q, k, v, seq_offsets, num_targets, max_attn_len, contextual_seq_len, min_full_attn_seq_len, sort_by_length,
+            q_scale, k_scale, v_scale, tile_config, kv_splits,
+        )
+        if out is not None:
+            return out
+    return _hstu_mha(
+        max_seq_len, alpha, q, k, v, seq_offsets, causal, dropout_pr, num_targets, attn_scale, max_attn_len, contextual_seq_len,
+        min_full_attn_seq_len, sort_by_length, q_scale, k_scale, v_scale, tile_config, kv_splits, bwd_workspace,
+    )
+
+
+@_profiled("hstu_mha")
+def _hstu_mha(
+    max_seq_len, alpha, q, k, v, seq_offsets, causal, dropout_pr, num_targets, attn_scale, max_attn_len, contextual_seq_len,
+    min_full_attn_seq_len, sort_by_length, q_scale, k_scale, v_scale, tile_config, kv_splits, bwd_workspace,
+) -> torch.Tensor:
+    """``hstu_mha`` for every call that the native front leaves: the checks, gradients, ``attn_scale``, copies."""
     torch._assert(max_seq_len > 0, "max_seq_len must be larger than 0")
     torch._assert(q.dim() == 3, "q must be 3-D")
     torch._assert(k.shape == q.shape, "k must be the same shape as q")
@@ -229,7 +247,6 @@ def hstu_mha(
     return out
 
 
-@_profiled("delta_hstu_mha")
 def delta_hstu_mha(
     max_seq_len: int,
     alpha: float,
@@ -252,6 +269,23 @@ def delta_hstu_mha(
 
     Returns ``[B * delta_size, H, Dv]`` in the dtype of ``delta_q`` (bf16 for fp8 inputs).
     """
+    out = native.front.delta_hstu_mha(
+        max_seq_len, alpha, delta_q, k, v, seq_offsets, num_targets, max_attn_len, contextual_seq_len, q_scale, k_scale, v_scale, tile_config,
+        kv_splits,
+    )
+    if out is not None:
+        return out
+    return _delta_hstu_mha(
+        max_seq_len, alpha, delta_q, k, v, seq_offsets, num_targets, max_attn_len, contextual_seq_len, q_scale, k_scale, v_scale, tile_config,
+        kv_splits,
+    )
+
+
+@_profiled("delta_hstu_mha")
+def _delta_hstu_mha(
+    max_seq_len, alpha, delta_q, k, v, seq_offsets, num_targets, max_attn_len, contextual_seq_len, q_scale, k_scale, v_scale, tile_config, kv_splits,
+) -> torch.Tensor:
+    """``delta_hstu_mha`` for every call that the native front leaves."""
     torch._assert(delta_q.dim() == 3, "delta_q must be 3-D")
     L, H, D = delta_q.shape
     B = seq_offsets.size(0) - 1

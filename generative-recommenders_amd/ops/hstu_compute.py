@@ -23,6 +23,7 @@ import torch.nn.functional as F
 
 from ..build import LINEAR_LIB_PATH
 from ..common import HammerKernel
+from . import native
 
 
 class HstuUqvkArgs(ctypes.Structure):
@@ -281,6 +282,9 @@ def hstu_compute_uqvk(
     hipBLASLt; 1 = layer-norm kernel + hipBLASLt; 2 = the fused kernel; 3 = layer-norm kernel + hand-written GEMM
     (d_model a multiple of 64, hidden * H and the output width multiples of 256; slower than 1 at the sizes measured);
     2 and 3 raise ``NotImplementedError`` where they do not apply."""
+    parts = native.front.compute_uqvk(x, norm_weight, norm_bias, norm_eps, num_heads, attn_dim, hidden_dim, uvqk_weight, uvqk_bias, path)
+    if parts is not None:
+        return parts
     torch._assert(x.dim() == 2, "x must be 2-D")
     n_out = (2 * hidden_dim + 2 * attn_dim) * num_heads
     torch._assert(uvqk_weight.shape == (x.shape[1], n_out), "uvqk_weight must be [d_model, (2*hidden + 2*attn) * heads]")
@@ -540,6 +544,13 @@ def hstu_compute_output(
     reads ``u`` and ``attn`` where they are (``NotImplementedError`` if the shape does not fit: d_model a multiple of 256,
     heads * linear_dim a multiple of 64 -- or with dropout, whose mask covers the copied blocks too); 0 = whichever is
     faster for the shape (2 where it fits, rows >= 32768 and nothing is dropped).  Dropout as in ``norm_mul_dropout``."""
+    if not training or dropout_ratio <= 0.0:
+        out = native.front.compute_output(
+            attn, u, x, norm_weight, norm_bias, norm_eps, output_weight, num_heads, linear_dim, concat_u, concat_x,
+            MUL_U_ACTIVATIONS.get(mul_u_activation_type, -1), group_norm, path,
+        )
+        if out is not None:
+            return out
     torch._assert(x.dim() == 2 and x.shape[0] == attn.shape[0], "x must be 2-D with attn's row count")
     _check(x, attn, u, norm_weight, norm_bias, output_weight)
     torch._assert(mul_u_activation_type in MUL_U_ACTIVATIONS, "mul_u_activation_type must be none, sigmoid or silu")

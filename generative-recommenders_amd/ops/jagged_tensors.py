@@ -17,7 +17,7 @@ from typing import Optional, Tuple
 import torch
 
 from ..common import HammerKernel, switch_to_contiguous_if_needed
-from . import hip_backend
+from . import hip_backend, native
 
 
 def _needs_grad(*tensors: torch.Tensor) -> bool:
@@ -91,6 +91,9 @@ def concat_2D_jagged(
     """Per batch: rows of ``values_left`` followed by rows of ``values_right``; returns ``[L_left + L_right, D]``.
 
     A side without offsets is dense: exactly ``max_len_*`` rows per batch."""
+    out = native.front.concat_2d_jagged(values_left, values_right, max_len_left, max_len_right, offsets_left, offsets_right)
+    if out is not None:
+        return out
     torch._assert(values_left.dim() == 2, "values_left must be 2D")
     torch._assert(values_right.dim() == 2, "values_right must be 2D")
     torch._assert(
@@ -132,6 +135,9 @@ def split_2D_jagged(
     kernel: HammerKernel = HammerKernel.HIP,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Inverse of ``concat_2D_jagged``: returns ``(values_left, values_right)``."""
+    parts = native.front.split_2d_jagged(values, total_len_left, total_len_right, max_len_left, max_len_right, offsets_left, offsets_right)
+    if parts is not None:
+        return parts
     torch._assert(values.dim() == 2, "values must be 2D")
     torch._assert(
         offsets_left is not None or offsets_right is not None,
@@ -185,6 +191,8 @@ def write_kv_tail(full_values: torch.Tensor, full_offsets: torch.Tensor, delta_v
     sequence are overwritten with its block of ``delta_values``; the history rows are not touched, so the next
     micro-batch of candidates only repeats this call.  Returns ``full_values``.
     """
+    if native.front.write_kv_tail(full_values, full_offsets, delta_values):
+        return full_values
     torch._assert(full_values.dim() == 2 and delta_values.dim() == 2, "values must be 2D")
     torch._assert(full_values.shape[1] == delta_values.shape[1], "row widths must match")
     torch._assert(full_values.dtype == delta_values.dtype, "dtypes must match")
