@@ -56,24 +56,27 @@ def _native_commands():
 
 def build_library(verbose: bool = False) -> str:
     """Always recompiles; returns the path of the attention library.  The translation units compile side by side
-    (forward, backward, dense steps, native front), then libhstu_hip.so is linked from the first two and the front against
-    both libraries."""
+    (attention forward and backward, dense steps forward and backward, native front), then the two libraries are linked
+    and the front against both."""
     from concurrent.futures import ThreadPoolExecutor
 
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     common = [hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + ["-I", INCLUDE, "-I", CSRC]
     objs = [os.path.join(CSRC, "hstu_api.o"), os.path.join(CSRC, "hstu_bwd_api.o")]
+    linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o")]
     jobs = [
         common + ["-c", os.path.join(CSRC, "hstu_api.hip"), "-o", objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_bwd_api.hip"), "-o", objs[1]],
-        common + ["-shared", os.path.join(CSRC, "hstu_linear.hip"), "-o", LINEAR_LIB_PATH, "-lhipblaslt"],
+        common + ["-c", os.path.join(CSRC, "hstu_linear.hip"), "-o", linear_objs[0]],
+        common + ["-c", os.path.join(CSRC, "hstu_linear_bwd.hip"), "-o", linear_objs[1]],
     ]
     native_compile, native_link, native_obj = _native_commands()
     jobs.append(native_compile)
-    with ThreadPoolExecutor(max_workers=4) as pool:
+    with ThreadPoolExecutor(max_workers=5) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB_PATH], verbose)
+    _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + linear_objs + ["-o", LINEAR_LIB_PATH, "-lhipblaslt"], verbose)
     _run(native_link, verbose)
-    for o in objs + [native_obj]:
+    for o in objs + linear_objs + [native_obj]:
         os.remove(o)
     return LIB_PATH

@@ -12,23 +12,22 @@
 #include <mutex>
 #include <tuple>
 
-#include "hstu_philox.h"
+#include "hstu_rows.h"
 #include "hstu_uqvk_kernel.h"
 #include "hstu_output_kernel.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+using hstu::bf16x8_t;
+using hstu::f16x8_t;
+using hstu::dropout8;
+using hstu::dropout_params;
+using hstu::NormMulParams;
+using hstu::output_blocks;
+using hstu::sigmoid_f;
+using hstu::wave_sum;
 
 thread_local char g_last_error[256] = "";
-
-// Sum over the 64 lanes of a wave, result in every lane.
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
-}
 
 // One wave per row, rows dealt to the waves of the grid with a stride.  A lane holds NCH chunks of 8 elements
 // (chunk c of the row goes to lane c % 64), loaded once; mean and variance in fp32 (two passes over the
@@ -117,33 +116,6 @@ int launch_layer_norm(const void* x, int64_t x_rs, const void* weight, const voi
     return 0;
 }
 
-// ---- norm * u, concatenated with the copied blocks ------------------------------------------------------------------
-struct NormMulParams {
-    const char *attn, *u, *weight, *bias;
-    char* joined;
-    int64_t attn_rs, u_rs, joined_rs, rows;  // strides in elements
-    float eps;
-    int d, group_lanes;                      // row width; lanes per head (group norm)
-    int off_u, off_x, off_y;                 // column offsets of the blocks in `joined`, -1 = block absent
-    int silu_u, mul_act;
-    hstu::DropoutParams drop;                // thresh 0: no dropout
-    int64_t width;                           // logical width of `joined` (all blocks): the mask's row pitch
-};
-
-// Eight consecutive elements starting at column `col` (a multiple of 8) of row r: dropped or scaled, in fp32.
-template <class V8, class E>
-__device__ __forceinline__ V8 dropout8(const hstu::DropoutParams& d, int64_t r, int64_t width, int64_t col, const float (&x)[8]) {
-    const uint64_t group = (uint64_t)(r * width + col) >> 2;
-    const hstu::PhiloxWords a = hstu::dropout_words(d, group), b = hstu::dropout_words(d, group + 1);
-    V8 out;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        out[j] = (E)(a.w[j] >= d.thresh ? x[j] * d.scale : 0.f);
-        out[4 + j] = (E)(b.w[j] >= d.thresh ? x[4 + j] * d.scale : 0.f);
-    }
-    return out;
-}
-
 // keep[r * width + c] = 1 where the element survives: what the backward pass multiplies by (times the scale).
 __global__ __launch_bounds__(256) void hstu_dropout_mask_kernel(hstu::DropoutParams d, int64_t groups, unsigned char* keep) {
     for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += (int64_t)gridDim.x * 256) {
@@ -153,8 +125,6 @@ __global__ __launch_bounds__(256) void hstu_dropout_mask_kernel(hstu::DropoutPar
         ((uchar4*)keep)[g] = k;
     }
 }
-
-__device__ __forceinline__ float sigmoid_f(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
 // One wave per row as in the layer norm kernel.  GROUP: statistics per head (aligned groups of `group_lanes` lanes hold
 // one head's chunks, so the sums run over xor distances below group_lanes) and one weight / bias per head.
@@ -291,20 +261,6 @@ __global__ __launch_bounds__(256) void hstu_norm_mul_kernel(NormMulParams p) {
     }
 }
 
-// False: the ratio is not in [0, 1).
-bool dropout_params(float ratio, uint64_t seed, uint64_t offset, hstu::DropoutParams& d) {
-    if (!(ratio >= 0.f && ratio < 1.f)) return false;
-    d.seed = seed, d.offset = offset;
-    d.thresh = (uint32_t)((double)ratio * 4294967296.0);
-    d.scale = 1.0f / (1.0f - ratio);
-    return true;
-}
-
-int output_blocks(const HstuOutputArgs* a) {
-    if (a->group_norm) return (a->concat_u && a->concat_x) ? 3 : 1;
-    return 1 + (a->concat_u ? 1 : 0) + (a->concat_x ? 1 : 0);
-}
-
 int launch_norm_mul(const HstuOutputArgs* a, void* joined, int64_t joined_rs, hipStream_t stream);
 
 // path = 2: which shapes the concatenating GEMM kernel takes, and what the norm-multiply kernel has to leave for it.
@@ -381,35 +337,10 @@ int launch_output_fused(const HstuOutputArgs* a, hipStream_t stream) {
 }
 
 int launch_norm_mul(const HstuOutputArgs* a, void* joined, int64_t joined_rs, hipStream_t stream) {
-    if (a->rows < 0 || a->heads <= 0 || a->linear_dim <= 0) return -5;
-    const int64_t d64 = (int64_t)a->heads * a->linear_dim;
-    if (d64 > 4096 || (d64 & 7) != 0) return -5;
-    const int d = (int)d64, blocks = output_blocks(a);
-    if (a->attn_row_stride < d || a->u_row_stride < d || joined_rs < (int64_t)blocks * d) return -5;
-    if (((a->attn_row_stride | a->u_row_stride | joined_rs) & 7) != 0) return -4;
-    if (a->dtype != 0 && a->dtype != 1) return -2;
-    if (a->mul_u_activation < 0 || a->mul_u_activation > 2) return -5;
-    int group_lanes = 0;
-    if (a->group_norm) {
-        group_lanes = a->linear_dim / 8;
-        if ((a->linear_dim & 7) != 0 || group_lanes > 64 || (group_lanes & (group_lanes - 1)) != 0) return -6;
-    }
-    if (a->rows == 0) return 0;
-    if (!a->attn || !a->u || !a->norm_weight || !a->norm_bias || !joined) return -1;
-    if ((((uintptr_t)a->attn | (uintptr_t)a->u | (uintptr_t)joined) & 15) != 0) return -4;
-    if (!a->group_norm && (((uintptr_t)a->norm_weight | (uintptr_t)a->norm_bias) & 15) != 0) return -4;
     NormMulParams p;
-    p.attn = (const char*)a->attn, p.u = (const char*)a->u, p.weight = (const char*)a->norm_weight, p.bias = (const char*)a->norm_bias;
-    p.joined = (char*)joined;
-    p.attn_rs = a->attn_row_stride, p.u_rs = a->u_row_stride, p.joined_rs = joined_rs, p.rows = a->rows;
-    p.eps = a->norm_eps, p.d = d, p.group_lanes = group_lanes;
-    const bool cu = blocks == 3 || (!a->group_norm && a->concat_u), cx = blocks == 3 || (!a->group_norm && a->concat_x);
-    p.off_u = cu ? 0 : -1;
-    p.off_x = cx ? (cu ? d : 0) : -1;
-    p.off_y = (blocks - 1) * d;
-    p.silu_u = a->silu_u ? 1 : 0, p.mul_act = a->mul_u_activation;
-    p.width = (int64_t)blocks * d;
-    if (!dropout_params(a->dropout_ratio, a->dropout_seed, a->dropout_offset, p.drop)) return -5;
+    int rc = hstu::norm_mul_params(a, joined, joined_rs, true, p);
+    if (rc != 0 || a->rows == 0) return rc;
+    const int d = p.d;
     long long wgs = (a->rows + 3) / 4;
     if (wgs > 256 * 16) wgs = 256 * 16;
     const int nch = (d / 8 + 63) / 64;
@@ -684,6 +615,11 @@ size_t joined_bytes(const HstuOutputArgs* a) {
 }
 
 }  // namespace
+
+// for the library's other translation unit; not exported
+extern "C" __attribute__((visibility("hidden"))) void hstu_linear_set_last_error(const char* text) {
+    snprintf(g_last_error, sizeof(g_last_error), "%s", text);
+}
 
 extern "C" {
 

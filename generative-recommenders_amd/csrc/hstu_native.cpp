@@ -2,6 +2,9 @@
 // result and the scratch memory and calls the C ABI (hstu_hip.h, hstu_linear.h) -- the work that ops/*.py does through
 // ctypes for every argument it has to look at, in a few microseconds instead of ten to thirty.
 //
+// The operators that are differentiable record a backward node of their own here (torch::autograd::Function): nothing but inputs
+// is saved, the gradients come from the library's backward kernels and plain products.
+//
 // Every function serves the usual call only and returns nothing (None) for any other: tensors that need a copy first
 // (rows not dense or not 16-byte aligned), dtypes it does not know, gradients it does not form, arguments the caller got
 // wrong, HSTU_HIP_CHECK_CONTRACT, a status other than 0.  The Python operator then goes through its own checks and raises,
@@ -23,6 +26,10 @@ namespace {
 
 using at::Tensor;
 using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+struct Declined {};  // thrown where a call turns out, on the way, to be the Python operator's
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
@@ -112,15 +119,87 @@ bool attention_operands(const Tensor& q, const Tensor& k, const Tensor& v, const
 
 at::ScalarType result_type(const Tensor& q) { return q.scalar_type() == at::kFloat8_e4m3fn ? at::kBFloat16 : q.scalar_type(); }
 
+Tensor attention_result(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& offsets, const OptTensor& targets, const AttentionCall& call) {
+    Tensor out = at::empty({v.size(0), v.size(1), v.size(2)}, v.options().dtype(result_type(q)));
+    if (attention_forward(q, k, v, out, offsets, targets, call) != HSTU_OK) throw Declined();
+    return out;
+}
+
+// dq, dk, dv (any rows the kernels can write) from dout.  `workspace`: the caller's dS scratch, else scores are recomputed.
+void attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dq, const Tensor& dk, const Tensor& dv,
+                        const Tensor& offsets, const OptTensor& targets, AttentionCall call, const OptTensor& workspace) {
+    HstuFwdArgs a{};
+    call.tile_config = call.kv_splits = 0;
+    call.sort = false;
+    fill_attention(a, q, k, v, offsets, targets, call);
+    Tensor scratch;
+    if (workspace) {
+        TORCH_CHECK(workspace->scalar_type() == at::kByte && workspace->is_contiguous() && workspace->device() == q.device(),
+                    "workspace must be a contiguous uint8 tensor on the inputs' device");
+        a.workspace = workspace->data_ptr(), a.workspace_bytes = workspace->numel(), a.sort_by_length = 1;
+    } else if (a.batch >= 2) {
+        scratch = at::empty({4 * (int64_t)a.batch}, q.options().dtype(at::kByte));
+        a.workspace = scratch.data_ptr(), a.workspace_bytes = 4 * (int64_t)a.batch, a.sort_by_length = 1;
+    }
+    HstuBwdGrads g{};
+    g.dout = dout.const_data_ptr(), g.dq = dq.data_ptr(), g.dk = dk.data_ptr(), g.dv = dv.data_ptr();
+    g.do_row_stride = dout.stride(0), g.do_head_stride = dout.stride(1);
+    g.dq_row_stride = dq.stride(0), g.dq_head_stride = dq.stride(1);
+    g.dk_row_stride = dk.stride(0), g.dk_head_stride = dk.stride(1);
+    g.dv_row_stride = dv.stride(0), g.dv_head_stride = dv.stride(1);
+    const c10::DeviceGuard guard(q.device());
+    const int rc = hstu_hip_mha_bwd(&a, &g, stream_of(q));
+    TORCH_CHECK(rc == HSTU_OK, "hstu_hip: ", hstu_hip_status_string(rc), " (", hstu_hip_last_error(), ") [status ", rc, "]");
+}
+
+Tensor kernel_rows(const Tensor& t) { return kernel_layout(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+
+std::vector<int64_t> pack(const AttentionCall& c) { return {c.max_seq_len, c.w, c.c, c.f}; }
+AttentionCall unpack(const std::vector<int64_t>& i, double alpha) { return {i[0], 0, i[1], i[2], i[3], alpha, 1.0, 1.0, 1.0, 0, 0, false}; }
+
+struct MhaFunction : torch::autograd::Function<MhaFunction> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& offsets, const OptTensor& targets,
+                          const AttentionCall& call, const OptTensor& workspace) {
+        Tensor out = attention_result(q, k, v, offsets, targets, call);
+        ctx->save_for_backward({q, k, v, offsets, targets ? *targets : Tensor()});
+        ctx->saved_data["call"] = pack(call);
+        ctx->saved_data["alpha"] = call.alpha;
+        if (workspace) ctx->saved_data["workspace"] = *workspace;
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        Tensor q = saved[0], k = saved[1], v = saved[2];
+        const OptTensor targets = saved[4].defined() ? OptTensor(saved[4]) : OptTensor();
+        const auto ws = ctx->saved_data.find("workspace");
+        const OptTensor workspace = ws == ctx->saved_data.end() ? OptTensor() : OptTensor(ws->second.toTensor());
+        // fp32 inputs: the backward kernels take 16-bit operands, so they run on bf16 copies (fp32's range: dout can be tiny) and
+        // the gradients are widened again
+        const bool wide = q.scalar_type() == at::kFloat;
+        if (wide) q = q.to(at::kBFloat16), k = k.to(at::kBFloat16), v = v.to(at::kBFloat16);
+        const Tensor dout = kernel_rows(grads[0].to(q.scalar_type()));
+        Tensor dq = at::empty_like(q, at::MemoryFormat::Contiguous), dk = at::empty_like(k, at::MemoryFormat::Contiguous),
+               dv = at::empty_like(v, at::MemoryFormat::Contiguous);
+        attention_backward(dout, q, k, v, dq, dk, dv, saved[3], targets,
+                           unpack(ctx->saved_data["call"].toIntVector(), ctx->saved_data["alpha"].toDouble()), workspace);
+        if (wide) dq = dq.to(at::kFloat), dk = dk.to(at::kFloat), dv = dv.to(at::kFloat);
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
 OptTensor hstu_mha(int64_t max_seq_len, double alpha, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& offsets,
                    const OptTensor& targets, int64_t w, int64_t c, int64_t f, bool sort, double q_scale, double k_scale, double v_scale,
-                   int64_t tile_config, int64_t kv_splits) {
-    if (max_seq_len <= 0 || !attention_operands(q, k, v, offsets, targets) || q.size(0) != k.size(0) || wants_grad({&q, &k, &v})) return {};
-    RECORD_USER_SCOPE("hstu_mha");
-    Tensor out = at::empty({v.size(0), v.size(1), v.size(2)}, v.options().dtype(result_type(q)));
+                   int64_t tile_config, int64_t kv_splits, const OptTensor& bwd_workspace) {
+    if (max_seq_len <= 0 || !attention_operands(q, k, v, offsets, targets) || q.size(0) != k.size(0)) return {};
     const AttentionCall call{max_seq_len, 0, w, c, f, alpha, q_scale, k_scale, v_scale, tile_config, kv_splits, sort};
-    if (attention_forward(q, k, v, out, offsets, targets, call) != HSTU_OK) return {};
-    return out;
+    const bool grad = wants_grad({&q, &k, &v});
+    if (grad && q.scalar_type() == at::kFloat8_e4m3fn) return {};
+    RECORD_USER_SCOPE("hstu_mha");
+    try {
+        return grad ? MhaFunction::apply(q, k, v, offsets, targets, call, bwd_workspace) : attention_result(q, k, v, offsets, targets, call);
+    } catch (const Declined&) {
+        return {};
+    }
 }
 
 OptTensor delta_hstu_mha(int64_t max_seq_len, double alpha, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& offsets,
@@ -226,61 +305,277 @@ Tensor aligned_scratch(size_t bytes, const Tensor& like, void** ptr) {
 std::tuple<Tensor, Tensor, Tensor, Tensor> uqvk_views(const Tensor& buf, int64_t heads, int64_t attn, int64_t hidden) {
     const int64_t rows = buf.size(0), pitch = buf.size(1), nu = hidden * heads, na = attn * heads;
     const at::AutoDispatchBelowADInplaceOrView below;
-    return {buf.as_strided({rows, nu}, {pitch, 1}, 0), buf.as_strided({rows, heads, attn}, {pitch, attn, 1}, 2 * nu),
-            buf.as_strided({rows, heads, attn}, {pitch, attn, 1}, 2 * nu + na), buf.as_strided({rows, heads, hidden}, {pitch, hidden, 1}, nu)};
+    auto view = [&](at::IntArrayRef sizes, at::IntArrayRef strides, int64_t offset) {
+        Tensor t = buf.as_strided(sizes, strides, offset);
+        // a change through one of them is a change of the buffer that a backward node has saved
+        if (!buf.is_inference()) t.unsafeGetTensorImpl()->set_version_counter(buf.unsafeGetTensorImpl()->version_counter());
+        return t;
+    };
+    return {view({rows, nu}, {pitch, 1}, 0), view({rows, heads, attn}, {pitch, attn, 1}, 2 * nu),
+            view({rows, heads, attn}, {pitch, attn, 1}, 2 * nu + na), view({rows, heads, hidden}, {pitch, hidden, 1}, nu)};
 }
 
-std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> compute_uqvk(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias,
-                                                                       double eps, int64_t heads, int64_t attn, int64_t hidden,
-                                                                       const Tensor& weight, const Tensor& bias, int64_t path) {
-    const int64_t n_out = (2 * hidden + 2 * attn) * heads;
-    if (!matrix_rows(x) || dense_dtype(x) < 0 || heads <= 0 || attn <= 0 || hidden <= 0) return {};
-    if (weight.dim() != 2 || weight.size(0) != x.size(1) || weight.size(1) != n_out || bias.dim() != 1 || bias.size(0) != n_out) return {};
-    if (!parameter(norm_weight, x) || !parameter(norm_bias, x) || !parameter(weight, x) || !parameter(bias, x)) return {};
-    if (wants_grad({&x, &norm_weight, &norm_bias, &weight, &bias})) return {};
-    Tensor buf = at::empty({x.size(0), n_out}, x.options());
+struct UqvkShape {
+    int64_t heads, attn, hidden;
+    int64_t n_u() const { return hidden * heads; }
+    int64_t n_out() const { return (2 * hidden + 2 * attn) * heads; }
+};
+
+bool uqvk_operands(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight, const Tensor& bias, const UqvkShape& s) {
+    if (!matrix_rows(x) || dense_dtype(x) < 0 || s.heads <= 0 || s.attn <= 0 || s.hidden <= 0) return false;
+    if (weight.dim() != 2 || weight.size(0) != x.size(1) || weight.size(1) != s.n_out() || bias.dim() != 1 || bias.size(0) != s.n_out()) return false;
+    if (norm_weight.dim() != 1 || norm_weight.size(0) != x.size(1) || norm_bias.dim() != 1 || norm_bias.size(0) != x.size(1)) return false;
+    return parameter(norm_weight, x) && parameter(norm_bias, x) && parameter(weight, x) && parameter(bias, x);
+}
+
+// The buffer u | v | q | k, u through SiLU.
+Tensor uqvk_buffer(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight, const Tensor& bias, double eps,
+                   const UqvkShape& s, int64_t path) {
+    Tensor buf = at::empty({x.size(0), s.n_out()}, x.options());
     HstuUqvkArgs a{};
     a.x = x.const_data_ptr(), a.x_row_stride = x.stride(0);
     a.norm_weight = norm_weight.const_data_ptr(), a.norm_bias = norm_bias.const_data_ptr(), a.norm_eps = (float)eps;
     a.uvqk_weight = weight.const_data_ptr(), a.uvqk_bias = bias.const_data_ptr(), a.uvqk = buf.data_ptr();
-    a.rows = x.size(0), a.d_model = (int32_t)x.size(1), a.heads = (int32_t)heads, a.attn_dim = (int32_t)attn, a.hidden_dim = (int32_t)hidden;
+    a.rows = x.size(0), a.d_model = (int32_t)x.size(1);
+    a.heads = (int32_t)s.heads, a.attn_dim = (int32_t)s.attn, a.hidden_dim = (int32_t)s.hidden;
     a.dtype = dense_dtype(x), a.path = (int32_t)path;
     const size_t need = hstu_uqvk_workspace_bytes(&a);
     Tensor scratch;
     if (need > 0) scratch = aligned_scratch(need, x, &a.workspace), a.workspace_bytes = (int64_t)need;
     const c10::DeviceGuard guard(x.device());
-    if (hstu_uqvk_forward(&a, stream_of(x)) != 0) return {};
-    return uqvk_views(buf, heads, attn, hidden);
+    if (hstu_uqvk_forward(&a, stream_of(x)) != 0) throw Declined();
+    return buf;
 }
 
-// The output step without dropout.
-OptTensor compute_output(const Tensor& attn, const Tensor& u, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, double eps,
-                         const Tensor& weight, int64_t heads, int64_t linear_dim, bool concat_u, bool concat_x, int64_t activation,
-                         bool group_norm, int64_t path) {
-    if (!matrix_rows(attn) || !matrix_rows(u) || !matrix_rows(x) || dense_dtype(x) < 0) return {};
-    if (attn.scalar_type() != x.scalar_type() || u.scalar_type() != x.scalar_type()) return {};
-    const int64_t rows = attn.size(0), width = attn.size(1);
-    if (u.size(0) != rows || u.size(1) != width || x.size(0) != rows || width != heads * linear_dim || heads <= 0 || activation < 0) return {};
-    const int64_t norm = group_norm ? heads : width, blocks = group_norm ? (concat_u && concat_x ? 3 : 1) : 1 + concat_u + concat_x;
-    if (norm_weight.dim() != 1 || norm_weight.size(0) != norm || norm_bias.dim() != 1 || norm_bias.size(0) != norm) return {};
-    if (weight.dim() != 2 || weight.size(0) != blocks * width || weight.size(1) != x.size(1)) return {};
-    if (!parameter(norm_weight, x) || !parameter(norm_bias, x) || !parameter(weight, x)) return {};
-    if (wants_grad({&attn, &u, &x, &norm_weight, &norm_bias, &weight})) return {};
-    Tensor out = at::empty({rows, x.size(1)}, x.options());
-    HstuOutputArgs a{};
+void check_linear(int rc) { TORCH_CHECK(rc == 0, "hstu_linear: status ", rc, " (", hstu_linear_last_error(), ")"); }
+
+// Gradients of x, norm_weight, norm_bias, weight, bias from `d`, the gradient of the producer's buffer u | v | q | k: its v, q and k
+// columns are filled in, the u columns are formed here from `du` (the gradient behind SiLU; undefined: zero).
+variable_list uqvk_backward(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight, const Tensor& bias, double eps,
+                            int64_t n_u, Tensor d, Tensor du) {
+    const int64_t rows = x.size(0), dm = x.size(1);
+    const c10::DeviceGuard guard(x.device());
+    void* stream = stream_of(x);
+    Tensor normed = at::empty({rows, dm}, x.options());
+    check_linear(hstu_uqvk_layer_norm(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
+                                      normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
+    Tensor d_u = d.narrow(1, 0, n_u);
+    if (du.defined()) {
+        if (!matrix_rows(du)) du = du.contiguous();
+        at::mm_out(d_u, normed, weight.narrow(1, 0, n_u));
+        check_linear(hstu_uqvk_silu_bwd(d_u.data_ptr(), d_u.stride(0), bias.const_data_ptr(), du.const_data_ptr(), du.stride(0), rows, n_u,
+                                        dense_dtype(x), stream));
+    } else {
+        d_u.zero_();
+    }
+    Tensor dy = at::mm(d, weight.t()), dx = at::empty({rows, dm}, x.options());
+    Tensor dnw = at::empty_like(norm_weight), dnb = at::empty_like(norm_bias);
+    const int64_t need = (int64_t)hstu_uqvk_layer_norm_bwd_workspace_bytes(rows, (int32_t)dm);
+    Tensor scratch = at::empty({need}, x.options().dtype(at::kByte));
+    check_linear(hstu_uqvk_layer_norm_bwd(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), (float)eps, dy.const_data_ptr(), dm,
+                                          dx.data_ptr(), dm, dnw.data_ptr(), dnb.data_ptr(), rows, (int32_t)dm, dense_dtype(x), scratch.data_ptr(),
+                                          need, stream));
+    return {dx, dnw, dnb, at::mm(normed.t(), d), d.sum(0)};
+}
+
+struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight,
+                                 const Tensor& bias, double eps, const UqvkShape& s, int64_t path) {
+        Tensor buf = uqvk_buffer(x, norm_weight, norm_bias, weight, bias, eps, s, path);
+        ctx->save_for_backward({x, norm_weight, norm_bias, weight, bias});
+        ctx->saved_data["shape"] = std::vector<int64_t>{s.heads, s.attn, s.hidden};
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        auto [u, q, k, v] = uqvk_views(buf, s.heads, s.attn, s.hidden);
+        return {u, q, k, v};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        const auto i = ctx->saved_data["shape"].toIntVector();
+        const UqvkShape s{i[0], i[1], i[2]};
+        Tensor d = at::empty({saved[0].size(0), s.n_out()}, saved[0].options());
+        auto views = uqvk_views(d, s.heads, s.attn, s.hidden);
+        auto put = [](Tensor to, const Tensor& from) { from.defined() ? to.copy_(from) : to.zero_(); };
+        put(std::get<1>(views), grads[1]);
+        put(std::get<2>(views), grads[2]);
+        put(std::get<3>(views), grads[3]);
+        variable_list got = uqvk_backward(saved[0], saved[1], saved[2], saved[3], saved[4], ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
+        got.resize(8);
+        return got;
+    }
+};
+
+// Producer and attention as one node: the attention's gradients are written straight into the producer's gradient buffer.
+struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight,
+                                 const Tensor& bias, const Tensor& offsets, const OptTensor& targets, double eps, const UqvkShape& s,
+                                 const AttentionCall& call) {
+        Tensor buf = uqvk_buffer(x, norm_weight, norm_bias, weight, bias, eps, s, 0);
+        auto [u, q, k, v] = uqvk_views(buf, s.heads, s.attn, s.hidden);
+        if (!attention_operands(q, k, v, offsets, targets)) throw Declined();
+        Tensor out = attention_result(q, k, v, offsets, targets, call).view({x.size(0), s.n_u()});
+        ctx->save_for_backward({x, norm_weight, norm_bias, weight, bias, offsets, targets ? *targets : Tensor(), buf});
+        ctx->saved_data["shape"] = std::vector<int64_t>{s.heads, s.attn, s.hidden};
+        ctx->saved_data["call"] = pack(call);
+        ctx->saved_data["alpha"] = call.alpha;
+        ctx->saved_data["eps"] = eps;
+        ctx->set_materialize_grads(false);
+        return {u, out, k, v};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        const auto i = ctx->saved_data["shape"].toIntVector();
+        const UqvkShape s{i[0], i[1], i[2]};
+        const Tensor& x = saved[0];
+        const OptTensor targets = saved[6].defined() ? OptTensor(saved[6]) : OptTensor();
+        Tensor d = at::empty({x.size(0), s.n_out()}, x.options());
+        const auto grad = uqvk_views(d, s.heads, s.attn, s.hidden), value = uqvk_views(saved[7], s.heads, s.attn, s.hidden);
+        const Tensor &dq = std::get<1>(grad), &dk = std::get<2>(grad), &dv = std::get<3>(grad);
+        if (grads[1].defined()) {
+            const Tensor dout = kernel_rows(grads[1].reshape({x.size(0), s.heads, s.hidden}));
+            attention_backward(dout, std::get<1>(value), std::get<2>(value), std::get<3>(value), dq, dk, dv, saved[5], targets,
+                               unpack(ctx->saved_data["call"].toIntVector(), ctx->saved_data["alpha"].toDouble()), {});
+            if (grads[2].defined()) dk.add_(grads[2]);
+            if (grads[3].defined()) dv.add_(grads[3]);
+        } else {
+            dq.zero_();
+            grads[2].defined() ? dk.copy_(grads[2]) : dk.zero_();
+            grads[3].defined() ? dv.copy_(grads[3]) : dv.zero_();
+        }
+        variable_list got = uqvk_backward(x, saved[1], saved[2], saved[3], saved[4], ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
+        got.resize(10);
+        return got;
+    }
+};
+
+typedef std::tuple<Tensor, Tensor, Tensor, Tensor> FourTensors;
+
+std::optional<FourTensors> compute_uqvk(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, double eps, int64_t heads, int64_t attn,
+                                        int64_t hidden, const Tensor& weight, const Tensor& bias, int64_t path) {
+    const UqvkShape s{heads, attn, hidden};
+    if (!uqvk_operands(x, norm_weight, norm_bias, weight, bias, s)) return {};
+    try {
+        if (wants_grad({&x, &norm_weight, &norm_bias, &weight, &bias})) {
+            const variable_list o = UqvkFunction::apply(x, norm_weight, norm_bias, weight, bias, eps, s, path);
+            return FourTensors(o[0], o[1], o[2], o[3]);
+        }
+        return uqvk_views(uqvk_buffer(x, norm_weight, norm_bias, weight, bias, eps, s, path), heads, attn, hidden);
+    } catch (const Declined&) {
+        return {};
+    }
+}
+
+// Producer and attention with gradients: (u, attention output [L, hidden * H], k, v).  Without gradients the two operators do.
+std::optional<FourTensors> preprocess_and_attention(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, double eps, int64_t heads,
+                                                    int64_t attn, int64_t hidden, const Tensor& weight, const Tensor& bias, int64_t max_seq_len,
+                                                    const Tensor& offsets, double alpha, const OptTensor& targets, int64_t w, int64_t c, bool sort) {
+    const UqvkShape s{heads, attn, hidden};
+    if (max_seq_len <= 0 || !wants_grad({&x, &norm_weight, &norm_bias, &weight, &bias})) return {};
+    if (!uqvk_operands(x, norm_weight, norm_bias, weight, bias, s)) return {};
+    const AttentionCall call{max_seq_len, 0, w, c, 0, alpha, 1.0, 1.0, 1.0, 0, 0, sort};
+    RECORD_USER_SCOPE("hstu_preprocess_and_attention");
+    try {
+        const variable_list o = PreprocessFunction::apply(x, norm_weight, norm_bias, weight, bias, offsets, targets, eps, s, call);
+        return FourTensors(o[0], o[1], o[2], o[3]);
+    } catch (const Declined&) {
+        return {};
+    }
+}
+
+struct OutputCall {
+    int64_t heads, linear_dim, activation, path;
+    bool concat_u, concat_x, group_norm;
+    double eps, dropout;
+    uint64_t seed, offset;
+    int64_t blocks() const { return group_norm ? (concat_u && concat_x ? 3 : 1) : 1 + concat_u + concat_x; }
+};
+
+void fill_output(HstuOutputArgs& a, const Tensor& attn, const Tensor& u, const Tensor& norm_weight, const Tensor& norm_bias, const OutputCall& c) {
     a.attn = attn.const_data_ptr(), a.attn_row_stride = attn.stride(0), a.u = u.const_data_ptr(), a.u_row_stride = u.stride(0);
-    a.x = x.const_data_ptr(), a.x_row_stride = x.stride(0);
-    a.norm_weight = norm_weight.const_data_ptr(), a.norm_bias = norm_bias.const_data_ptr(), a.norm_eps = (float)eps;
-    a.output_weight = weight.const_data_ptr(), a.out = out.data_ptr();
-    a.rows = rows, a.d_out = (int32_t)x.size(1), a.heads = (int32_t)heads, a.linear_dim = (int32_t)linear_dim;
-    a.concat_u = concat_u, a.concat_x = concat_x, a.group_norm = group_norm, a.mul_u_activation = (int32_t)activation;
-    a.dtype = dense_dtype(x), a.path = (int32_t)path;
+    a.norm_weight = norm_weight.const_data_ptr(), a.norm_bias = norm_bias.const_data_ptr(), a.norm_eps = (float)c.eps;
+    a.rows = attn.size(0), a.heads = (int32_t)c.heads, a.linear_dim = (int32_t)c.linear_dim;
+    a.concat_u = c.concat_u, a.concat_x = c.concat_x, a.group_norm = c.group_norm, a.mul_u_activation = (int32_t)c.activation;
+    a.dtype = dense_dtype(attn), a.path = (int32_t)c.path;
+    a.dropout_ratio = (float)c.dropout, a.dropout_seed = c.seed, a.dropout_offset = c.offset;
+}
+
+Tensor output_result(const Tensor& attn, const Tensor& u, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight,
+                     const OutputCall& c) {
+    Tensor out = at::empty({x.size(0), x.size(1)}, x.options());
+    HstuOutputArgs a{};
+    fill_output(a, attn, u, norm_weight, norm_bias, c);
+    a.x = x.const_data_ptr(), a.x_row_stride = x.stride(0), a.output_weight = weight.const_data_ptr(), a.out = out.data_ptr();
+    a.d_out = (int32_t)x.size(1);
     const size_t need = hstu_output_workspace_bytes(&a);
     Tensor scratch;
     if (need > 0) scratch = aligned_scratch(need, x, &a.workspace), a.workspace_bytes = (int64_t)need;
     const c10::DeviceGuard guard(x.device());
-    if (hstu_output_forward(&a, stream_of(x)) != 0) return {};
+    if (hstu_output_forward(&a, stream_of(x)) != 0) throw Declined();
     return out;
+}
+
+struct OutputFunction : torch::autograd::Function<OutputFunction> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& attn, const Tensor& u, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias,
+                          const Tensor& weight, const OutputCall& c) {
+        Tensor out = output_result(attn, u, x, norm_weight, norm_bias, weight, c);
+        ctx->save_for_backward({attn, u, norm_weight, norm_bias, weight});
+        ctx->saved_data["sizes"] = std::vector<int64_t>{c.heads, c.linear_dim, c.activation, c.concat_u, c.concat_x, c.group_norm, (int64_t)c.seed,
+                                                        (int64_t)c.offset};
+        ctx->saved_data["floats"] = std::vector<double>{c.eps, c.dropout};
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &attn = saved[0], &u = saved[1], &norm_weight = saved[2], &norm_bias = saved[3], &weight = saved[4];
+        const auto i = ctx->saved_data["sizes"].toIntVector();
+        const auto f = ctx->saved_data["floats"].toDoubleVector();
+        const OutputCall c{i[0], i[1], i[2], 0, i[3] != 0, i[4] != 0, i[5] != 0, f[0], f[1], (uint64_t)i[6], (uint64_t)i[7]};
+        const Tensor dout = grads[0].contiguous();
+        const int64_t rows = attn.size(0), width = attn.size(1);
+        variable_list got(7);
+        got[2] = dout;  // the residual
+        const bool weight_too = ctx->needs_input_grad(5);
+        if (weight_too || ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4)) {
+            const Tensor dj = at::mm(dout, weight.t());
+            Tensor joined = weight_too ? at::empty_like(dj) : Tensor();
+            got[0] = at::empty({rows, width}, attn.options()), got[1] = at::empty({rows, width}, attn.options());
+            got[3] = at::empty_like(norm_weight), got[4] = at::empty_like(norm_bias);
+            HstuOutputArgs a{};
+            fill_output(a, attn, u, norm_weight, norm_bias, c);
+            HstuNormMulGrads g{};
+            g.d_joined = dj.const_data_ptr(), g.d_joined_row_stride = dj.size(1);
+            if (weight_too) g.joined = joined.data_ptr(), g.joined_row_stride = joined.size(1);
+            g.d_attn = got[0].data_ptr(), g.d_u = got[1].data_ptr(), g.d_attn_row_stride = g.d_u_row_stride = width;
+            g.d_norm_weight = got[3].data_ptr(), g.d_norm_bias = got[4].data_ptr();
+            g.workspace_bytes = (int64_t)hstu_output_norm_mul_bwd_workspace_bytes(&a);
+            Tensor scratch = at::empty({g.workspace_bytes}, attn.options().dtype(at::kByte));
+            g.workspace = scratch.data_ptr();
+            const c10::DeviceGuard guard(attn.device());
+            check_linear(hstu_output_norm_mul_bwd(&a, &g, stream_of(attn)));
+            if (weight_too) got[5] = at::mm(joined.t(), dout);
+        }
+        return got;
+    }
+};
+
+OptTensor compute_output(const Tensor& attn, const Tensor& u, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, double eps,
+                         const Tensor& weight, int64_t heads, int64_t linear_dim, bool concat_u, bool concat_x, int64_t activation,
+                         bool group_norm, int64_t path, double dropout, uint64_t seed, uint64_t offset) {
+    const OutputCall c{heads, linear_dim, activation, path, concat_u, concat_x, group_norm, eps, dropout, seed, offset};
+    if (!matrix_rows(attn) || !matrix_rows(u) || !matrix_rows(x) || dense_dtype(x) < 0) return {};
+    if (attn.scalar_type() != x.scalar_type() || u.scalar_type() != x.scalar_type()) return {};
+    const int64_t rows = attn.size(0), width = attn.size(1), norm = group_norm ? heads : width;
+    if (u.size(0) != rows || u.size(1) != width || x.size(0) != rows || width != heads * linear_dim || heads <= 0 || activation < 0) return {};
+    if (norm_weight.dim() != 1 || norm_weight.size(0) != norm || norm_bias.dim() != 1 || norm_bias.size(0) != norm) return {};
+    if (weight.dim() != 2 || weight.size(0) != c.blocks() * width || weight.size(1) != x.size(1)) return {};
+    if (!parameter(norm_weight, x) || !parameter(norm_bias, x) || !parameter(weight, x)) return {};
+    try {
+        return wants_grad({&attn, &u, &x, &norm_weight, &norm_bias, &weight})
+                   ? OutputFunction::apply(attn, u, x, norm_weight, norm_bias, weight, c)
+                   : output_result(attn, u, x, norm_weight, norm_bias, weight, c);
+    } catch (const Declined&) {
+        return {};
+    }
 }
 
 }  // namespace
@@ -294,5 +589,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("split_2d_jagged", &split_2d_jagged, nogil);
     m.def("write_kv_tail", &write_kv_tail, nogil);
     m.def("compute_uqvk", &compute_uqvk, nogil);
+    m.def("preprocess_and_attention", &preprocess_and_attention, nogil);
     m.def("compute_output", &compute_output, nogil);
 }

@@ -166,7 +166,7 @@ def hstu_mha(
     if causal and dropout_pr < 1e-6 and attn_scale is None:
         out = native.front.hstu_mha(
             max_seq_len, alpha, q, k, v, seq_offsets, num_targets, max_attn_len, contextual_seq_len, min_full_attn_seq_len, sort_by_length,
-            q_scale, k_scale, v_scale, tile_config, kv_splits,
+            q_scale, k_scale, v_scale, tile_config, kv_splits, bwd_workspace,
         )
         if out is not None:
             return out

@@ -10,8 +10,10 @@ epilogue.  ``u, q, k, v`` come back as column slices of one ``[L, (2*hidden + 2*
 normalises, multiplies and writes the concatenated operand; the product, with the residual as the GEMM's C operand,
 runs on hipBLASLt.  (``csrc/hstu_linear.hip``, ``include/hstu_linear.h``.)
 
-Device tensors only, bf16 or fp16; ``kernel`` is accepted and ignored.  The forward runs on the kernels above; the
-gradients come from a recomputation with the framework's operators (see ``_grads_by_recomputation``).
+Device tensors only, bf16 or fp16; ``kernel`` is accepted and ignored.  The usual call, with or without gradients, goes through
+the native front (``csrc/hstu_native.cpp``): backward kernels for the row-wise parts (``csrc/hstu_linear_bwd.hip``), plain
+products around them.  What it leaves -- operands that need a copy first -- is handled here; its gradients come from a
+recomputation with the framework's operators (see ``_grads_by_recomputation``).
 """
 
 import ctypes
@@ -91,9 +93,12 @@ class HstuOutputArgs(ctypes.Structure):
 
 EXPORTS = (
     "hstu_uqvk_workspace_bytes", "hstu_uqvk_forward", "hstu_uqvk_layer_norm", "hstu_output_workspace_bytes", "hstu_output_forward",
-    "hstu_output_norm_mul", "hstu_output_dropout_mask", "hstu_linear_last_error", "hstu_linear_version",
+    "hstu_output_norm_mul", "hstu_output_dropout_mask", "hstu_output_norm_mul_bwd_workspace_bytes", "hstu_output_norm_mul_bwd",
+    "hstu_uqvk_layer_norm_bwd_workspace_bytes", "hstu_uqvk_layer_norm_bwd", "hstu_uqvk_silu_bwd", "hstu_linear_last_error",
+    "hstu_linear_version",
 )
 MUL_U_ACTIVATIONS = {"none": 0, "sigmoid": 1, "silu": 2}
+_WORD64 = (1 << 64) - 1  # a Philox seed or offset as the library takes it
 
 _lib: Optional[ctypes.CDLL] = None
 
@@ -164,9 +169,9 @@ def _needs_grad(*tensors: torch.Tensor) -> bool:
     return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
 
 
-# ---- gradients of the dense steps -----------------------------------------------------------------------------------
-# The forward of every function below runs on this package's kernels.  Their gradients are NOT hand-written: the
-# backward recomputes the step with the framework's own operators (layer / group norm, addmm on hipBLASLt) in the
+# ---- gradients of the calls that the native front leaves ----------------------------------------------------------------
+# (parameters or rows that are not dense and 16-byte aligned, and ``layer_norm`` / ``norm_mul_dropout`` on their own.)  The
+# forward runs on this package's kernels; the gradients here are not hand-written: the backward recomputes the step with the framework's own operators (layer / group norm, addmm on hipBLASLt) in the
 # arithmetic of the reference's PyTorch backend (fp32 norm and product with u, result rounded to the input type, then the
 # product with the weight: ops/pytorch/pt_layer_norm.py:24-39, pt_hstu_linear.py:24-124, ops/hstu_compute.py:54-104) and
 # lets autograd differentiate that -- nothing but the inputs is saved, which is what the reference's recompute_* flags
@@ -544,17 +549,19 @@ def hstu_compute_output(
     reads ``u`` and ``attn`` where they are (``NotImplementedError`` if the shape does not fit: d_model a multiple of 256,
     heads * linear_dim a multiple of 64 -- or with dropout, whose mask covers the copied blocks too); 0 = whichever is
     faster for the shape (2 where it fits, rows >= 32768 and nothing is dropped).  Dropout as in ``norm_mul_dropout``."""
-    if not training or dropout_ratio <= 0.0:
-        out = native.front.compute_output(
-            attn, u, x, norm_weight, norm_bias, norm_eps, output_weight, num_heads, linear_dim, concat_u, concat_x,
-            MUL_U_ACTIVATIONS.get(mul_u_activation_type, -1), group_norm, path,
-        )
-        if out is not None:
-            return out
+    state = None
+    if training and dropout_ratio > 0.0:
+        state = _dropout_state(dropout_ratio, training, attn.shape[0] * attn.shape[1] * _blocks(concat_u, concat_x, group_norm), attn.device, seed)
+    ratio, word_seed, word_offset = state or (0.0, 0, 0)
+    out = native.front.compute_output(
+        attn, u, x, norm_weight, norm_bias, norm_eps, output_weight, num_heads, linear_dim, concat_u, concat_x,
+        MUL_U_ACTIVATIONS.get(mul_u_activation_type, -1), group_norm, path, ratio, word_seed & _WORD64, word_offset & _WORD64,
+    )
+    if out is not None:
+        return out
     torch._assert(x.dim() == 2 and x.shape[0] == attn.shape[0], "x must be 2-D with attn's row count")
     _check(x, attn, u, norm_weight, norm_bias, output_weight)
     torch._assert(mul_u_activation_type in MUL_U_ACTIVATIONS, "mul_u_activation_type must be none, sigmoid or silu")
-    state = _dropout_state(dropout_ratio, training, attn.shape[0] * attn.shape[1] * _blocks(concat_u, concat_x, group_norm), attn.device, seed)
     if _needs_grad(x, attn, u, norm_weight, norm_bias, output_weight):
         return _OutputFunction.apply(attn, u, x, norm_weight, norm_bias, output_weight, norm_eps, num_heads, linear_dim, concat_u,
                                      concat_x, mul_u_activation_type, group_norm, path, state)
@@ -622,6 +629,12 @@ def hstu_preprocess_and_attention(
         "uvqk_weight.shape[1] must equal 2 * num_heads * (hidden_dim + attn_dim)",
     )
     torch._assert(causal is True, "only causal attention is supported.")
+    parts = native.front.preprocess_and_attention(
+        x, norm_weight, norm_bias, norm_eps, num_heads, attn_dim, hidden_dim, uvqk_weight, uvqk_bias, max_seq_len, seq_offsets, attn_alpha,
+        num_targets, max_attn_len, contextual_seq_len, sort_by_length,
+    )
+    if parts is not None:
+        return parts
     u, q, k, v = hstu_compute_uqvk(x, norm_weight, norm_bias, norm_eps, num_heads, attn_dim, hidden_dim, uvqk_weight, uvqk_bias, kernel)
     attn_output = hstu_mha(
         max_seq_len=max_seq_len, alpha=attn_alpha, q=q, k=k, v=v, seq_offsets=seq_offsets, causal=causal, dropout_pr=0.0,

@@ -147,6 +147,44 @@ int hstu_output_norm_mul(const HstuOutputArgs* args, void* joined, int64_t joine
  * `keep`: rows * width bytes of device memory, 4-byte aligned. */
 int hstu_output_dropout_mask(float ratio, uint64_t seed, uint64_t offset, int64_t rows, int64_t width, void* keep, void* stream);
 
+/*
+ * ---- Backward of the row-wise parts ----
+ * (the products are plain GEMMs and the caller's: d_joined = d_out @ W^T, d_W = joined^T @ d_out, and the like for the producer).
+ * Statistics and the dropout mask are recomputed from the forward's inputs; nothing is saved.  The gradients of a norm's weight
+ * and bias are summed over the rows in fp32 in a fixed order through `workspace` (16-byte aligned) and rounded once.
+ */
+
+/* Gradients of hstu_output_norm_mul for the call described by its HstuOutputArgs (dropout fields included), from the gradient of
+ * `joined`.  Row strides in elements, rows 16-byte aligned.  rows must be > 0 (-5). */
+typedef struct HstuNormMulGrads {
+    const void* d_joined;      /* [rows, blocks * heads * linear_dim] */
+    int64_t d_joined_row_stride;
+    void* joined;              /* NULL, or where `joined` itself goes (recomputed): the operand of the weight's gradient */
+    int64_t joined_row_stride;
+    void* d_attn;              /* [rows, heads * linear_dim] */
+    int64_t d_attn_row_stride;
+    void* d_u;                 /* [rows, heads * linear_dim] */
+    int64_t d_u_row_stride;
+    void* d_norm_weight;       /* as norm_weight */
+    void* d_norm_bias;
+    void* workspace;           /* hstu_output_norm_mul_bwd_workspace_bytes() bytes */
+    int64_t workspace_bytes;
+} HstuNormMulGrads;
+
+size_t hstu_output_norm_mul_bwd_workspace_bytes(const HstuOutputArgs* args);
+int hstu_output_norm_mul_bwd(const HstuOutputArgs* args, const HstuNormMulGrads* grads, void* stream);
+
+/* dx, d_weight, d_bias of hstu_uqvk_layer_norm from dy.  rows must be > 0 (-5). */
+size_t hstu_uqvk_layer_norm_bwd_workspace_bytes(int64_t rows, int32_t d_model);
+int hstu_uqvk_layer_norm_bwd(const void* x, int64_t x_row_stride, const void* weight, float eps, const void* dy, int64_t dy_row_stride, void* dx,
+                             int64_t dx_row_stride, void* d_weight, void* d_bias, int64_t rows, int32_t d_model, int32_t dtype, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+
+/* In place: pre[r, c] = du[r, c] * (derivative of SiLU at pre[r, c] + bias[c]) for c < width (a multiple of 8): from the product
+ * LN(x) @ W of the u columns to their gradient in front of SiLU. */
+int hstu_uqvk_silu_bwd(void* pre, int64_t pre_row_stride, const void* bias, const void* du, int64_t du_row_stride, int64_t rows, int64_t width,
+                       int32_t dtype, void* stream);
+
 const char* hstu_linear_last_error(void);
 
 /* Library version, major*10000 + minor*100 + patch.  101: HstuUqvkArgs gained qkv_fp8 / v_scale / q_scale / k_scale /

@@ -1,5 +1,5 @@
 """The operators' native front: it serves the usual call with the same bits as the Python path, and leaves (returns None
-for) every call that path has to copy for, refuse or differentiate."""
+for) every call that path has to copy for or refuse; gradients of the dense steps against the recomputation in Python."""
 
 import pytest
 import torch
@@ -31,7 +31,7 @@ def test_attention_through_the_front_and_through_python(pkg, dev, front, dtype, 
         wide = front.delta_hstu_mha(150, 0.1, q.transpose(1, 2).contiguous().transpose(1, 2), *args[3:])
         wrong = front.delta_hstu_mha(150, 0.1, q[:-1], *args[3:])
     else:
-        args = (150, 0.1, q, k, v, offs, t, 20, 3, 0, True, 0.5, 2.0, 1.5, 0, 0)
+        args = (150, 0.1, q, k, v, offs, t, 20, 3, 0, True, 0.5, 2.0, 1.5, 0, 0, None)
         got = front.hstu_mha(*args)
         want = A._hstu_mha(150, 0.1, q, k, v, offs, True, 0.0, t, None, 20, 3, 0, True, 0.5, 2.0, 1.5, 0, 0, None)
         wide = front.hstu_mha(150, 0.1, q.transpose(1, 2).contiguous().transpose(1, 2), *args[3:])
@@ -47,12 +47,79 @@ def test_dense_steps_and_row_copies_leave_what_they_cannot_serve(pkg, dev, front
     print("[case] native front, calls it leaves", flush=True)
     assert front.compute_uqvk(*args) is not None
     assert front.compute_uqvk(x.float(), *args[1:]) is None and front.compute_uqvk(x[:, 1:], *args[1:]) is None
-    assert front.compute_uqvk(x.clone().requires_grad_(), *args[1:]) is None  # gradients: the Python operator
+    assert all(t.requires_grad for t in front.compute_uqvk(x.clone().requires_grad_(), *args[1:]))
     attn, wo, ow = x[:, :64], torch.randn(192, 128, device=dev).bfloat16(), nw[:64]
-    out = (attn, attn, x, ow, ow, 1e-6, wo, 1, 64, True, True, 0, False, 0)
-    assert front.compute_output(*out) is not None and front.compute_output(*out[:11], -1, False, 0) is None
+    out = (attn, attn, x, ow, ow, 1e-6, wo, 1, 64, True, True, 0, False, 0, 0.0, 0, 0)
+    assert front.compute_output(*out) is not None and front.compute_output(*out[:11], -1, *out[12:]) is None
     offs = torch.tensor([0, 12, 20], device=dev)
     assert front.concat_2d_jagged(x, x, 12, 12, offs, offs) is not None and front.concat_2d_jagged(x, x, None, 12, offs, offs) is None
     assert front.split_2d_jagged(torch.cat([x, x]), 20, 20, 12, 12, offs, offs) is not None and front.split_2d_jagged(x, 12, 9, 12, 8, offs, offs) is None
     assert front.write_kv_tail(x, offs, x[:4].clone()) and not front.write_kv_tail(x, offs, x[:3].clone())
     torch.cuda.synchronize()
+
+
+def _grads(fn, tensors, d_out):
+    leaves = [t.detach().clone().requires_grad_() for t in tensors]
+    return torch.autograd.grad(fn(*leaves), leaves, d_out)
+
+
+def _close(got, want, what):
+    """Both are sums of the same terms with the same roundings of the operands, accumulated in fp32 in another order and rounded
+    once: a matrix of results in bf16 differs by its last bit here and there (2^-9 relative, half of it on average), a vector
+    that is summed over the rows by the cancellation on top, so four times that."""
+    assert got.shape == want.shape and torch.isfinite(got).all(), what
+    rel = float((got.float() - want.float()).norm() / want.float().norm())
+    assert rel <= (4e-3 if got.dim() > 1 else 1.6e-2), f"{what}: {rel:.2e}"
+
+
+@pytest.mark.parametrize("rows,heads,dim,cu,cx,act,group,silu_u,drop", [
+    (1, 1, 8, True, True, "none", False, False, 0.0), (5, 2, 64, True, True, "silu", False, False, 0.3), (300, 3, 168, False, True, "sigmoid", False, False, 0.0),
+    (4100, 4, 128, True, False, "none", False, False, 0.2), (77, 8, 128, True, True, "none", True, False, 0.1), (9, 8, 512, True, True, "none", False, False, 0.0),
+    (513, 2, 8, False, False, "none", True, False, 0.0), (260, 1, 512, True, True, "none", True, False, 0.5),
+])
+def test_output_step_gradients_against_the_recomputation(dev, rows, heads, dim, cu, cx, act, group, silu_u, drop):
+    """The norm-multiply backward kernel and the products around it, at widths of one lane to the widest row, one row to more
+    rows than waves, against the package's own restatement with torch operators (same operands, same mask)."""
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    print(f"[case] output gradients {rows} {heads} {dim} {cu} {cx} {act} group={group} drop={drop}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows)
+    width, d = heads * dim, 64
+    blocks = hc._blocks(cu, cx, group)
+    norm = heads if group else width
+    shapes = ((rows, width), (rows, width), (rows, d), (norm,), (norm,), (blocks * width, d))
+    ins = [torch.randn(s, generator=g, device=dev).bfloat16() for s in shapes]
+    d_out = torch.randn((rows, d), generator=g, device=dev).bfloat16()
+    state = hc._dropout_state(drop, True, 0, dev, (3, 8))
+    mask = hc._keep_scaled(state, rows, blocks * width, dev)
+    got = _grads(lambda a, u, x, nw, nb, w: hc.hstu_compute_output(a, u, x, nw, nb, 1e-6, w, heads, dim, drop, True, cu, cx, act, group, True, seed=(3, 8)),
+                 ins, d_out)
+    want = _grads(lambda a, u, x, nw, nb, w: torch.addmm(x, hc._norm_mul_math(a, u, nw, nb, 1e-6, False, cu, cx, act, group, heads, dim, keep_scaled=mask), w),
+                  ins, d_out)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("attn", "u", "x", "norm_weight", "norm_bias", "weight"), got, want):
+        _close(a, b, f"d/d{name}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,d,heads,attn,hidden", [(1, 64, 1, 16, 16), (4101, 128, 2, 32, 64), (63, 1024, 1, 64, 64), (20, 4096, 1, 8, 8), (300, 520, 3, 16, 8)])
+def test_producer_gradients_against_the_recomputation(dev, dtype, rows, d, heads, attn, hidden):
+    """Layer-norm and SiLU backward kernels, at widths up to the widest row and with rows past the waves of the grid."""
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    print(f"[case] producer gradients {rows} {d} {heads} {attn} {hidden} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows)
+    n = (2 * attn + 2 * hidden) * heads
+    ins = [torch.randn(s, generator=g, device=dev).to(dtype) for s in ((rows, d), (d,), (d,), (d, n), (n,))]
+    ins[3] = (ins[3] / d**0.5).contiguous()
+    d_out = torch.randn((rows, n), generator=g, device=dev).to(dtype)
+
+    def through_kernels(x, nw, nb, w, b):
+        u, q, k, v = hc.hstu_compute_uqvk(x, nw, nb, 1e-6, heads, attn, hidden, w, b)
+        return torch.cat([u, v.flatten(1), q.flatten(1), k.flatten(1)], dim=1)
+
+    got = _grads(through_kernels, ins, d_out)
+    want = _grads(lambda x, nw, nb, w, b: hc._uqvk_math(x, nw, nb, 1e-6, hidden * heads, w, b), ins, d_out)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("x", "norm_weight", "norm_bias", "weight", "bias"), got, want):
+        _close(a, b, f"d/d{name}")
