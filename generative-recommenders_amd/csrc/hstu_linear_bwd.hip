@@ -1,12 +1,14 @@
-// Backward of the row-wise parts of the dense steps (libhstu_linear.so): the norm-multiply step of the output projection, the
-// layer norm of the producer and the SiLU on its u columns.  The products around them are plain GEMMs and the caller's.
+// Backward of the dense steps (libhstu_linear.so): the norm-multiply step of the output projection, the layer norm of the producer,
+// the SiLU on its u columns, and the gradients of the weights (hstu_wgrad_kernel.h).  The other products are plain GEMMs and the
+// caller's.
 //
-// All of it is bound by HBM, so every kernel reads each row once and writes each result once: one wave per row with 16-byte
+// The row-wise kernels are bound by HBM, so every kernel reads each row once and writes each result once: one wave per row with 16-byte
 // accesses as in the forward kernels, statistics recomputed from the row in registers (nothing is saved by the forward), the
 // dropout mask regenerated from its Philox stream.  The gradients of the norm's weight and bias are sums over all rows: a wave
 // keeps its share in fp32 registers, a workgroup adds its four waves in LDS and writes one partial row, and a second small
 // kernel adds the partial rows in order -- no atomics, the same bits from run to run.
 #include "hstu_rows.h"
+#include "hstu_wgrad_kernel.h"
 
 #include <cstdio>
 
@@ -373,6 +375,50 @@ __global__ __launch_bounds__(256) void hstu_silu_bwd_kernel(char* v, int64_t v_r
     }
 }
 
+// How the rows of a weight gradient are split: as many workgroups as the chip has CUs (one fits a CU) where the rows allow at
+// least two tiles of 32 rows each; more only repeats fp32 sums (256 KB each, written and read once).  The byte offsets inside a
+// split stay below 2^31.
+struct WgradPlan {
+    int tiles_m, tiles_n, splits, rows_per_split;
+    size_t partial_bytes, colsum_bytes;
+};
+WgradPlan wgrad_plan(int m, int n, int64_t rows, int64_t stride) {
+    WgradPlan pl;
+    pl.tiles_m = (m + kWgTile - 1) / kWgTile, pl.tiles_n = (n + kWgTile - 1) / kWgTile;
+    const int64_t tiles = (int64_t)pl.tiles_m * pl.tiles_n;
+    int64_t want = 256 / tiles;
+    if (want > rows / (2 * kWgDepth)) want = rows / (2 * kWgDepth);
+    const int64_t most_rows = ((int64_t)1 << 30) / (stride * 2);  // of a split
+    if (want < (rows + most_rows - 1) / most_rows) want = (rows + most_rows - 1) / most_rows;
+    if (want < 1) want = 1;
+    pl.rows_per_split = (int)(((rows + want - 1) / want + kWgDepth - 1) / kWgDepth * kWgDepth);
+    pl.splits = (int)((rows + pl.rows_per_split - 1) / pl.rows_per_split);
+    pl.partial_bytes = (size_t)pl.splits * tiles * kWgTileFloats * sizeof(float);
+    pl.colsum_bytes = (size_t)pl.splits * n * sizeof(float);
+    return pl;
+}
+
+template <class TT>
+int launch_wgrad(const WgradParams& p, typename TT::elem* out, typename TT::elem* colsum, hipStream_t stream) {
+    auto kern = hstu_wgrad_kernel<TT>;
+    static bool attr_done[64];  // (a function attribute belongs to the device it was set on)
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
+    if (dev < 0 || !attr_done[dev]) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds) != hipSuccess)
+            return launch_status("weight gradient kernel attribute");
+        if (dev >= 0) attr_done[dev] = true;
+    }
+    const int tiles = p.tiles_m * p.tiles_n;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((tiles * p.splits + 7) / 8 * 8)), dim3(kWgWaves * 64), kWgLds, stream, p);
+    int rc = launch_status("weight gradient kernel launch");
+    if (rc != 0) return rc;
+    const int tile_blocks = tiles * (kWgTileFloats / 4 / 256), sum_blocks = colsum ? (p.n + 255) / 256 : 0;
+    hipLaunchKernelGGL((hstu_wgrad_reduce_kernel<typename TT::elem>), dim3((unsigned)(tile_blocks + sum_blocks)), dim3(256), 0, stream, p, out, colsum,
+                       tile_blocks);
+    return launch_status("weight gradient reduce kernel launch");
+}
+
 template <class E>
 void sum_partials(const float* partial, long long n, int cols, int half, void* out0, void* out1, hipStream_t stream) {
     hipLaunchKernelGGL((hstu_sum_partials_kernel<E>), dim3((unsigned)((cols + 63) / 64)), dim3(1024), 0, stream, partial, (int)n, cols, half, (E*)out0,
@@ -483,6 +529,33 @@ int hstu_uqvk_silu_bwd(void* pre, int64_t pre_row_stride, const void* bias, cons
         hipLaunchKernelGGL((hstu_silu_bwd_kernel<f16x8_t>), dim3((unsigned)wgs), dim3(256), 0, stream, (char*)pre, pre_row_stride, (const char*)bias,
                            (const char*)du, du_row_stride, rows, (int)(width / 8));
     return launch_status("SiLU backward kernel launch");
+}
+
+size_t hstu_linear_weight_grad_workspace_bytes(int32_t m, int32_t n, int64_t rows, int64_t a_row_stride, int64_t b_row_stride) {
+    if (m <= 0 || n <= 0 || rows <= 0 || a_row_stride < m || b_row_stride < n) return 0;
+    const WgradPlan pl = wgrad_plan(m, n, rows, a_row_stride > b_row_stride ? a_row_stride : b_row_stride);
+    return pl.partial_bytes + pl.colsum_bytes;
+}
+
+int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, const void* b, int64_t b_row_stride, int32_t n, int64_t rows,
+                            int32_t dtype, void* out, void* b_sums, void* workspace, int64_t workspace_bytes, void* stream_) {
+    if (m <= 0 || n <= 0 || (m & 7) != 0 || (n & 7) != 0 || m > 65536 || n > 65536 || rows <= 0 || rows > 0x7fffffffLL) return -5;
+    if (a_row_stride < m || b_row_stride < n || a_row_stride > (1 << 22) || b_row_stride > (1 << 22)) return -5;
+    if (dtype != 0 && dtype != 1) return -2;
+    if (!a || !b || !out || !workspace) return -1;
+    if (misaligned({a, b, out, workspace}, {a_row_stride, b_row_stride})) return -4;
+    if (workspace_bytes < (int64_t)hstu_linear_weight_grad_workspace_bytes(m, n, rows, a_row_stride, b_row_stride)) return -5;
+    const WgradPlan pl = wgrad_plan(m, n, rows, a_row_stride > b_row_stride ? a_row_stride : b_row_stride);
+    WgradParams p;
+    p.a = (const char*)a, p.b = (const char*)b;
+    p.a_rsb = (unsigned)(a_row_stride * 2), p.b_rsb = (unsigned)(b_row_stride * 2);
+    p.m = m, p.n = n, p.rows = rows, p.rows_per_split = pl.rows_per_split;
+    p.tiles_m = pl.tiles_m, p.tiles_n = pl.tiles_n, p.splits = pl.splits;
+    p.partial = (float*)workspace;
+    p.colsum = b_sums ? (float*)((char*)workspace + pl.partial_bytes) : nullptr;
+    hipStream_t stream = (hipStream_t)stream_;
+    if (dtype == 0) return launch_wgrad<Bf16>(p, (__bf16*)out, (__bf16*)b_sums, stream);
+    return launch_wgrad<Fp16>(p, (_Float16*)out, (_Float16*)b_sums, stream);
 }
 
 }  // extern "C"

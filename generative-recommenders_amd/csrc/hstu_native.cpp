@@ -349,6 +349,17 @@ Tensor uqvk_buffer(const Tensor& x, const Tensor& norm_weight, const Tensor& nor
 
 void check_linear(int rc) { TORCH_CHECK(rc == 0, "hstu_linear: status ", rc, " (", hstu_linear_last_error(), ")"); }
 
+// a^T @ b, and the column sums of b where `b_sums` is defined.
+Tensor weight_grad(const Tensor& a, const Tensor& b, const Tensor& b_sums) {
+    Tensor out = at::empty({a.size(1), b.size(1)}, a.options());
+    const int32_t m = (int32_t)a.size(1), n = (int32_t)b.size(1);
+    const int64_t need = (int64_t)hstu_linear_weight_grad_workspace_bytes(m, n, a.size(0), a.stride(0), b.stride(0));
+    Tensor scratch = at::empty({need}, a.options().dtype(at::kByte));
+    check_linear(hstu_linear_weight_grad(a.const_data_ptr(), a.stride(0), m, b.const_data_ptr(), b.stride(0), n, a.size(0), dense_dtype(a),
+                                         out.data_ptr(), b_sums.defined() ? b_sums.data_ptr() : nullptr, scratch.data_ptr(), need, stream_of(a)));
+    return out;
+}
+
 // Gradients of x, norm_weight, norm_bias, weight, bias from `d`, the gradient of the producer's buffer u | v | q | k: its v, q and k
 // columns are filled in, the u columns are formed here from `du` (the gradient behind SiLU; undefined: zero).
 variable_list uqvk_backward(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight, const Tensor& bias, double eps,
@@ -375,7 +386,9 @@ variable_list uqvk_backward(const Tensor& x, const Tensor& norm_weight, const Te
     check_linear(hstu_uqvk_layer_norm_bwd(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), (float)eps, dy.const_data_ptr(), dm,
                                           dx.data_ptr(), dm, dnw.data_ptr(), dnb.data_ptr(), rows, (int32_t)dm, dense_dtype(x), scratch.data_ptr(),
                                           need, stream));
-    return {dx, dnw, dnb, at::mm(normed.t(), d), d.sum(0)};
+    Tensor d_bias = at::empty_like(bias);
+    Tensor d_weight = weight_grad(normed, d, d_bias);
+    return {dx, dnw, dnb, d_weight, d_bias};
 }
 
 struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
@@ -552,7 +565,7 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
             g.workspace = scratch.data_ptr();
             const c10::DeviceGuard guard(attn.device());
             check_linear(hstu_output_norm_mul_bwd(&a, &g, stream_of(attn)));
-            if (weight_too) got[5] = at::mm(joined.t(), dout);
+            if (weight_too) got[5] = weight_grad(joined, dout, Tensor());
         }
         return got;
     }

@@ -94,7 +94,8 @@ class HstuOutputArgs(ctypes.Structure):
 EXPORTS = (
     "hstu_uqvk_workspace_bytes", "hstu_uqvk_forward", "hstu_uqvk_layer_norm", "hstu_output_workspace_bytes", "hstu_output_forward",
     "hstu_output_norm_mul", "hstu_output_dropout_mask", "hstu_output_norm_mul_bwd_workspace_bytes", "hstu_output_norm_mul_bwd",
-    "hstu_uqvk_layer_norm_bwd_workspace_bytes", "hstu_uqvk_layer_norm_bwd", "hstu_uqvk_silu_bwd", "hstu_linear_last_error",
+    "hstu_uqvk_layer_norm_bwd_workspace_bytes", "hstu_uqvk_layer_norm_bwd", "hstu_uqvk_silu_bwd",
+    "hstu_linear_weight_grad_workspace_bytes", "hstu_linear_weight_grad", "hstu_linear_last_error",
     "hstu_linear_version",
 )
 MUL_U_ACTIVATIONS = {"none": 0, "sigmoid": 1, "silu": 2}
@@ -171,8 +172,8 @@ def _needs_grad(*tensors: torch.Tensor) -> bool:
 
 # ---- gradients of the calls that the native front leaves ----------------------------------------------------------------
 # (parameters or rows that are not dense and 16-byte aligned, and ``layer_norm`` / ``norm_mul_dropout`` on their own.)  The
-# forward runs on this package's kernels; the gradients here are not hand-written: the backward recomputes the step with the framework's own operators (layer / group norm, addmm on hipBLASLt) in the
-# arithmetic of the reference's PyTorch backend (fp32 norm and product with u, result rounded to the input type, then the
+# forward runs on this package's kernels; the gradients here are not hand-written: the backward recomputes the step with the
+# framework's own operators (layer / group norm, addmm on hipBLASLt) in the arithmetic of the reference's PyTorch backend (fp32 norm and product with u, result rounded to the input type, then the
 # product with the weight: ops/pytorch/pt_layer_norm.py:24-39, pt_hstu_linear.py:24-124, ops/hstu_compute.py:54-104) and
 # lets autograd differentiate that -- nothing but the inputs is saved, which is what the reference's recompute_* flags
 # ask for.  It is there so that a training step can run through the package.

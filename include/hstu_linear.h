@@ -149,7 +149,7 @@ int hstu_output_dropout_mask(float ratio, uint64_t seed, uint64_t offset, int64_
 
 /*
  * ---- Backward of the row-wise parts ----
- * (the products are plain GEMMs and the caller's: d_joined = d_out @ W^T, d_W = joined^T @ d_out, and the like for the producer).
+ * (the products with a weight, d_joined = d_out @ W^T and the like, are plain GEMMs and the caller's).
  * Statistics and the dropout mask are recomputed from the forward's inputs; nothing is saved.  The gradients of a norm's weight
  * and bias are summed over the rows in fp32 in a fixed order through `workspace` (16-byte aligned) and rounded once.
  */
@@ -184,6 +184,13 @@ int hstu_uqvk_layer_norm_bwd(const void* x, int64_t x_row_stride, const void* we
  * LN(x) @ W of the u columns to their gradient in front of SiLU. */
 int hstu_uqvk_silu_bwd(void* pre, int64_t pre_row_stride, const void* bias, const void* du, int64_t du_row_stride, int64_t rows, int64_t width,
                        int32_t dtype, void* stream);
+
+/* Gradient of a weight: out[m, n] = a^T @ b for a [rows, m] and b [rows, n] (strides in elements, rows 16-byte aligned; m and n
+ * multiples of 8), fp32 sums rounded once; `b_sums`, if not NULL, gets the column sums of b [n] (the gradient of a bias).  The rows
+ * are split over workgroups whose sums are added in a fixed order through `workspace` (16-byte aligned). */
+size_t hstu_linear_weight_grad_workspace_bytes(int32_t m, int32_t n, int64_t rows, int64_t a_row_stride, int64_t b_row_stride);
+int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, const void* b, int64_t b_row_stride, int32_t n, int64_t rows,
+                            int32_t dtype, void* out, void* b_sums, void* workspace, int64_t workspace_bytes, void* stream);
 
 const char* hstu_linear_last_error(void);
 

@@ -123,3 +123,37 @@ def test_producer_gradients_against_the_recomputation(dev, dtype, rows, d, heads
     torch.cuda.synchronize()
     for name, a, b in zip(("x", "norm_weight", "norm_bias", "weight", "bias"), got, want):
         _close(a, b, f"d/d{name}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,m,n,sliced", [(1, 8, 8, False), (33, 264, 248, False), (64, 256, 512, True), (1000, 72, 776, False), (40000, 520, 256, True)])
+def test_weight_gradient_kernel(dev, dtype, rows, m, n, sliced):
+    """out = a^T b and the column sums of b, against fp64: one row, part tiles in both directions, rows that fill no tile, more
+    splits than one, operands that are column slices.  The bound: rounding the result to nearest moves a value by at
+    most half a unit of its last place, 2^-8 of it in bf16 (8 bits of significand) and 2^-11 in fp16 (11 bits), so the 2-norm of
+    the result by no more than that; a tenth of it more for the fp32 sums of at most 40000 products (each rounding 2^-24, random
+    in sign)."""
+    import ctypes
+
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    print(f"[case] weight gradient {rows} {m} {n} {sliced} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows + m)
+    pad = 40 if sliced else 0
+    a = torch.randn((rows, m + pad), generator=g, device=dev).to(dtype)[:, pad:]
+    b = torch.randn((rows, n + pad), generator=g, device=dev).to(dtype)[:, :n]
+    out, sums = torch.full((m, n), float("nan"), dtype=dtype, device=dev), torch.full((n,), float("nan"), dtype=dtype, device=dev)
+    L = hc.lib()
+    L.hstu_linear_weight_grad_workspace_bytes.restype = ctypes.c_size_t
+    L.hstu_linear_weight_grad_workspace_bytes.argtypes = [ctypes.c_int32, ctypes.c_int32] + [ctypes.c_int64] * 3
+    need = L.hstu_linear_weight_grad_workspace_bytes(m, n, rows, a.stride(0), b.stride(0))
+    ws = torch.full((need // 4,), float("nan"), device=dev)
+    P, I, Q = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
+    rc = L.hstu_linear_weight_grad(P(a.data_ptr()), Q(a.stride(0)), I(m), P(b.data_ptr()), Q(b.stride(0)), I(n), Q(rows), I(0 if dtype == torch.bfloat16 else 1),
+                                   P(out.data_ptr()), P(sums.data_ptr()), P(ws.data_ptr()), Q(need), P(torch.cuda.current_stream(dev).cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == 0, hc.lib().hstu_linear_last_error()
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for got, want in ((out, a.double().t() @ b.double()), (sums, b.double().sum(0))):
+        assert torch.isfinite(got).all()
+        assert float((got.double() - want).norm() / want.norm()) <= 1.1 * unit
