@@ -80,6 +80,10 @@ __global__ __launch_bounds__(256) void hstu_check_contract_kernel(const void* of
 
 }  // namespace hstu
 
+// The pipelined kernels' variant for fitted runs: a translation unit of its own (hstu_fwd_fitted.hip).
+extern "C" __attribute__((visibility("hidden"))) void hstu_hip_launch_fitted(const hstu::FwdParams* p, int dtype, int dim, int cfg, int grid_per_xcd,
+                                                                           hipStream_t stream);
+
 namespace {
 
 constexpr int kMaxSortBatch = 8192;  // beyond this the quadratic ranking is not worth its time
@@ -133,10 +137,12 @@ int launch(const hstu::FwdParams& p, hipStream_t stream) {
 
 template <class TT, int DQK, int DV, int BN, int NG>
 int launch_pp(const hstu::FwdParams& p, int grid_per_xcd, int64_t total_q, hipStream_t stream) {
-    if constexpr (NG == 0) {  // the streaming form of the 8-wave kernel
-        hipLaunchKernelGGL((hstu::hstu_fwd_stream_kernel<TT, DQK, DV, BN>), dim3((unsigned)grid_per_xcd * 8), dim3(512), 0, stream, p);
+    if (p.fit_runs > 0) {
+        hstu_hip_launch_fitted(&p, TT::CODE, DQK, NG == 0 ? 2 : 3, grid_per_xcd, stream);
+    } else if constexpr (NG == 0) {  // the streaming form of the 8-wave kernel
+        hipLaunchKernelGGL((hstu::hstu_fwd_stream_kernel<TT, DQK, DV, BN, false>), dim3((unsigned)grid_per_xcd * 8), dim3(512), 0, stream, p);
     } else {
-        hipLaunchKernelGGL((hstu::hstu_fwd_pp_kernel<TT, DQK, DV, BN, NG>), dim3((unsigned)grid_per_xcd * 8), dim3(NG * 256), 0, stream,
+        hipLaunchKernelGGL((hstu::hstu_fwd_pp_kernel<TT, DQK, DV, BN, NG, false>), dim3((unsigned)grid_per_xcd * 8), dim3(NG * 256), 0, stream,
                            p);  // LDS is a static array
     }
     hipError_t e = hipGetLastError();
@@ -144,7 +150,7 @@ int launch_pp(const hstu::FwdParams& p, int grid_per_xcd, int64_t total_q, hipSt
         set_last_error("kernel launch", e);
         return HSTU_ERR_LAUNCH;
     }
-    if (p.kv_splits > 1) {
+    if (p.kv_splits > 1 || p.fit_runs > 0) {
         const long long threads = (long long)total_q * p.H * (DV / 4);
         const long long blocks = (threads + 255) / 256;
         if (blocks > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
@@ -209,6 +215,8 @@ struct Plan {
     int cfg;               // tile configuration, 1-based
     int splits;            // workgroups per row block along kv (1 = no split)
     int chunk;             // kv tiles per run when split
+    int fit_runs;          // runs fitted to the lengths (decode_fitted): workgroups per (head, row block), 0 = off; `splits` is then
+                           // their average number per row block
     // the workspace, in this order:
     size_t queue_bytes;    // work-item counters and list lengths of the persistent kernels
     size_t order_bytes;    // sequence ranking
@@ -234,7 +242,8 @@ bool rows_fit_buffer_offsets(const HstuFwdArgs* a) {
 }
 
 Plan make_plan(const HstuFwdArgs* a) {
-    Plan pl = {0, 1, 0, 0, 0, 0, 0, 0, 0};
+    Plan pl{};
+    pl.splits = 1;
     // The streaming two-group kernel (256-row blocks, one workgroup per CU) wins when the average sequence is long;
     // the one-group pipeline (128-row blocks, two workgroups per CU) wastes less on short or very uneven sequences
     // and in delta mode.
@@ -252,9 +261,15 @@ Plan make_plan(const HstuFwdArgs* a) {
             // -- 1 to 3 % ahead; 1280 -- level; 1800 -- 3 % ahead; 2048 to 2560 -- 6 to 8 % ahead)
             pl.cfg = avg_tiles >= 960 / kTileRows ? 2 : 3;
         } else {
-            // few long histories: 256-row blocks, whose kv range is then split below so that every CU gets one
-            const long long blocks256 = (long long)a->batch * a->heads * ((a->delta_size + 255) / 256);
-            pl.cfg = (blocks256 * 2 <= 256 && avg_tiles >= 32) ? 2 : 3;
+            // Few long histories: 256-row blocks, whose kv range is then split below so that every CU gets one -- where their
+            // second half exists (5 histories of 8000 .. 16000 x 100 candidates, 4 heads: 44 us against 38 with 128-row blocks)
+            // and a CU's share is at least 8 tiles, below which what an item costs besides its steps counts for more
+            // (256 candidates: 2 and 8 histories of 1000 .. 4000: 25 and 35 us against 22 and 32; 5 of 8000 .. 16000: 51
+            // against 56; 32 of 1024 .. 4096: 73 against 78).
+            const long long mb256 = (a->delta_size + 255) / 256, blocks256 = (long long)a->batch * a->heads * mb256;
+            const bool half_empty = (a->delta_size - 1) % 256 < 128;
+            const bool long_runs = a->total_kv / kTileRows * a->heads * mb256 >= 8 * 256;
+            pl.cfg = (blocks256 * 2 <= 256 && avg_tiles >= 32 && !half_empty && long_runs) ? 2 : 3;
         }
     }
     if (a->sort_by_length && a->batch >= 2 && a->batch <= kMaxSortBatch) pl.order_bytes = (size_t)a->batch * sizeof(int);
@@ -272,6 +287,27 @@ Plan make_plan(const HstuFwdArgs* a) {
         // 256 CUs.  Cut the kv range so that the chip is just filled (more runs than that only add partial-sum
         // traffic: with every CU busy the clock drops and the time per tile rises), in runs of at least 16 tiles.
         const long long resident = pl.cfg == 2 ? 256 : 512;  // workgroups the chip holds at once
+        // Runs fitted to the lengths where the whole history is in reach of every row (no window, no contextual prefix), for at
+        // most 64 sequences (decode_fitted has a lane for each).  128-row blocks: one workgroup per CU (a second one halves
+        // the runs but not what an item costs, and both wait for the same HBM: 16 x 1000 .. 4000 x 128 candidates 31 us
+        // with 256 workgroups, 40 with 512; 5 x 8000 .. 16000 x 100: 37 and 45) unless the row blocks alone are more than 64
+        // (30 x 7300 .. 14600 x 91: 173 and 150).  Short runs still pay: 50 candidates x 400 rows, 16.7 us unsplit, 12.4 us in
+        // runs of one tile.  Below 6 tiles saved the extra kernel and the partial sums cost more than the shorter runs save;
+        // with fewer than four workgroups per sequence there is little to fit (32 x 1024 .. 4096 x 256: 76 us, equal counts 73).
+        if (a->max_attn_len == 0 && a->contextual_seq_len == 0 && a->batch <= 64 && max_tiles <= (1 << 20)) {
+            const long long chip = pl.cfg == 2 ? 256 : blocks * 4 <= 256 ? 256 : 512;
+            const long long num_mb = (rows_per_pair + bm - 1) / bm, planes = a->heads * num_mb;
+            const long long tiles = a->total_kv / kTileRows + a->batch;  // of a plane, at most
+            long long runs = chip / 8 / num_mb * 8 / a->heads;
+            if (runs > tiles) runs = tiles;
+            if (runs >= 4 * a->batch && max_tiles - (tiles + runs - 1) / runs >= 6) {
+                pl.fit_runs = (int)runs;
+                pl.splits = (int)(runs / a->batch);
+                pl.counts_bytes = (size_t)blocks * sizeof(int);
+                pl.partial_bytes = (size_t)planes * runs * (rows_per_pair < bm ? rows_per_pair : bm) * a->dv * sizeof(float);
+                return pl;
+            }
+        }
         long long want = resident / blocks;
         if (want > max_tiles / 16) want = max_tiles / 16;
         if (want > kMaxSplits) want = kMaxSplits;
@@ -329,6 +365,7 @@ void fill_decode_params(hstu::FwdParams& p) {
     d.delta = p.delta;
     d.w = p.w;
     d.f = p.f;
+    d.fit_runs = p.fit_runs;
     d.mb_magic = p.mb_magic;
     d.mb_shift = p.mb_shift;
     d.h_magic = p.h_magic;
@@ -579,6 +616,7 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
         }
     }
     if (plan.splits > 1 && !ws_ok) {
+        plan.fit_runs = 0;
         if (a->kv_splits > 1) return a->workspace ? HSTU_ERR_BAD_SHAPE : HSTU_ERR_NULL_POINTER;
         plan.splits = 1;
         plan.partial_bytes = plan.counts_bytes = 0;
@@ -593,6 +631,7 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
         p.partial = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(base + plan.counts_bytes) + 255) & ~(uintptr_t)255);
         p.partial_stride = (int64_t)a->total_q * a->heads * a->dv;
         p.kv_chunk = plan.chunk;
+        if (plan.fit_runs > 0) p.fit_runs = plan.fit_runs, plan.splits = 1;  // (an item is one run: decode_fitted)
     }
     p.kv_splits = plan.splits;
 
@@ -604,7 +643,8 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
     const int bm = cfg == 2 ? 256 : 128;
     p.num_mb = (rows_per_pair + bm - 1) / bm;
     const long long pairs_per_xcd = (num_pairs + 7) / 8;
-    const long long slots = pairs_per_xcd * p.num_mb * plan.splits;
+    const long long slots = p.fit_runs > 0 ? (((long long)p.fit_runs * a->heads + 7) / 8) * p.num_mb : pairs_per_xcd * p.num_mb * plan.splits;
+    p.fit_rows = rows_per_pair < bm ? rows_per_pair : bm;
     if (slots <= 0) return HSTU_OK;
     if (slots * 8 > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
     p.pairs_per_xcd = (int)pairs_per_xcd;

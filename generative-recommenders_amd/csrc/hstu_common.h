@@ -60,7 +60,7 @@ struct DecodeParams {
     const void* offsets;
     const void* targets;
     int items_cap, kv_splits, kv_chunk, c, pairs_per_xcd, num_mb, B, H;
-    int uniform, max_seq_len, offsets_i64, targets_i64, delta, w, f, pad0;
+    int uniform, max_seq_len, offsets_i64, targets_i64, delta, w, f, fit_runs;
     unsigned mb_magic, mb_shift, h_magic, h_shift;
     int pad1[2];
 };
@@ -111,6 +111,9 @@ struct FwdParams {
     float* partial;
     int64_t partial_stride;  // floats per split = total_q * H * dv
     int* split_counts;
+    // Delta form with few row blocks: runs fitted to the lengths (see decode_fitted).  fit_runs: workgroups per plane (0 = off);
+    // `partial` then holds [plane][workgroup][fit_rows][dv], and split_counts the first workgroup << 16 | number of runs.
+    int fit_runs, fit_rows;
     alignas(64) DecodeParams dec;  // copies of the fields above that decode_work reads
 };
 
@@ -127,6 +130,7 @@ struct FwdParams {
     "v_mul_f32 %4, " a ", %4\n\tv_mul_f32 %5, " b ", %5\n\tv_mul_f32 %6, " c ", %6\n\tv_mul_f32 %7, " d ", %7\n\t"     \
     "v_cvt_pk_bf16_f32 " p ", %4, %5\n\tv_cvt_pk_bf16_f32 " q ", %6, %7\n\t"
 struct Bf16 {
+    static constexpr int CODE = 0;  // HstuDtype
     static constexpr bool PAIRWISE = false;
     typedef bf16x8_t vec8;
     typedef __bf16 elem;
@@ -191,6 +195,7 @@ __device__ __forceinline__ void sigmoid_f16_pairs(const h2_t (&t)[4], h2_t (&r)[
 #undef HSTU_F16_PAIRS
 
 struct Fp16 {
+    static constexpr int CODE = 1;  // HstuDtype
     static constexpr bool PAIRWISE = false;
     static constexpr bool PINNED_SILU = false;
     typedef f16x8_t vec8;
@@ -226,6 +231,7 @@ struct Fp16F32 : Fp16 {
 // typical magnitudes (|t| around 1e-2) into the normal range of e4m3 (2^-6 .. 448); p is unbounded only
 // towards -inf (t -> -inf), where it is clamped to the largest finite e4m3 value.
 struct Fp8 {
+    static constexpr int CODE = 2;  // HstuDtype
     typedef long vec8;
     typedef unsigned char elem;
     typedef __bf16 out_elem;
@@ -378,6 +384,7 @@ struct Work {
     int u;            // number of non-target positions
     int split;        // which run of the kv range this workgroup takes (0 when the range is not split)
     int nsplit;       // number of non-empty runs of this row block
+    int fit_slot;     // fitted runs: number of the workgroup's partial sums, -1: stored directly (one run)
     int block_id;     // (b * H + h) * num_mb + row block
     int R0, R1;       // sequence positions of the workgroup's first and last row (inclusive)
     int jt_begin;     // first kv tile that can hold a valid pair
@@ -431,11 +438,24 @@ __device__ __forceinline__ int fast_div(int x, unsigned magic, unsigned shift) {
     return magic ? (int)(__umulhi((unsigned)x, magic) >> shift) : x;
 }
 
+// Runs fitted to the lengths, for the delta form when its row blocks are few (at most 64 sequences: a lane each).  A plane is a (head, row
+// block) pair; `fit_runs` workgroups share the kv tiles of its sequences.  Sequence b gets r_b = ceil(tiles_b / tau) of them, with the
+// smallest tau (tiles of the longest run) for which they suffice: a run count from max_seq_len alone is the same for all
+// histories, so that the longest one's runs are several times the shortest's, and the launch lasts as long as they do.
+// Every lane tries another tau between the mean and twice the mean, where the workgroups suffice for sure (the host gives at least
+// two per sequence).  Measured with the reduce kernel: 5 histories of 8000 .. 16000 rows x 100 candidates, 4 heads, d = 128, 256
+// workgroups: 38 us (2.8 TB/s of K and V) where the equal run counts took 55 us and 71 us with 256-row blocks.  Run 0 records the first workgroup and the number of runs for the reduce kernel; one run is stored directly.
+// The row blocks of a head, which read the same keys, share an XCD.
+template <int BM, int BN>
+__device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, int slot, int xcd, int64_t& seq_start, int64_t& seq_end, int& mb);
+
 // Decode work item `bid` (the workgroup id in a one-item-per-workgroup launch) of the launch whose FwdParams are the
 // kernel's first argument.  Workgroup ids go round-robin
 // over the 8 XCDs, so ids congruent mod 8 share an L2: all row blocks of one (sequence, head) pair stay on one
 // XCD, heaviest block first.  Returns false if the item holds no work.
-template <int BM, int BN>
+// FIT: the launch runs on fitted runs (decode_fitted).  A variant of the kernels of its own: the decoding, inlined at every place
+// that starts an item, made the others' code larger and the windowed ragged batch 0.7 % slower.
+template <int BM, int BN, bool FIT>
 __device__ __forceinline__ bool decode_work(Work& w, int bid) {
     // the block of parameters, straight from the kernel argument segment: FwdParams is the kernels' first argument
     typedef __attribute__((ext_vector_type(16))) int i32x16_t;
@@ -449,6 +469,7 @@ __device__ __forceinline__ bool decode_work(Work& w, int bid) {
     int slot = bid >> 3;
     // the splits of one row block are neighbours on one XCD
     w.split = 0;
+    w.fit_slot = -1;
     if (p.kv_splits > 1) {
         const int s0 = slot / p.kv_splits;
         w.split = slot - s0 * p.kv_splits;
@@ -460,7 +481,10 @@ __device__ __forceinline__ bool decode_work(Work& w, int bid) {
     int pair_local, mb;
     int64_t seq_start, seq_end;
     int t = 0;
-    if (p.items) {
+    if constexpr (FIT) {
+        if (!decode_fitted<BM, BN>(w, p, slot, xcd, seq_start, seq_end, mb)) return false;
+        if (p.targets) t = p.targets_i64 ? (int)HSTU_CONST(int64_t, p.targets)[w.b] : HSTU_CONST(int, p.targets)[w.b];
+    } else if (p.items) {
         // everything straight from the list: one load
         if (slot >= HSTU_CONST(int, p.nitems)[xcd]) return false;
         typedef __attribute__((ext_vector_type(8))) int i32x8_t;
@@ -530,8 +554,10 @@ __device__ __forceinline__ bool decode_work(Work& w, int bid) {
 
     w.R0 = w.rbase + w.m0;
     w.R1 = w.rbase + w.m1 - 1;
-    kv_tile_range(M, w.u, w.R0, w.R1, BN, w.jt_begin, w.jt_end);
-    w.nsplit = 1;
+    if constexpr (!FIT) {
+        kv_tile_range(M, w.u, w.R0, w.R1, BN, w.jt_begin, w.jt_end);
+        w.nsplit = 1;
+    }
     w.block_id = (w.b * p.H + w.h) * p.num_mb + mb;
     if (p.kv_splits > 1) {
         w.nsplit = (w.jt_end - w.jt_begin + p.kv_chunk - 1) / p.kv_chunk;
@@ -555,6 +581,57 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
     v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
     return v;
+}
+
+template <int BM, int BN>
+__device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, int slot, int xcd, int64_t& seq_start, int64_t& seq_end, int& mb) {
+    const int lane = threadIdx.x & 63;
+    const int g0 = fast_div(slot, p.mb_magic, p.mb_shift);
+    mb = slot - g0 * p.num_mb;
+    const int k = g0 * 8 + xcd;  // (head, workgroup of the plane)
+    const int h = k / p.fit_runs, i = k - h * p.fit_runs;
+    if (h >= p.H) return false;
+    int tiles = 0;  // of sequence `lane`, for this row block: its last row ends at n - delta + the block's end
+    if (lane < p.B) {
+        const int64_t n64 = p.offsets_i64 ? ((const int64_t*)p.offsets)[lane + 1] - ((const int64_t*)p.offsets)[lane]
+                                          : (int64_t)(((const int*)p.offsets)[lane + 1] - ((const int*)p.offsets)[lane]);
+        const int n = n64 > p.max_seq_len ? p.max_seq_len : (int)n64;
+        const int end = (mb + 1) * BM < p.delta ? (mb + 1) * BM : p.delta;
+        if (n > 0 && n >= p.delta) tiles = (n - p.delta + end + BN - 1) / BN;
+    }
+    const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(tiles), 63);
+    const int mean = (int)(((unsigned)total + (unsigned)p.fit_runs - 1) / (unsigned)p.fit_runs);
+    // (an approximate quotient serves as well as the exact one: every workgroup computes the same)
+    const int tau = mean + lane * ((mean + 62) / 63);
+    const float inv = __builtin_amdgcn_rcpf((float)tau);
+    auto runs_of = [](int t, int tau, float inv) { return (int)((float)(t + tau - 1) * inv); };
+    int need = 0;
+    for (int b = 0; b < p.B; ++b) need += runs_of(__builtin_amdgcn_readlane(tiles, b), tau, inv);
+    const uint64_t enough = __ballot(need <= p.fit_runs && tau > 0);
+    if (enough == 0) return false;  // (no sequence has anything to do; otherwise lane 63 suffices)
+    const int best = __builtin_ctzll(enough);
+    const int tau_b = __builtin_amdgcn_readlane(tau, best);
+    const float inv_b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv), best));
+    int runs = runs_of(tiles, tau_b, inv_b);
+    runs = tiles > 0 && runs < 1 ? 1 : runs > tiles ? tiles : runs;
+    const int upto = wave_inclusive_scan(runs);
+    const int b = __popcll(__ballot(upto <= i));
+    if (b >= p.B) return false;  // more workgroups than runs
+    const int r = __builtin_amdgcn_readlane(runs, b), first = __builtin_amdgcn_readlane(upto, b) - r, t = __builtin_amdgcn_readlane(tiles, b);
+    w.b = b, w.h = h;
+    w.split = i - first;
+    w.nsplit = r | first << 16;
+    w.jt_begin = (int)((unsigned)(w.split * t) / (unsigned)r);
+    w.jt_end = (int)((unsigned)((w.split + 1) * t) / (unsigned)r);
+    if (r > 1) w.fit_slot = (h * p.num_mb + mb) * p.fit_runs + i;
+    if (p.offsets_i64) {
+        seq_start = HSTU_CONST(int64_t, p.offsets)[b];
+        seq_end = HSTU_CONST(int64_t, p.offsets)[b + 1];
+    } else {
+        seq_start = HSTU_CONST(int, p.offsets)[b];
+        seq_end = HSTU_CONST(int, p.offsets)[b + 1];
+    }
+    return true;
 }
 
 #define HSTU_PLAN_THREADS 1024
@@ -953,12 +1030,21 @@ __device__ __forceinline__ void store_output_via_lds(const f32x16_t (&oacc)[DT][
     }
 }
 
-// Unscaled fp32 accumulators of one block of 32 query rows to partial[split][row][head][dv]; 16 bytes per store.
+// Where the partial sums of an item go (query row r of the sequence at + r * partial_pitch), or null: the item is stored directly.
+template <bool FIT>
+__device__ __forceinline__ int partial_pitch(const FwdParams& p, int dv) { return FIT ? dv : p.H * dv; }
+template <bool FIT>
+__device__ __forceinline__ float* partial_base(const FwdParams& p, const Work& w, int64_t orow0, int dv) {
+    if constexpr (FIT) return w.fit_slot >= 0 ? p.partial + ((int64_t)w.fit_slot * p.fit_rows - w.m0) * dv : nullptr;
+    if (p.kv_splits > 1) return p.partial + (int64_t)w.split * p.partial_stride + (orow0 * p.H + w.h) * dv;
+    return nullptr;
+}
+
+// Unscaled fp32 accumulators of one block of 32 query rows; 16 bytes per store.
 template <int DT, int QT>
-__device__ __forceinline__ void store_partial(const f32x16_t (&oacc)[DT][QT], int qt, float* partial, int64_t orow0, int ql,
-                                              int nq, int H, int h, int g) {
+__device__ __forceinline__ void store_partial(const f32x16_t (&oacc)[DT][QT], int qt, float* partial, int pitch, int ql, int nq, int g) {
     if (ql >= nq) return;
-    float* op = partial + ((orow0 + ql) * H + h) * (int64_t)(DT * 32) + g * 4;
+    float* op = partial + (int64_t)ql * pitch + g * 4;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -1007,12 +1093,26 @@ __global__ __launch_bounds__(256) void hstu_reduce_splits_kernel(const FwdParams
         if (row - start >= n) return;
         r = (int)(row - start);
     }
-    const int runs = p.split_counts[(b * p.H + h) * p.num_mb + r / bm];
-    f32x4_t acc = *(const f32x4_t*)(p.partial + idx * 4);
-    for (int s = 1; s < runs; ++s) {
-        const f32x4_t x = *(const f32x4_t*)(p.partial + s * p.partial_stride + idx * 4);
-        acc += x;
+    const int mb = r / bm;
+    int runs = p.split_counts[(b * p.H + h) * p.num_mb + mb];
+    const float* src = p.partial + idx * 4;
+    int64_t pitch = p.partial_stride;
+    if (p.fit_runs > 0) {
+        pitch = (int64_t)p.fit_rows * dv;
+        src = p.partial + ((int64_t)(h * p.num_mb + mb) * p.fit_runs + (runs >> 16)) * pitch + (int64_t)(r - mb * bm) * dv + c * 4;
+        runs &= 0xffff;
+        if (runs == 1) return;  // stored by its one workgroup
     }
+    f32x4_t acc = *(const f32x4_t*)src;
+    int s = 1;
+    for (; s + 4 <= runs; s += 4) {  // four loads in flight, added in order
+        f32x4_t x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = *(const f32x4_t*)(src + (s + j) * pitch);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc += x[j];
+    }
+    for (; s < runs; ++s) acc += *(const f32x4_t*)(src + s * pitch);
     elem4 o4;
     const float osc = output_scale(p, row);
 #pragma unroll

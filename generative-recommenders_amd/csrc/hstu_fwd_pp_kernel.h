@@ -86,7 +86,7 @@ __device__ __forceinline__ void prescale_q(typename TT::vec8 (&qreg)[KS], float 
 
 // NG = 1 (the only instantiation): a single wave group, 4 waves, 128 rows, 2 LDS slots, two workgroups per CU and one
 // barrier per tile.  It wastes less than 256-row blocks on short sequences, whose last block would be mostly empty.
-template <class TT, int DQK, int DV, int BN, int NG>
+template <class TT, int DQK, int DV, int BN, int NG, bool FIT>
 __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParams p_arg) {
     typedef typename TT::vec8 vec8;
     static_assert(DQK == DV, "the interleaved matrix phase assumes as many first-product as second-product MFMAs");
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
     asm volatile("" : "+s"(pk));
     const FwdParams& p = *(const FwdParams*)pk;
     Work W;
-    if (!decode_work<BM, BN>(W, bid)) return;
+    if (!decode_work<BM, BN, FIT>(W, bid)) return;
     const SeqMask& M = W.M;
     const int n = W.n;
     const int nq = W.m1;  // one past the last row of this item: rows from here on are never loaded or stored
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
     const int jt_end = W.jt_end;
     const int T = jt_end - W.jt_begin;  // steps
     const int64_t orow0 = p.delta > 0 ? (int64_t)W.b * p.delta : W.seq_start;
-    float* const my_partial = p.kv_splits > 1 ? p.partial + (int64_t)W.split * p.partial_stride : nullptr;
+    float* const my_partial = partial_base<FIT>(p, W, orow0, DV);
     if (T <= 0) return;  // cannot happen for a row block with rows (each row sees itself); kept for safety
     int t_cur = W.jt_begin;
 
@@ -456,9 +456,9 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
     // the redundant copies of the last steps may still be in flight: they must land before the LDS is released
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
+    if ((my_partial || FIT) && W.split == 0 && threadIdx.x == 0) p.split_counts[W.block_id] = W.nsplit;
     if (my_partial) {
-        store_partial<DT>(oacc, 0, my_partial, orow0, wq0 + l32, nq, p.H, W.h, g);
-        if (W.split == 0 && threadIdx.x == 0) p.split_counts[W.block_id] = W.nsplit;
+        store_partial<DT>(oacc, 0, my_partial, partial_pitch<FIT>(p, DV), wq0 + l32, nq, g);
     } else if constexpr (4 * 32 * (DT * 64 + 16) <= NSLOT * (KTILE + VTILE)) {
         // the K/V tiles are dead once every wave is through its last product; each wave then turns its output
         // tile around in its own piece of that LDS

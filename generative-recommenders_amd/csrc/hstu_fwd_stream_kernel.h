@@ -73,7 +73,7 @@ __device__ __forceinline__ void store_output_staged(const f32x16_t (&oacc)[DT][1
     }
 }
 
-template <class TT, int DQK, int DV, int BN>
+template <class TT, int DQK, int DV, int BN, bool FIT>
 __global__ __launch_bounds__(512, 2) void hstu_fwd_stream_kernel(const FwdParams p_arg) {
     typedef typename TT::vec8 vec8;
     static_assert(DQK == DV, "the interleaved matrix phase assumes as many first-product as second-product MFMAs");
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(512, 2) void hstu_fwd_stream_kernel(const FwdParams
     auto find_next = [&](const FwdParams& p, Work& W) __attribute__((always_inline)) -> bool {
         for (;;) {
             if (next_bid < 0) return false;
-            if (decode_work<BM, BN>(W, next_bid) && W.jt_end > W.jt_begin) return true;
+            if (decode_work<BM, BN, FIT>(W, next_bid) && W.jt_end > W.jt_begin) return true;
             if (queue) {
                 if (drawer) publish_next(resolve_ticket(draw_ticket()));
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(512, 2) void hstu_fwd_stream_kernel(const FwdParams
         drain_slot = (T - 1) % NSLOT;
         t_cur = W.jt_begin;
         orow0 = p.delta > 0 ? (int64_t)W.b * p.delta : W.seq_start;
-        my_partial = p.kv_splits > 1 ? p.partial + (int64_t)W.split * p.partial_stride : nullptr;
+        my_partial = partial_base<FIT>(p, W, orow0, DV);
         row.init(M, wR0 + l32);
         lds_read_offsets<TT, DQK, DV>(kaddr, vaddr, lane_v);
         // (only vaddr[0] is kept: the second transposing read of an operand lies 8 rows below the first for every lane,
@@ -476,9 +476,9 @@ __global__ __launch_bounds__(512, 2) void hstu_fwd_stream_kernel(const FwdParams
     };
     // `more`: the copies of a next item have been started.
     auto store_item = [&](const FwdParams& p, bool more) __attribute__((always_inline)) {
+        if ((my_partial || FIT) && split == 0 && threadIdx.x == 0) p.split_counts[block_id] = nsplit;
         if (my_partial) {
-            store_partial<DT>(oacc, 0, my_partial, orow0, wq0 + l32, nq, p.H, h_cur, g);
-            if (split == 0 && threadIdx.x == 0) p.split_counts[block_id] = nsplit;
+            store_partial<DT>(oacc, 0, my_partial, partial_pitch<FIT>(p, DV), wq0 + l32, nq, g);
             return;
         }
         const float osc = output_scale(p, orow0 + (wq0 + l32 < nq ? wq0 + l32 : nq - 1));

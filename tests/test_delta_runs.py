@@ -1,0 +1,43 @@
+"""The delta form with few row blocks: kv runs fitted to the lengths (decode_fitted), against the oracle and the unsplit kernel."""
+
+import pytest
+import torch
+
+from oracle import hstu_oracle as O
+from util import assert_parity, make_case
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # lengths (history + delta), delta, heads, dim
+    ([900], 1, 1, 32),                                   # one sequence, one row
+    ([450], 50, 4, 128),                                 # a run per tile
+    ([129, 2500], 129, 2, 64),                           # two row blocks, the second of one row; a sequence without history
+    ([2000, 100, 64, 1037, 700], 64, 3, 128),            # tile multiples, heads that do not divide the XCDs
+    ([5000, 300], 300, 1, 128),                          # row blocks of 128 and of 256 with a part over
+    ([6000, 40, 3513] + [65] * 61, 33, 1, 64),           # 64 sequences (every lane), most of them one or two tiles
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("lengths,delta,heads,dim", CASES)
+@pytest.mark.parametrize("cfg", [0, 2])
+def test_fitted_runs(pkg, dev, lengths, delta, heads, dim, dtype, cfg):
+    print(f"[case] fitted runs {len(lengths)} sequences up to {max(lengths)}, delta {delta}, {heads} x {dim} {dtype} cfg {cfg}", flush=True)
+    from generative_recommenders_amd.ops import hip_backend as hb
+
+    B, N, alpha = len(lengths), max(lengths) + 7, dim**-0.5
+    q, k, v, offs, t = make_case(11, lengths, heads, dim, targets=[min(delta, 5)] * B, delta_size=delta)
+    runs = hb.plan_for(B, heads, dim, dim, B * delta, int(offs[-1]), N, delta_size=delta, tile_config=cfg)[1]
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    args = [N, alpha] + [x.to(dev) for x in (q, k, v, offs)]
+    got = pkg.delta_hstu_mha(*args, num_targets=t.to(dev), tile_config=cfg)
+    again = pkg.delta_hstu_mha(*args, num_targets=t.to(dev), tile_config=cfg)
+    one = pkg.delta_hstu_mha(*args, num_targets=t.to(dev), tile_config=cfg, kv_splits=1)
+    torch.cuda.synchronize()
+    assert runs >= 2, "the automatic rule splits these"
+    assert torch.equal(got, again)
+    # the same products, summed in fp32 run by run: what is left is the rounding of the result (at most 2^-8 of it, in bf16)
+    assert float((got.float() - one.float()).norm() / one.float().norm()) <= 2.0**-8
+    if dtype == torch.bfloat16:
+        assert_parity(got, O.cached_hstu_mha_per_sequence(N, alpha, q.float(), k.float(), v.float(), offs, t), "fitted runs")
