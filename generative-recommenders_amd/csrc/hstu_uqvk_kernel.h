@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
         int64_t r = row0 + rg * 32 + l32;
-        r = r < p.rows ? r : p.rows - 1;  // rows past the end repeat the last one; they are never stored
+        r = r < p.rows ? r : p.rows - 1;  // rows past the end repeat the last one
         const char* xp = p.x + (r * p.x_rs + 8 * g) * 2;
         float sum = 0.f;
 #pragma unroll
@@ -229,8 +229,11 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
             for (int i = 0; i < 4; ++i) {
                 const int row = i * 8 + rsub;
                 const i32x4_t v = *HSTU_LDS(const i32x4_t, stage + row * kUqvkStageRow + chunk * 16);
-                if (row0 + rg * 32 + row < p.rows)
-                    *(i32x4_t*)(p.out + ((row0 + rg * 32 + row) * p.n_out + col0) * 2 + chunk * 16) = v;
+                // rows past the end are the last row once more, the same bits to the same place: a store that is left out where no lane has
+                // a row would be missing from the number of instructions in flight that the next tile's wait counts with
+                int64_t r = row0 + rg * 32 + row;
+                r = r < p.rows ? r : p.rows - 1;
+                *(i32x4_t*)(p.out + (r * p.n_out + col0) * 2 + chunk * 16) = v;
                 if (to8) {
                     // the rounded values once more, scaled, as e4m3: 8 lanes cover 64 bytes of a row
                     const vec8 e = __builtin_bit_cast(vec8, v);
@@ -251,10 +254,8 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
                     lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
                     hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
                     hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
-                    if (row0 + rg * 32 + row < p.rows) {
-                        typedef __attribute__((ext_vector_type(2))) int i32x2_t;
-                        *(i32x2_t*)(p.out8 + (row0 + rg * 32 + row) * (int64_t)(p.n_out - p.n_silu) + (col0 - p.n_silu) + chunk * 8) = i32x2_t{lo, hi};
-                    }
+                    typedef __attribute__((ext_vector_type(2))) int i32x2_t;
+                    *(i32x2_t*)(p.out8 + r * (int64_t)(p.n_out - p.n_silu) + (col0 - p.n_silu) + chunk * 8) = i32x2_t{lo, hi};
                 }
             }
         }
