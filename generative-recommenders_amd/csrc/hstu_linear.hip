@@ -11,10 +11,14 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 
 #include "hstu_rows.h"
 #include "hstu_uqvk_kernel.h"
 #include "hstu_output_kernel.h"
+
+// hstu_uqvk_wide.hip
+int hstu_uqvk_wide_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
 
 namespace {
 
@@ -599,8 +603,21 @@ int launch_uqvk_fused(hstu::UqvkFusedParams p, hipStream_t stream) {
     return 0;
 }
 
+// 64 rows per wave where that kernel's work, row blocks of 256 x column blocks of 64, gives each CU 16 units or more (8 at d_model 256,
+// where the rows are normalised in half the time); below that the rows' preparation, 256 at a time on one CU, outweighs
+// the faster matrix phase.  d_model 512 into 2048 columns, 32 -> 64 rows per wave: 26000 rows 87 -> 91 us, 32768 100 -> 85, 139264
+// 408 -> 329; into 4096: 12000 rows 83 -> 87, 16384 98 -> 88, 174000 957 -> 743; d_model 256 into 1024: 26000 rows 39 -> 40, 32768
+// 40 -> 34.  Columns: into 256 it is slower at every size (300000 rows of d_model 512: 177 -> 197), into 512 from 131072 rows on the faster
+// one (133 -> 125).
+bool uqvk_takes_wide(const hstu::UqvkFusedParams& p, int d_model) {
+    if (d_model < 256 || p.n_out < 512 || p.n_silu % 64 != 0) return false;
+    const long long units = (p.rows + 255) / 256 * (p.n_out / 64);
+    return units >= (d_model == 256 ? 2048 : 4096) && units <= 0x7fffffffLL;
+}
+
 template <class TT>
 int launch_uqvk_fused_k(const hstu::UqvkFusedParams& p, int d_model, hipStream_t stream) {
+    if (uqvk_takes_wide(p, d_model)) return hstu_uqvk_wide_launch(p, d_model, std::is_same<TT, hstu::Bf16>::value, stream);
     switch (d_model) {
         case 128: return launch_uqvk_fused<TT, 2>(p, stream);
         case 256: return launch_uqvk_fused<TT, 4>(p, stream);

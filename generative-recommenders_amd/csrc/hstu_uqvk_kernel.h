@@ -34,6 +34,7 @@ struct UqvkFusedParams {
     int n_out;   // multiple of 128
     int n_silu;  // multiple of 32: columns [0, n_silu) go through SiLU
     int chunks_per_wg;  // column blocks (of 128) a workgroup walks: the grid holds ceil(n_out / 128 / chunks_per_wg) workgroups per row block
+    int units;          // (64 rows per wave) row blocks x column blocks of 64, of which a workgroup takes chunks_per_wg or one more
     // Optional second output: the v | q | k columns (those from n_silu on) once more as e4m3 bytes,
     // out8[r, n - n_silu] = e4m3(rounded out[r, n] * inv_scale[t]), t = 0 (v: the next n_silu columns), 1 (q: the next
     // n_attn), 2 (k: the rest), clamped to +-448; and the largest |rounded out| of each of the three, for the scales of
@@ -55,6 +56,52 @@ constexpr int kUqvkLds = 3 * kUqvkSlot + kUqvkBiasRing + kUqvkWaves * 32 * kUqvk
 // for the two half-waves g: the four rows of a half-wave go to four different 64-byte bank groups (row bits 0-1 ->
 // chunk bits 2-3) and the two half-waves to different 32-byte halves of a group (row bit 3 -> chunk bit 1).
 __device__ __forceinline__ int swz_w(int row) { return ((row & 3) << 2) | (((row >> 3) & 1) << 1); }
+
+// Row r (rows past the end repeat the last one) through the layer norm, as the B operands of a lane: 8 consecutive k of every 16,
+// from 8 g on; the two half-waves share the row.
+template <class TT, int KS>
+__device__ __forceinline__ void uqvk_normalised_row(const UqvkFusedParams& p, int64_t r, int g, typename TT::vec8 (&xr)[KS]) {
+    typedef typename TT::vec8 vec8;
+    typedef typename TT::elem elem;
+    constexpr int K = KS * 16;
+    r = r < p.rows ? r : p.rows - 1;
+    const char* xp = p.x + (r * p.x_rs + 8 * g) * 2;
+    float sum = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        xr[ks] = *(const vec8*)(xp + ks * 32);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum += (float)xr[ks][j];
+    }
+    sum += __shfl_xor(sum, 32, 64);
+    float mean = sum * (1.0f / K);
+    // (rounded here: folded into the subtractions below, in one kernel and not in the other, a row's bits would depend on the batch)
+    asm volatile("" : "+v"(mean));
+    // the rows stay packed between the passes: without this the compiler keeps all their fp32 conversions alive
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xr[ks]));
+    float sq = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float d = (float)xr[ks][j] - mean;
+            sq += d * d;
+        }
+    sq += __shfl_xor(sq, 32, 64);
+    const float rstd = __builtin_amdgcn_rsqf(__builtin_fmaf(sq, 1.0f / K, p.eps));
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xr[ks]));
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const vec8 wv = *(const vec8*)(p.norm_weight + (ks * 16 + 8 * g) * 2);
+        const vec8 bv = *(const vec8*)(p.norm_bias + (ks * 16 + 8 * g) * 2);
+        vec8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = (elem)(((float)xr[ks][j] - mean) * rstd * (float)wv[j] + (float)bv[j]);
+        xr[ks] = o;
+    }
+}
 
 template <class TT, int KT>  // KT = d_model / 64: k tiles per column block
 __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(const UqvkFusedParams p) {
@@ -102,44 +149,7 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
     // ---- this wave's rows: load, normalise, keep as B operands
     vec8 xreg[RG][KS];
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg) {
-        int64_t r = row0 + rg * 32 + l32;
-        r = r < p.rows ? r : p.rows - 1;  // rows past the end repeat the last one
-        const char* xp = p.x + (r * p.x_rs + 8 * g) * 2;
-        float sum = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            xreg[rg][ks] = *(const vec8*)(xp + ks * 32);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) sum += (float)xreg[rg][ks][j];
-        }
-        sum += __shfl_xor(sum, 32, 64);
-        const float mean = sum * (1.0f / K);
-        // the rows stay packed between the passes: without this the compiler keeps all their fp32 conversions alive
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xreg[rg][ks]));
-        float sq = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float d = (float)xreg[rg][ks][j] - mean;
-                sq += d * d;
-            }
-        sq += __shfl_xor(sq, 32, 64);
-        const float rstd = __builtin_amdgcn_rsqf(sq * (1.0f / K) + p.eps);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xreg[rg][ks]));
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const vec8 wv = *(const vec8*)(p.norm_weight + (ks * 16 + 8 * g) * 2);
-            const vec8 bv = *(const vec8*)(p.norm_bias + (ks * 16 + 8 * g) * 2);
-            vec8 o;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = (elem)(((float)xreg[rg][ks][j] - mean) * rstd * (float)wv[j] + (float)bv[j]);
-            xreg[rg][ks] = o;
-        }
-    }
+    for (int rg = 0; rg < RG; ++rg) uqvk_normalised_row<TT, KS>(p, row0 + rg * 32 + l32, g, xreg[rg]);
 
     // transposing reads of a W tile: lane supplies the address of 4 consecutive n of k row 8g + 4sec + j
     int waddr[2][4];

@@ -226,6 +226,37 @@ def test_uqvk_columns_divided_over_workgroups_give_the_same_bits(pkg, dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "L,d_model,H,attn,hidden",
+    # at least 16 row blocks of 256 x column blocks of 64 per CU (8 at d_model 256), with remainders 0, 1 and 255 of the rows; units that
+    # the 256 workgroups share evenly and not; the u columns a whole and an odd number of blocks; the fewest columns
+    [(32768, 512, 4, 128, 128), (65537, 512, 2, 128, 128), (44031, 384, 3, 128, 128), (32769, 256, 4, 64, 64), (65791, 256, 2, 64, 64),
+     (131073, 512, 2, 64, 64), (52000, 384, 1, 512, 320)],
+)
+def test_uqvk_with_64_rows_per_wave_gives_the_bits_of_32(pkg, dev, L, d_model, H, attn, hidden, dtype):
+    """The sums run in the same order, so every row is bit for bit what the kernel for few rows gives for it (which the tests
+    above hold against the oracle); the e4m3 copy and the maxima likewise."""
+    print(f"[case] uqvk 64 rows per wave {L} {d_model} {H} {attn} {hidden} {dtype}", flush=True)
+    x, nw, nb, w, b = [t.to(dev) for t in _inputs(L + d_model, L, d_model, H, attn, hidden, dtype)]
+    whole = pkg.hstu_compute_uqvk(x, nw, nb, 1e-6, H, attn, hidden, w, b, path=2)
+    whole8 = pkg.hstu_compute_uqvk_fp8(x, nw, nb, 1e-6, H, attn, hidden, w, b, 0.01, 0.011, 0.012) if hidden * H % 128 == 0 else None
+    top = torch.zeros(3, device=dev)
+    for i in range(0, L, 8000):
+        rows = slice(i, min(i + 8000, L))
+        part = pkg.hstu_compute_uqvk(x[rows], nw, nb, 1e-6, H, attn, hidden, w, b, path=2)
+        for g_, p_ in zip(whole, part):
+            assert torch.equal(g_[rows], p_)
+        if whole8 is not None:
+            part8 = pkg.hstu_compute_uqvk_fp8(x[rows], nw, nb, 1e-6, H, attn, hidden, w, b, 0.01, 0.011, 0.012)
+            for g_, p_ in zip(whole8[:4], part8[:4]):
+                assert torch.equal(g_[rows].contiguous().view(torch.uint8), p_.contiguous().view(torch.uint8))
+            top = torch.maximum(top, part8[4])
+    torch.cuda.synchronize()
+    assert whole8 is None or torch.equal(whole8[4], top)
+
+
+@pytest.mark.gpu
 def test_uqvk_with_a_total_length_that_changes_from_batch_to_batch(pkg, dev):
     """The hipBLASLt path keeps one plan per size class of the row count, not per row count: lengths of one class
     (1100, 1101, 1279), of others (640, 5000), and the first again, each against the oracle."""
