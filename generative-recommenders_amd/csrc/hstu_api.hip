@@ -668,8 +668,10 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
         order = nullptr;
     }
 
-    // ahead of the forward kernel: sequence ranking and / or the start value of the work-item counters
-    if (order || queue) {
+    // ahead of the forward kernel: sequence ranking and / or the start value of the work-item counters; where work lists are built, the
+    // kernel that builds them does both (up to a number of sequences)
+    const bool plan_ranks = items && queue && (!order || a->batch <= hstu::kPlanRank);
+    if (!plan_ranks && (order || queue)) {
         const int blocks = order ? (a->batch + 3) / 4 : 1;
         hipLaunchKernelGGL(hstu::hstu_prep_kernel, dim3(blocks), dim3(256), 0, stream, a->seq_offsets, a->seq_offsets_i64,
                            a->batch, order, queue, grid_per_xcd);
@@ -679,13 +681,14 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
             return HSTU_ERR_LAUNCH;
         }
     }
-    p.order = order;
+    p.order = plan_ranks ? nullptr : order;  // (the lists name the sequences)
     p.queue = queue;
     if (items && queue) {
         // the lists are 32-byte records behind everything else in the workspace; align them
         items = (int*)((reinterpret_cast<uintptr_t>(items) + 31) & ~(uintptr_t)31);
         p.items_cap = (int)slots;
-        hipLaunchKernelGGL(hstu::hstu_plan_kernel, dim3(8), dim3(HSTU_PLAN_THREADS), 0, stream, p, bm, 64, queue + 8 * 16, items);
+        hipLaunchKernelGGL(hstu::hstu_plan_kernel, dim3(8), dim3(HSTU_PLAN_THREADS), 0, stream, p, bm, 64, queue + 8 * 16, items,
+                           plan_ranks && order ? 1 : 0, queue, grid_per_xcd);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) {
             set_last_error("plan kernel launch", e);

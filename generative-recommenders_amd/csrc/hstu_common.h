@@ -641,8 +641,14 @@ __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, in
 // pair heaviest block first).  Heavy-first across the whole list keeps the end of the launch made of small
 // items, items of one class and pair stay neighbours (they share K/V through the L2), and row blocks past the
 // end of short sequences never become items.  A stable counting sort: the candidate items in pair-major order
-// are cut into 256 equal runs, one per thread; count per thread and class, scan over the threads, place.
-static __global__ __launch_bounds__(HSTU_PLAN_THREADS) void hstu_plan_kernel(const FwdParams p, int bm, int bn, int* nitems, int* items) {
+// are cut into equal runs, one per thread; count per thread and class, scan over the threads, place.
+// It also gives the XCD's item counter its start value and, for `rank` (at most kPlanRank sequences), ranks the sequences by
+// length itself, as hstu_prep_kernel does: a launch before this one, which short calls notice (96 sequences of
+// 20 .. 276 rows through a layer 79.9 -> 78.4 us).  Every workgroup repeats the ranking, 16 waves
+// with a ballot per 64 others: 64 ballots each at 256 sequences, four times that at 512.
+constexpr int kPlanRank = 256;
+static __global__ __launch_bounds__(HSTU_PLAN_THREADS) void hstu_plan_kernel(const FwdParams p, int bm, int bn, int* nitems, int* items, int rank,
+                                                                             int* queue, int queue_start) {
     constexpr int NC = 12;    // classes: up to 2^11 = 2048 tiles and more
     constexpr int NT = HSTU_PLAN_THREADS, NW = NT / 64;
     constexpr int CACHE = 32768;  // candidates whose class is remembered between the two walks
@@ -651,6 +657,22 @@ static __global__ __launch_bounds__(HSTU_PLAN_THREADS) void hstu_plan_kernel(con
     __shared__ int cbase[NC];
     __shared__ signed char cls[CACHE];  // weight class of candidate k, -1 = no such row block
     const int xcd = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ long long lengths[kPlanRank];
+    __shared__ int order[kPlanRank];  // (rank) longest sequence first, ties by index
+    if (tid == 0) queue[xcd * 16] = queue_start;
+    if (rank) {
+        if (tid < p.B)
+            lengths[tid] = p.offsets_i64 ? ((const int64_t*)p.offsets)[tid + 1] - ((const int64_t*)p.offsets)[tid]
+                                         : (int64_t)(((const int*)p.offsets)[tid + 1] - ((const int*)p.offsets)[tid]);
+        __syncthreads();
+        for (int i = wave; i < p.B; i += NW) {
+            const long long ni = lengths[i];
+            int before = 0;
+            for (int j = lane; j - lane < p.B; j += 64) before += __popcll(__ballot(j < p.B && (lengths[j] > ni || (lengths[j] == ni && j < i))));
+            if (lane == 0) order[before] = i;
+        }
+        __syncthreads();
+    }
     for (int c = 0; c < NC; ++c) cnt[c][tid] = 0;
     const int num_mb = p.num_mb;
     const int total = p.pairs_per_xcd * num_mb;  // candidates: every row block a pair could have
@@ -680,7 +702,7 @@ static __global__ __launch_bounds__(HSTU_PLAN_THREADS) void hstu_plan_kernel(con
                 live = pair < p.B * p.H;
                 if (live) {
                     const int rseq = pair / p.H;
-                    b = p.order ? p.order[rseq] : rseq;
+                    b = rank ? order[rseq] : p.order ? p.order[rseq] : rseq;
                     h = pair - rseq * p.H;
                     seq_start = p.offsets_i64 ? ((const int64_t*)p.offsets)[b] : (int64_t)((const int*)p.offsets)[b];
                     const int64_t len = (p.offsets_i64 ? ((const int64_t*)p.offsets)[b + 1] : (int64_t)((const int*)p.offsets)[b + 1]) - seq_start;
