@@ -17,7 +17,9 @@
 // 139264 rows of d_model 512 into 2048 columns: 408 -> 329 us (0.89 PFLOP/s); 300000 rows into 4096 columns 1593 -> 1249 us
 // (1.01 PFLOP/s, the matrix pipe busy 56 % of the cycles; a large library product reaches 1.36).  On the way: the barrier without a
 // wait for LDS reads 347 -> 329, no branches inside a column block and column blocks in turned order (see below) 65536 rows into
-// 4096 columns 364 -> 292.  What is left: the rows' preparation, which nothing overlaps, about a fifth of the time.
+// 4096 columns 364 -> 292; the addresses of the stores computed where they are used (no spills, whose reloads wait for all
+// copies) and the e4m3 copy in halves behind the store: the 8-bit layer of 16 sequences of 4096 .. 16384 rows 1.013 -> 1.064 of its
+// former speed.  What is left: the rows' preparation, which nothing overlaps, about a fifth of the time.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -48,6 +50,7 @@ struct WideSchedule {
     static constexpr int piece(int i) { return at(3 + 11 * i / 4); }  // 16 pieces, eight per 32 rows: bias, SiLU, rounding, staging
     static constexpr int read(int i) { return at((i < 4 ? 25 : 47 - 12) + 3 * i); }  // 8: a store's rows out of the staging area
     static constexpr int store(int i) { return at((i < 4 ? 29 : 51 - 12) + 3 * i); }
+    static constexpr int convert(int i, int half) { return at((i < 4 ? 30 : 52 - 12) + 3 * i + half); }  // the e4m3 copy, behind the store
     static constexpr int stores_in(int first, int last) {
         int n = 0;
         for (int i = 0; i < 8; ++i) n += store(i) >= first && store(i) <= last;
@@ -148,17 +151,19 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         const int64_t base_row = row0 < p.rows ? row0 : p.rows - 1;
         char* const obase = p.out + base_row * p.n_out * 2;
         unsigned char* const obase8 = OUT8 ? p.out8 + base_row * (p.n_out - p.n_silu) : nullptr;
-        unsigned orow[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            int64_t r = row0 + i * 8 + rsub;
-            r = r < p.rows ? r : p.rows - 1;
-            orow[i] = (unsigned)(r - base_row);
-        }
+        const int64_t below = p.rows - 1 - base_row;
+        const int last = below < 63 ? (int)below : 63;
+        // (computed where it is used: hoisted out of the loop, the addresses of all stores take registers that the rows need)
+        auto orow = [&](int i) __attribute__((always_inline)) {
+            int r = rsub;
+            asm volatile("" : "+v"(r));
+            return (unsigned)(i * 8 + r < last ? i * 8 + r : last);
+        };
 
         f32x16_t acc[2][2][2];  // [set][row group][32 columns]
         elem4 b4[2][4];
         i32x4_t rd[8];
+        float blockmax = 0.f;  // (e4m3 output) the largest |value| of the column block in progress
         auto read_bias = [&](int c) __attribute__((always_inline)) {
             const char* b = smem + RING * kWideSlot + (c & 3) * 128 + g * 8;
 #pragma unroll
@@ -184,32 +189,37 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         auto read_rows = [&](int i) __attribute__((always_inline)) {
             rd[i] = *HSTU_LDS(const i32x4_t, stage + (i >> 2) * kWideStage + ((i & 3) * 8 + rsub) * kUqvkStageRow + chunk * 16);
         };
-        auto store_rows = [&](int i, int c, auto Silu) __attribute__((always_inline)) {
+        auto store_rows = [&](int i, int c) __attribute__((always_inline)) {
             const int col0 = col_of(c);
-            *(i32x4_t*)(obase + (int64_t)col0 * 2 + (orow[i] * (unsigned)(p.n_out * 2) + chunk * 16)) = rd[i];
-            if constexpr (OUT8 && !decltype(Silu)::value) {
-                {
-                    // the rounded values once more, scaled, as e4m3: 8 lanes cover 64 bytes of a row
-                    const int tensor = col0 < 2 * p.n_silu ? 0 : col0 < 2 * p.n_silu + p.n_attn ? 1 : 2;
-                    const vec8 e = __builtin_bit_cast(vec8, rd[i]);
-                    const float is = p.inv_scale[tensor];
-                    float f[8], m8 = 0.f;
+            *(i32x4_t*)(obase + (int64_t)col0 * 2 + (orow(i) * (unsigned)(p.n_out * 2) + chunk * 16)) = rd[i];
+        };
+        // The rounded values of store i once more, scaled, as e4m3, in two halves (a step of two MFMAs has
+        // room for about twelve vector instructions): 8 lanes cover 64 bytes of a row.
+        int half8[2];
+        auto convert8 = [&](int i, int h, int c) __attribute__((always_inline)) {
+            const int col0 = col_of(c);
+            const int tensor = col0 < 2 * p.n_silu ? 0 : col0 < 2 * p.n_silu + p.n_attn ? 1 : 2;
+            const float is = p.inv_scale[tensor];
+            const vec8 e = __builtin_bit_cast(vec8, rd[i]);
+            float f[4];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const float x = (float)e[j];
-                        m8 = __builtin_fmaxf(m8, __builtin_fabsf(x));
-                        f[j] = __builtin_fminf(__builtin_fmaxf(x * is, -448.0f), 448.0f);
-                    }
-                    amax[0] = tensor == 0 ? __builtin_fmaxf(amax[0], m8) : amax[0];
-                    amax[1] = tensor == 1 ? __builtin_fmaxf(amax[1], m8) : amax[1];
-                    amax[2] = tensor == 2 ? __builtin_fmaxf(amax[2], m8) : amax[2];
-                    int lo = 0, hi = 0;
-                    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
-                    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
-                    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
-                    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
-                    typedef __attribute__((ext_vector_type(2))) int i32x2_t;
-                    *(i32x2_t*)(obase8 + (col0 - p.n_silu) + (orow[i] * (unsigned)(p.n_out - p.n_silu) + chunk * 8)) = i32x2_t{lo, hi};
+            for (int j = 0; j < 4; ++j) {
+                const float x = (float)e[4 * h + j];
+                blockmax = __builtin_fmaxf(blockmax, __builtin_fabsf(x));
+                f[j] = __builtin_fminf(__builtin_fmaxf(x * is, -448.0f), 448.0f);
+            }
+            int v = 0;
+            v = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], v, false);
+            v = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], v, true);
+            half8[h] = v;
+            if (h == 1) {
+                typedef __attribute__((ext_vector_type(2))) int i32x2_t;
+                *(i32x2_t*)(obase8 + (col0 - p.n_silu) + (orow(i) * (unsigned)(p.n_out - p.n_silu) + chunk * 8)) = i32x2_t{half8[0], half8[1]};
+                if (i == 7) {
+                    amax[0] = tensor == 0 ? __builtin_fmaxf(amax[0], blockmax) : amax[0];
+                    amax[1] = tensor == 1 ? __builtin_fmaxf(amax[1], blockmax) : amax[1];
+                    amax[2] = tensor == 2 ? __builtin_fmaxf(amax[2], blockmax) : amax[2];
+                    blockmax = 0.f;
                 }
             }
         };
@@ -262,7 +272,14 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
                             if (Plan::read(i) == s) read_rows(i);
 #pragma unroll
                         for (int i = 0; i < 8; ++i)
-                            if (Plan::store(i) == s) store_rows(i, c - 1, Silu);
+                            if (Plan::store(i) == s) store_rows(i, c - 1);
+                        if constexpr (OUT8 && !decltype(Silu)::value) {
+#pragma unroll
+                            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                                for (int h = 0; h < 2; ++h)
+                                    if (Plan::convert(i, h) == s) convert8(i, h, c - 1);
+                        }
                     }
                     if (m < 12 && m % 3 == 1) issue(c + 1, kt, prev2, m / 3);
                 }
@@ -277,7 +294,10 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
 #pragma unroll
             for (int i = 0; i < 8; ++i) read_rows(i);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) store_rows(i, c, Silu);
+            for (int i = 0; i < 8; ++i) {
+                store_rows(i, c);
+                if constexpr (OUT8 && !decltype(Silu)::value) convert8(i, 0, c), convert8(i, 1, c);
+            }
         };
 
         auto next_block = [&](f32x16_t(&now)[2][2], const f32x16_t(&before)[2][2], int c) __attribute__((always_inline)) {
