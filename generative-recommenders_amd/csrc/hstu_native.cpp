@@ -168,6 +168,7 @@ struct MhaFunction : torch::autograd::Function<MhaFunction> {
         return out;
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
         const auto saved = ctx->get_saved_variables();
         Tensor q = saved[0], k = saved[1], v = saved[2];
         const OptTensor targets = saved[4].defined() ? OptTensor(saved[4]) : OptTensor();
@@ -403,6 +404,7 @@ struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
         return {u, q, k, v};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
         const auto saved = ctx->get_saved_variables();
         const auto i = ctx->saved_data["shape"].toIntVector();
         const UqvkShape s{i[0], i[1], i[2]};
@@ -436,6 +438,7 @@ struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
         return {u, out, k, v};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
         const auto saved = ctx->get_saved_variables();
         const auto i = ctx->saved_data["shape"].toIntVector();
         const UqvkShape s{i[0], i[1], i[2]};
@@ -538,12 +541,13 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
         return out;
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
         const auto saved = ctx->get_saved_variables();
         const Tensor &attn = saved[0], &u = saved[1], &norm_weight = saved[2], &norm_bias = saved[3], &weight = saved[4];
         const auto i = ctx->saved_data["sizes"].toIntVector();
         const auto f = ctx->saved_data["floats"].toDoubleVector();
         const OutputCall c{i[0], i[1], i[2], 0, i[3] != 0, i[4] != 0, i[5] != 0, f[0], f[1], (uint64_t)i[6], (uint64_t)i[7]};
-        const Tensor dout = grads[0].contiguous();
+        const Tensor dout = grads[0].detach().contiguous();
         const int64_t rows = attn.size(0), width = attn.size(1);
         variable_list got(7);
         got[2] = dout;  // the residual

@@ -157,3 +157,25 @@ def test_weight_gradient_kernel(dev, dtype, rows, m, n, sliced):
     for got, want in ((out, a.double().t() @ b.double()), (sums, b.double().sum(0))):
         assert torch.isfinite(got).all()
         assert float((got.double() - want).norm() / want.norm()) <= 1.1 * unit
+
+
+def test_gradients_under_create_graph_are_the_plain_ones_without_a_graph(pkg, dev):
+    """The backward kernels are not differentiable: with ``create_graph`` the gradients are those of the plain call and carry no
+    graph, not part of one."""
+    print("[case] gradients with create_graph", flush=True)
+    g = torch.Generator(device=dev).manual_seed(5)
+    H, D, d, L = 2, 64, 128, 90
+    shapes = ((L, d), (d,), (d,), (d, 4 * H * D), (4 * H * D,), (H * D,), (H * D,), (3 * H * D, d))
+    ins = [(0.1 * torch.randn(s, generator=g, device=dev)).bfloat16().requires_grad_() for s in shapes]
+    offsets = torch.tensor([0, 30, 90], device=dev)
+    d_out = torch.randn((L, d), generator=g, device=dev).bfloat16().requires_grad_()
+
+    def layer(x, nw, nb, w, b, onw, onb, ow):
+        u, attn, _, _ = pkg.hstu_preprocess_and_attention(x, nw, nb, 1e-6, H, D, D, w, b, 60, offsets, D**-0.5, True, None, 0, 0, True, True, False)
+        return pkg.hstu_compute_output(attn, u, x, onw, onb, 1e-6, ow, H, D, 0.0, True, True, True, "none", False, True)
+
+    plain = torch.autograd.grad(layer(*ins), ins, d_out.detach())
+    graph = torch.autograd.grad(layer(*ins), ins, d_out, create_graph=True)
+    torch.cuda.synchronize()
+    for a, b in zip(plain, graph):
+        assert torch.equal(a, b) and not b.requires_grad
