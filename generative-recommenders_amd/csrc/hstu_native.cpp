@@ -348,6 +348,9 @@ Tensor uqvk_buffer(const Tensor& x, const Tensor& norm_weight, const Tensor& nor
     return buf;
 }
 
+// what the weight gradient takes: result columns (wider ones get their gradients from the Python operator)
+constexpr int64_t kWeightGradColumns = 65536;
+
 void check_linear(int rc) { TORCH_CHECK(rc == 0, "hstu_linear: status ", rc, " (", hstu_linear_last_error(), ")"); }
 
 // a^T @ b, and the column sums of b where `b_sums` is defined.
@@ -472,6 +475,7 @@ std::optional<FourTensors> compute_uqvk(const Tensor& x, const Tensor& norm_weig
     if (!uqvk_operands(x, norm_weight, norm_bias, weight, bias, s)) return {};
     try {
         if (wants_grad({&x, &norm_weight, &norm_bias, &weight, &bias})) {
+            if (s.n_out() > kWeightGradColumns) return {};
             const variable_list o = UqvkFunction::apply(x, norm_weight, norm_bias, weight, bias, eps, s, path);
             return FourTensors(o[0], o[1], o[2], o[3]);
         }
@@ -487,7 +491,7 @@ std::optional<FourTensors> preprocess_and_attention(const Tensor& x, const Tenso
                                                     const Tensor& offsets, double alpha, const OptTensor& targets, int64_t w, int64_t c, bool sort) {
     const UqvkShape s{heads, attn, hidden};
     if (max_seq_len <= 0 || !wants_grad({&x, &norm_weight, &norm_bias, &weight, &bias})) return {};
-    if (!uqvk_operands(x, norm_weight, norm_bias, weight, bias, s)) return {};
+    if (!uqvk_operands(x, norm_weight, norm_bias, weight, bias, s) || s.n_out() > kWeightGradColumns) return {};
     const AttentionCall call{max_seq_len, 0, w, c, 0, alpha, 1.0, 1.0, 1.0, 0, 0, sort};
     RECORD_USER_SCOPE("hstu_preprocess_and_attention");
     try {
@@ -586,9 +590,10 @@ OptTensor compute_output(const Tensor& attn, const Tensor& u, const Tensor& x, c
     if (norm_weight.dim() != 1 || norm_weight.size(0) != norm || norm_bias.dim() != 1 || norm_bias.size(0) != norm) return {};
     if (weight.dim() != 2 || weight.size(0) != c.blocks() * width || weight.size(1) != x.size(1)) return {};
     if (!parameter(norm_weight, x) || !parameter(norm_bias, x) || !parameter(weight, x)) return {};
+    const bool grad = wants_grad({&attn, &u, &x, &norm_weight, &norm_bias, &weight});
+    if (grad && x.size(1) > kWeightGradColumns) return {};
     try {
-        return wants_grad({&attn, &u, &x, &norm_weight, &norm_bias, &weight})
-                   ? OutputFunction::apply(attn, u, x, norm_weight, norm_bias, weight, c)
+        return grad ? OutputFunction::apply(attn, u, x, norm_weight, norm_bias, weight, c)
                    : output_result(attn, u, x, norm_weight, norm_bias, weight, c);
     } catch (const Declined&) {
         return {};

@@ -102,9 +102,10 @@ def test_output_step_gradients_against_the_recomputation(dev, rows, heads, dim, 
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("rows,d,heads,attn,hidden", [(1, 64, 1, 16, 16), (4101, 128, 2, 32, 64), (63, 1024, 1, 64, 64), (20, 4096, 1, 8, 8), (300, 520, 3, 16, 8)])
+@pytest.mark.parametrize("rows,d,heads,attn,hidden", [(1, 64, 1, 16, 16), (4101, 128, 2, 32, 64), (63, 1024, 1, 64, 64), (20, 4096, 1, 8, 8), (300, 520, 3, 16, 8), (3, 64, 1, 32768, 16)])
 def test_producer_gradients_against_the_recomputation(dev, dtype, rows, d, heads, attn, hidden):
-    """Layer-norm and SiLU backward kernels, at widths up to the widest row and with rows past the waves of the grid."""
+    """Layer-norm and SiLU backward kernels, at widths up to the widest row, with rows past the waves of the grid, and at more columns
+    than the weight gradient takes."""
     from generative_recommenders_amd.ops import hstu_compute as hc
 
     print(f"[case] producer gradients {rows} {d} {heads} {attn} {hidden} {dtype}", flush=True)
