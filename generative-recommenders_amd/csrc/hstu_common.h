@@ -601,10 +601,14 @@ __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, in
     }
     const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(tiles), 63);
     const int mean = (int)(((unsigned)total + (unsigned)p.fit_runs - 1) / (unsigned)p.fit_runs);
-    // (an approximate quotient serves as well as the exact one: every workgroup computes the same)
+    // (An approximate quotient serves as well as the exact one: every workgroup computes the same.  But a sequence of one tile has
+    // one run also where tau * (1 / tau) rounds below 1, and must count as one here, or the runs exceed the workgroups.)
     const int tau = mean + lane * ((mean + 62) / 63);
     const float inv = __builtin_amdgcn_rcpf((float)tau);
-    auto runs_of = [](int t, int tau, float inv) { return (int)((float)(t + tau - 1) * inv); };
+    auto runs_of = [](int t, int tau, float inv) {
+        const int r = (int)((float)(t + tau - 1) * inv);
+        return t <= 0 ? 0 : r < 1 ? 1 : r > t ? t : r;
+    };
     int need = 0;
     for (int b = 0; b < p.B; ++b) need += runs_of(__builtin_amdgcn_readlane(tiles, b), tau, inv);
     const uint64_t enough = __ballot(need <= p.fit_runs && tau > 0);
@@ -612,8 +616,7 @@ __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, in
     const int best = __builtin_ctzll(enough);
     const int tau_b = __builtin_amdgcn_readlane(tau, best);
     const float inv_b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv), best));
-    int runs = runs_of(tiles, tau_b, inv_b);
-    runs = tiles > 0 && runs < 1 ? 1 : runs > tiles ? tiles : runs;
+    const int runs = runs_of(tiles, tau_b, inv_b);
     const int upto = wave_inclusive_scan(runs);
     const int b = __popcll(__ballot(upto <= i));
     if (b >= p.B) return false;  // more workgroups than runs

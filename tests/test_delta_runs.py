@@ -16,6 +16,8 @@ CASES = [
     ([2000, 100, 64, 1037, 700], 64, 3, 128),            # tile multiples, heads that do not divide the XCDs
     ([5000, 300], 300, 1, 128),                          # row blocks of 128 and of 256 with a part over
     ([6000, 40, 3513] + [65] * 61, 33, 1, 64),           # 64 sequences (every lane), most of them one or two tiles
+    # one tile among long histories, whose longest runs are 41 tiles (41 * (1 / 41) is below 1 in fp32): not a run more than workgroups
+    ([204 * 64 - 5, 164 * 64 - 3] * 3 + [204 * 64, 40], 16, 8, 32),
 ]
 
 
