@@ -290,7 +290,7 @@ def run_linear(name, args, pkg, torch):
         cpu = None
         flops = 2.0 * L * d_model * n_out + workloads.algorithmic_flops(wl)
         nbytes = 2.0 * (L * d_model + d_model * n_out + L * n_out) + 1.0 * L * 3 * H * D + 2.0 * L * H * D
-        kernel = "hstu_uqvk_fused_kernel (e4m3 epilogue) + hstu_fwd_stream_kernel (fp8)"
+        kernel = "hstu_uqvk_wide_kernel (e4m3 epilogue) + hstu_fwd_stream_kernel (fp8)"
         metric = "fused q/k/v producer -> fp8 attention, TFLOP/s (cfg5: 16 sequences of 4096..16384, H8 d128, d_model 512)"
     elif name == "layer":
         # one STU layer forward on the headline batch (64 sequences of 8192): hstu_preprocess_and_attention, then
@@ -313,7 +313,7 @@ def run_linear(name, args, pkg, torch):
         attn_flops = workloads.algorithmic_flops(wl)
         flops = 2.0 * L * d_model * n_out + attn_flops + 2.0 * L * 3 * H * D * d_model
         nbytes = 2.0 * (L * d_model * 3 + d_model * n_out + 3 * H * D * d_model)  # x in (twice: the residual), out
-        kernel = "hstu_uqvk_fused_kernel + hstu_fwd_stream_kernel + hstu_norm_mul_kernel + hstu_output_gemm_kernel"
+        kernel = "hstu_uqvk_wide_kernel + hstu_fwd_stream_kernel + hstu_norm_mul_kernel + hstu_output_gemm_kernel"
         metric = "STU layer fwd TFLOP/s (uqvk, attention, output; 64 x 8192 tokens, d_model 512, H4 d128)"
     elif name in ("uqvk", "layernorm"):
         nw, nb = rnd(d_model, scale=0.1, shift=1.0), rnd(d_model, scale=0.1)
@@ -323,7 +323,7 @@ def run_linear(name, args, pkg, torch):
             cpu = lambda r: uqvk_oracle.compute_uqvk(x[:r].float().cpu(), nw.float().cpu(), nb.float().cpu(), 1e-6, H, D, D, w.float().cpu(), b.float().cpu())  # noqa: E731
             flops, nbytes = 2.0 * L * d_model * n_out, 2.0 * (L * d_model + d_model * n_out + L * n_out)
             kernel = ("hstu_layer_norm_kernel + 2 hipBLASLt GEMMs (bias, bias + SiLU epilogues)" if args.uqvk_path == 1
-                      else "hstu_uqvk_fused_kernel")
+                      else "hstu_uqvk_wide_kernel")
             metric = "hstu_compute_uqvk fwd TFLOP/s (524288 tokens, d_model 512 -> 2048)"
         else:
             step = lambda: hstu_compute.layer_norm(x, nw, nb, 1e-6)  # noqa: E731
