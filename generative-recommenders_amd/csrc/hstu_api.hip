@@ -595,24 +595,29 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
         const char** dst[3] = {&p.q, &p.k, &p.v};
         int64_t* prs[3] = {&p.q_rs, &p.k_rs, &p.v_rs};
         int64_t* phs[3] = {&p.q_hs, &p.k_hs, &p.v_hs};
+        hstu::CastParams cast{};
+        cast.H = a->heads;
+        long long blocks = 0;
         for (int i = 0; i < 3; ++i) {
             cur = (char*)((reinterpret_cast<uintptr_t>(cur) + 255) & ~(uintptr_t)255);
             const long long threads = (long long)rows[i] * a->heads * (d[i] / 8);
-            const long long blocks = (threads + 255) / 256;
+            cast.src[i] = (const float*)src[i], cast.dst[i] = (_Float16*)cur;
+            cast.rs[i] = rs[i], cast.hs[i] = hs[i], cast.rows[i] = rows[i], cast.d[i] = d[i];
+            cast.first[i] = (unsigned)blocks;
+            blocks += (threads + 255) / 256;
             if (blocks > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
-            if (blocks > 0) {
-                hipLaunchKernelGGL(hstu::hstu_cast_f32_f16_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (const float*)src[i],
-                                   rs[i], hs[i], rows[i], a->heads, d[i], (_Float16*)cur);
-                hipError_t e = hipGetLastError();
-                if (e != hipSuccess) {
-                    set_last_error("cast kernel launch", e);
-                    return HSTU_ERR_LAUNCH;
-                }
-            }
             *dst[i] = cur;
             *prs[i] = (int64_t)a->heads * d[i];
             *phs[i] = d[i];
             cur += (size_t)rows[i] * a->heads * d[i] * 2;
+        }
+        if (blocks > 0) {
+            hipLaunchKernelGGL(hstu::hstu_cast_f32_f16_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, cast);
+            hipError_t e = hipGetLastError();
+            if (e != hipSuccess) {
+                set_last_error("cast kernel launch", e);
+                return HSTU_ERR_LAUNCH;
+            }
         }
     }
     if (plan.splits > 1 && !ws_ok) {

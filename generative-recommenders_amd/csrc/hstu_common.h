@@ -1001,10 +1001,22 @@ __device__ __forceinline__ void store_output(const f32x16_t (&oacc)[DT][QT], int
         }
 }
 
-// dst[row][h][0..d) (dense, fp16) = src[row * rs + h * hs + 0..d) (fp32, strides in elements); 8 elements per thread.
-static __global__ __launch_bounds__(256) void hstu_cast_f32_f16_kernel(const float* src, int64_t rs, int64_t hs, int64_t rows, int H,
-                                                                int d, _Float16* dst) {
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over rows * H * d / 8
+// q, k, v: dst[row][h][0..d) (dense, fp16) = src[row * rs + h * hs + 0..d) (fp32, strides in elements); 8 elements per thread,
+// the workgroups of k and v behind those of q.  One launch for the three: a small call pays 4 us for each, whatever it copies.
+struct CastParams {
+    const float* src[3];
+    _Float16* dst[3];
+    int64_t rs[3], hs[3], rows[3];
+    int d[3];
+    unsigned first[3];  // first workgroup of the operand
+    int H;
+};
+static __global__ __launch_bounds__(256) void hstu_cast_f32_f16_kernel(const CastParams p) {
+    const int which = blockIdx.x >= p.first[2] ? 2 : blockIdx.x >= p.first[1] ? 1 : 0, d = p.d[which], H = p.H;
+    const float* src = p.src[which];
+    _Float16* dst = p.dst[which];
+    const int64_t rs = p.rs[which], hs = p.hs[which], rows = p.rows[which];
+    const int64_t idx = (int64_t)(blockIdx.x - p.first[which]) * 256 + threadIdx.x;  // over rows * H * d / 8
     const int d8 = d >> 3;
     if (idx >= rows * H * d8) return;
     const int c = (int)(idx % d8);
