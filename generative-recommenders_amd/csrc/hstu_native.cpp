@@ -554,7 +554,9 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
         const Tensor dout = grads[0].detach().contiguous();
         const int64_t rows = attn.size(0), width = attn.size(1);
         variable_list got(7);
-        got[2] = dout;  // the residual
+        // The residual: the tensor that came in, for a leaf's accumulation to see that others hold it too and copy it.  (Another
+        // tensor on the same memory would be taken over, and the next gradient added into the caller's.)
+        got[2] = grads[0].requires_grad() ? grads[0].clone() : grads[0];
         const bool weight_too = ctx->needs_input_grad(5);
         if (weight_too || ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4)) {
             const Tensor dj = at::mm(dout, weight.t());

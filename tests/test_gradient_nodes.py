@@ -1,0 +1,64 @@
+"""The autograd nodes of the operators' native front: what they hand back to autograd and what they take from it."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hc():
+    from generative_recommenders_amd.ops import hstu_compute
+
+    return hstu_compute
+
+
+H, D, D_MODEL = 2, 64, 128
+N_OUT = 4 * H * D
+
+
+def _rand(dev, seed, shapes, dtype=torch.bfloat16):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return [torch.randn(s, generator=g, device=dev).to(dtype) for s in shapes]
+
+
+def _output_inputs(dev, rows, dtype=torch.bfloat16):
+    """attn, u, x, norm weight, norm bias, weight"""
+    return _rand(dev, rows, ((rows, H * D), (rows, H * D), (rows, D_MODEL), (H * D,), (H * D,), (3 * H * D, D_MODEL)), dtype)
+
+
+def _output(hc, attn, u, x, nw, nb, w):
+    return hc.hstu_compute_output(attn, u, x, nw, nb, 1e-6, w, H, D, 0.0, True, True, True, "none", False, True)
+
+
+def _producer_inputs(dev, rows, dtype=torch.bfloat16):
+    """x, norm weight, norm bias, weight, bias"""
+    ins = _rand(dev, rows + 1, ((rows, D_MODEL), (D_MODEL,), (D_MODEL,), (D_MODEL, N_OUT), (N_OUT,)), dtype)
+    ins[3] = ins[3] / D_MODEL**0.5
+    return ins
+
+
+def _producer(hc, x, nw, nb, w, b):
+    return hc.hstu_compute_uqvk(x, nw, nb, 1e-6, H, D, D, w, b)
+
+
+def _first_half(hc, dev, x, nw, nb, w, b):
+    """(u, attention output, k, v) of one sequence"""
+    offsets = torch.tensor([0, x.shape[0]], device=dev)
+    return hc.hstu_preprocess_and_attention(x, nw, nb, 1e-6, H, D, D, w, b, x.shape[0], offsets, D**-0.5, True, None, 0, 0, True, True, False)
+
+
+def _leaves(tensors):
+    return [t.detach().clone().requires_grad_() for t in tensors]
+
+
+def test_the_residuals_gradient_is_not_the_callers_tensor(dev, hc):
+    """Autograd adds later gradients to a leaf's first one in place: it must not share the memory of the gradient that came in."""
+    print("[case] residual gradient of a leaf", flush=True)
+    attn, u, x, nw, nb, w = _output_inputs(dev, 40)
+    x.requires_grad_()
+    d_out = torch.ones_like(x)
+    for _ in range(3):
+        _output(hc, attn, u, x, nw, nb, w).backward(d_out)
+    torch.cuda.synchronize()
+    assert (d_out == 1).all() and (x.grad == 3).all()
