@@ -29,6 +29,13 @@ using OptTensor = std::optional<Tensor>;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
+// Every backward node runs in one.  No graph, with create_graph too: the kernels' gradients are not differentiable.  And no autocast: the
+// kernels read a product as the inputs' type, which autocast to another one would change.
+struct BackwardScope {
+    torch::NoGradGuard no_graph;
+    c10::impl::ExcludeDispatchKeyGuard no_autocast{c10::autocast_dispatch_keyset};
+};
+
 struct Declined {};  // thrown where a call turns out, on the way, to be the Python operator's
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
@@ -168,7 +175,7 @@ struct MhaFunction : torch::autograd::Function<MhaFunction> {
         return out;
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
+        const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
         Tensor q = saved[0], k = saved[1], v = saved[2];
         const OptTensor targets = saved[4].defined() ? OptTensor(saved[4]) : OptTensor();
@@ -407,7 +414,7 @@ struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
         return {u, q, k, v};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
+        const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
         const auto i = ctx->saved_data["shape"].toIntVector();
         const UqvkShape s{i[0], i[1], i[2]};
@@ -441,7 +448,7 @@ struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
         return {u, out, k, v};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
+        const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
         const auto i = ctx->saved_data["shape"].toIntVector();
         const UqvkShape s{i[0], i[1], i[2]};
@@ -545,7 +552,7 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
         return out;
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-        const torch::NoGradGuard no_graph;  // (with create_graph too: the kernels' gradients are not differentiable)
+        const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
         const Tensor &attn = saved[0], &u = saved[1], &norm_weight = saved[2], &norm_bias = saved[3], &weight = saved[4];
         const auto i = ctx->saved_data["sizes"].toIntVector();

@@ -62,3 +62,23 @@ def test_the_residuals_gradient_is_not_the_callers_tensor(dev, hc):
         _output(hc, attn, u, x, nw, nb, w).backward(d_out)
     torch.cuda.synchronize()
     assert (d_out == 1).all() and (x.grad == 3).all()
+
+
+@pytest.mark.parametrize("dtype,other", [(torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)])
+def test_backward_inside_autocast_of_the_other_type(dev, hc, dtype, other):
+    """The nodes' products are of the inputs' type whatever autocast would make of them: the kernels read that type."""
+    print(f"[case] backward of {dtype} under autocast to {other}", flush=True)
+    ins = _leaves([0.1 * t for t in _producer_inputs(dev, 50, dtype) + _output_inputs(dev, 50, dtype)[3:]])
+
+    def layer():
+        u, attn, _, _ = _first_half(hc, dev, *ins[:5])
+        return _output(hc, attn, u, ins[0], *ins[5:])
+
+    (d_out,) = _rand(dev, 9, ((50, D_MODEL),), dtype)
+    want = torch.autograd.grad(layer(), ins, d_out) + torch.autograd.grad(_producer(hc, *ins[:5])[0], ins[:5], d_out)
+    first, second = layer(), _producer(hc, *ins[:5])[0]
+    with torch.autocast("cuda", dtype=other):
+        got = torch.autograd.grad(first, ins, d_out) + torch.autograd.grad(second, ins[:5], d_out)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype and torch.equal(a, b)
