@@ -303,6 +303,13 @@ bool matrix_rows(const Tensor& t) {
     return t.dim() == 2 && t.is_cuda() && t.size(0) > 0 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && aligned16(t);
 }
 
+// An incoming gradient as the kernels read it.  (contiguous() is no help: a view of a flat gradient at an odd offset and a single
+// row of any row stride are contiguous.)
+Tensor gradient_rows(const Tensor& t) { return matrix_rows(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+Tensor dense_gradient(const Tensor& t) {
+    return t.stride(1) == 1 && t.stride(0) == t.size(1) && aligned16(t) ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 Tensor aligned_scratch(size_t bytes, const Tensor& like, void** ptr) {
     Tensor t = at::empty({(int64_t)bytes + 256}, like.options().dtype(at::kByte));
     *ptr = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(t.data_ptr()) + 255) & ~(uintptr_t)255);
@@ -383,7 +390,7 @@ variable_list uqvk_backward(const Tensor& x, const Tensor& norm_weight, const Te
                                       normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
     Tensor d_u = d.narrow(1, 0, n_u);
     if (du.defined()) {
-        if (!matrix_rows(du)) du = du.contiguous();
+        du = gradient_rows(du);
         at::mm_out(d_u, normed, weight.narrow(1, 0, n_u));
         check_linear(hstu_uqvk_silu_bwd(d_u.data_ptr(), d_u.stride(0), bias.const_data_ptr(), du.const_data_ptr(), du.stride(0), rows, n_u,
                                         dense_dtype(x), stream));
@@ -558,7 +565,7 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
         const auto i = ctx->saved_data["sizes"].toIntVector();
         const auto f = ctx->saved_data["floats"].toDoubleVector();
         const OutputCall c{i[0], i[1], i[2], 0, i[3] != 0, i[4] != 0, i[5] != 0, f[0], f[1], (uint64_t)i[6], (uint64_t)i[7]};
-        const Tensor dout = grads[0].detach().contiguous();
+        const Tensor dout = dense_gradient(grads[0]);
         const int64_t rows = attn.size(0), width = attn.size(1);
         variable_list got(7);
         // The residual: the tensor that came in, for a leaf's accumulation to see that others hold it too and copy it.  (Another

@@ -82,3 +82,37 @@ def test_backward_inside_autocast_of_the_other_type(dev, hc, dtype, other):
     torch.cuda.synchronize()
     for a, b in zip(got, want):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+def _odd_offset(t):
+    """The same values, contiguous, two bytes past a 16-byte boundary."""
+    return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+
+def _one_row_of_a_wider_buffer(t):
+    """The same values; strides that count as contiguous although the row stride is odd, and for the last form below the row's width."""
+    return t.as_strided(t.shape, (t.shape[1] + 5, 1))
+
+
+def _one_row_overlapping(t):
+    return t.as_strided(t.shape, (1, 1))
+
+
+@pytest.mark.parametrize("rows,layout", [(40, _odd_offset), (1, _odd_offset), (1, _one_row_of_a_wider_buffer), (1, _one_row_overlapping)])
+def test_gradients_that_are_not_as_the_kernels_read_rows(dev, hc, rows, layout):
+    """Slices of a flat gradient and single rows of wider ones, for the output step and for u: the result of a dense copy."""
+    print(f"[case] gradient layout {rows} {layout.__name__}", flush=True)
+    out_ins, ins = _leaves(_output_inputs(dev, rows)), _leaves(_producer_inputs(dev, rows))
+    d_out, du = _rand(dev, 4, ((rows, D_MODEL), (rows, H * D)))
+    calls = (
+        (lambda: _output(hc, *out_ins), out_ins, d_out),
+        (lambda: _producer(hc, *ins)[0], ins, du),
+        (lambda: _first_half(hc, dev, *ins)[0], ins, du),
+        (lambda: _first_half(hc, dev, *ins)[1], ins, du),
+    )
+    for fn, tensors, d in calls:
+        want = torch.autograd.grad(fn(), tensors, d)
+        got = torch.autograd.grad(fn(), tensors, layout(d))
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
