@@ -177,8 +177,8 @@ struct MhaFunction : torch::autograd::Function<MhaFunction> {
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
-        Tensor q = saved[0], k = saved[1], v = saved[2];
-        const OptTensor targets = saved[4].defined() ? OptTensor(saved[4]) : OptTensor();
+        Tensor q = kernel_rows(saved[0]), k = kernel_rows(saved[1]), v = kernel_rows(saved[2]);
+        const OptTensor targets = saved[4].defined() ? OptTensor(saved[4].contiguous()) : OptTensor();
         const auto ws = ctx->saved_data.find("workspace");
         const OptTensor workspace = ws == ctx->saved_data.end() ? OptTensor() : OptTensor(ws->second.toTensor());
         // fp32 inputs: the backward kernels take 16-bit operands, so they run on bf16 copies (fp32's range: dout can be tiny) and
@@ -188,7 +188,7 @@ struct MhaFunction : torch::autograd::Function<MhaFunction> {
         const Tensor dout = kernel_rows(grads[0].to(q.scalar_type()));
         Tensor dq = at::empty_like(q, at::MemoryFormat::Contiguous), dk = at::empty_like(k, at::MemoryFormat::Contiguous),
                dv = at::empty_like(v, at::MemoryFormat::Contiguous);
-        attention_backward(dout, q, k, v, dq, dk, dv, saved[3], targets,
+        attention_backward(dout, q, k, v, dq, dk, dv, saved[3].contiguous(), targets,
                            unpack(ctx->saved_data["call"].toIntVector(), ctx->saved_data["alpha"].toDouble()), workspace);
         if (wide) dq = dq.to(at::kFloat), dk = dk.to(at::kFloat), dv = dv.to(at::kFloat);
         return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
@@ -309,6 +309,10 @@ Tensor gradient_rows(const Tensor& t) { return matrix_rows(t) ? t : t.clone(at::
 Tensor dense_gradient(const Tensor& t) {
     return t.stride(1) == 1 && t.stride(0) == t.size(1) && aligned16(t) ? t : t.clone(at::MemoryFormat::Contiguous);
 }
+
+// Saved tensors as the kernels read them: what saved-tensor hooks give back has the values of what was saved, in any layout.
+Tensor saved_rows(const Tensor& t) { return gradient_rows(t); }
+Tensor saved_dense(const Tensor& t) { return t.is_contiguous() && aligned16(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
 
 Tensor aligned_scratch(size_t bytes, const Tensor& like, void** ptr) {
     Tensor t = at::empty({(int64_t)bytes + 256}, like.options().dtype(at::kByte));
@@ -431,7 +435,8 @@ struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
         put(std::get<1>(views), grads[1]);
         put(std::get<2>(views), grads[2]);
         put(std::get<3>(views), grads[3]);
-        variable_list got = uqvk_backward(saved[0], saved[1], saved[2], saved[3], saved[4], ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
+        variable_list got = uqvk_backward(saved_rows(saved[0]), saved_dense(saved[1]), saved_dense(saved[2]), saved_dense(saved[3]),
+                                          saved_dense(saved[4]), ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
         got.resize(8);
         return got;
     }
@@ -459,14 +464,14 @@ struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
         const auto saved = ctx->get_saved_variables();
         const auto i = ctx->saved_data["shape"].toIntVector();
         const UqvkShape s{i[0], i[1], i[2]};
-        const Tensor& x = saved[0];
-        const OptTensor targets = saved[6].defined() ? OptTensor(saved[6]) : OptTensor();
+        const Tensor x = saved_rows(saved[0]), offsets = saved[5].contiguous(), buf = saved_dense(saved[7]);
+        const OptTensor targets = saved[6].defined() ? OptTensor(saved[6].contiguous()) : OptTensor();
         Tensor d = at::empty({x.size(0), s.n_out()}, x.options());
-        const auto grad = uqvk_views(d, s.heads, s.attn, s.hidden), value = uqvk_views(saved[7], s.heads, s.attn, s.hidden);
+        const auto grad = uqvk_views(d, s.heads, s.attn, s.hidden), value = uqvk_views(buf, s.heads, s.attn, s.hidden);
         const Tensor &dq = std::get<1>(grad), &dk = std::get<2>(grad), &dv = std::get<3>(grad);
         if (grads[1].defined()) {
             const Tensor dout = kernel_rows(grads[1].reshape({x.size(0), s.heads, s.hidden}));
-            attention_backward(dout, std::get<1>(value), std::get<2>(value), std::get<3>(value), dq, dk, dv, saved[5], targets,
+            attention_backward(dout, std::get<1>(value), std::get<2>(value), std::get<3>(value), dq, dk, dv, offsets, targets,
                                unpack(ctx->saved_data["call"].toIntVector(), ctx->saved_data["alpha"].toDouble()), {});
             if (grads[2].defined()) dk.add_(grads[2]);
             if (grads[3].defined()) dv.add_(grads[3]);
@@ -475,7 +480,8 @@ struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
             grads[2].defined() ? dk.copy_(grads[2]) : dk.zero_();
             grads[3].defined() ? dv.copy_(grads[3]) : dv.zero_();
         }
-        variable_list got = uqvk_backward(x, saved[1], saved[2], saved[3], saved[4], ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
+        variable_list got = uqvk_backward(x, saved_dense(saved[1]), saved_dense(saved[2]), saved_dense(saved[3]), saved_dense(saved[4]),
+                                          ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
         got.resize(10);
         return got;
     }
@@ -561,7 +567,8 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
-        const Tensor &attn = saved[0], &u = saved[1], &norm_weight = saved[2], &norm_bias = saved[3], &weight = saved[4];
+        const Tensor attn = saved_rows(saved[0]), u = saved_rows(saved[1]), norm_weight = saved_dense(saved[2]), norm_bias = saved_dense(saved[3]),
+                     weight = saved_dense(saved[4]);
         const auto i = ctx->saved_data["sizes"].toIntVector();
         const auto f = ctx->saved_data["floats"].toDoubleVector();
         const OutputCall c{i[0], i[1], i[2], 0, i[3] != 0, i[4] != 0, i[5] != 0, f[0], f[1], (uint64_t)i[6], (uint64_t)i[7]};

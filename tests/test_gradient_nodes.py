@@ -116,3 +116,23 @@ def test_gradients_that_are_not_as_the_kernels_read_rows(dev, hc, rows, layout):
         torch.cuda.synchronize()
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+def test_saved_tensors_that_come_back_in_another_layout(dev, hc):
+    """What saved-tensor hooks give back (from a flat store, say) has the values, not the alignment, of what was saved."""
+    print("[case] saved tensors at odd offsets", flush=True)
+    out_ins, ins = _leaves(_output_inputs(dev, 40)), _leaves(_producer_inputs(dev, 40))
+    d_out, du = _rand(dev, 4, ((40, D_MODEL), (40, H * D)))
+    calls = (
+        (lambda: _output(hc, *out_ins), out_ins, d_out),
+        (lambda: _producer(hc, *ins)[0], ins, du),
+        (lambda: _first_half(hc, dev, *ins)[1], ins, du),
+    )
+    for fn, tensors, d in calls:
+        want = torch.autograd.grad(fn(), tensors, d)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), lambda t: _odd_offset(t) if t.is_floating_point() else t):
+            out = fn()
+        got = torch.autograd.grad(out, tensors, d)
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
