@@ -382,16 +382,23 @@ Tensor weight_grad(const Tensor& a, const Tensor& b, const Tensor& b_sums) {
     return out;
 }
 
-// Gradients of x, norm_weight, norm_bias, weight, bias from `d`, the gradient of the producer's buffer u | v | q | k: its v, q and k
-// columns are filled in, the u columns are formed here from `du` (the gradient behind SiLU; undefined: zero).
-variable_list uqvk_backward(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight, const Tensor& bias, double eps,
-                            int64_t n_u, Tensor d, Tensor du) {
+// Gradients of x, norm_weight, norm_bias, weight, bias (those of `ctx`'s first five inputs that are wanted) from `d`, the gradient of
+// the producer's buffer u | v | q | k: its v, q and k columns are filled in, the u columns are formed here from `du` (the gradient
+// behind SiLU; undefined: zero).
+variable_list uqvk_backward(const AutogradContext* ctx, const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, const Tensor& weight,
+                            const Tensor& bias, double eps, int64_t n_u, Tensor d, Tensor du) {
+    const bool rows_wanted = ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(2);
+    const bool weight_wanted = ctx->needs_input_grad(3) || ctx->needs_input_grad(4);
     const int64_t rows = x.size(0), dm = x.size(1);
     const c10::DeviceGuard guard(x.device());
     void* stream = stream_of(x);
-    Tensor normed = at::empty({rows, dm}, x.options());
-    check_linear(hstu_uqvk_layer_norm(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
-                                      normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
+    variable_list got(5);
+    Tensor normed;
+    if (du.defined() || weight_wanted) {
+        normed = at::empty({rows, dm}, x.options());
+        check_linear(hstu_uqvk_layer_norm(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
+                                          normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
+    }
     Tensor d_u = d.narrow(1, 0, n_u);
     if (du.defined()) {
         du = gradient_rows(du);
@@ -401,16 +408,20 @@ variable_list uqvk_backward(const Tensor& x, const Tensor& norm_weight, const Te
     } else {
         d_u.zero_();
     }
-    Tensor dy = at::mm(d, weight.t()), dx = at::empty({rows, dm}, x.options());
-    Tensor dnw = at::empty_like(norm_weight), dnb = at::empty_like(norm_bias);
-    const int64_t need = (int64_t)hstu_uqvk_layer_norm_bwd_workspace_bytes(rows, (int32_t)dm);
-    Tensor scratch = at::empty({need}, x.options().dtype(at::kByte));
-    check_linear(hstu_uqvk_layer_norm_bwd(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), (float)eps, dy.const_data_ptr(), dm,
-                                          dx.data_ptr(), dm, dnw.data_ptr(), dnb.data_ptr(), rows, (int32_t)dm, dense_dtype(x), scratch.data_ptr(),
-                                          need, stream));
-    Tensor d_bias = at::empty_like(bias);
-    Tensor d_weight = weight_grad(normed, d, d_bias);
-    return {dx, dnw, dnb, d_weight, d_bias};
+    if (rows_wanted) {
+        Tensor dy = at::mm(d, weight.t());
+        got[0] = at::empty({rows, dm}, x.options()), got[1] = at::empty_like(norm_weight), got[2] = at::empty_like(norm_bias);
+        const int64_t need = (int64_t)hstu_uqvk_layer_norm_bwd_workspace_bytes(rows, (int32_t)dm);
+        Tensor scratch = at::empty({need}, x.options().dtype(at::kByte));
+        check_linear(hstu_uqvk_layer_norm_bwd(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), (float)eps, dy.const_data_ptr(), dm,
+                                              got[0].data_ptr(), dm, got[1].data_ptr(), got[2].data_ptr(), rows, (int32_t)dm, dense_dtype(x),
+                                              scratch.data_ptr(), need, stream));
+    }
+    if (weight_wanted) {
+        got[4] = at::empty_like(bias);
+        got[3] = weight_grad(normed, d, got[4]);
+    }
+    return got;
 }
 
 struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
@@ -435,7 +446,7 @@ struct UqvkFunction : torch::autograd::Function<UqvkFunction> {
         put(std::get<1>(views), grads[1]);
         put(std::get<2>(views), grads[2]);
         put(std::get<3>(views), grads[3]);
-        variable_list got = uqvk_backward(saved_rows(saved[0]), saved_dense(saved[1]), saved_dense(saved[2]), saved_dense(saved[3]),
+        variable_list got = uqvk_backward(ctx, saved_rows(saved[0]), saved_dense(saved[1]), saved_dense(saved[2]), saved_dense(saved[3]),
                                           saved_dense(saved[4]), ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
         got.resize(8);
         return got;
@@ -480,7 +491,7 @@ struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
             grads[2].defined() ? dk.copy_(grads[2]) : dk.zero_();
             grads[3].defined() ? dv.copy_(grads[3]) : dv.zero_();
         }
-        variable_list got = uqvk_backward(x, saved_dense(saved[1]), saved_dense(saved[2]), saved_dense(saved[3]), saved_dense(saved[4]),
+        variable_list got = uqvk_backward(ctx, x, saved_dense(saved[1]), saved_dense(saved[2]), saved_dense(saved[3]), saved_dense(saved[4]),
                                           ctx->saved_data["eps"].toDouble(), s.n_u(), d, grads[0]);
         got.resize(10);
         return got;
@@ -579,7 +590,7 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
         // tensor on the same memory would be taken over, and the next gradient added into the caller's.)
         got[2] = grads[0].requires_grad() ? grads[0].clone() : grads[0];
         const bool weight_too = ctx->needs_input_grad(5);
-        if (weight_too || ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4)) {
+        if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4)) {
             const Tensor dj = at::mm(dout, weight.t());
             Tensor joined = weight_too ? at::empty_like(dj) : Tensor();
             got[0] = at::empty({rows, width}, attn.options()), got[1] = at::empty({rows, width}, attn.options());
@@ -597,6 +608,13 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
             const c10::DeviceGuard guard(attn.device());
             check_linear(hstu_output_norm_mul_bwd(&a, &g, stream_of(attn)));
             if (weight_too) got[5] = weight_grad(joined, dout, Tensor());
+        } else if (weight_too) {
+            const c10::DeviceGuard guard(attn.device());
+            Tensor joined = at::empty({rows, c.blocks() * width}, attn.options());
+            HstuOutputArgs a{};
+            fill_output(a, attn, u, norm_weight, norm_bias, c);
+            check_linear(hstu_output_norm_mul(&a, joined.data_ptr(), joined.size(1), stream_of(attn)));
+            got[5] = weight_grad(joined, dout, Tensor());
         }
         return got;
     }

@@ -136,3 +136,47 @@ def test_saved_tensors_that_come_back_in_another_layout(dev, hc):
         torch.cuda.synchronize()
         for a, b in zip(got, want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("wanted,d_model,heads,dim,limit_mb", [((0,), 128, 2, 64, 16), ((3,), 2048, 1, 16, 96), ((1, 2), 128, 2, 64, 16)])
+def test_gradients_that_nobody_asked_for_are_not_formed(dev, hc, wanted, d_model, heads, dim, limit_mb):
+    """Seen by the memory that the backward takes at its peak, 4096 rows.  d_model 128, 512 columns: 10 MB without the weight's
+    gradient, whose partial sums take 32 MB.  d_model 2048, 64 columns, the weight alone: LN(x) and the partial sums, 16 + 64 MB; the
+    layer norm's backward would add 16 MB for its operand and 32 for its results."""
+    print(f"[case] gradients wanted {wanted} of d_model {d_model}", flush=True)
+    n = 4 * heads * dim
+    ins = _rand(dev, 3, ((4096, d_model), (d_model,), (d_model,), (d_model, n), (n,)))
+    (du,) = _rand(dev, 4, ((4096, heads * dim),))
+    everything = _leaves(ins)
+    want = torch.autograd.grad(hc.hstu_compute_uqvk(*everything[:3], 1e-6, heads, dim, dim, *everything[3:])[0], everything, du)
+    want = [want[i].clone() for i in wanted]
+    some = [t.detach().clone().requires_grad_(i in wanted) for i, t in enumerate(ins)]
+    u = hc.hstu_compute_uqvk(*some[:3], 1e-6, heads, dim, dim, *some[3:])[0]
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats(dev)
+    before = torch.cuda.memory_allocated(dev)
+    got = torch.autograd.grad(u, [some[i] for i in wanted], du)
+    torch.cuda.synchronize()
+    peak = torch.cuda.max_memory_allocated(dev) - before
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert peak <= limit_mb << 20, f"{peak / 2**20:.0f} MB"
+
+
+@pytest.mark.parametrize("wanted,drop", [((2,), 0.0), ((5,), 0.0), ((5,), 0.3), ((0, 1), 0.0)])
+def test_output_step_with_part_of_its_gradients_wanted(dev, hc, wanted, drop):
+    """The weight's gradient alone comes from the forward's kernel (the joined operand) without the product that the others need."""
+    print(f"[case] output gradients wanted {wanted} dropout {drop}", flush=True)
+    ins = _output_inputs(dev, 300)
+    (d_out,) = _rand(dev, 4, ((300, D_MODEL),))
+
+    def step(t):
+        return hc.hstu_compute_output(*t[:5], 1e-6, t[5], H, D, drop, True, True, True, "silu", False, True, seed=(3, 8))
+
+    everything = _leaves(ins)
+    want = torch.autograd.grad(step(everything), everything, d_out)
+    some = [t.detach().clone().requires_grad_(i in wanted) for i, t in enumerate(ins)]
+    got = torch.autograd.grad(step(some), [some[i] for i in wanted], d_out)
+    torch.cuda.synchronize()
+    for i, a in zip(wanted, got):
+        assert torch.equal(a, want[i])
