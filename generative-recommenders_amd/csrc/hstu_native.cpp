@@ -115,12 +115,16 @@ int attention_forward(const Tensor& q, const Tensor& k, const Tensor& v, const T
     return hstu_hip_mha_fwd(&a, stream_of(q));
 }
 
+bool index_operands(const Tensor& offsets, const OptTensor& targets) {
+    if (!index_tensor(offsets) || offsets.dim() != 1 || offsets.numel() < 2) return false;
+    return !targets || (index_tensor(*targets) && targets->numel() == offsets.numel() - 1);
+}
+
 bool attention_operands(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& offsets, const OptTensor& targets) {
-    if (q.dim() != 3 || k.dim() != 3 || v.dim() != 3 || !q.is_cuda() || !k.is_cuda() || !v.is_cuda() || !index_tensor(offsets)) return false;
+    if (q.dim() != 3 || k.dim() != 3 || v.dim() != 3 || !q.is_cuda() || !k.is_cuda() || !v.is_cuda() || !index_operands(offsets, targets)) return false;
     if (attention_dtype(q.scalar_type()) < 0 || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type()) return false;
     if (k.size(1) != q.size(1) || k.size(2) != q.size(2) || v.size(0) != k.size(0) || v.size(1) != q.size(1)) return false;
-    if (offsets.dim() != 1 || offsets.numel() < 2 || q.numel() == 0 || k.numel() == 0 || v.numel() == 0) return false;
-    if (targets && (!index_tensor(*targets) || targets->numel() != offsets.numel() - 1)) return false;
+    if (q.numel() == 0 || k.numel() == 0 || v.numel() == 0) return false;
     return kernel_layout(q) && kernel_layout(k) && kernel_layout(v) && !contract_checks();
 }
 
@@ -460,7 +464,6 @@ struct PreprocessFunction : torch::autograd::Function<PreprocessFunction> {
                                  const AttentionCall& call) {
         Tensor buf = uqvk_buffer(x, norm_weight, norm_bias, weight, bias, eps, s, 0);
         auto [u, q, k, v] = uqvk_views(buf, s.heads, s.attn, s.hidden);
-        if (!attention_operands(q, k, v, offsets, targets)) throw Declined();
         Tensor out = attention_result(q, k, v, offsets, targets, call).view({x.size(0), s.n_u()});
         ctx->save_for_backward({x, norm_weight, norm_bias, weight, bias, offsets, targets ? *targets : Tensor(), buf});
         ctx->saved_data["shape"] = std::vector<int64_t>{s.heads, s.attn, s.hidden};
@@ -516,6 +519,23 @@ std::optional<FourTensors> compute_uqvk(const Tensor& x, const Tensor& norm_weig
     }
 }
 
+// Whether the attention will take the views of a producer's buffer: asked before the producer runs, which the Python operators
+// would otherwise repeat.  The library looks at sizes, strides and alignment alone; the buffer is allocated, so it is aligned
+// as x is here.
+bool attention_takes(const Tensor& x, const UqvkShape& s, const Tensor& offsets, const OptTensor& targets, const AttentionCall& call) {
+    if (!index_operands(offsets, targets) || contract_checks()) return false;
+    HstuFwdArgs a{};
+    a.q = a.k = a.v = x.const_data_ptr(), a.out = const_cast<void*>(x.const_data_ptr());
+    a.q_row_stride = a.k_row_stride = a.v_row_stride = s.n_out(), a.o_row_stride = s.n_u();
+    a.q_head_stride = a.k_head_stride = s.attn, a.v_head_stride = a.o_head_stride = s.hidden;
+    a.seq_offsets = offsets.const_data_ptr();
+    a.batch = (int32_t)(offsets.numel() - 1), a.heads = (int32_t)s.heads, a.dqk = (int32_t)s.attn, a.dv = (int32_t)s.hidden;
+    a.total_q = a.total_kv = x.size(0);
+    a.max_seq_len = (int32_t)call.max_seq_len, a.max_attn_len = (int32_t)call.w, a.contextual_seq_len = (int32_t)call.c;
+    a.dtype = attention_dtype(x.scalar_type());
+    return hstu_hip_check_args(&a) == HSTU_OK;
+}
+
 // Producer and attention with gradients: (u, attention output [L, hidden * H], k, v).  Without gradients the two operators do.
 std::optional<FourTensors> preprocess_and_attention(const Tensor& x, const Tensor& norm_weight, const Tensor& norm_bias, double eps, int64_t heads,
                                                     int64_t attn, int64_t hidden, const Tensor& weight, const Tensor& bias, int64_t max_seq_len,
@@ -524,6 +544,7 @@ std::optional<FourTensors> preprocess_and_attention(const Tensor& x, const Tenso
     if (max_seq_len <= 0 || !wants_grad({&x, &norm_weight, &norm_bias, &weight, &bias})) return {};
     if (!uqvk_operands(x, norm_weight, norm_bias, weight, bias, s) || s.n_out() > kWeightGradColumns) return {};
     const AttentionCall call{max_seq_len, 0, w, c, 0, alpha, 1.0, 1.0, 1.0, 0, 0, sort};
+    if (!attention_takes(x, s, offsets, targets, call)) return {};
     RECORD_USER_SCOPE("hstu_preprocess_and_attention");
     try {
         const variable_list o = PreprocessFunction::apply(x, norm_weight, norm_bias, weight, bias, offsets, targets, eps, s, call);

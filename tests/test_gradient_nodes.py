@@ -180,3 +180,29 @@ def test_output_step_with_part_of_its_gradients_wanted(dev, hc, wanted, drop):
     torch.cuda.synchronize()
     for i, a in zip(wanted, got):
         assert torch.equal(a, want[i])
+
+
+def test_producer_does_not_run_for_an_attention_that_is_left_to_python(dev, hc):
+    """Head dims without a kernel, offsets that need a copy, too few target counts, a negative window: known before the producer's buffer is
+    allocated."""
+    from generative_recommenders_amd.ops import native
+
+    print("[case] attention declined ahead of the producer", flush=True)
+    rows = 512
+
+    def declined(heads, dim, offsets, targets=None, window=0):
+        n = 4 * heads * dim
+        x, nw, nb, w, b = _rand(dev, 2, ((rows, D_MODEL), (D_MODEL,), (D_MODEL,), (D_MODEL, n), (n,)))
+        x.requires_grad_()
+        torch.cuda.reset_peak_memory_stats(dev)
+        before = torch.cuda.memory_allocated(dev)
+        got = native.front.preprocess_and_attention(x, nw, nb, 1e-6, heads, dim, dim, w, b, rows, offsets, 0.1, targets, window, 0, False)
+        torch.cuda.synchronize()
+        return got is None and torch.cuda.max_memory_allocated(dev) == before
+
+    offsets = torch.tensor([0, rows], device=dev)
+    assert declined(2, 24, offsets)
+    assert declined(2, 64, torch.tensor([0, 1, rows, 1], device=dev)[::2])
+    assert declined(2, 64, offsets, targets=offsets)
+    assert declined(2, 64, offsets, window=-1)
+    assert not declined(2, 64, offsets)
