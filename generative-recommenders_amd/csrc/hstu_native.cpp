@@ -145,8 +145,6 @@ void attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, co
     fill_attention(a, q, k, v, offsets, targets, call);
     Tensor scratch;
     if (workspace) {
-        TORCH_CHECK(workspace->scalar_type() == at::kByte && workspace->is_contiguous() && workspace->device() == q.device(),
-                    "workspace must be a contiguous uint8 tensor on the inputs' device");
         a.workspace = workspace->data_ptr(), a.workspace_bytes = workspace->numel(), a.sort_by_length = 1;
     } else if (a.batch >= 2) {
         scratch = at::empty({4 * (int64_t)a.batch}, q.options().dtype(at::kByte));
@@ -160,7 +158,12 @@ void attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, co
     g.dv_row_stride = dv.stride(0), g.dv_head_stride = dv.stride(1);
     const c10::DeviceGuard guard(q.device());
     const int rc = hstu_hip_mha_bwd(&a, &g, stream_of(q));
-    TORCH_CHECK(rc == HSTU_OK, "hstu_hip: ", hstu_hip_status_string(rc), " (", hstu_hip_last_error(), ") [status ", rc, "]");
+    if (rc == HSTU_OK) return;
+    // (the classes that the Python operators raise for a status)
+    const std::string what = c10::str("hstu_hip: ", hstu_hip_status_string(rc), " (", hstu_hip_last_error(), ") [status ", rc, "]");
+    TORCH_CHECK_VALUE(rc != HSTU_ERR_NULL_POINTER && rc != HSTU_ERR_BAD_SHAPE, what);
+    TORCH_CHECK_NOT_IMPLEMENTED(rc != HSTU_ERR_UNSUPPORTED, what);
+    TORCH_CHECK(false, what);
 }
 
 Tensor kernel_rows(const Tensor& t) { return kernel_layout(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
@@ -206,6 +209,8 @@ OptTensor hstu_mha(int64_t max_seq_len, double alpha, const Tensor& q, const Ten
     const AttentionCall call{max_seq_len, 0, w, c, f, alpha, q_scale, k_scale, v_scale, tile_config, kv_splits, sort};
     const bool grad = wants_grad({&q, &k, &v});
     if (grad && q.scalar_type() == at::kFloat8_e4m3fn) return {};
+    // (a workspace of the wrong kind is refused by the Python operator's backward)
+    if (grad && bwd_workspace && (bwd_workspace->scalar_type() != at::kByte || !bwd_workspace->is_contiguous() || bwd_workspace->device() != q.device())) return {};
     RECORD_USER_SCOPE("hstu_mha");
     try {
         return grad ? MhaFunction::apply(q, k, v, offsets, targets, call, bwd_workspace) : attention_result(q, k, v, offsets, targets, call);

@@ -206,3 +206,14 @@ def test_producer_does_not_run_for_an_attention_that_is_left_to_python(dev, hc):
     assert declined(2, 64, offsets, targets=offsets)
     assert declined(2, 64, offsets, window=-1)
     assert not declined(2, 64, offsets)
+
+
+def test_a_workspace_that_is_none_is_refused_as_before(pkg, dev):
+    print("[case] dS workspace of another type", flush=True)
+    q, k, v = _leaves(_rand(dev, 1, ((20, 2, 64),) * 3))
+    offsets = torch.tensor([0, 20], device=dev)
+    for bad in (torch.empty(1 << 20, dtype=torch.int8, device=dev), torch.empty((1 << 10, 1 << 10), dtype=torch.uint8, device=dev).t(),
+                torch.empty(1 << 20, dtype=torch.uint8)):
+        out = pkg.hstu_mha(20, 0.1, q, k, v, offsets, bwd_workspace=bad)
+        with pytest.raises(AssertionError, match="workspace must be"):
+            torch.autograd.grad(out, [q, k, v], torch.ones_like(out))
