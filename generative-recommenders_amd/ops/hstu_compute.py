@@ -523,6 +523,12 @@ def norm_mul_dropout(
     return _norm_mul_forward(x, u, weight, bias, eps, state, *flags)
 
 
+def _check_output(attn, u, x, norm_weight, norm_bias, output_weight, mul_u_activation_type) -> None:
+    torch._assert(x.dim() == 2 and x.shape[0] == attn.shape[0], "x must be 2-D with attn's row count")
+    _check(x, attn, u, norm_weight, norm_bias, output_weight)
+    torch._assert(mul_u_activation_type in MUL_U_ACTIVATIONS, "mul_u_activation_type must be none, sigmoid or silu")
+
+
 def hstu_compute_output(
     attn: torch.Tensor,
     u: torch.Tensor,
@@ -552,6 +558,7 @@ def hstu_compute_output(
     faster for the shape (2 where it fits, rows >= 32768 and nothing is dropped).  Dropout as in ``norm_mul_dropout``."""
     state = None
     if training and dropout_ratio > 0.0:
+        _check_output(attn, u, x, norm_weight, norm_bias, output_weight, mul_u_activation_type)  # before the generator moves on
         state = _dropout_state(dropout_ratio, training, attn.shape[0] * attn.shape[1] * _blocks(concat_u, concat_x, group_norm), attn.device, seed)
     ratio, word_seed, word_offset = state or (0.0, 0, 0)
     out = native.front.compute_output(
@@ -560,9 +567,7 @@ def hstu_compute_output(
     )
     if out is not None:
         return out
-    torch._assert(x.dim() == 2 and x.shape[0] == attn.shape[0], "x must be 2-D with attn's row count")
-    _check(x, attn, u, norm_weight, norm_bias, output_weight)
-    torch._assert(mul_u_activation_type in MUL_U_ACTIVATIONS, "mul_u_activation_type must be none, sigmoid or silu")
+    _check_output(attn, u, x, norm_weight, norm_bias, output_weight, mul_u_activation_type)
     if _needs_grad(x, attn, u, norm_weight, norm_bias, output_weight):
         return _OutputFunction.apply(attn, u, x, norm_weight, norm_bias, output_weight, norm_eps, num_heads, linear_dim, concat_u,
                                      concat_x, mul_u_activation_type, group_norm, path, state)

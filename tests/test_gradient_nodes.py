@@ -217,3 +217,16 @@ def test_a_workspace_that_is_none_is_refused_as_before(pkg, dev):
         out = pkg.hstu_mha(20, 0.1, q, k, v, offsets, bwd_workspace=bad)
         with pytest.raises(AssertionError, match="workspace must be"):
             torch.autograd.grad(out, [q, k, v], torch.ones_like(out))
+
+
+def test_a_refused_dropout_leaves_the_generator_where_it_was(dev, hc):
+    print("[case] refused calls and the dropout generator", flush=True)
+    attn, u, x, nw, nb, w = _output_inputs(dev, 8)
+    gen = torch.cuda.default_generators[0]
+    gen.set_offset(8)
+    for wrong in (dict(act="tanh"), dict(x=x[:-1]), dict(nw=nw.half()), dict(attn=attn.cpu())):
+        a = dict(attn=attn, x=x, nw=nw, act="none")
+        a.update(wrong)
+        with pytest.raises(AssertionError):
+            hc.hstu_compute_output(a["attn"], u, a["x"], a["nw"], nb, 1e-6, w, H, D, 0.1, True, True, True, a["act"], False, True)
+        assert gen.get_offset() == 8
