@@ -443,6 +443,7 @@ size_t hstu_uqvk_layer_norm_bwd_workspace_bytes(int64_t rows, int32_t d_model) {
 int hstu_uqvk_layer_norm_bwd(const void* x, int64_t x_row_stride, const void* weight, float eps, const void* dy, int64_t dy_row_stride, void* dx,
                              int64_t dx_row_stride, void* d_weight, void* d_bias, int64_t rows, int32_t d, int32_t dtype, void* workspace,
                              int64_t workspace_bytes, void* stream_) {
+    hstu_linear_set_last_error("");
     if (rows <= 0 || d <= 0 || (d & 7) != 0 || d > 4096 || x_row_stride < d || dy_row_stride < d || dx_row_stride < d) return -5;
     if (dtype != 0 && dtype != 1) return -2;
     if (!x || !weight || !dy || !dx || !d_weight || !d_bias || !workspace) return -1;
@@ -476,6 +477,7 @@ size_t hstu_output_norm_mul_bwd_workspace_bytes(const HstuOutputArgs* a) {
 }
 
 int hstu_output_norm_mul_bwd(const HstuOutputArgs* a, const HstuNormMulGrads* g, void* stream_) {
+    hstu_linear_set_last_error("");
     if (!a || !g) return -1;
     NormMulBwdParams q;
     int rc = norm_mul_params(a, g->joined, g->joined ? g->joined_row_stride : (int64_t)output_blocks(a) * a->heads * a->linear_dim, false, q.f);
@@ -514,6 +516,7 @@ int hstu_output_norm_mul_bwd(const HstuOutputArgs* a, const HstuNormMulGrads* g,
 
 int hstu_uqvk_silu_bwd(void* pre, int64_t pre_row_stride, const void* bias, const void* du, int64_t du_row_stride, int64_t rows, int64_t width, int32_t dtype,
                        void* stream_) {
+    hstu_linear_set_last_error("");
     if (rows < 0 || width <= 0 || (width & 7) != 0 || width > (1 << 30) || pre_row_stride < width || du_row_stride < width) return -5;
     if (dtype != 0 && dtype != 1) return -2;
     if (rows == 0) return 0;
@@ -539,6 +542,7 @@ size_t hstu_linear_weight_grad_workspace_bytes(int32_t m, int32_t n, int64_t row
 
 int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, const void* b, int64_t b_row_stride, int32_t n, int64_t rows,
                             int32_t dtype, void* out, void* b_sums, void* workspace, int64_t workspace_bytes, void* stream_) {
+    hstu_linear_set_last_error("");
     if (m <= 0 || n <= 0 || (m & 7) != 0 || (n & 7) != 0 || m > 65536 || n > 65536 || rows <= 0 || rows > 0x7fffffffLL) return -5;
     if (a_row_stride < m || b_row_stride < n || a_row_stride > (1 << 22) || b_row_stride > (1 << 22)) return -5;
     if (dtype != 0 && dtype != 1) return -2;

@@ -281,3 +281,25 @@ def test_native_operator_schemas_are_the_references():
 
     with pytest.raises(NotImplementedError):
         torch.ops.hstu.hstu_mha(8, 0.1, z, z, z, torch.tensor([0, 4]), True, None, None, 0, 0, 0, None, None, None, False, False)
+
+
+def test_dense_backward_entries_clear_an_older_calls_error_text():
+    """A refused call's text is its own or empty, not what the call before it left."""
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    L = hc.lib()
+    P, I, Q, F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_float
+    a = hc.HstuUqvkArgs()
+    a.rows, a.d_model, a.heads, a.attn_dim, a.hidden_dim, a.path = 8, 24, 1, 8, 8, 3
+    a.uvqk_weight = a.uvqk_bias = a.uvqk = 256
+    null = P(None)
+    refused = (
+        lambda: L.hstu_uqvk_layer_norm_bwd(null, Q(8), null, F(0), null, Q(8), null, Q(8), null, null, Q(0), I(8), I(0), null, Q(0), null),
+        lambda: L.hstu_output_norm_mul_bwd(null, null, null),
+        lambda: L.hstu_uqvk_silu_bwd(null, Q(8), null, null, Q(8), Q(8), Q(4), I(0), null),
+        lambda: L.hstu_linear_weight_grad(null, Q(8), I(8), null, Q(8), I(8), Q(0), I(0), null, null, null, Q(0), null),
+    )
+    for call in refused:
+        assert L.hstu_uqvk_forward(ctypes.byref(a), null) == -6 and L.hstu_linear_last_error() != b""
+        assert call() < 0
+        assert L.hstu_linear_last_error() == b""
