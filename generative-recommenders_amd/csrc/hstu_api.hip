@@ -241,7 +241,8 @@ bool rows_fit_buffer_offsets(const HstuFwdArgs* a) {
     return (int64_t)a->max_seq_len * rs * es < (1LL << 32);
 }
 
-Plan make_plan(const HstuFwdArgs* a) {
+// `scratch`: bytes of workspace at hand; an automatic kv-split is one that fits.
+Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX) {
     Plan pl{};
     pl.splits = 1;
     // The streaming two-group kernel (256-row blocks, one workgroup per CU) wins when the average sequence is long;
@@ -279,6 +280,7 @@ Plan make_plan(const HstuFwdArgs* a) {
     const int rows_per_pair = a->delta_size > 0 ? a->delta_size : a->max_seq_len;
     const long long blocks = (long long)a->batch * a->heads * ((rows_per_pair + bm - 1) / bm);
     const int max_tiles = (a->max_seq_len + kTileRows - 1) / kTileRows;
+    const size_t split_counts_bytes = (size_t)blocks * sizeof(int), split_bytes = (size_t)a->total_q * a->heads * a->dv * sizeof(float);
     int s = 1;
     if (a->kv_splits > 0) {
         s = a->kv_splits;
@@ -303,14 +305,17 @@ Plan make_plan(const HstuFwdArgs* a) {
             if (runs >= 4 * a->batch && max_tiles - (tiles + runs - 1) / runs >= 6) {
                 pl.fit_runs = (int)runs;
                 pl.splits = (int)(runs / a->batch);
-                pl.counts_bytes = (size_t)blocks * sizeof(int);
+                pl.counts_bytes = split_counts_bytes;
                 pl.partial_bytes = (size_t)planes * runs * (rows_per_pair < bm ? rows_per_pair : bm) * a->dv * sizeof(float);
-                return pl;
+                if (pl.total() <= scratch) return pl;
+                pl.fit_runs = 0, pl.splits = 1;  // their partial sums take more than those of equal counts can
+                pl.counts_bytes = pl.partial_bytes = 0;
             }
         }
         long long want = resident / blocks;
         if (want > max_tiles / 16) want = max_tiles / 16;
         if (want > kMaxSplits) want = kMaxSplits;
+        while (want >= 2 && pl.total() + split_counts_bytes + want * split_bytes + 256 > scratch) --want;
         if (want >= 2) s = (int)want;
     }
     // Work lists for ragged batches (equal lengths are dealt arithmetically, a kv-split enumerates its runs
@@ -323,11 +328,13 @@ Plan make_plan(const HstuFwdArgs* a) {
     if (s > 1) {
         pl.splits = s;
         pl.chunk = (max_tiles + s - 1) / s;
-        pl.counts_bytes = (size_t)blocks * sizeof(int);
-        pl.partial_bytes = (size_t)s * (size_t)a->total_q * a->heads * a->dv * sizeof(float);
+        pl.counts_bytes = split_counts_bytes;
+        pl.partial_bytes = (size_t)s * split_bytes;
     }
     return pl;
 }
+
+size_t scratch_bytes(const HstuFwdArgs* a) { return a->workspace ? (size_t)a->workspace_bytes : 0; }
 
 // Constants for fast_div (device side): x / d == (x * magic) >> (32 + shift) for 0 <= x < 2^31; magic 0 means d == 1.
 void fast_div_constants(unsigned d, unsigned* magic, unsigned* shift) {
@@ -456,8 +463,7 @@ size_t hstu_hip_workspace_bytes(const HstuFwdArgs* a) {
 int hstu_hip_plan(const HstuFwdArgs* a, int32_t* tile_config, int32_t* kv_splits) {
     int rc = hstu_hip_check_args(a);
     if (rc != HSTU_OK) return rc;
-    Plan pl = make_plan(a);
-    if (pl.splits > 1 && !(a->workspace && (size_t)a->workspace_bytes >= pl.total()) && a->kv_splits <= 1) pl.splits = 1;
+    const Plan pl = make_plan(a, scratch_bytes(a));
     if (tile_config) *tile_config = pl.cfg;
     if (kv_splits) *kv_splits = pl.splits;
     return HSTU_OK;
@@ -581,7 +587,7 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
 
     // Every use of the caller's scratch memory is an optimisation that never changes the result: without enough of
     // it an automatic choice falls back to the plain schedule, an explicit kv_splits > 1 is an error.
-    Plan plan = make_plan(a);
+    Plan plan = make_plan(a, scratch_bytes(a));
     const bool ws_ok = a->workspace && (size_t)a->workspace_bytes >= plan.total();
     if (a->dtype == HSTU_FP32) {
         // the one use of the workspace that is not optional: rounded copies of the inputs
@@ -620,12 +626,7 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
             }
         }
     }
-    if (plan.splits > 1 && !ws_ok) {
-        plan.fit_runs = 0;
-        if (a->kv_splits > 1) return a->workspace ? HSTU_ERR_BAD_SHAPE : HSTU_ERR_NULL_POINTER;
-        plan.splits = 1;
-        plan.partial_bytes = plan.counts_bytes = 0;
-    }
+    if (plan.splits > 1 && !ws_ok) return a->workspace ? HSTU_ERR_BAD_SHAPE : HSTU_ERR_NULL_POINTER;  // (asked for: make_plan's own fit)
     char* ws = (char*)a->workspace;
     const size_t ws_bytes = a->workspace ? (size_t)a->workspace_bytes : 0;
     int* queue = plan.queue_bytes > 0 && ws_bytes >= plan.queue_bytes ? (int*)ws : nullptr;

@@ -43,3 +43,21 @@ def test_fitted_runs(pkg, dev, lengths, delta, heads, dim, dtype, cfg):
     assert float((got.float() - one.float()).norm() / one.float().norm()) <= 2.0**-8
     if dtype == torch.bfloat16:
         assert_parity(got, O.cached_hstu_mha_per_sequence(N, alpha, q.float(), k.float(), v.float(), offs, t), "fitted runs")
+
+
+def test_runs_at_scratch_limits(pkg, dev):
+    """Workspaces that hold the fitted runs, fewer equal ones, none: the same products in another order."""
+    from generative_recommenders_amd.ops import hip_backend as hb
+
+    lengths, delta, heads, dim = [2000, 100, 64, 1037, 7000], 64, 3, 128
+    B, N, alpha = len(lengths), max(lengths) + 7, dim**-0.5
+    q, k, v, offs, _ = make_case(12, lengths, heads, dim, delta_size=delta)
+    want = O.cached_hstu_mha_per_sequence(N, alpha, q.float(), k.float(), v.float(), offs, None)
+    q, k, v, offs = (x.to(dev) for x in (q, k, v, offs))
+    run = B * delta * heads * dim * 4
+    for limit in (None, 8 * run + 4096, 3 * run + 4096, 2 * run + 4096, run, 600, 0):
+        print(f"[case] runs with {limit} bytes of scratch memory", flush=True)
+        out = torch.full((B * delta, heads, dim), float("nan"), dtype=q.dtype, device=dev)
+        hb.mha_fwd(q, k, v, out, offs, None, N, alpha, delta, 0, 0, 0, workspace_bytes=limit)
+        torch.cuda.synchronize()
+        assert_parity(out, want, f"{limit} bytes")

@@ -303,3 +303,29 @@ def test_dense_backward_entries_clear_an_older_calls_error_text():
         assert L.hstu_uqvk_forward(ctypes.byref(a), null) == -6 and L.hstu_linear_last_error() != b""
         assert call() < 0
         assert L.hstu_linear_last_error() == b""
+
+
+def test_a_kv_split_is_cut_to_the_workspace_at_hand(backend):
+    """Delta form, 5 histories of up to 15000 rows x 100 rows: 64 fitted runs per head want 13.1 MB of partial sums, eight equal runs 8.2
+    MB, two 2 MB; with less the split goes, never the call."""
+    L, (B, H, D, delta, N) = backend.lib(), (5, 4, 128, 100, 15000)
+    a = backend.HstuFwdArgs()
+    a.batch, a.heads, a.dqk, a.dv, a.total_q, a.total_kv, a.max_seq_len, a.delta_size = B, H, D, D, B * delta, B * 12000, N, delta
+    a.q = a.k = a.v = a.out = a.seq_offsets = 256
+    a.q_row_stride = a.k_row_stride = a.v_row_stride = a.o_row_stride = H * D
+    a.q_head_stride = a.k_head_stride = a.v_head_stride = a.o_head_stride = D
+    need = L.hstu_hip_workspace_bytes(ctypes.byref(a))
+    run = B * delta * H * D * 4  # the partial sums of one run of equal counts
+    other = 4 * B * H + 256 + 576  # counts, alignment, counters
+
+    def runs(bytes_):
+        a.workspace, a.workspace_bytes = (256, bytes_) if bytes_ else (None, 0)
+        splits = ctypes.c_int32()
+        assert L.hstu_hip_plan(ctypes.byref(a), None, ctypes.byref(splits)) == 0
+        return splits.value
+
+    assert need > 8 * run + other and runs(need) == 64 // B
+    assert runs(need - 1) == 8 and runs(8 * run + other) == 8 and runs(8 * run + other - 1) == 7
+    assert runs(2 * run + other) == 2 and runs(2 * run + other - 1) == 1 and runs(0) == 1
+    a.kv_splits = 4
+    assert runs(2 * run) == 4  # asked for: the call itself refuses a workspace that is too small
