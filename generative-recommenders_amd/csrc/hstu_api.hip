@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <initializer_list>
@@ -114,7 +115,7 @@ int launch(const hstu::FwdParams& p, hipStream_t stream) {
     auto kern = hstu::hstu_fwd_kernel<TT, DQK, DV, QT, NW, BN, OCC>;
     // once per device (the attribute belongs to the device's copy of the kernel); raising the dynamic LDS limit is
     // idempotent, so racing threads only set the same value twice
-    static bool attr_done[64];
+    static std::atomic<bool> attr_done[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
     if (dev < 0 || !attr_done[dev]) {
@@ -384,7 +385,7 @@ bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15)
 // 1 if the current device is gfx950, 0 if not, cached per device ordinal (the kernels use gfx950-only
 // instructions; the reference's native op makes the same kind of check, flash_common.cpp:420-422).
 int current_device_is_gfx950() {
-    static int cache[64];  // 0 unknown, 1 yes, 2 no; racing threads store the same value
+    static std::atomic<int> cache[64];  // 0 unknown, 1 yes, 2 no; racing threads store the same value
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (dev < 0 || dev >= 64) return 0;
@@ -398,7 +399,7 @@ int current_device_is_gfx950() {
 
 // Compute units of the current device (256 on MI355X), cached per device ordinal.
 int current_device_cus() {
-    static int cache[64];
+    static std::atomic<int> cache[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
     if (cache[dev] == 0) {

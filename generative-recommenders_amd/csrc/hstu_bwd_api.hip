@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 
@@ -56,7 +57,7 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     auto k2 = hstu::hstu_bwd_dq_kernel<TT, DQK, DV, kBwdWaves, kBwdTile>;
     auto k3 = hstu::hstu_bwd_dq_stored_kernel<TT, DQK, kStoredWaves, kBwdTile>;
     // (a function attribute belongs to the device it was set on: one flag per device)
-    static bool attr_done[64];
+    static std::atomic<bool> attr_done[64];
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
     if (dev < 0 || !attr_done[dev]) {

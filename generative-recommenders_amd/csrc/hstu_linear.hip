@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -295,7 +296,7 @@ template <class TT, bool BIAS>
 int launch_output_gemm_t(const hstu::OutputGemmParams& p, hipStream_t stream) {
     auto kern = hstu::hstu_output_gemm_kernel<TT, BIAS>;
     // (a function attribute belongs to the device it was set on: one flag per device)
-    static bool attr_done[64];
+    static std::atomic<bool> attr_done[64];
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
     if (dev < 0 || !attr_done[dev]) {
@@ -578,7 +579,7 @@ template <class TT, int KT>
 int launch_uqvk_fused(hstu::UqvkFusedParams p, hipStream_t stream) {
     auto kern = hstu::hstu_uqvk_fused_kernel<TT, KT>;
     // (a function attribute belongs to the device it was set on: one flag per device)
-    static bool attr_done[64];
+    static std::atomic<bool> attr_done[64];
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
     if (dev < 0 || !attr_done[dev]) {

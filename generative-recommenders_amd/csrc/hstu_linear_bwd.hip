@@ -10,6 +10,7 @@
 #include "hstu_rows.h"
 #include "hstu_wgrad_kernel.h"
 
+#include <atomic>
 #include <cstdio>
 
 // defined in hstu_linear.hip; internal to the library
@@ -401,7 +402,7 @@ WgradPlan wgrad_plan(int m, int n, int64_t rows, int64_t stride) {
 template <class TT>
 int launch_wgrad(const WgradParams& p, typename TT::elem* out, typename TT::elem* colsum, hipStream_t stream) {
     auto kern = hstu_wgrad_kernel<TT>;
-    static bool attr_done[64];  // (a function attribute belongs to the device it was set on)
+    static std::atomic<bool> attr_done[64];  // (a function attribute belongs to the device it was set on)
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
     if (dev < 0 || !attr_done[dev]) {

@@ -3,6 +3,7 @@
 // instructions can read them (with the other form the kernel copies 64 registers per column block and spills).
 #include "hstu_uqvk_wide_kernel.h"
 
+#include <atomic>
 #include <cstdio>
 
 // defined in hstu_linear.hip; internal to the library
@@ -20,7 +21,7 @@ int fail(const char* what, hipError_t e) {
 template <class TT, int KT, bool OUT8>
 int launch(hstu::UqvkFusedParams p, hipStream_t stream) {
     auto kern = hstu::hstu_uqvk_wide_kernel<TT, KT, OUT8>;
-    static bool attr_done[64];  // (a function attribute belongs to the device it was set on)
+    static std::atomic<bool> attr_done[64];  // (a function attribute belongs to the device it was set on)
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
     if (dev < 0 || !attr_done[dev]) {
