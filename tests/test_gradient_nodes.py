@@ -230,3 +230,26 @@ def test_a_refused_dropout_leaves_the_generator_where_it_was(dev, hc):
         with pytest.raises(AssertionError):
             hc.hstu_compute_output(a["attn"], u, a["x"], a["nw"], nb, 1e-6, w, H, D, 0.1, True, True, True, a["act"], False, True)
         assert gen.get_offset() == 8
+
+
+@pytest.mark.parametrize("arrive", ["u", "out", "k", "v", "kv", "out k", "out v", "u out k v"])
+def test_gradients_that_arrive_through_any_of_the_outputs(dev, hc, arrive):
+    """The one node for producer and attention against the two operators one after the other: the same kernels, but with the attention's
+    and the callers' gradients of k and v added in bf16 by autograd there, as here."""
+    print(f"[case] gradients through {arrive}", flush=True)
+    rows = 70
+    one, two = _leaves(_producer_inputs(dev, rows)), _leaves(_producer_inputs(dev, rows))
+    offsets = torch.tensor([0, rows], device=dev)
+    from generative_recommenders_amd.ops import hstu_attention
+
+    u, q, k, v = _producer(hc, *two)
+    attn = hstu_attention.hstu_mha(rows, D**-0.5, q, k, v, offsets).view(rows, H * D)
+    first, second = _first_half(hc, dev, *one), (u, attn, k, v)
+    picked = [i for i, name in enumerate(("u", "out", "k", "v")) if name in arrive.split() or (arrive == "kv" and name in "kv")]
+    assert picked
+    d = _rand(dev, 5, [first[i].shape for i in picked])
+    got = torch.autograd.grad([first[i] for i in picked], one, d)
+    want = torch.autograd.grad([second[i] for i in picked], two, d)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -72,12 +72,12 @@ def _close(got, want, what):
     assert rel <= (4e-3 if got.dim() > 1 else 1.6e-2), f"{what}: {rel:.2e}"
 
 
-@pytest.mark.parametrize("rows,heads,dim,cu,cx,act,group,silu_u,drop", [
-    (1, 1, 8, True, True, "none", False, False, 0.0), (5, 2, 64, True, True, "silu", False, False, 0.3), (300, 3, 168, False, True, "sigmoid", False, False, 0.0),
-    (4100, 4, 128, True, False, "none", False, False, 0.2), (77, 8, 128, True, True, "none", True, False, 0.1), (9, 8, 512, True, True, "none", False, False, 0.0),
-    (513, 2, 8, False, False, "none", True, False, 0.0), (260, 1, 512, True, True, "none", True, False, 0.5),
+@pytest.mark.parametrize("rows,heads,dim,cu,cx,act,group,drop", [
+    (1, 1, 8, True, True, "none", False, 0.0), (5, 2, 64, True, True, "silu", False, 0.3), (300, 3, 168, False, True, "sigmoid", False, 0.0),
+    (4100, 4, 128, True, False, "none", False, 0.2), (77, 8, 128, True, True, "none", True, 0.1), (9, 8, 512, True, True, "none", False, 0.0),
+    (513, 2, 8, False, False, "none", True, 0.0), (260, 1, 512, True, True, "none", True, 0.5),
 ])
-def test_output_step_gradients_against_the_recomputation(dev, rows, heads, dim, cu, cx, act, group, silu_u, drop):
+def test_output_step_gradients_against_the_recomputation(dev, rows, heads, dim, cu, cx, act, group, drop):
     """The norm-multiply backward kernel and the products around it, at widths of one lane to the widest row, one row to more
     rows than waves, against the package's own restatement with torch operators (same operands, same mask)."""
     from generative_recommenders_amd.ops import hstu_compute as hc
@@ -99,6 +99,50 @@ def test_output_step_gradients_against_the_recomputation(dev, rows, heads, dim, 
     torch.cuda.synchronize()
     for name, a, b in zip(("attn", "u", "x", "norm_weight", "norm_bias", "weight"), got, want):
         _close(a, b, f"d/d{name}")
+
+
+@pytest.mark.parametrize("rows,heads,dim,cx,act,group,drop", [
+    (5, 2, 64, True, "none", False, 0.0), (300, 4, 128, False, "sigmoid", False, 0.2), (77, 8, 128, True, "none", True, 0.0), (260, 1, 512, True, "none", True, 0.3),
+])
+def test_norm_multiply_backward_with_silu_on_the_copied_u(dev, rows, heads, dim, cx, act, group, drop):
+    """``silu_u``, which only the C entry passes on to its kernel (the Python operator that has the flag differentiates the restatement):
+    d attn, d u, the norm's gradients and the recomputed operand."""
+    import ctypes
+
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    print(f"[case] norm-multiply backward, silu_u {rows} {heads} {dim} {cx} {act} group={group} drop={drop}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows)
+    width, norm = heads * dim, heads if group else heads * dim
+    ins = [torch.randn(s, generator=g, device=dev).bfloat16() for s in ((rows, width), (rows, width), (norm,), (norm,))]
+    a, keep, blocks = hc._output_args(*ins, 1e-6, heads, dim, True, cx, act, group, True)
+    d_joined = torch.randn((rows, blocks * width), generator=g, device=dev).bfloat16()
+    state = hc._dropout_state(drop, True, 0, dev, (3, 8))
+    hc._set_dropout(a, state)
+    mask = hc._keep_scaled(state, rows, blocks * width, dev)
+
+    got = [torch.full_like(t, float("nan")) for t in ins]
+    joined = torch.full_like(d_joined, float("nan"))
+    L, P, Q = hc.lib(), ctypes.c_void_p, ctypes.c_int64
+    L.hstu_output_norm_mul_bwd_workspace_bytes.restype = ctypes.c_size_t
+    need = L.hstu_output_norm_mul_bwd_workspace_bytes(ctypes.byref(a))
+    ws = torch.full((need // 4,), float("nan"), device=dev)
+
+    class Grads(ctypes.Structure):  # HstuNormMulGrads
+        _fields_ = [(f"f{i}", P if i not in (1, 3, 5, 7, 11) else Q) for i in range(12)]
+
+    grads = Grads(d_joined.data_ptr(), d_joined.stride(0), joined.data_ptr(), joined.stride(0), got[0].data_ptr(), width, got[1].data_ptr(), width,
+                  got[2].data_ptr(), got[3].data_ptr(), ws.data_ptr(), need)
+    rc = L.hstu_output_norm_mul_bwd(ctypes.byref(a), ctypes.byref(grads), P(torch.cuda.current_stream(dev).cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == 0, L.hstu_linear_last_error()
+
+    def restated(attn, u, nw, nb):
+        return hc._norm_mul_math(attn, u, nw, nb, 1e-6, True, True, cx, act, group, heads, dim, keep_scaled=mask)
+
+    _close(joined, restated(*ins), "joined")
+    for name, x, y in zip(("attn", "u", "norm_weight", "norm_bias"), got, _grads(restated, ins, d_joined)):
+        _close(x, y, f"d/d{name}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
