@@ -12,14 +12,16 @@
 // stores in flight is known wherever a copy is waited for.
 //
 // The work, row blocks of 256 x column blocks of 64, is one line that is cut into equal parts, one per CU; a part that crosses
-// into the next row block normalises that block's rows too (5 to 6 column blocks' time: 6000 vector instructions and the wait for HBM).
+// into the next row block normalises that block's rows too (12 us, three column blocks' time: 6000 vector instructions and the wait for HBM).
 //
 // 139264 rows of d_model 512 into 2048 columns: 408 -> 329 us (0.89 PFLOP/s); 300000 rows into 4096 columns 1593 -> 1249 us
-// (1.01 PFLOP/s, the matrix pipe busy 56 % of the cycles; a large library product reaches 1.36).  On the way: the barrier without a
+// (1.01 PFLOP/s; a large library product reaches 1.36); 524288 rows into 2048 columns 1.20 ms, the matrix pipe busy 56 % of the
+// cycles (SQ_VALU_MFMA_BUSY_CYCLES / 4 SQ_BUSY_CU_CYCLES).  On the way: the barrier without a
 // wait for LDS reads 347 -> 329, no branches inside a column block and column blocks in turned order (see below) 65536 rows into
 // 4096 columns 364 -> 292; the addresses of the stores computed where they are used (no spills, whose reloads wait for all
 // copies) and the e4m3 copy in halves behind the store: the 8-bit layer of 16 sequences of 4096 .. 16384 rows 1.013 -> 1.064 of its
-// former speed.  What is left: the rows' preparation, which nothing overlaps, about a fifth of the time.
+// former speed.  What is left: the rows' preparation, which nothing overlaps, 8 % of the time (with other rows of the matrix prepared
+// first, as a measurement, 1.20 -> 1.31 ms at 524288 rows), and the column blocks themselves, where the matrix pipe is idle for 39 % of it.
 #pragma once
 #include <type_traits>
 #include <utility>

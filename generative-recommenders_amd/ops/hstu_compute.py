@@ -1,14 +1,15 @@
 """``hstu_compute_uqvk``, ``hstu_compute_output`` and ``hstu_preprocess_and_attention`` with the reference's
 signatures (``generative_recommenders/ops/hstu_compute.py:54-104``, ``:107-214``, ``:217-334``).
 
-``hstu_compute_uqvk``: layer norm + uvqk projection + split + SiLU(u).  The layer norm is a hand-written gfx950
-kernel; the projection is a plain GEMM and runs on hipBLASLt with the bias and, for the u columns, the SiLU in its
-epilogue.  ``u, q, k, v`` come back as column slices of one ``[L, (2*hidden + 2*attn) * H]`` buffer, which
-``hstu_mha`` / ``delta_hstu_mha`` read in place.
+``hstu_compute_uqvk``: layer norm + uvqk projection + split + SiLU(u), in one hand-written gfx950 kernel for d_model 128,
+256, 384 and 512 (``csrc/hstu_uqvk_kernel.h``, ``csrc/hstu_uqvk_wide_kernel.h``); other shapes take a layer-norm kernel and hipBLASLt
+with the bias and, for the u columns, the SiLU in its epilogue.  ``u, q, k, v`` come back as column slices of one
+``[L, (2*hidden + 2*attn) * H]`` buffer, which ``hstu_mha`` / ``delta_hstu_mha`` read in place.
 
-``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  One hand-written kernel
-normalises, multiplies and writes the concatenated operand; the product, with the residual as the GEMM's C operand,
-runs on hipBLASLt.  (``csrc/hstu_linear.hip``, ``include/hstu_linear.h``.)
+``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  From 32768 rows on a hand-written GEMM reads u
+and attn where they are and ``act(u) * norm(attn)`` from a row-wise kernel; below, and for widths it does not take or with dropout, that
+kernel writes the concatenated operand and hipBLASLt multiplies it with the residual as its C operand.
+(``csrc/hstu_linear.hip``, ``csrc/hstu_output_kernel.h``, ``include/hstu_linear.h``.)
 
 Device tensors only, bf16 or fp16; ``kernel`` is accepted and ignored.  The usual call, with or without gradients, goes through
 the native front (``csrc/hstu_native.cpp``): backward kernels for the row-wise parts (``csrc/hstu_linear_bwd.hip``), plain
@@ -173,10 +174,10 @@ def _needs_grad(*tensors: torch.Tensor) -> bool:
 # ---- gradients of the calls that the native front leaves ----------------------------------------------------------------
 # (parameters or rows that are not dense and 16-byte aligned, and ``layer_norm`` / ``norm_mul_dropout`` on their own.)  The
 # forward runs on this package's kernels; the gradients here are not hand-written: the backward recomputes the step with the
-# framework's own operators (layer / group norm, addmm on hipBLASLt) in the arithmetic of the reference's PyTorch backend (fp32 norm and product with u, result rounded to the input type, then the
-# product with the weight: ops/pytorch/pt_layer_norm.py:24-39, pt_hstu_linear.py:24-124, ops/hstu_compute.py:54-104) and
-# lets autograd differentiate that -- nothing but the inputs is saved, which is what the reference's recompute_* flags
-# ask for.  It is there so that a training step can run through the package.
+# framework's own operators (layer / group norm, addmm on hipBLASLt) in the arithmetic of the reference's PyTorch backend (fp32
+# norm and product with u, result rounded to the input type, then the product with the weight: ops/pytorch/pt_layer_norm.py:24-39,
+# pt_hstu_linear.py:24-124, ops/hstu_compute.py:54-104) and lets autograd differentiate that -- nothing but the inputs is saved,
+# which is what the reference's recompute_* flags ask for.
 
 def _layer_norm_math(x, weight, bias, eps):
     return F.layer_norm(x.float(), (x.shape[-1],), weight.float(), bias.float(), eps).to(x.dtype)

@@ -89,7 +89,8 @@ typedef struct HstuFwdArgs {
     int64_t workspace_bytes;
     int32_t kv_splits;               /* 0 = choose automatically (delta mode with too few row blocks to fill and
                                         balance the chip is split when the workspace allows, in runs fitted to the
-                                        lengths of the sequences where it can); 1 = never split;
+                                        lengths of the sequences where it can, else in as many equal
+                                        ones as it holds); 1 = never split;
                                         S = 2..8: cut the kv range of every row block into runs of
                                         ceil(ceil(max_seq_len / 64) / S) tiles of 64 rows, each run taken by its own
                                         workgroup, and add the fp32 partial results in a second kernel.  Needs

@@ -10,7 +10,7 @@
  * All four results stay column slices of ONE [L, n_out] buffer -- the layout the attention entry points read in
  * place through their row / head strides -- so nothing is copied on the way to `hstu_hip_mha_fwd`.
  *
- * Two paths.  Fused (the usual shapes, see `path`): one hand-written kernel that keeps a wave's 32 normalised rows in
+ * Two paths.  Fused (the usual shapes, see `path`): one hand-written kernel that keeps a wave's 32 or 64 normalised rows in
  * registers as MFMA operands, streams the weight through LDS and applies bias and SiLU before the store -- x is read
  * once, uvqk written once, nothing else touches HBM.  Library path (any shape): a layer-norm kernel (one wave per row)
  * and hipBLASLt with the bias and, for the u columns, the SiLU in the GEMM's epilogue.  This library is separate from
@@ -48,8 +48,9 @@ typedef struct HstuUqvkArgs {
                                   GEMM's scratch (unused by the fused kernel; may then be NULL) */
     int64_t workspace_bytes;
     int32_t path;              /* 0 = automatic: the fused kernel (layer norm, product, bias, SiLU in one pass, the
-                                  normalised rows held in registers) when d_model is 128, 256, 384 or 512 and
-                                  hidden_dim * heads and n_out are multiples of 128, else the library path;
+                                  normalised rows held in registers) when d_model is 128, 256, 384 or 512,
+                                  hidden_dim * heads is a multiple of 32 (128 with the e4m3 copy below) and n_out one
+                                  of 128, else the library path;
                                   1 = library path (layer-norm kernel + hipBLASLt); 2 = fused kernel or status -6;
                                   3 = layer-norm kernel + the hand-written GEMM kernel of the output projection with the
                                   bias as the start of the sums and SiLU(u) in its epilogue (d_model a multiple of 64,
