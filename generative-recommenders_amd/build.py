@@ -63,7 +63,7 @@ def build_library(verbose: bool = False) -> str:
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     common = [hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + ["-I", INCLUDE, "-I", CSRC]
     objs = [os.path.join(CSRC, name) for name in ("hstu_api.o", "hstu_bwd_api.o", "hstu_fwd_fitted.o")]
-    linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o"), os.path.join(CSRC, "hstu_uqvk_wide.o")]
+    linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o"), os.path.join(CSRC, "hstu_uqvk.o")]
     jobs = [
         common + ["-c", os.path.join(CSRC, "hstu_api.hip"), "-o", objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_bwd_api.hip"), "-o", objs[1]],
@@ -71,7 +71,7 @@ def build_library(verbose: bool = False) -> str:
         common + ["-c", os.path.join(CSRC, "hstu_linear.hip"), "-o", linear_objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_linear_bwd.hip"), "-o", linear_objs[1]],
         # (matrix results in vector registers: see the file)
-        common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_uqvk_wide.hip"), "-o", linear_objs[2]],
+        common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_uqvk.hip"), "-o", linear_objs[2]],
     ]
     native_compile, native_link, native_obj = _native_commands()
     jobs.append(native_compile)

@@ -353,6 +353,11 @@ __device__ __forceinline__ int swz_v(int row) {
     return half_swap;
 }
 
+// Chunk swizzle of a tile of a dense product (rows of 256 bytes = 16 chunks).  A transposing read touches rows {8g + 4sec + j}, j = 0..3,
+// for the two half-waves g: the four rows of a half-wave go to four different 64-byte bank groups (row bits 0-1 ->
+// chunk bits 2-3) and the two half-waves to different 32-byte halves of a group (row bit 3 -> chunk bit 1).
+__device__ __forceinline__ int swz_w(int row) { return ((row & 3) << 2) | (((row >> 3) & 1) << 1); }
+
 // 16 bytes per lane, global memory -> LDS at lds_base + 16*lane (lds_base is wave-uniform and goes
 // through M0).  Written as inline assembly on purpose: the compiler then does not know that an LDS
 // write is in flight and does not put a vmcnt(0) wait in front of the next LDS read, which would

@@ -18,8 +18,8 @@
 #include "hstu_uqvk_kernel.h"
 #include "hstu_output_kernel.h"
 
-// hstu_uqvk_wide.hip
-int hstu_uqvk_wide_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
+// hstu_uqvk.hip
+int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
 
 namespace {
 
@@ -593,8 +593,8 @@ int launch_uqvk_fused(hstu::UqvkFusedParams p, hipStream_t stream) {
     constexpr int kRows = hstu::kUqvkWaves * hstu::kUqvkRowsPerWave;
     const long long grid = (p.rows + kRows - 1) / kRows;
     const int nchunks = p.n_out / hstu::kUqvkTileN;
-    p.chunks_per_wg = uqvk_chunks_per_wg(grid, nchunks);
-    const unsigned splits = (unsigned)((nchunks + p.chunks_per_wg - 1) / p.chunks_per_wg);
+    p.units_per_wave = uqvk_chunks_per_wg(grid, nchunks);
+    const unsigned splits = (unsigned)((nchunks + p.units_per_wave - 1) / p.units_per_wave);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid, splits), dim3(hstu::kUqvkWaves * 64), hstu::kUqvkLds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -604,29 +604,6 @@ int launch_uqvk_fused(hstu::UqvkFusedParams p, hipStream_t stream) {
     return 0;
 }
 
-// 64 rows per wave where that kernel's work, row blocks of 256 x column blocks of 64, gives each CU 16 units or more (8 at d_model 256,
-// where the rows are normalised in half the time); below that the rows' preparation, 256 at a time on one CU, outweighs
-// the faster matrix phase.  d_model 512 into 2048 columns, 32 -> 64 rows per wave: 26000 rows 87 -> 91 us, 32768 100 -> 85, 139264
-// 408 -> 329; into 4096: 12000 rows 83 -> 87, 16384 98 -> 88, 174000 957 -> 743; d_model 256 into 1024: 26000 rows 39 -> 40, 32768
-// 40 -> 34.  Columns: into 256 it is slower at every size (300000 rows of d_model 512: 177 -> 197), into 512 from 131072 rows on the faster
-// one (133 -> 125).
-bool uqvk_takes_wide(const hstu::UqvkFusedParams& p, int d_model) {
-    if (d_model < 256 || p.n_out < 512 || p.n_silu % 64 != 0) return false;
-    const long long units = (p.rows + 255) / 256 * (p.n_out / 64);
-    return units >= (d_model == 256 ? 2048 : 4096) && units <= 0x7fffffffLL;
-}
-
-template <class TT>
-int launch_uqvk_fused_k(const hstu::UqvkFusedParams& p, int d_model, hipStream_t stream) {
-    if (uqvk_takes_wide(p, d_model)) return hstu_uqvk_wide_launch(p, d_model, std::is_same<TT, hstu::Bf16>::value, stream);
-    switch (d_model) {
-        case 128: return launch_uqvk_fused<TT, 2>(p, stream);
-        case 256: return launch_uqvk_fused<TT, 4>(p, stream);
-        case 384: return launch_uqvk_fused<TT, 6>(p, stream);
-        default: return launch_uqvk_fused<TT, 8>(p, stream);
-    }
-}
-
 size_t normed_bytes(const HstuUqvkArgs* a) { return (((size_t)a->rows * a->d_model * 2) + 255) & ~(size_t)255; }
 size_t joined_bytes(const HstuOutputArgs* a) {
     return (((size_t)a->rows * output_blocks(a) * a->heads * a->linear_dim * 2) + 255) & ~(size_t)255;
@@ -634,7 +611,13 @@ size_t joined_bytes(const HstuOutputArgs* a) {
 
 }  // namespace
 
-// for the library's other translation unit; not exported
+// for the library's other translation units; not exported
+// d_model: 384 or 512.  (Here and not beside the other kernels: it is built and measured with the general form of the matrix instructions.)
+__attribute__((visibility("hidden"))) int hstu_uqvk_fused_launch(hstu::UqvkFusedParams p, int d_model, bool bf16, hipStream_t stream) {
+    if (d_model == 384) return bf16 ? launch_uqvk_fused<hstu::Bf16, 6>(p, stream) : launch_uqvk_fused<hstu::Fp16, 6>(p, stream);
+    return bf16 ? launch_uqvk_fused<hstu::Bf16, 8>(p, stream) : launch_uqvk_fused<hstu::Fp16, 8>(p, stream);
+}
+
 extern "C" __attribute__((visibility("hidden"))) void hstu_linear_set_last_error(const char* text) {
     snprintf(g_last_error, sizeof(g_last_error), "%s", text);
 }
@@ -706,7 +689,7 @@ int hstu_uqvk_forward(const HstuUqvkArgs* a, void* stream_) {
                 p.inv_scale[i] = 1.0f / sc[i];
             }
         }
-        return a->dtype == 0 ? launch_uqvk_fused_k<hstu::Bf16>(p, a->d_model, stream) : launch_uqvk_fused_k<hstu::Fp16>(p, a->d_model, stream);
+        return hstu_uqvk_launch(p, a->d_model, a->dtype == 0, stream);
     }
     if (!a->workspace) return -1;
     if ((size_t)a->workspace_bytes < hstu_uqvk_workspace_bytes(a) || ((uintptr_t)a->workspace & 255) != 0) return -4;

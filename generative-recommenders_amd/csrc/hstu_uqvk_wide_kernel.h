@@ -40,11 +40,6 @@ constexpr int kWideRing = KT / 2 + 2;
 template <int KT>
 constexpr int kWideLds = kWideRing<KT> * kWideSlot + kWideBias + 4 * 2 * kWideStage;
 
-// Chunk swizzle of a W tile (rows of 128 bytes = 8 chunks): the rows 8g + 4sec + j of a transposing read lie in different
-// 64-byte bank groups (odd rows by the pitch, row bit 1 -> chunk bit 2), the two half-waves in different halves of a group
-// (row bit 3 -> chunk bit 1).
-__device__ __forceinline__ int swz_w64(int row) { return (((row >> 1) & 1) << 2) | (((row >> 3) & 1) << 1); }
-
 // When the epilogue of the previous column block does what, in steps of the S a column block has.
 template <int S>
 struct WideSchedule {
@@ -86,9 +81,9 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
     const int g = lane >> 5, l32 = lane & 31;
     const int nblk = p.n_out / kWideCols;
     // this workgroup's part of the line of units
-    const int extra = p.units - p.chunks_per_wg * (int)gridDim.x;  // parts that are one unit longer
-    int unit = (int)blockIdx.x * p.chunks_per_wg + ((int)blockIdx.x < extra ? (int)blockIdx.x : extra);
-    const int unit_end = unit + p.chunks_per_wg + ((int)blockIdx.x < extra ? 1 : 0);
+    const int extra = p.units - p.units_per_wave * (int)gridDim.x;  // parts that are one unit longer
+    int unit = (int)blockIdx.x * p.units_per_wave + ((int)blockIdx.x < extra ? (int)blockIdx.x : extra);
+    const int unit_end = unit + p.units_per_wave + ((int)blockIdx.x < extra ? 1 : 0);
 
     // copy instruction i of this wave brings rows (wave + 4 i) * 8 + lane / 8 of a tile, physical chunk lane % 8
     unsigned coff[4];
@@ -183,10 +178,7 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = v[j] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v[j]));
             }
-            elem4 o4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o4[j] = (elem)v[j];
-            *HSTU_LDS(elem4, stage + rg * kWideStage + l32 * kUqvkStageRow + (dt * 32 + r4 * 8 + g * 4) * 2) = o4;
+            *HSTU_LDS(elem4, stage + rg * kWideStage + l32 * kUqvkStageRow + (dt * 32 + r4 * 8 + g * 4) * 2) = round_to<elem>(v);
         };
         auto read_rows = [&](int i) __attribute__((always_inline)) {
             rd[i] = *HSTU_LDS(const i32x4_t, stage + (i >> 2) * kWideStage + ((i & 3) * 8 + rsub) * kUqvkStageRow + chunk * 16);

@@ -257,6 +257,41 @@ def test_uqvk_with_64_rows_per_wave_gives_the_bits_of_32(pkg, dev, L, d_model, H
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "d_model,H,attn,hidden,whole,parts",
+    # several rounds of 128 rows per workgroup (d_model 384, 512) or of 64 (below), against: units of their own for 32 rows, up to the last
+    # size that takes; 64 rows with 1, 2, 4, 8 units per wave; sizes with a remainder of 1, 31, 33, 63 rows; u columns that end inside
+    # a block of 64; one column block
+    [(512, 4, 128, 128, 17000, (1, 33, 1024, 1025, 2048, 4095, 8129, 16351)), (512, 2, 64, 64, 24001, (63, 4096, 4097, 8193, 16384)),
+     (384, 3, 96, 32, 24000, (1, 95, 5000, 16001)), (512, 1, 32, 32, 40001, (31, 16384, 32768)), (512, 1, 64, 64, 40000, (1, 8192, 8193, 32700)),
+     (256, 4, 64, 64, 30001, (1, 2048, 2049, 4097, 8193, 16385)), (128, 3, 32, 96, 30000, (33, 5461, 5462, 20000))],
+)
+def test_uqvk_kernels_for_few_rows_give_the_same_bits(pkg, dev, d_model, H, attn, hidden, whole, parts):
+    """All the fused kernels sum in the same order: a row's bits are the same in every batch.  The rows are compared from both ends of
+    the large batch, whose last rows are held against the oracle."""
+    print(f"[case] uqvk few rows {d_model} {H} {attn} {hidden} {whole} {parts}", flush=True)
+    host = _inputs(whole, whole, d_model, H, attn, hidden, torch.bfloat16)
+    x, nw, nb, w, b = [t.to(dev) for t in host]
+    fp8 = hidden * H % 128 == 0
+    ref = pkg.hstu_compute_uqvk(x, nw, nb, 1e-6, H, attn, hidden, w, b, path=2)
+    ref8 = pkg.hstu_compute_uqvk_fp8(x, nw, nb, 1e-6, H, attn, hidden, w, b, 0.01, 0.011, 0.012) if fp8 else None
+    for n in parts:
+        for rows in (slice(0, n), slice(whole - n, whole)):
+            got = pkg.hstu_compute_uqvk(x[rows], nw, nb, 1e-6, H, attn, hidden, w, b, path=2)
+            for g_, r_ in zip(got, ref):
+                assert torch.equal(g_, r_[rows]), n
+        if fp8:
+            got8 = pkg.hstu_compute_uqvk_fp8(x[rows], nw, nb, 1e-6, H, attn, hidden, w, b, 0.01, 0.011, 0.012)
+            for g_, r_ in zip(got8[:4], ref8[:4]):
+                assert torch.equal(g_.contiguous().view(torch.uint8), r_[rows].contiguous().view(torch.uint8)), n
+            assert torch.equal(got8[4], torch.stack([t[rows].float().abs().max() for t in (ref[3], ref[1], ref[2])])), n
+    torch.cuda.synchronize()
+    end = U.compute_uqvk(host[0][-100:], *host[1:3], 1e-6, H, attn, hidden, *host[3:])
+    for name, g_, r_ in zip("uqkv", ref, end):
+        _close(g_[-100:], r_, name)
+
+
+@pytest.mark.gpu
 def test_uqvk_with_a_total_length_that_changes_from_batch_to_batch(pkg, dev):
     """The hipBLASLt path keeps one plan per size class of the row count, not per row count: lengths of one class
     (1100, 1101, 1279), of others (640, 5000), and the first again, each against the oracle."""
