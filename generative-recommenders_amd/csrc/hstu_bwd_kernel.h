@@ -62,12 +62,41 @@ __device__ __forceinline__ char* ds_pair_base(const BwdParams& bp, const Work& W
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
 constexpr int kKeyBlock = 128, kQueryTile = 64;  // geometry of the key-stationary kernel
 
+// Where blocks hold valid pairs only, as an interval of their first positions: what SeqMask::classify answers with 2, once per
+// workgroup instead of some forty scalar instructions per block.
+struct FullRange {
+    int lo, hi;
+    __device__ __forceinline__ bool has(int first) const { return first >= lo && first <= hi; }
+};
+// the blocks of `nr` query rows all of which see all keys of [s_lo, s_lo + ns)
+__device__ __forceinline__ FullRange full_rows(const SeqMask& M, int s_lo, int ns, int nr) {
+    const int s_hi = s_lo + ns - 1;
+    if (s_hi >= M.n) return {1, 0};
+    const int ids_lo = M.id(s_lo), ids_hi = M.id(s_hi);
+    if (ids_hi >= M.idclamp) return {1, 0};  // (ids stop there: no row is past it)
+    int hi = M.n - nr;
+    if (M.w > 0 && M.w < (1 << 30) && M.w < M.idclamp - ids_lo) {
+        const int last = ids_lo + M.w + M.shift - (nr - 1);
+        hi = last < hi ? last : hi;
+    }
+    return {ids_hi + 1 + M.shift, hi};
+}
+// the blocks of `ns` keys all of which every row of [r_lo, r_hi] sees
+__device__ __forceinline__ FullRange full_keys(const SeqMask& M, int r_lo, int r_hi, int ns) {
+    if (r_hi < r_lo) return {1, 0};
+    const int idr_lo = M.id(r_lo), idr_hi = M.id(r_hi);
+    if (idr_lo < 1) return {1, 0};
+    const int last = idr_lo - 1 + M.shift - (ns - 1), hi = M.n - ns < last ? M.n - ns : last;
+    return {M.w > 0 && idr_hi - M.w > 0 ? idr_hi - M.w + M.shift : 0, hi};
+}
+
 // The tiles of 64 query rows that the key-stationary kernel visits for the 128 keys starting at S0: rows at or after
 // the first key (all rows if a contextual prefix sees every key), up to the last row whose window still reaches the
 // block (targets sit at id max_id); inside that range a tile without a valid pair is passed over.
 struct KeyBlockWalk {
     int first, end;
     bool scan;
+    FullRange full;  // first rows of tiles that hold valid pairs only
     __device__ __forceinline__ void init(const SeqMask& M, bool has_targets, int S0, int n) {
         const int S1 = (S0 + kKeyBlock < n ? S0 + kKeyBlock : n) - 1;
         int q_hi = n - 1;
@@ -82,10 +111,11 @@ struct KeyBlockWalk {
         end = q_hi / kQueryTile + 1;
         first = M.c > 0 ? 0 : S0 / kQueryTile;
         scan = M.w > 0 || M.c > 0 || has_targets;
+        full = full_rows(M, S0, kKeyBlock, kQueryTile);
     }
     __device__ __forceinline__ bool visits(const SeqMask& M, int jt, int S0, int n) const {
         if (jt < first || jt >= end) return false;
-        if (!scan) return true;
+        if (!scan || full.has(jt * kQueryTile)) return true;
         const int r1 = (jt + 1) * kQueryTile < n ? (jt + 1) * kQueryTile - 1 : n - 1;
         return M.classify(jt * kQueryTile, r1, S0, kKeyBlock) != 0;
     }
@@ -170,7 +200,10 @@ __device__ __forceinline__ bool bwd_decode(const FwdParams& p, Work& w, int bid,
     const int pair_local = slot / p.num_mb;
     const int j = slot - pair_local * p.num_mb;
     const int mb = low_first ? j : p.num_mb - 1 - j;
-    const int pair = pair_local * 8 + xcd;
+    // Every other round of eight pairs is dealt the other way round: in order of length, and with the heads of a sequence next to each
+    // other, the first XCDs would get the longer sequences every time (32 sequences of 1024 .. 8192 rows, 4 heads: 1 / 8 of the CU
+    // cycles were idle).
+    const int pair = pair_local * 8 + ((pair_local & 1) ? 7 - xcd : xcd);
     if (pair >= p.B * p.H) return false;
     const int rseq = pair / p.H;
     w.h = pair - rseq * p.H;
@@ -213,11 +246,11 @@ __device__ __forceinline__ bool bwd_decode(const FwdParams& p, Work& w, int bid,
 
 // sigma and its companions for one score: t = c1 * s = -x * log2(e).
 //   p = t * sigma                      (P up to the constant 1 / (c1 * N) * alpha)
-//   g = sigma * (1 + x * (1 - sigma))  = sigma + ln2 * p * (sigma - 1)
+//   g = sigma * (1 + x * (1 - sigma))  = sigma + p * (ln2 * sigma - ln2)
 __device__ __forceinline__ void silu_and_slope(float t, float& p, float& g) {
     const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
     p = t * sig;
-    g = __builtin_fmaf(0.6931471805599453f * p, sig - 1.0f, sig);
+    g = __builtin_fmaf(p, __builtin_fmaf(sig, 0.6931471805599453f, -0.6931471805599453f), sig);
 }
 
 // The same in two pieces whose instructions stay where they are written (the compiler does not look into the asm, so
@@ -620,7 +653,10 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
     const int wR0 = wq0;
     const int wR1 = (wq0 + 32 < n ? wq0 + 32 : n) - 1;
 
-    int jt = next_valid_tile<BN>(W, W.jt_begin);
+    // key tiles and the wave's blocks of 32 keys that hold valid pairs only
+    const FullRange full_tile = full_keys(M, W.R0, W.R1, BN), full_block = full_keys(M, wR0, wR1, 32);
+    auto next_tile = [&](int t) { return t < W.jt_end && full_tile.has(t * BN) ? t : next_valid_tile<BN>(W, t); };
+    int jt = next_tile(W.jt_begin);
     const int jt_end = W.jt_end;
 
     const char* kbase = p.k + (W.seq_start * p.k_rs + (int64_t)W.h * p.k_hs) * 2;
@@ -650,7 +686,7 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
 
     int stage = 0;
     while (jt < jt_end) {
-        const int jn = next_valid_tile<BN>(W, jt + 1);
+        const int jn = next_tile(jt + 1);
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
         if (jn < jt_end) {
@@ -665,7 +701,7 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
             const int s0 = jt * BN + sub * 32;  // first key row of the block of 32
             // one instruction stream for every kind of block (see the key-stationary kernel): a block without a valid
             // pair runs like the others and its dS is cleared afterwards
-            const int cls = M.classify(wR0, wR1, s0, 32);
+            const int cls = full_block.has(s0) ? 2 : M.classify(wR0, wR1, s0, 32);
             f32x16_t s, dp;
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;

@@ -61,7 +61,8 @@ __global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(c
     walk.init(M, p.targets != nullptr, S0, n);
     const int jt_end = walk.end;
     auto next_tile = [&](int jt) { return walk.next(M, jt, S0, n); };
-    auto block_class = [&](int r0) { return block_class32(M, !walk.scan, r0, wS0, n); };
+    const FullRange full = full_rows(M, wS0, 32, 32);
+    auto block_class = [&](int r0) { return full.has(r0) ? 2 : block_class32(M, !walk.scan, r0, wS0, n); };
 
     KeyMask key;
     key.init(M, wS0 + l32);
@@ -325,8 +326,9 @@ __global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(c
                 for (int j = 0; j < 4; ++j) {
                     const unsigned gj = g4[j];  // (a bit_cast of the vector element itself reads element 0)
                     const h2_t g2 = __builtin_bit_cast(h2_t, gj);
-                    d8[2 * j] = dp[8 * h + 2 * j] * (float)g2[0];
-                    d8[2 * j + 1] = dp[8 * h + 2 * j + 1] * (float)g2[1];
+                    // (with the addition one instruction takes the fp16 factor as it is; a product of -0 becomes +0)
+                    d8[2 * j] = __builtin_fmaf(dp[8 * h + 2 * j], (float)g2[0], 0.0f);
+                    d8[2 * j + 1] = __builtin_fmaf(dp[8 * h + 2 * j + 1], (float)g2[1], 0.0f);
                 }
                 dsb[h] = TT::pack8(d8);
             }

@@ -142,3 +142,60 @@ def test_kernel_source_bits_equal_the_kernel_source_predicate(tmp_path):
     subprocess.run([gxx, "-O1", "-std=c++17", str(src), "-o", str(exe)], check=True)
     total, bad = (int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
     assert total > 100_000_000 and bad == 0
+
+
+_FULL_HARNESS = """
+#include <cstdio>
+#define __device__
+#define __forceinline__
+%s
+int main() {
+    long total = 0, bad = 0;
+    const int ws[] = {0, 1, 7, 33, 70, 0x7fffffff};
+    for (int n = 1; n <= 150; n += n < 20 ? 1 : 13) for (int tg = -1; tg <= n && tg < 60; tg += tg < 3 ? 1 : 11) for (int w : ws) for (int c = 0; c <= 12; c += 4)
+    for (int f = 0; f <= 20; f += 20) {
+        SeqMask M; M.n = n; M.w = w; M.c = c; M.f = f; M.shift = c > 0 ? c - 1 : 0;
+        const int t = tg < 0 ? 0 : tg;
+        M.max_id = n - t - M.shift; M.idclamp = tg >= 0 ? M.max_id : 0x7fffffff;
+        for (int s = 0; s < n + 40; s += 5) for (int ns = 32; ns <= 128; ns += 96) for (int nr = 32; nr <= 64; nr += 32) {
+            const FullRange F = full_rows(M, s, ns, nr);
+            for (int r = 0; r < n + 70; ++r, ++total) bad += F.has(r) != (r + nr <= n && M.classify(r, r + nr - 1, s, ns) == 2);
+        }
+        for (int r = 0; r < n; r += 3) for (int nr = 32; nr <= 128; nr += 96) for (int ns = 32; ns <= 64; ns += 32) {
+            const int r1 = (r + nr < n ? r + nr : n) - 1;
+            const FullRange F = full_keys(M, r, r1, ns);
+            for (int s = 0; s < n + 70; ++s, ++total) bad += F.has(s) != (M.classify(r, r1, s, ns) == 2);
+        }
+    }
+    printf("%%ld %%ld\\n", total, bad);
+    return 0;
+}
+"""
+
+
+def test_kernel_source_intervals_of_full_blocks_equal_the_kernel_source_classes(tmp_path):
+    """full_rows() and full_keys() against SeqMask::classify() == 2, for every block start and small mask setting: both ways, so that no
+    block that needs the mask passes without it and none is masked for nothing."""
+    import os
+    import shutil
+    import subprocess
+
+    import pytest
+
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("needs g++")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "generative-recommenders_amd", "csrc")
+    common = open(os.path.join(csrc, "hstu_common.h")).read()
+    bwd = open(os.path.join(csrc, "hstu_bwd_kernel.h")).read()
+
+    def cut(text, begin, end):
+        return text[text.index(begin) : text.index(end)]
+
+    structs = cut(common, "// Per-sequence mask state", "// Chunk swizzles.") + cut(bwd, "// Where blocks hold valid pairs only", "// The tiles of 64 query rows")
+    src = tmp_path / "full.cpp"
+    src.write_text(_FULL_HARNESS % structs)
+    exe = tmp_path / "full"
+    subprocess.run([gxx, "-O1", "-std=c++17", str(src), "-o", str(exe)], check=True)
+    total, bad = (int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
+    assert total > 10_000_000 and bad == 0, (total, bad)
