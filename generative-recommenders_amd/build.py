@@ -63,7 +63,8 @@ def build_library(verbose: bool = False) -> str:
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     common = [hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + ["-I", INCLUDE, "-I", CSRC]
     objs = [os.path.join(CSRC, name) for name in ("hstu_api.o", "hstu_bwd_api.o", "hstu_fwd_fitted.o")]
-    linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o"), os.path.join(CSRC, "hstu_uqvk.o")]
+    linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o"), os.path.join(CSRC, "hstu_uqvk.o"),
+                   os.path.join(CSRC, "hstu_uqvk_bwd.o")]
     jobs = [
         common + ["-c", os.path.join(CSRC, "hstu_api.hip"), "-o", objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_bwd_api.hip"), "-o", objs[1]],
@@ -72,10 +73,11 @@ def build_library(verbose: bool = False) -> str:
         common + ["-c", os.path.join(CSRC, "hstu_linear_bwd.hip"), "-o", linear_objs[1]],
         # (matrix results in vector registers: see the file)
         common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_uqvk.hip"), "-o", linear_objs[2]],
+        common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_uqvk_bwd.hip"), "-o", linear_objs[3]],
     ]
     native_compile, native_link, native_obj = _native_commands()
     jobs.append(native_compile)
-    with ThreadPoolExecutor(max_workers=7) as pool:
+    with ThreadPoolExecutor(max_workers=8) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB_PATH], verbose)
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + linear_objs + ["-o", LINEAR_LIB_PATH, "-lhipblaslt"], verbose)

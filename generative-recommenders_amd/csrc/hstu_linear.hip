@@ -18,8 +18,11 @@
 #include "hstu_uqvk_kernel.h"
 #include "hstu_output_kernel.h"
 
-// hstu_uqvk.hip
+// hstu_uqvk.hip, hstu_uqvk_bwd.hip
 int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
+int hstu_uqvk_grad_u_launch(const hstu::UqvkFusedParams& p, int depth, bool bf16, hipStream_t stream);
+bool hstu_product_t_takes(int64_t rows, int depth, int n);
+int hstu_product_t_launch(const hstu::UqvkFusedParams& p, int depth, bool bf16, hipStream_t stream);
 
 namespace {
 
@@ -403,9 +406,10 @@ int rows_class(long long rows) {
 struct GemmShape {
     long long ldw, ldact, ldres, ldd;
     int rows_class, k, n, dtype, epi, device;
+    bool trans;
     bool operator<(const GemmShape& o) const {
-        return std::tie(rows_class, ldw, ldact, ldres, ldd, k, n, dtype, epi, device) <
-               std::tie(o.rows_class, o.ldw, o.ldact, o.ldres, o.ldd, o.k, o.n, o.dtype, o.epi, o.device);
+        return std::tie(rows_class, ldw, ldact, ldres, ldd, k, n, dtype, epi, device, trans) <
+               std::tie(o.rows_class, o.ldw, o.ldact, o.ldres, o.ldd, o.k, o.n, o.dtype, o.epi, o.device, o.trans);
     }
 };
 
@@ -418,16 +422,16 @@ int blaslt_fail(const char* what, hipblasStatus_t st) {
     return HSTU_LINEAR_ERR_BLASLT;
 }
 
-// `residual` (row stride ldres) may be null: then ldres must be 0 and beta is 0.
+// `residual` (row stride ldres) may be null: then ldres must be 0 and beta is 0.  `trans`: weight is [n, k].
 int gemm(const void* act, int64_t ldact, const void* weight, int64_t ldw, const void* bias, const void* residual, int64_t ldres,
-         void* out, int64_t ldd, int64_t rows, int k, int n, int dtype, int epi, void* scratch, hipStream_t stream) {
+         void* out, int64_t ldd, int64_t rows, int k, int n, int dtype, int epi, void* scratch, hipStream_t stream, bool trans = false) {
     if (n == 0 || rows == 0) return 0;
     std::lock_guard<std::mutex> lock(g_mutex);
     hipblasStatus_t st;
     if (!g_handle && (st = hipblasLtCreate(&g_handle)) != HIPBLAS_STATUS_SUCCESS) return blaslt_fail("hipblasLtCreate", st);
     int dev = 0;
     (void)hipGetDevice(&dev);
-    const GemmShape key{(long long)ldw, (long long)ldact, (long long)ldres, (long long)ldd, rows_class(rows), k, n, dtype, epi, dev};
+    const GemmShape key{(long long)ldw, (long long)ldact, (long long)ldres, (long long)ldd, rows_class(rows), k, n, dtype, epi, dev, trans};
     const hipDataType t = dtype == 0 ? HIP_R_16BF : HIP_R_16F;
     auto set_rows = [&](GemmPlan& pl) -> hipblasStatus_t {
         if (pl.rows == rows) return HIPBLAS_STATUS_SUCCESS;
@@ -465,6 +469,11 @@ int gemm(const void* act, int64_t ldact, const void* weight, int64_t ldw, const 
         GemmPlan pl;
         if ((st = hipblasLtMatmulDescCreate(&pl.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F)) != HIPBLAS_STATUS_SUCCESS)
             return blaslt_fail("hipblasLtMatmulDescCreate", st);
+        if (trans) {
+            const hipblasOperation_t op = HIPBLAS_OP_T;
+            if ((st = hipblasLtMatmulDescSetAttribute(pl.desc, HIPBLASLT_MATMUL_DESC_TRANSA, &op, sizeof(op))) != HIPBLAS_STATUS_SUCCESS)
+                return blaslt_fail("hipblasLtMatmulDescSetAttribute", st);
+        }
         if (epi != kEpiNone) {
             const hipblasLtEpilogue_t e = epi == kEpiBiasSilu ? HIPBLASLT_EPILOGUE_SWISH_BIAS_EXT : HIPBLASLT_EPILOGUE_BIAS;
             st = hipblasLtMatmulDescSetAttribute(pl.desc, HIPBLASLT_MATMUL_DESC_EPILOGUE, &e, sizeof(e));
@@ -477,7 +486,7 @@ int gemm(const void* act, int64_t ldact, const void* weight, int64_t ldw, const 
                 st = hipblasLtMatmulDescSetAttribute(pl.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias, sizeof(bias));
             if (st != HIPBLAS_STATUS_SUCCESS) return blaslt_fail("hipblasLtMatmulDescSetAttribute", st);
         }
-        if ((st = hipblasLtMatrixLayoutCreate(&pl.a, t, n, k, ldw)) != HIPBLAS_STATUS_SUCCESS || (st = set_rows(pl)) != HIPBLAS_STATUS_SUCCESS)
+        if ((st = hipblasLtMatrixLayoutCreate(&pl.a, t, trans ? k : n, trans ? n : k, ldw)) != HIPBLAS_STATUS_SUCCESS || (st = set_rows(pl)) != HIPBLAS_STATUS_SUCCESS)
             return blaslt_fail("hipblasLtMatrixLayoutCreate", st);
         if ((st = ask_heuristic(pl)) != HIPBLAS_STATUS_SUCCESS) return blaslt_fail("hipblasLtMatmulAlgoGetHeuristic", st);
         it = g_plans.emplace(key, pl).first;
@@ -604,6 +613,9 @@ int launch_uqvk_fused(hstu::UqvkFusedParams p, hipStream_t stream) {
     return 0;
 }
 
+// (byte offsets inside 64 rows have 32 bits)
+bool product_stride(int64_t stride, int64_t width) { return stride >= width && (stride & 7) == 0 && stride < (1 << 22); }
+
 size_t normed_bytes(const HstuUqvkArgs* a) { return (((size_t)a->rows * a->d_model * 2) + 255) & ~(size_t)255; }
 size_t joined_bytes(const HstuOutputArgs* a) {
     return (((size_t)a->rows * output_blocks(a) * a->heads * a->linear_dim * 2) + 255) & ~(size_t)255;
@@ -678,6 +690,7 @@ int hstu_uqvk_forward(const HstuUqvkArgs* a, void* stream_) {
         p.x = (const char*)a->x, p.x_rs = a->x_row_stride;
         p.norm_weight = (const char*)a->norm_weight, p.norm_bias = (const char*)a->norm_bias, p.eps = a->norm_eps;
         p.w = (const char*)a->uvqk_weight, p.bias = (const char*)a->uvqk_bias, p.out = (char*)a->uvqk;
+        p.w_rs = p.out_rs = n_out, p.du = nullptr, p.du_rs = 0;
         p.rows = a->rows, p.n_out = n_out, p.n_silu = n_u;
         p.out8 = (unsigned char*)a->qkv_fp8, p.absmax = (unsigned*)a->qkv_absmax, p.n_attn = a->attn_dim * a->heads;
         if (a->qkv_fp8) {
@@ -715,6 +728,48 @@ int hstu_uqvk_forward(const HstuUqvkArgs* a, void* stream_) {
     if (rc != 0) return rc;
     return gemm(normed, a->d_model, w + (int64_t)n_u * 2, n_out, b + (int64_t)n_u * 2, nullptr, 0, o + (int64_t)n_u * 2, n_out, a->rows,
                 a->d_model, n_out - n_u, a->dtype, kEpiBias, scratch, stream);
+}
+
+int hstu_uqvk_u_grad(const void* x, int64_t x_row_stride, const void* norm_weight, const void* norm_bias, float eps, const void* weight,
+                     int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride, int64_t rows,
+                     int32_t d_model, int32_t width, int32_t dtype, void* stream) {
+    g_last_error[0] = 0;
+    if (rows < 0 || rows > 0x7fffffffLL || d_model <= 0 || width <= 0 || (dtype != 0 && dtype != 1)) return -5;
+    if ((d_model != 128 && d_model != 256 && d_model != 384 && d_model != 512) || width % 128 != 0 || width > (1 << 20)) return -6;
+    if (rows == 0) return 0;
+    if (!x || !norm_weight || !norm_bias || !weight || !bias || !du || !out) return -1;
+    const uintptr_t ptrs = (uintptr_t)x | (uintptr_t)norm_weight | (uintptr_t)norm_bias | (uintptr_t)weight | (uintptr_t)bias | (uintptr_t)du | (uintptr_t)out;
+    if ((ptrs & 15) != 0) return -4;
+    if (!product_stride(x_row_stride, d_model) || !product_stride(weight_row_stride, width) || !product_stride(du_row_stride, width) ||
+        !product_stride(out_row_stride, width))
+        return -5;
+    hstu::UqvkFusedParams p{};
+    p.x = (const char*)x, p.x_rs = x_row_stride, p.norm_weight = (const char*)norm_weight, p.norm_bias = (const char*)norm_bias, p.eps = eps;
+    p.w = (const char*)weight, p.w_rs = weight_row_stride, p.bias = (const char*)bias, p.du = (const char*)du, p.du_rs = du_row_stride;
+    p.out = (char*)out, p.out_rs = out_row_stride, p.rows = rows, p.n_out = width;
+    return hstu_uqvk_grad_u_launch(p, d_model, dtype == 0, (hipStream_t)stream);
+}
+
+size_t hstu_linear_product_t_workspace_bytes(int64_t rows, int32_t k, int32_t n) { return hstu_product_t_takes(rows, k, n) ? 0 : kGemmScratch; }
+
+int hstu_linear_product_t(const void* a, int64_t a_row_stride, const void* weight, int64_t weight_row_stride, int64_t rows, int32_t k, int32_t n,
+                          int32_t dtype, void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes, void* stream) {
+    g_last_error[0] = 0;
+    if (rows < 0 || rows > 0x7fffffffLL || k <= 0 || n <= 0 || (k & 7) != 0 || (n & 7) != 0 || (dtype != 0 && dtype != 1)) return -5;
+    if (rows == 0) return 0;
+    if (!a || !weight || !out) return -1;
+    if ((((uintptr_t)a | (uintptr_t)weight | (uintptr_t)out) & 15) != 0) return -4;
+    if (!product_stride(a_row_stride, k) || !product_stride(weight_row_stride, k) || !product_stride(out_row_stride, n)) return -5;
+    if (!hstu_product_t_takes(rows, k, n)) {
+        if (!workspace) return -1;
+        if ((size_t)workspace_bytes < kGemmScratch || ((uintptr_t)workspace & 255) != 0) return -4;
+        return gemm(a, a_row_stride, weight, weight_row_stride, nullptr, nullptr, 0, out, out_row_stride, rows, k, n, dtype, kEpiNone, workspace,
+                    (hipStream_t)stream, true);
+    }
+    hstu::UqvkFusedParams p{};
+    p.x = (const char*)a, p.x_rs = a_row_stride, p.w = (const char*)weight, p.w_rs = weight_row_stride;
+    p.out = (char*)out, p.out_rs = out_row_stride, p.rows = rows, p.n_out = n;
+    return hstu_product_t_launch(p, k, dtype == 0, (hipStream_t)stream);
 }
 
 size_t hstu_output_workspace_bytes(const HstuOutputArgs* a) {

@@ -380,6 +380,19 @@ constexpr int64_t kWeightGradColumns = 65536;
 
 void check_linear(int rc) { TORCH_CHECK(rc == 0, "hstu_linear: status ", rc, " (", hstu_linear_last_error(), ")"); }
 
+// a @ weight^T
+Tensor product_t(const Tensor& a, const Tensor& weight) {
+    const int64_t rows = a.size(0), n = weight.size(0);
+    const int32_t k = (int32_t)a.size(1);
+    Tensor out = at::empty({rows, n}, a.options()), scratch;
+    const size_t need = hstu_linear_product_t_workspace_bytes(rows, k, (int32_t)n);
+    void* workspace = nullptr;
+    if (need > 0) scratch = aligned_scratch(need, a, &workspace);
+    check_linear(hstu_linear_product_t(a.const_data_ptr(), a.stride(0), weight.const_data_ptr(), weight.stride(0), rows, k, (int32_t)n, dense_dtype(a),
+                                       out.data_ptr(), n, workspace, (int64_t)need, stream_of(a)));
+    return out;
+}
+
 // a^T @ b, and the column sums of b where `b_sums` is defined.
 Tensor weight_grad(const Tensor& a, const Tensor& b, const Tensor& b_sums) {
     Tensor out = at::empty({a.size(1), b.size(1)}, a.options());
@@ -402,23 +415,31 @@ variable_list uqvk_backward(const AutogradContext* ctx, const Tensor& x, const T
     const c10::DeviceGuard guard(x.device());
     void* stream = stream_of(x);
     variable_list got(5);
+    Tensor d_u = d.narrow(1, 0, n_u);
+    bool u_done = !du.defined();
+    if (u_done) {
+        d_u.zero_();
+    } else {
+        du = gradient_rows(du);
+        const int rc = hstu_uqvk_u_grad(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
+                                        weight.const_data_ptr(), weight.stride(0), bias.const_data_ptr(), du.const_data_ptr(), du.stride(0), d_u.data_ptr(),
+                                        d_u.stride(0), rows, (int32_t)dm, (int32_t)n_u, dense_dtype(x), stream);
+        if (rc != -6 && rc != -5) check_linear(rc);  // (another shape: the product and what follows it below)
+        u_done = rc == 0;
+    }
     Tensor normed;
-    if (du.defined() || weight_wanted) {
+    if (!u_done || weight_wanted) {
         normed = at::empty({rows, dm}, x.options());
         check_linear(hstu_uqvk_layer_norm(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
                                           normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
     }
-    Tensor d_u = d.narrow(1, 0, n_u);
-    if (du.defined()) {
-        du = gradient_rows(du);
+    if (!u_done) {
         at::mm_out(d_u, normed, weight.narrow(1, 0, n_u));
         check_linear(hstu_uqvk_silu_bwd(d_u.data_ptr(), d_u.stride(0), bias.const_data_ptr(), du.const_data_ptr(), du.stride(0), rows, n_u,
                                         dense_dtype(x), stream));
-    } else {
-        d_u.zero_();
     }
     if (rows_wanted) {
-        Tensor dy = at::mm(d, weight.t());
+        Tensor dy = product_t(d, weight);
         got[0] = at::empty({rows, dm}, x.options()), got[1] = at::empty_like(norm_weight), got[2] = at::empty_like(norm_bias);
         const int64_t need = (int64_t)hstu_uqvk_layer_norm_bwd_workspace_bytes(rows, (int32_t)dm);
         Tensor scratch = at::empty({need}, x.options().dtype(at::kByte));
@@ -617,7 +638,8 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
         got[2] = grads[0].requires_grad() ? grads[0].clone() : grads[0];
         const bool weight_too = ctx->needs_input_grad(5);
         if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4)) {
-            const Tensor dj = at::mm(dout, weight.t());
+            const c10::DeviceGuard guard(attn.device());
+            const Tensor dj = product_t(dout, weight);
             Tensor joined = weight_too ? at::empty_like(dj) : Tensor();
             got[0] = at::empty({rows, width}, attn.options()), got[1] = at::empty({rows, width}, attn.options());
             got[3] = at::empty_like(norm_weight), got[4] = at::empty_like(norm_bias);
@@ -631,7 +653,6 @@ struct OutputFunction : torch::autograd::Function<OutputFunction> {
             g.workspace_bytes = (int64_t)hstu_output_norm_mul_bwd_workspace_bytes(&a);
             Tensor scratch = at::empty({g.workspace_bytes}, attn.options().dtype(at::kByte));
             g.workspace = scratch.data_ptr();
-            const c10::DeviceGuard guard(attn.device());
             check_linear(hstu_output_norm_mul_bwd(&a, &g, stream_of(attn)));
             if (weight_too) got[5] = weight_grad(joined, dout, Tensor());
         } else if (weight_too) {

@@ -1,121 +1,7 @@
-// The producer's kernels and which of them a call takes (libhstu_linear.so).  A translation unit of its own because it is compiled with the
-// matrix instructions' VGPR form: the normalised rows fill the accumulation registers, the sums stay where vector
-// instructions can read them (with the other form the kernels copy their sums per column block and spill).
-#include "hstu_uqvk_kernel.h"
-#include "hstu_uqvk_wide_kernel.h"
-
-#include <atomic>
-#include <cstdio>
-#include <type_traits>
-
-// defined in hstu_linear.hip; internal to the library
-extern "C" __attribute__((visibility("hidden"))) void hstu_linear_set_last_error(const char* text);
-int hstu_uqvk_fused_launch(hstu::UqvkFusedParams p, int d_model, bool bf16, hipStream_t stream);
-
-namespace {
-
-int fail(const char* what, hipError_t e) {
-    char text[256];
-    snprintf(text, sizeof(text), "%s: %s", what, hipGetErrorString(e));
-    hstu_linear_set_last_error(text);
-    return -7;
-}
-
-// Launches `kern` with `lds` bytes of dynamic LDS, of which it never asks for more than `most`.
-int launch(void (*kern)(hstu::UqvkFusedParams), std::atomic<bool> (&attr_done)[64], int most, int lds, dim3 grid, const hstu::UqvkFusedParams& p,
-           hipStream_t stream) {
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
-    if (dev < 0 || !attr_done[dev]) {  // (a function attribute belongs to the device it was set on)
-        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, most);
-        if (e != hipSuccess) return fail("fused uqvk kernel attribute", e);
-        if (dev >= 0) attr_done[dev] = true;
-    }
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, p);
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : fail("fused uqvk kernel launch", e);
-}
-
-template <class TT, int KT, bool OUT8>
-int launch_wide(hstu::UqvkFusedParams p, hipStream_t stream) {
-    static std::atomic<bool> attr_done[64];
-    p.units = (int)((p.rows + hstu::kWideRows - 1) / hstu::kWideRows) * (p.n_out / hstu::kWideCols);
-    const int grid = p.units < 256 ? p.units : 256;  // one workgroup per CU
-    p.units_per_wave = p.units / grid;
-    return launch(hstu::hstu_uqvk_wide_kernel<TT, KT, OUT8>, attr_done, hstu::kWideLds<KT>, hstu::kWideLds<KT>, dim3((unsigned)grid), p, stream);
-}
-
-template <class TT, int KT, int RB, int NB, bool OUT8>
-int launch_rows(hstu::UqvkFusedParams p, int units_per_wave, hipStream_t stream) {
-    static std::atomic<bool> attr_done[64];
-    typedef hstu::UqvkRows<KT, RB, NB> Geo;
-    const long long blocks = (p.rows + RB * 32 - 1) / (RB * 32);
-    const int units = (p.n_out / NB + 3) / 4;  // of a wave that walks its quarter of all columns
-    p.units_per_wave = units_per_wave < units ? units_per_wave : units;
-    const unsigned splits = (unsigned)((units + p.units_per_wave - 1) / p.units_per_wave);
-    return launch(hstu::hstu_uqvk_rows_kernel<TT, KT, RB, NB, OUT8>, attr_done, Geo::lds(hstu::kUqvkMostUnits), Geo::lds(p.units_per_wave),
-                  dim3((unsigned)blocks, splits), p, stream);
-}
-
-enum class Kernel { kRows32, kRows64, kFused, kWide };
-struct Choice {
-    Kernel kernel;
-    int units_per_wave;
-};
-
-// The kernel of a call.  All sizes in us, this rule's choice against the kernel on the other side of the line.
-//   * kWide where its work, row blocks of 256 x column blocks of 64, gives each CU 16 units or more; below that the rows' preparation, 256
-//     at a time on one CU, outweighs the faster matrix phase.  Against kFused, d_model 512 into 2048 columns: 26000 rows 91 / 87, 32768
-//     85 / 100, 139264 329 / 408; into 4096: 12000 rows 87 / 83, 16384 88 / 98.  Against kRows64, d_model 256 into 2048: 24000 rows 52 / 48,
-//     45000 77 / 88; into 512: 90000 rows 61 / 52.  Columns: into 256 it is slower at every size (300000 rows of d_model 512: 197 / 177).
-//   * kRows32 while all column units can be waves of their own in one round of workgroups, two per CU: d_model 512 into 2048 columns, 1000
-//     rows 10.3, kRows64 12.4; 2000 rows (two rounds) 18.5 / 13.8.  Few columns, up to 256: up to two rounds of workgroups that hold all of
-//     them: d_model 512 into 128 columns, 24000 rows 14.5, kRows64 23.0, kFused 17.8; 90000 rows 45.5 / 72.1 / 41.1.
-//   * kRows64, dividing the columns over as many workgroups as one round holds (one per CU, two up to d_model 256): d_model 512 into 2048,
-//     4000 rows with 2 units per wave 21.3, with 1 29.0, with 4 27.5.  More rounds, and more than 8 units per wave, are kFused's at d_model 384 and 512 (into 512 columns, 24000
-//     rows 35.1 / 33.4, 90000 rows 109 / 88; into 4096, 12000 rows 92 / 81) and kRows64's below (d_model 256 into 512 columns, 45000 rows 29.3 / 38.3).
-Choice choose(const hstu::UqvkFusedParams& p, int kt) {
-    const long long wide_units = (p.rows + 255) / 256 * (p.n_out / 64);
-    const bool whole64 = p.n_silu % 64 == 0;  // (SiLU per 64 columns)
-    if (kt >= 4 && p.n_out >= 512 && whole64 && wide_units >= 4096 && wide_units <= 0x7fffffffLL) return {Kernel::kWide, 0};
-    const int quarter32 = p.n_out / 128;  // column units of a wave that walks a quarter of the columns
-    const long long blocks32 = (p.rows + 31) / 32, blocks64 = (p.rows + 63) / 64;
-    if (blocks32 * quarter32 <= 512) return {Kernel::kRows32, 1};
-    if (p.n_out <= 256 && kt > 4 && blocks32 <= 1024) return {Kernel::kRows32, quarter32};
-    const int quarter = kt <= 4 ? quarter32 : (quarter32 + 1) / 2, round = kt <= 4 ? 512 : 256;
-    if (kt <= 4 || whole64) {
-        for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2)
-            if (blocks64 * ((quarter + per - 1) / per) <= round) return {Kernel::kRows64, per};
-        if (kt <= 4) return {Kernel::kRows64, hstu::kUqvkMostUnits};
-    }
-    return {Kernel::kFused, 0};
-}
-
-template <class TT, int KT, bool OUT8>
-int launch_depth(const hstu::UqvkFusedParams& p, hipStream_t stream) {
-    const Choice c = choose(p, KT);
-    if constexpr (KT >= 4)
-        if (c.kernel == Kernel::kWide) return launch_wide<TT, KT, OUT8>(p, stream);
-    if constexpr (KT > 4)
-        if (c.kernel == Kernel::kFused) return hstu_uqvk_fused_launch(p, KT * 64, std::is_same<TT, hstu::Bf16>::value, stream);
-    if (c.kernel == Kernel::kRows32) return launch_rows<TT, KT, 1, 32, OUT8>(p, c.units_per_wave, stream);
-    return launch_rows<TT, KT, 2, (KT <= 4 ? 32 : 64), OUT8>(p, c.units_per_wave, stream);
-}
-
-template <class TT, bool OUT8>
-int launch_type(const hstu::UqvkFusedParams& p, int d_model, hipStream_t stream) {
-    switch (d_model) {
-        case 128: return launch_depth<TT, 2, OUT8>(p, stream);
-        case 256: return launch_depth<TT, 4, OUT8>(p, stream);
-        case 384: return launch_depth<TT, 6, OUT8>(p, stream);
-        default: return launch_depth<TT, 8, OUT8>(p, stream);
-    }
-}
-
-}  // namespace
+// The producer's kernels (libhstu_linear.so).  A translation unit of its own because of how it is compiled: see hstu_uqvk_launch.h.
+#include "hstu_uqvk_launch.h"
 
 // d_model: 128, 256, 384 or 512
 int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream) {
-    if (bf16) return p.out8 ? launch_type<hstu::Bf16, true>(p, d_model, stream) : launch_type<hstu::Bf16, false>(p, d_model, stream);
-    return p.out8 ? launch_type<hstu::Fp16, true>(p, d_model, stream) : launch_type<hstu::Fp16, false>(p, d_model, stream);
+    return p.out8 ? launch_mode<hstu::kUqvkForward8>(p, d_model, bf16, stream) : launch_mode<hstu::kUqvkForward>(p, d_model, bf16, stream);
 }

@@ -38,9 +38,13 @@ struct UqvkFusedParams {
     const char* norm_weight;
     const char* norm_bias;
     float eps;
-    const char* w;     // [K, n_out] row-major
+    const char* w;     // [K, n_out] row-major (the product with a transposed matrix: [n_out, K])
+    int64_t w_rs;      // its row stride in elements
     const char* bias;  // [n_out]
-    char* out;         // [rows, n_out] dense
+    char* out;         // [rows, n_out]
+    int64_t out_rs;    // its row stride in elements
+    const char* du;    // (gradient of u) [rows, n_out]
+    int64_t du_rs;
     int64_t rows;
     int n_out;   // multiple of 128
     int n_silu;  // multiple of 32: columns [0, n_silu) go through SiLU
@@ -214,12 +218,19 @@ struct UqvkRows {
     static constexpr int lds(int units_per_wave) { return kBias + units_per_wave * 4 * NB * 2; }
 };
 
-template <class TT, int KT, int RB, int NB, bool OUT8>  // KT = d_model / 64
+// What the kernel computes from its products.
+//   kUqvkForward, kUqvkForward8: the producer, without and with the e4m3 copy
+//   kUqvkGradU: out = du * SiLU'(LN(x) W + bias), the gradient of the u columns' products; nothing of the forward is read but x
+//   kProductT: out = x W^T, no norm, no bias: W's k run along its rows, so its tiles are read as they lie
+enum { kUqvkForward, kUqvkForward8, kUqvkGradU, kProductT };
+
+template <class TT, int KT, int RB, int NB, int MODE>  // KT = d_model / 64
 __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk_rows_kernel(const UqvkFusedParams p) {
     typedef typename TT::vec8 vec8;
     typedef typename TT::elem elem;
     typedef __attribute__((ext_vector_type(4))) elem elem4;
     typedef UqvkRows<KT, RB, NB> Geo;
+    constexpr bool OUT8 = MODE == kUqvkForward8, BIAS = MODE != kProductT, TRANS = MODE == kProductT;
     constexpr int K = Geo::K, KS = K / 16, DT = NB / 32, RING = Geo::kRing, TILES = K / 32;  // TILES: of a unit
     constexpr int COPIES = Geo::kTile / 1024, RPC = 1024 / (NB * 2), CH = NB / 8;             // copies of a tile, k rows of a copy, chunks of a k row
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -228,17 +239,17 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 5, l32 = lane & 31;
     const int64_t row0 = (int64_t)blockIdx.x * (RB * 32);
-    // Units: number (w units_per_wave + i) splits + y is the i-th of wave w in workgroup y of a row block's `splits`, as far as there are
-    // columns.  All lines of a unit's W tiles lie a row of W apart, often a multiple of the interleave of the L2's channels: the waves that
-    // run together should be at columns that are far apart, and the workgroups of an XCD start at different ones of theirs.
-    const int splits = (int)gridDim.y, of_y = (p.n_out / NB - (int)blockIdx.y + splits - 1) / splits;
-    const int left = of_y - wave * p.units_per_wave;
+    // Units: number (y units_per_wave + i) 4 + w is the i-th of wave w in workgroup y of a row block, as far as there are columns.  All lines of a
+    // unit's W tiles lie a row of W apart, often a multiple of the interleave of the L2's channels: the workgroups of an XCD start at
+    // different ones of their units.
+    const int left = (p.n_out / NB - wave + 3) / 4 - (int)blockIdx.y * p.units_per_wave;
     const int units = left < 0 ? 0 : left < p.units_per_wave ? left : p.units_per_wave;
     const int ntiles = units * TILES;
     const int turn = units > 0 ? (int)(blockIdx.x >> 3) % units : 0;
+    const int col0_wg = (int)blockIdx.y * p.units_per_wave * 4 * NB;  // first column of the workgroup
     auto col_of = [&](int u) __attribute__((always_inline)) {
         const int i = u + turn < units ? u + turn : u + turn - units;
-        return ((wave * p.units_per_wave + i) * splits + (int)blockIdx.y) * NB;
+        return col0_wg + (i * 4 + wave) * NB;
     };
 
     // ---- the rows, a quarter for each wave: a row lies across LANES x 2 lanes
@@ -255,12 +266,11 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
         if (holds) xv[i] = *(const vec8*)(p.x + (r * p.x_rs + chunk_of * 8) * 2);
     }
     wv = vec8{}, bv = vec8{};
-    if (holds) wv = *(const vec8*)(p.norm_weight + chunk_of * 16), bv = *(const vec8*)(p.norm_bias + chunk_of * 16);
-    {  // the bias values of the workgroup's columns
+    if (MODE != kProductT && holds) wv = *(const vec8*)(p.norm_weight + chunk_of * 16), bv = *(const vec8*)(p.norm_bias + chunk_of * 16);
+    if constexpr (BIAS) {  // the bias values of the workgroup's columns
         const int cols = p.units_per_wave * 4 * NB;
         for (int c = threadIdx.x * 8; c < cols; c += 256 * 8) {
-            const int col = (c / NB * splits + (int)blockIdx.y) * NB + c % NB;
-            if (col < p.n_out) *HSTU_LDS(vec8, smem + Geo::kBias + c * 2) = *(const vec8*)(p.bias + (int64_t)col * 2);
+            if (col0_wg + c < p.n_out) *HSTU_LDS(vec8, smem + Geo::kBias + c * 2) = *(const vec8*)(p.bias + (int64_t)(col0_wg + c) * 2);
         }
     }
 
@@ -268,13 +278,19 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     unsigned coff[COPIES];
 #pragma unroll
     for (int i = 0; i < COPIES; ++i) {
-        const int row = i * RPC + lane / CH, c = lane % CH;
-        coff[i] = (unsigned)row * (unsigned)(p.n_out * 2) + (unsigned)((NB == 64 ? c ^ swz_w64(row) : c) * 16);
+        if constexpr (TRANS) {  // NB rows of 64 bytes, swizzled for 16 rows' reads of one chunk
+            const int row = i * 16 + lane / 4, c = (lane & 3) ^ ((row >> 2) & 3);
+            coff[i] = (unsigned)row * (unsigned)(p.w_rs * 2) + (unsigned)(c * 16);
+        } else {
+            const int row = i * RPC + lane / CH, c = lane % CH;
+            coff[i] = (unsigned)row * (unsigned)(p.w_rs * 2) + (unsigned)((NB == 64 ? c ^ swz_w64(row) : c) * 16);
+        }
     }
     auto slot_at = [&](int slot) __attribute__((always_inline)) { return smem + (slot * 4 + wave) * Geo::kTile; };
     auto issue_one = [&](int t, int slot, int i) __attribute__((always_inline)) {
         const int u = t / TILES, kt = t - u * TILES;
-        global_load_lds16_soff(p.w + ((int64_t)kt * 32 * p.n_out + col_of(u)) * 2, coff[i], slot_at(slot) + i * 1024);
+        const int64_t first = TRANS ? (int64_t)col_of(u) * p.w_rs + kt * 32 : (int64_t)kt * 32 * p.w_rs + col_of(u);
+        global_load_lds16_soff(p.w + first * 2, coff[i], slot_at(slot) + i * 1024);
     };
     auto issue = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
@@ -287,11 +303,14 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     char* const panel = smem + Geo::kEarly * 4 * Geo::kTile;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-        const float mean = ln_mean<K>(ln_tree_lanes<LANES>(ln_chunk_sum(xv[i])));
-        const float sq = ln_chunk_squares(xv[i], mean);
-        const float rstd = ln_rstd<K>(ln_tree_lanes<LANES>(holds ? sq : 0.f), p.eps);
+        if constexpr (MODE != kProductT) {
+            const float mean = ln_mean<K>(ln_tree_lanes<LANES>(ln_chunk_sum(xv[i])));
+            const float sq = ln_chunk_squares(xv[i], mean);
+            const float rstd = ln_rstd<K>(ln_tree_lanes<LANES>(holds ? sq : 0.f), p.eps);
+            xv[i] = ln_chunk_apply<vec8, elem>(xv[i], mean, rstd, wv, bv);
+        }
         const int row = (wave * NP + i) * RPI + sub;
-        if (holds) *HSTU_LDS(vec8, panel + row * (K * 2) + ((chunk_of ^ (row & 15)) * 16)) = ln_chunk_apply<vec8, elem>(xv[i], mean, rstd, wv, bv);
+        if (holds) *HSTU_LDS(vec8, panel + row * (K * 2) + ((chunk_of ^ (row & 15)) * 16)) = xv[i];
     }
     __syncthreads();
     vec8 xreg[RB][KS];
@@ -327,7 +346,14 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     // the operands of a tile, each of which RB MFMAs use: 16 k, 32 columns
     constexpr int OPS = 2 * DT;
     vec8 fr[OPS];
+    int taddr[2];  // (transposed W: the lane's column, chunk 2 kk + g of its 32 k)
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) taddr[kk] = l32 * 64 + (((2 * kk + g) ^ ((l32 >> 2) & 3)) * 16);
     auto load_op = [&](int slot, int op) __attribute__((always_inline)) {
+        if constexpr (TRANS) {
+            fr[op] = *HSTU_LDS(const vec8, slot_at(slot) + (op % DT) * 2048 + taddr[op / DT]);
+            return;
+        }
         const char* tile = slot_at(slot) + (op / DT) * 16 * (NB * 2);
         fr[op] = read_vt_operand<TT>(tile + waddr[0][op % DT], tile + waddr[1][op % DT]);
     };
@@ -347,8 +373,7 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     elem4 b4[DT][4];
     i32x4_t rd[STORES];
     auto read_bias = [&](int u) __attribute__((always_inline)) {
-        const int i = u + turn < units ? u + turn : u + turn - units;
-        const char* b = smem + Geo::kBias + (wave * p.units_per_wave + i) * NB * 2 + g * 8;
+        const char* b = smem + Geo::kBias + (col_of(u) - col0_wg) * 2 + g * 8;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -358,7 +383,7 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
         const int rb = i / (4 * DT), dt = i / 4 % DT, r4 = i % 4;
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = sums[rb][dt][r4 * 4 + j] + (float)b4[dt][r4][j];
+        for (int j = 0; j < 4; ++j) v[j] = BIAS ? sums[rb][dt][r4 * 4 + j] + (float)b4[dt][r4][j] : sums[rb][dt][r4 * 4 + j];
         if (silu) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = v[j] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v[j]));
@@ -368,7 +393,8 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     auto read_rows = [&](int i) __attribute__((always_inline)) {
         rd[i % STORES] = *HSTU_LDS(const i32x4_t, stage + (i % STORES * RPS + rsub) * Geo::kStageRow + chunk * 16);
     };
-    char* const obase = p.out + row0 * p.n_out * 2;
+    char* const obase = p.out + row0 * p.out_rs * 2;
+    const char* const dbase = MODE == kUqvkGradU ? p.du + row0 * p.du_rs * 2 : nullptr;
     unsigned char* const obase8 = OUT8 ? p.out8 + row0 * (p.n_out - p.n_silu) : nullptr;
     const int rows_here = p.rows - row0 < RB * 32 ? (int)(p.rows - row0) : RB * 32;
     // (computed where it is used: hoisted out of the loop, the addresses of all stores take registers that the rows need)
@@ -377,9 +403,25 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
         asm volatile("" : "+v"(r));
         return i * RPS + r;
     };
+    vec8 dv[RB * STORES];
+    auto read_du = [&](int i, int col0) __attribute__((always_inline)) {
+        int r = orow(i);
+        r = r < rows_here ? r : rows_here - 1;
+        dv[i] = *(const vec8*)(dbase + (int64_t)col0 * 2 + ((unsigned)r * (unsigned)(p.du_rs * 2) + chunk * 16));
+    };
     auto store_rows = [&](int i, int col0) __attribute__((always_inline)) {
         const int r = orow(i);
-        if (r < rows_here) *(i32x4_t*)(obase + (int64_t)col0 * 2 + ((unsigned)r * (unsigned)(p.n_out * 2) + chunk * 16)) = rd[i % STORES];
+        if constexpr (MODE == kUqvkGradU) {  // (the rounded sums, as a product of its own would leave them)
+            const vec8 f8 = __builtin_bit_cast(vec8, rd[i % STORES]);
+            vec8 o;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float f = (float)f8[j], sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * f));
+                o[j] = (elem)((float)dv[i][j] * sg * (1.f + f * (1.f - sg)));
+            }
+            rd[i % STORES] = __builtin_bit_cast(i32x4_t, o);
+        }
+        if (r < rows_here) *(i32x4_t*)(obase + (int64_t)col0 * 2 + ((unsigned)r * (unsigned)(p.out_rs * 2) + chunk * 16)) = rd[i % STORES];
     };
     // the rounded values once more, scaled, as e4m3
     auto convert8 = [&](int i, int col0) __attribute__((always_inline)) {
@@ -406,10 +448,14 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
     };
     auto finish = [&](const f32x16_t(&sums)[RB][DT], int u) __attribute__((always_inline)) {
         const int col0 = col_of(u);
-        read_bias(u);
+        if constexpr (BIAS) read_bias(u);
+        if constexpr (MODE == kUqvkGradU) {
+#pragma unroll
+            for (int i = 0; i < RB * STORES; ++i) read_du(i, col0);
+        }
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            if (col0 < p.n_silu) {  // (a unit's columns are all u's or none)
+            if ((MODE == kUqvkForward || MODE == kUqvkForward8) && col0 < p.n_silu) {  // (a unit's columns are all u's or none)
 #pragma unroll
                 for (int i = 0; i < 4 * DT; ++i) piece(rb * 4 * DT + i, sums, true);
             } else {
@@ -462,13 +508,20 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
         __builtin_amdgcn_sched_barrier(0);
         finish(acc, u);
     }
-    if constexpr (OUT8) {
+    if constexpr (OUT8) {  // one maximum per workgroup and tensor: hundreds of workgroups end together, on three addresses
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             float m = amax[t];
 #pragma unroll
             for (int d = 32; d >= 1; d >>= 1) m = __builtin_fmaxf(m, __shfl_xor(m, d, 64));
-            if (lane == 0 && m > 0.f) atomicMax(p.absmax + t, __builtin_bit_cast(unsigned, m));
+            if (lane == 0) *HSTU_LDS(float, stage + t * 4) = m;
+        }
+        __syncthreads();
+        if (threadIdx.x < 3) {
+            float m = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) m = __builtin_fmaxf(m, *HSTU_LDS(const float, smem + 4 * RING * Geo::kTile + w * Geo::kStage + threadIdx.x * 4));
+            if (m > 0.f) atomicMax(p.absmax + threadIdx.x, __builtin_bit_cast(unsigned, m));
         }
     }
 }

@@ -67,11 +67,12 @@ __device__ __forceinline__ void wide_for(F&& f, std::integer_sequence<int, I...>
     (f(std::integral_constant<int, I>{}), ...);
 }
 
-template <class TT, int KT, bool OUT8>  // KT = d_model / 64
+template <class TT, int KT, int MODE>  // KT = d_model / 64; MODE: not kUqvkGradU
 __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedParams p) {
     typedef typename TT::vec8 vec8;
     typedef typename TT::elem elem;
     typedef __attribute__((ext_vector_type(4))) elem elem4;
+    constexpr bool OUT8 = MODE == kUqvkForward8, TRANS = MODE == kProductT;
     constexpr int KS = KT * 4, TPB = KT / 2, S = 16 * TPB, PD = 4, RING = kWideRing<KT>;
     typedef WideSchedule<S> Plan;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -89,8 +90,13 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
     unsigned coff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int row = (wave + 4 * i) * 8 + (lane >> 3);
-        coff[i] = (unsigned)row * (unsigned)(p.n_out * 2) + ((lane & 7) ^ swz_w64(row)) * 16;
+        if constexpr (TRANS) {  // 64 columns' rows of 256 bytes
+            const int row = (wave + 4 * i) * 4 + (lane >> 4);
+            coff[i] = (unsigned)row * (unsigned)(p.w_rs * 2) + ((lane & 15) ^ (row & 15)) * 16;
+        } else {
+            const int row = (wave + 4 * i) * 8 + (lane >> 3);
+            coff[i] = (unsigned)row * (unsigned)(p.w_rs * 2) + ((lane & 7) ^ swz_w64(row)) * 16;
+        }
     }
     // transposing reads: lane supplies the address of 4 consecutive n of k row 8g + 4sec + j (+ 16 per k step)
     int waddr[2][2];
@@ -103,6 +109,9 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
             for (int dt = 0; dt < 2; ++dt) waddr[sec][dt] = row * 128 + (((dt * 4 + 2 * half + (q4 >> 1)) ^ swz_w64(row)) * 16) + (q4 & 1) * 8;
         }
     }
+    int taddr[8];  // (transposed W: the lane's column, chunk 2 k step + g)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) taddr[k] = l32 * 256 + (((2 * k + g) ^ (l32 & 15)) * 16);
     char* const stage = smem + RING * kWideSlot + kWideBias + wave * 2 * kWideStage;
     const int chunk = lane & 7, rsub = lane >> 3;  // 8 lanes cover one row's 128 bytes, 8 rows per store
     float amax[3] = {0.f, 0.f, 0.f};                 // (e4m3 output) the largest |value| this lane has stored of v, q, k
@@ -121,11 +130,11 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         auto col_of = [&](int c) __attribute__((always_inline)) { return (c_begin + (c + turn < n ? c + turn : c + turn - n)) * kWideCols; };
         // ---- copies: tile kt of column block c into ring slot s, one instruction of the four at a time; past the last block that one's
         // tiles again, into slots nobody reads
-        const int64_t tile_bytes = (int64_t)kWideTileK * p.n_out * 2;
+        const int64_t tile_bytes = TRANS ? kWideTileK * 2 : (int64_t)kWideTileK * p.w_rs * 2;
         auto issue = [&](int c, int kt, int s, int i) __attribute__((always_inline)) {
-            const char* src = p.w + (int64_t)col_of(c < n ? c : n - 1) * 2 + kt * tile_bytes;
+            const char* src = p.w + (int64_t)col_of(c < n ? c : n - 1) * 2 * (TRANS ? p.w_rs : 1) + kt * tile_bytes;
             // (block c's bias is read at the start of block c + 1, before the copies of block c + 4 are issued)
-            if (i == 0 && kt == 0 && wave == 0 && lane < 8 && c < n)
+            if (!TRANS && i == 0 && kt == 0 && wave == 0 && lane < 8 && c < n)
                 global_load_lds16(p.bias + (int64_t)col_of(c) * 2 + lane * 16, smem + RING * kWideSlot + (c & 3) * 128);
             global_load_lds16_soff(src, coff[i], smem + __builtin_amdgcn_readfirstlane(s * kWideSlot + (wave + 4 * i) * 1024));
         };
@@ -137,7 +146,14 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         vec8 xreg[2][KS];
 #pragma unroll
         for (int rg = 0; rg < 2; ++rg) {
-            uqvk_normalised_row<TT, KS>(p, row0 + rg * 32 + l32, g, xreg[rg]);
+            if constexpr (TRANS) {
+                int64_t r = row0 + rg * 32 + l32;
+                r = r < p.rows ? r : p.rows - 1;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) xreg[rg][ks] = *(const vec8*)(p.x + (r * p.x_rs + ks * 16 + 8 * g) * 2);
+            } else {
+                uqvk_normalised_row<TT, KS>(p, row0 + rg * 32 + l32, g, xreg[rg]);
+            }
             // all of it here: the compiler would otherwise move the arithmetic of the second half into the first column block
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+a"(xreg[rg][ks]));
@@ -146,7 +162,7 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
 
         // where this lane's stores go: rows past the end are the last row
         const int64_t base_row = row0 < p.rows ? row0 : p.rows - 1;
-        char* const obase = p.out + base_row * p.n_out * 2;
+        char* const obase = p.out + base_row * p.out_rs * 2;
         unsigned char* const obase8 = OUT8 ? p.out8 + base_row * (p.n_out - p.n_silu) : nullptr;
         const int64_t below = p.rows - 1 - base_row;
         const int last = below < 63 ? (int)below : 63;
@@ -162,6 +178,7 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         i32x4_t rd[8];
         float blockmax = 0.f;  // (e4m3 output) the largest |value| of the column block in progress
         auto read_bias = [&](int c) __attribute__((always_inline)) {
+            if constexpr (TRANS) return;
             const char* b = smem + RING * kWideSlot + (c & 3) * 128 + g * 8;
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt)
@@ -173,7 +190,7 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
             const int rg = i >> 3, dt = (i >> 2) & 1, r4 = i & 3;
             float v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = sums[rg][dt][r4 * 4 + j] + (float)b4[dt][r4][j];
+            for (int j = 0; j < 4; ++j) v[j] = TRANS ? sums[rg][dt][r4 * 4 + j] : sums[rg][dt][r4 * 4 + j] + (float)b4[dt][r4][j];
             if constexpr (decltype(Silu)::value) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = v[j] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v[j]));
@@ -185,7 +202,7 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         };
         auto store_rows = [&](int i, int c) __attribute__((always_inline)) {
             const int col0 = col_of(c);
-            *(i32x4_t*)(obase + (int64_t)col0 * 2 + (orow(i) * (unsigned)(p.n_out * 2) + chunk * 16)) = rd[i];
+            *(i32x4_t*)(obase + (int64_t)col0 * 2 + (orow(i) * (unsigned)(p.out_rs * 2) + chunk * 16)) = rd[i];
         };
         // The rounded values of store i once more, scaled, as e4m3, in two halves (a step of two MFMAs has
         // room for about twelve vector instructions): 8 lanes cover 64 bytes of a row.
@@ -222,6 +239,10 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         int slot = 0;  // of the tile in progress
         vec8 fr[PD];
         auto load_op = [&](int s, int m) __attribute__((always_inline)) {
+            if constexpr (TRANS) {
+                fr[m % PD] = *HSTU_LDS(const vec8, smem + s * kWideSlot + (m & 1) * 8192 + taddr[m >> 1]);
+                return;
+            }
             const char* b = smem + s * kWideSlot + (m >> 1) * 16 * 128;
             fr[m % PD] = read_vt_operand<TT>(b + waddr[0][m & 1], b + waddr[1][m & 1]);
         };
@@ -295,11 +316,11 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
         };
 
         auto next_block = [&](f32x16_t(&now)[2][2], const f32x16_t(&before)[2][2], int c) __attribute__((always_inline)) {
-            if (col_of(c - 1) < p.n_silu) block(now, before, c, std::true_type{}, std::true_type{});
+            if (!TRANS && col_of(c - 1) < p.n_silu) block(now, before, c, std::true_type{}, std::true_type{});
             else block(now, before, c, std::true_type{}, std::false_type{});
         };
         auto last_epilogue = [&](const f32x16_t(&sums)[2][2], int c) __attribute__((always_inline)) {
-            if (col_of(c) < p.n_silu) finish(sums, c, std::true_type{});
+            if (!TRANS && col_of(c) < p.n_silu) finish(sums, c, std::true_type{});
             else finish(sums, c, std::false_type{});
         };
         block(acc[0], acc[1], 0, std::false_type{}, std::false_type{});

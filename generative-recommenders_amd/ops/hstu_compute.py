@@ -96,6 +96,7 @@ EXPORTS = (
     "hstu_uqvk_workspace_bytes", "hstu_uqvk_forward", "hstu_uqvk_layer_norm", "hstu_output_workspace_bytes", "hstu_output_forward",
     "hstu_output_norm_mul", "hstu_output_dropout_mask", "hstu_output_norm_mul_bwd_workspace_bytes", "hstu_output_norm_mul_bwd",
     "hstu_uqvk_layer_norm_bwd_workspace_bytes", "hstu_uqvk_layer_norm_bwd", "hstu_uqvk_silu_bwd",
+    "hstu_uqvk_u_grad", "hstu_linear_product_t_workspace_bytes", "hstu_linear_product_t",
     "hstu_linear_weight_grad_workspace_bytes", "hstu_linear_weight_grad", "hstu_linear_last_error",
     "hstu_linear_version",
 )

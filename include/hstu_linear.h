@@ -150,7 +150,6 @@ int hstu_output_dropout_mask(float ratio, uint64_t seed, uint64_t offset, int64_
 
 /*
  * ---- Backward of the row-wise parts ----
- * (the products with a weight, d_joined = d_out @ W^T and the like, are plain GEMMs and the caller's).
  * Statistics and the dropout mask are recomputed from the forward's inputs; nothing is saved.  The gradients of a norm's weight
  * and bias are summed over the rows in fp32 in a fixed order through `workspace` (16-byte aligned) and rounded once.
  */
@@ -192,6 +191,20 @@ int hstu_uqvk_silu_bwd(void* pre, int64_t pre_row_stride, const void* bias, cons
 size_t hstu_linear_weight_grad_workspace_bytes(int32_t m, int32_t n, int64_t rows, int64_t a_row_stride, int64_t b_row_stride);
 int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, const void* b, int64_t b_row_stride, int32_t n, int64_t rows,
                             int32_t dtype, void* out, void* b_sums, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* The same gradient without that product in memory: out = du * (derivative of SiLU at LN(x) @ weight + bias) for a depth d_model of 128, 256,
+ * 384 or 512 and a width that is a multiple of 128 (-6 otherwise).  weight [d_model, width] and the rows of x, du and out with strides in
+ * elements, 16-byte aligned, below 2^22. */
+int hstu_uqvk_u_grad(const void* x, int64_t x_row_stride, const void* norm_weight, const void* norm_bias, float eps, const void* weight,
+                     int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride, int64_t rows,
+                     int32_t d_model, int32_t width, int32_t dtype, void* stream);
+
+/* out [rows, n] = a [rows, k] @ weight [n, k]^T (strides in elements, rows 16-byte aligned, strides below 2^22; k and n multiples of 8), fp32
+ * sums rounded once: d_joined = d_out @ output_weight^T and the like.  `workspace` (256-byte aligned) is for the shapes that the library's GEMM
+ * takes; the others need none. */
+size_t hstu_linear_product_t_workspace_bytes(int64_t rows, int32_t k, int32_t n);
+int hstu_linear_product_t(const void* a, int64_t a_row_stride, const void* weight, int64_t weight_row_stride, int64_t rows, int32_t k, int32_t n,
+                          int32_t dtype, void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes, void* stream);
 
 const char* hstu_linear_last_error(void);
 

@@ -292,6 +292,64 @@ def test_uqvk_kernels_for_few_rows_give_the_same_bits(pkg, dev, d_model, H, attn
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 3e-3), (torch.float16, 4e-4)])  # half a unit in the last place, uniform: 1.7e-3, 2.1e-4
+@pytest.mark.parametrize(
+    "rows,k,n",
+    # one row; remainders of 32 and 64 rows; units of their own, several per wave, 64 rows per wave with shares that differ (depths 256, 384,
+    # 512); more columns than the waves of a workgroup have units for; the library's shapes (depths 64 and 1152, few columns)
+    [(1, 512, 1536), (33, 128, 128), (65, 256, 384), (4097, 512, 1024), (2049, 384, 1152), (8193, 128, 640), (20001, 512, 1536), (30001, 256, 768),
+     (33333, 384, 512), (70, 64, 64), (300, 1152, 256), (20000, 512, 128)],
+)
+def test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound):
+    """hstu_linear_product_t on rows that are slices of wider buffers, against the product in 64 bits."""
+    import ctypes
+
+    print(f"[case] product_t {rows} {k} {n} {dtype}", flush=True)
+    L, V, I, J = pkg.lib(), ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32
+    L.hstu_linear_product_t_workspace_bytes.restype = ctypes.c_size_t
+    g = torch.Generator(device=dev).manual_seed(rows + k)
+    a = torch.randn(rows, k + 64, generator=g, device=dev).to(dtype)[:, 32 : 32 + k]
+    w = (torch.randn(n, k + 8, generator=g, device=dev) / k**0.5).to(dtype)[:, :k]
+    out = torch.full((rows, n + 8), 7.0, device=dev, dtype=dtype)
+    need = L.hstu_linear_product_t_workspace_bytes(I(rows), J(k), J(n))
+    scratch = torch.empty(need + 256, dtype=torch.uint8, device=dev)
+    ws = (scratch.data_ptr() + 255) // 256 * 256
+    rc = L.hstu_linear_product_t(V(a.data_ptr()), I(a.stride(0)), V(w.data_ptr()), I(w.stride(0)), I(rows), J(k), J(n), J(0 if dtype is torch.bfloat16 else 1),
+                                 V(out.data_ptr()), I(out.stride(0)), V(ws), I(need), V(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == 0, pkg.lib().hstu_linear_last_error()
+    ref = a.double() @ w.double().t()
+    assert float((out[:, :n].double() - ref).norm() / ref.norm()) <= bound
+    assert bool((out[:, n:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])  # the rounded norm, sums and result: 2.0e-3, 2.6e-4
+@pytest.mark.parametrize("rows,k,n", [(1, 512, 128), (33, 128, 384), (65, 256, 128), (4097, 512, 512), (2049, 384, 640), (20001, 512, 256), (40001, 256, 256)])
+def test_gradient_of_u_in_front_of_silu(pkg, dev, rows, k, n, dtype, bound):
+    """hstu_uqvk_u_grad (du a slice of a wider buffer, the result a slice of the producer's gradient buffer) against 64 bits."""
+    import ctypes
+
+    print(f"[case] u_grad {rows} {k} {n} {dtype}", flush=True)
+    V, I, J = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32
+    g = torch.Generator(device=dev).manual_seed(rows + k)
+    r = lambda *shape: torch.randn(*shape, generator=g, device=dev)
+    x, nw, nb = r(rows, k).to(dtype), (1 + 0.1 * r(k)).to(dtype), (0.1 * r(k)).to(dtype)
+    w, b, du = (r(k, 3 * n) / k**0.5).to(dtype), (0.1 * r(3 * n)).to(dtype), r(rows, n + 8).to(dtype)[:, 8:]
+    out = torch.full((rows, 3 * n), 7.0, device=dev, dtype=dtype)
+    rc = pkg.lib().hstu_uqvk_u_grad(V(x.data_ptr()), I(k), V(nw.data_ptr()), V(nb.data_ptr()), ctypes.c_float(1e-6), V(w.data_ptr()), I(3 * n), V(b.data_ptr()),
+                                    V(du.data_ptr()), I(du.stride(0)), V(out.data_ptr()), I(3 * n), I(rows), J(k), J(n), J(0 if dtype is torch.bfloat16 else 1),
+                                    V(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == 0
+    z = torch.nn.functional.layer_norm(x.double(), (k,), nw.double(), nb.double(), 1e-6) @ w[:, :n].double() + b[:n].double()
+    s = torch.sigmoid(z)
+    ref = du.double() * s * (1 + z * (1 - s))
+    assert float((out[:, :n].double() - ref).norm() / ref.norm()) <= bound
+    assert bool((out[:, n:] == 7.0).all())
+
+
+@pytest.mark.gpu
 def test_uqvk_with_a_total_length_that_changes_from_batch_to_batch(pkg, dev):
     """The hipBLASLt path keeps one plan per size class of the row count, not per row count: lengths of one class
     (1100, 1101, 1279), of others (640, 5000), and the first again, each against the oracle."""
