@@ -17,6 +17,7 @@
 #include "hstu_rows.h"
 #include "hstu_uqvk_kernel.h"
 #include "hstu_output_kernel.h"
+#include "hstu_output_rows_kernel.h"
 
 // hstu_uqvk.hip, hstu_uqvk_bwd.hip
 int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
@@ -288,6 +289,47 @@ bool output_fused_u_made(const HstuOutputArgs* a) { return !a->group_norm && a->
 // measured against the library path it wins from 32768 rows on: 70 against 77 us there, 37 against 32 us at 2048).
 bool output_takes_fused(const HstuOutputArgs* a) {
     return a->path == 2 || (a->path == 0 && a->rows >= 32768 && a->dropout_ratio == 0.f && output_fused_shape(a));
+}
+
+// path = 0: the one kernel for a few rows, where a row's chunks are one per lane and the joined rows fit the LDS.  Up to 256 rows it is latency
+// for both (50 rows 7.8 us a pass, the two kernels of the library path 10.2; 256 rows 8.1 / 11.9); beyond, its workgroups of 32 x 32 would read W
+// once per 32 rows (1.5 MB of it for 3 x 512 into 512 columns) and need more than one round on the chip.
+bool output_takes_rows(const HstuOutputArgs* a) {
+    const int64_t d = (int64_t)a->heads * a->linear_dim;
+    if (a->path != 0 || a->rows > 256 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1)) return false;
+    if (a->d_out % 32 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512 || output_blocks(a) * d > hstu::kOutRowsMostK) return false;
+    if (!a->group_norm) return true;
+    const int lanes = a->linear_dim / 8;
+    return a->linear_dim % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0;
+}
+
+template <class TT, bool GROUP>
+int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
+    hstu::OutputRowsParams p;
+    const int rc = hstu::norm_mul_params(a, nullptr, (int64_t)output_blocks(a) * a->heads * a->linear_dim, false, p.nm);
+    if (rc != 0) return rc;
+    p.x = (const char*)a->x, p.x_rs = a->x_row_stride, p.w = (const char*)a->output_weight, p.out = (char*)a->out;
+    p.n = a->d_out, p.k = output_blocks(a) * p.nm.d;
+    auto kern = hstu::hstu_output_rows_kernel<TT, GROUP>;
+    // (a function attribute belongs to the device it was set on: one flag per device)
+    static std::atomic<bool> attr_done[64];
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
+    if (dev < 0 || !attr_done[dev]) {
+        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, hstu::out_rows_lds(hstu::kOutRowsMostK));
+        if (e != hipSuccess) {
+            snprintf(g_last_error, sizeof(g_last_error), "hipFuncSetAttribute: %s", hipGetErrorString(e));
+            return -7;
+        }
+        if (dev >= 0) attr_done[dev] = true;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)(a->d_out / 32), (unsigned)((a->rows + 31) / 32)), dim3(256), hstu::out_rows_lds(p.k), stream, p);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        snprintf(g_last_error, sizeof(g_last_error), "output kernel launch: %s", hipGetErrorString(e));
+        return -7;
+    }
+    return 0;
 }
 
 size_t output_fused_workspace(const HstuOutputArgs* a) {
@@ -774,6 +816,7 @@ int hstu_linear_product_t(const void* a, int64_t a_row_stride, const void* weigh
 
 size_t hstu_output_workspace_bytes(const HstuOutputArgs* a) {
     if (!a || a->rows <= 0 || a->heads <= 0 || a->linear_dim <= 0) return 0;
+    if (output_takes_rows(a)) return 0;
     if (output_takes_fused(a)) return output_fused_shape(a) ? output_fused_workspace(a) : 0;
     return joined_bytes(a) + kGemmScratch;
 }
@@ -822,6 +865,10 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
         snprintf(g_last_error, sizeof(g_last_error), "the concatenating output kernel reads u and attn where they are and cannot drop their "
                  "elements: dropout runs on the library path (path 0 or 1)");
         return -6;
+    }
+    if (output_takes_rows(a)) {
+        if (a->dtype == 0) return a->group_norm ? launch_output_rows<hstu::Bf16, true>(a, stream) : launch_output_rows<hstu::Bf16, false>(a, stream);
+        return a->group_norm ? launch_output_rows<hstu::Fp16, true>(a, stream) : launch_output_rows<hstu::Fp16, false>(a, stream);
     }
     if (output_takes_fused(a)) {
         if (!a->workspace) return -1;

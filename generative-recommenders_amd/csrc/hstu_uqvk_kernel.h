@@ -62,24 +62,6 @@ struct UqvkFusedParams {
 
 constexpr int kUqvkStageRow = 64 * 2 + 16;  // staging row: 64 outputs + pad
 
-// x + (x of the lane whose number differs in bit 5, bit 4)
-__device__ __forceinline__ float add_xor32(float x) {
-    const unsigned u = __builtin_bit_cast(unsigned, x);
-    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    const unsigned lo = r[0], hi = r[1];
-    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
-}
-__device__ __forceinline__ float add_xor16(float x) {
-    const unsigned u = __builtin_bit_cast(unsigned, x);
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    const unsigned lo = r[0], hi = r[1];
-    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
-}
-template <int CTRL>
-__device__ __forceinline__ float add_dpp(float x) {
-    return x + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
-
 // N values as they are in fp32, rounded to E.  (fp16: left to itself the compiler makes one rounding of the last operation and this one, in
 // one kernel and not in the other.)
 template <class E, int N>

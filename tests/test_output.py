@@ -248,6 +248,30 @@ def test_compute_output_fused_kernel(pkg, dev, N, H, ld, cu, cx, act, group_norm
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "N,H,ld,D,cu,cx,act,group_norm",
+    # one row; the edges of the blocks of 32 rows and the last size; depths of 1, 2 and 3 blocks from 128 to 1536, i.e. one to twelve tiles per
+    # wave, fewer and more than a ring holds; one block of columns; heads of one, four and sixteen lanes; every activation
+    [(1, 4, 128, 512, True, True, "none", False), (31, 2, 64, 256, True, True, "silu", False), (33, 1, 128, 32, False, False, "sigmoid", False),
+     (255, 4, 128, 512, True, True, "none", True), (256, 4, 32, 640, True, True, "none", True), (64, 16, 8, 96, False, False, "none", True),
+     (65, 3, 128, 512, True, False, "silu", False), (200, 2, 256, 512, False, True, "none", False)],
+)
+def test_compute_output_of_a_few_rows(pkg, dev, N, H, ld, D, cu, cx, act, group_norm, dtype):
+    """The one kernel for a few rows (chosen without being asked for) on strided views: against the fp32 oracle and the library path."""
+    print(f"[case] output of a few rows {N} {H} {ld} {D} {cu} {cx} {act} group={group_norm} {dtype}", flush=True)
+    attn, u, x, nw, nb, w = _inputs(N + D, N, H, ld, D, _blocks(cu, cx, group_norm), group_norm, dtype)
+    wide = torch.cat([u, attn, x], dim=1).to(dev)
+    L = H * ld
+    args = (wide[:, L : 2 * L], wide[:, :L], wide[:, 2 * L :], nw.to(dev), nb.to(dev), 1e-6, w.to(dev), H, ld, 0.0, False, cu, cx, act, group_norm, False)
+    got, lib = pkg.hstu_compute_output(*args), pkg.hstu_compute_output(*args, path=1)
+    torch.cuda.synchronize()
+    kw = dict(concat_u=cu, concat_x=cx, mul_u_activation_type=act, group_norm=group_norm, num_heads=H, linear_dim=ld)
+    _close(got, O.compute_output(attn, u, x, nw, nb, w, 1e-6, **kw), "few rows vs fp32 oracle")
+    _close(got, lib.float().cpu(), "few rows vs library path")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N", [33000, 257])
 def test_compute_output_concat_gemm_on_views_of_wider_buffers(pkg, dev, N):
     """u as the column slice of a [N, 4 * 512] buffer (what the producer leaves), attn as a slice of a padded one: the
