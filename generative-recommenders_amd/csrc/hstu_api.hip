@@ -800,7 +800,8 @@ int common_vector_bytes(std::initializer_list<uint64_t> values) {
     return vec;
 }
 
-constexpr int kJaggedRows = 32;  // joined rows per workgroup
+constexpr int kJaggedRows = 32, kTailRows = 16;  // rows per workgroup of the two kernels
+constexpr int64_t kShortRow = 1 << 26;           // bytes of a row up to which a block's accesses are counted in 32 bits
 
 int check_jagged_args(const HstuJaggedCopyArgs* a) {
     if (!a) return HSTU_ERR_NULL_POINTER;
@@ -844,13 +845,19 @@ int launch_jagged_copy(const HstuJaggedCopyArgs* a, hipStream_t stream) {
     const int vec = common_vector_bytes({(uint64_t)(uintptr_t)a->left, (uint64_t)(uintptr_t)a->right, (uint64_t)(uintptr_t)a->joined,
                                          (uint64_t)a->left_row_stride, (uint64_t)a->right_row_stride,
                                          (uint64_t)a->joined_row_stride, (uint64_t)a->row_bytes});
-    switch (vec) {
-        case 16: hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, 16, kJaggedRows>), grid, dim3(256), 0, stream, p); break;
-        case 8: hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, 8, kJaggedRows>), grid, dim3(256), 0, stream, p); break;
-        case 4: hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, 4, kJaggedRows>), grid, dim3(256), 0, stream, p); break;
-        case 2: hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, 2, kJaggedRows>), grid, dim3(256), 0, stream, p); break;
-        default: hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, 1, kJaggedRows>), grid, dim3(256), 0, stream, p); break;
+#define HSTU_COPY_LAUNCH(V, INDEX) hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, V, kJaggedRows, INDEX>), grid, dim3(256), 0, stream, p)
+    if (a->row_bytes > kShortRow) {
+        HSTU_COPY_LAUNCH(1, uint64_t);
+    } else {
+        switch (vec) {
+            case 16: HSTU_COPY_LAUNCH(16, unsigned); break;
+            case 8: HSTU_COPY_LAUNCH(8, unsigned); break;
+            case 4: HSTU_COPY_LAUNCH(4, unsigned); break;
+            case 2: HSTU_COPY_LAUNCH(2, unsigned); break;
+            default: HSTU_COPY_LAUNCH(1, unsigned); break;
+        }
     }
+#undef HSTU_COPY_LAUNCH
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_last_error("jagged copy kernel launch", e);
@@ -874,19 +881,23 @@ int hstu_hip_jagged_write_tail(void* joined, int64_t joined_row_stride, const vo
     if (batch == 0 || tail_len == 0 || row_bytes == 0) return HSTU_OK;
     if (!joined || !offsets || !tail) return HSTU_ERR_NULL_POINTER;
     if (batch > 65535) return HSTU_ERR_BAD_SHAPE;
-    const dim3 grid((unsigned)((tail_len + kJaggedRows - 1) / kJaggedRows), (unsigned)batch);
+    const dim3 grid((unsigned)((tail_len + kTailRows - 1) / kTailRows), (unsigned)batch);
     hipStream_t stream = (hipStream_t)stream_;
     const int vec = common_vector_bytes({(uint64_t)(uintptr_t)joined, (uint64_t)(uintptr_t)tail, (uint64_t)joined_row_stride,
                                          (uint64_t)tail_row_stride, (uint64_t)row_bytes});
-#define HSTU_TAIL_LAUNCH(V)                                                                                                   \
-    hipLaunchKernelGGL((hstu::hstu_jagged_write_tail_kernel<V, kJaggedRows>), grid, dim3(256), 0, stream, (char*)joined,        \
+#define HSTU_TAIL_LAUNCH(V, INDEX)                                                                                            \
+    hipLaunchKernelGGL((hstu::hstu_jagged_write_tail_kernel<V, kTailRows, INDEX>), grid, dim3(256), 0, stream, (char*)joined,   \
                        joined_row_stride, offsets, offsets_i64, (const char*)tail, tail_row_stride, row_bytes, tail_len)
-    switch (vec) {
-        case 16: HSTU_TAIL_LAUNCH(16); break;
-        case 8: HSTU_TAIL_LAUNCH(8); break;
-        case 4: HSTU_TAIL_LAUNCH(4); break;
-        case 2: HSTU_TAIL_LAUNCH(2); break;
-        default: HSTU_TAIL_LAUNCH(1); break;
+    if (row_bytes > kShortRow) {
+        HSTU_TAIL_LAUNCH(1, uint64_t);
+    } else {
+        switch (vec) {
+            case 16: HSTU_TAIL_LAUNCH(16, unsigned); break;
+            case 8: HSTU_TAIL_LAUNCH(8, unsigned); break;
+            case 4: HSTU_TAIL_LAUNCH(4, unsigned); break;
+            case 2: HSTU_TAIL_LAUNCH(2, unsigned); break;
+            default: HSTU_TAIL_LAUNCH(1, unsigned); break;
+        }
     }
 #undef HSTU_TAIL_LAUNCH
     hipError_t e = hipGetLastError();

@@ -206,6 +206,28 @@ def test_write_kv_tail_equals_concat_and_feeds_delta_attention(pkg, dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "batch,tail,columns,dtype",
+    # blocks of 16 rows with a remainder of 1, 15 and none; rows of fewer accesses than threads and of more than one round; odd widths; a row
+    # whose accesses are counted in 64 bits
+    [(3, 17, 512, torch.bfloat16), (2, 15, 7, torch.bfloat16), (1, 1, 3000, torch.float32), (4, 32, 33, torch.float16), (2, 1, (1 << 26) + 3, torch.uint8)],
+)
+def test_write_kv_tail_blocks(pkg, dev, batch, tail, columns, dtype):
+    print(f"[case] write_kv_tail {batch} {tail} {columns} {dtype}", flush=True)
+    history = [3 * b for b in range(batch)]
+    ends = np.cumsum([h + tail for h in history])
+    offs = torch.tensor(np.concatenate([[0], ends]), dtype=torch.int64, device=dev)
+    full = torch.arange(int(ends[-1]) * columns, device=dev).remainder(251).view(-1, columns).to(dtype)
+    new = (torch.arange(batch * tail * columns, device=dev).remainder(239) + 3).view(-1, columns).to(dtype)
+    want = full.clone()
+    for b in range(batch):
+        want[int(ends[b]) - tail : int(ends[b])] = new[b * tail : (b + 1) * tail]
+    pkg.write_kv_tail(full, offs, new)
+    torch.cuda.synchronize()
+    assert torch.equal(full, want)
+
+
+@pytest.mark.gpu
 def test_jagged_wrapper_rejections(pkg, dev):
     a = torch.zeros((4, 8), device=dev)
     with pytest.raises(AssertionError, match="values_left must be 2D"):
