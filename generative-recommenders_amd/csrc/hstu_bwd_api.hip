@@ -189,7 +189,8 @@ extern "C" int hstu_hip_mha_bwd(const HstuFwdArgs* a, const HstuBwdGrads* g, voi
     p.slots_per_xcd = (int)slots;
 
     // `sort_by_length`: long sequences first (their blocks are the long-running ones); needs 4 * batch bytes of workspace
-    if (a->sort_by_length && a->batch >= 2 && a->batch <= 8192 && a->workspace &&
+    // (not where all blocks start together, one workgroup per CU: 8 sequences of 150 rows, 2 heads, save the launch)
+    if (a->sort_by_length && a->batch >= 2 && a->batch <= 8192 && slots * 8 > 256 && a->workspace &&
         (size_t)a->workspace_bytes >= (size_t)a->batch * sizeof(int)) {
         rc = hstu_hip_launch_rank(a->seq_offsets, a->seq_offsets_i64, a->batch, (int*)a->workspace, stream_);
         if (rc != HSTU_OK) return rc;

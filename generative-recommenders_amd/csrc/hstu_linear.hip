@@ -773,14 +773,15 @@ int hstu_uqvk_forward(const HstuUqvkArgs* a, void* stream_) {
 }
 
 int hstu_uqvk_u_grad(const void* x, int64_t x_row_stride, const void* norm_weight, const void* norm_bias, float eps, const void* weight,
-                     int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride, int64_t rows,
-                     int32_t d_model, int32_t width, int32_t dtype, void* stream) {
+                     int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride,
+                     void* normed, int64_t rows, int32_t d_model, int32_t width, int32_t dtype, void* stream) {
     g_last_error[0] = 0;
     if (rows < 0 || rows > 0x7fffffffLL || d_model <= 0 || width <= 0 || (dtype != 0 && dtype != 1)) return -5;
     if ((d_model != 128 && d_model != 256 && d_model != 384 && d_model != 512) || width % 128 != 0 || width > (1 << 20)) return -6;
     if (rows == 0) return 0;
     if (!x || !norm_weight || !norm_bias || !weight || !bias || !du || !out) return -1;
-    const uintptr_t ptrs = (uintptr_t)x | (uintptr_t)norm_weight | (uintptr_t)norm_bias | (uintptr_t)weight | (uintptr_t)bias | (uintptr_t)du | (uintptr_t)out;
+    const uintptr_t ptrs = (uintptr_t)x | (uintptr_t)norm_weight | (uintptr_t)norm_bias | (uintptr_t)weight | (uintptr_t)bias | (uintptr_t)du | (uintptr_t)out |
+                           (uintptr_t)normed;
     if ((ptrs & 15) != 0) return -4;
     if (!product_stride(x_row_stride, d_model) || !product_stride(weight_row_stride, width) || !product_stride(du_row_stride, width) ||
         !product_stride(out_row_stride, width))
@@ -788,7 +789,7 @@ int hstu_uqvk_u_grad(const void* x, int64_t x_row_stride, const void* norm_weigh
     hstu::UqvkFusedParams p{};
     p.x = (const char*)x, p.x_rs = x_row_stride, p.norm_weight = (const char*)norm_weight, p.norm_bias = (const char*)norm_bias, p.eps = eps;
     p.w = (const char*)weight, p.w_rs = weight_row_stride, p.bias = (const char*)bias, p.du = (const char*)du, p.du_rs = du_row_stride;
-    p.out = (char*)out, p.out_rs = out_row_stride, p.rows = rows, p.n_out = width;
+    p.out = (char*)out, p.out_rs = out_row_stride, p.normed = (char*)normed, p.rows = rows, p.n_out = width;
     return hstu_uqvk_grad_u_launch(p, d_model, dtype == 0, (hipStream_t)stream);
 }
 

@@ -416,20 +416,20 @@ variable_list uqvk_backward(const AutogradContext* ctx, const Tensor& x, const T
     void* stream = stream_of(x);
     variable_list got(5);
     Tensor d_u = d.narrow(1, 0, n_u);
-    bool u_done = !du.defined();
+    Tensor normed;
+    if (du.defined() || weight_wanted) normed = at::empty({rows, dm}, x.options());
+    bool u_done = !du.defined(), normed_done = false;
     if (u_done) {
         d_u.zero_();
     } else {
         du = gradient_rows(du);
         const int rc = hstu_uqvk_u_grad(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
                                         weight.const_data_ptr(), weight.stride(0), bias.const_data_ptr(), du.const_data_ptr(), du.stride(0), d_u.data_ptr(),
-                                        d_u.stride(0), rows, (int32_t)dm, (int32_t)n_u, dense_dtype(x), stream);
+                                        d_u.stride(0), weight_wanted ? normed.data_ptr() : nullptr, rows, (int32_t)dm, (int32_t)n_u, dense_dtype(x), stream);
         if (rc != -6 && rc != -5) check_linear(rc);  // (another shape: the product and what follows it below)
-        u_done = rc == 0;
+        u_done = normed_done = rc == 0;
     }
-    Tensor normed;
-    if (!u_done || weight_wanted) {
-        normed = at::empty({rows, dm}, x.options());
+    if (!normed_done && (!u_done || weight_wanted)) {
         check_linear(hstu_uqvk_layer_norm(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
                                           normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
     }

@@ -45,6 +45,7 @@ struct UqvkFusedParams {
     int64_t out_rs;    // its row stride in elements
     const char* du;    // (gradient of u) [rows, n_out]
     int64_t du_rs;
+    char* normed;      // (gradient of u) NULL, or where LN(x) goes: [rows, K] dense
     int64_t rows;
     int n_out;   // multiple of 128
     int n_silu;  // multiple of 32: columns [0, n_silu) go through SiLU
@@ -202,7 +203,8 @@ struct UqvkRows {
 
 // What the kernel computes from its products.
 //   kUqvkForward, kUqvkForward8: the producer, without and with the e4m3 copy
-//   kUqvkGradU: out = du * SiLU'(LN(x) W + bias), the gradient of the u columns' products; nothing of the forward is read but x
+//   kUqvkGradU: out = du * SiLU'(LN(x) W + bias), the gradient of the u columns' products, and LN(x) itself, an operand of W's gradient; nothing of the
+//     forward is read but x
 //   kProductT: out = x W^T, no norm, no bias: W's k run along its rows, so its tiles are read as they lie
 enum { kUqvkForward, kUqvkForward8, kUqvkGradU, kProductT };
 
@@ -292,6 +294,9 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
             xv[i] = ln_chunk_apply<vec8, elem>(xv[i], mean, rstd, wv, bv);
         }
         const int row = (wave * NP + i) * RPI + sub;
+        if constexpr (MODE == kUqvkGradU) {
+            if (p.normed && blockIdx.y == 0 && holds && row0 + row < p.rows) *(vec8*)(p.normed + ((row0 + row) * K + chunk_of * 8) * 2) = xv[i];
+        }
         if (holds) *HSTU_LDS(vec8, panel + row * (K * 2) + ((chunk_of ^ (row & 15)) * 16)) = xv[i];
     }
     __syncthreads();

@@ -194,10 +194,10 @@ int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, cons
 
 /* The same gradient without that product in memory: out = du * (derivative of SiLU at LN(x) @ weight + bias) for a depth d_model of 128, 256,
  * 384 or 512 and a width that is a multiple of 128 (-6 otherwise).  weight [d_model, width] and the rows of x, du and out with strides in
- * elements, 16-byte aligned, below 2^22. */
+ * elements, 16-byte aligned, below 2^22.  `normed`, if not NULL, gets LN(x) as hstu_uqvk_layer_norm writes it, [rows, d_model] dense. */
 int hstu_uqvk_u_grad(const void* x, int64_t x_row_stride, const void* norm_weight, const void* norm_bias, float eps, const void* weight,
-                     int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride, int64_t rows,
-                     int32_t d_model, int32_t width, int32_t dtype, void* stream);
+                     int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride,
+                     void* normed, int64_t rows, int32_t d_model, int32_t width, int32_t dtype, void* stream);
 
 /* out [rows, n] = a [rows, k] @ weight [n, k]^T (strides in elements, rows 16-byte aligned, strides below 2^22; k and n multiples of 8), fp32
  * sums rounded once: d_joined = d_out @ output_weight^T and the like.  `workspace` (256-byte aligned) is for the shapes that the library's GEMM

@@ -337,12 +337,15 @@ def test_gradient_of_u_in_front_of_silu(pkg, dev, rows, k, n, dtype, bound):
     x, nw, nb = r(rows, k).to(dtype), (1 + 0.1 * r(k)).to(dtype), (0.1 * r(k)).to(dtype)
     w, b, du = (r(k, 3 * n) / k**0.5).to(dtype), (0.1 * r(3 * n)).to(dtype), r(rows, n + 8).to(dtype)[:, 8:]
     out = torch.full((rows, 3 * n), 7.0, device=dev, dtype=dtype)
+    normed = torch.full((rows + 1, k), 7.0, device=dev, dtype=dtype)
     rc = pkg.lib().hstu_uqvk_u_grad(V(x.data_ptr()), I(k), V(nw.data_ptr()), V(nb.data_ptr()), ctypes.c_float(1e-6), V(w.data_ptr()), I(3 * n), V(b.data_ptr()),
-                                    V(du.data_ptr()), I(du.stride(0)), V(out.data_ptr()), I(3 * n), I(rows), J(k), J(n), J(0 if dtype is torch.bfloat16 else 1),
-                                    V(torch.cuda.current_stream().cuda_stream))
+                                    V(du.data_ptr()), I(du.stride(0)), V(out.data_ptr()), I(3 * n), V(normed.data_ptr()), I(rows), J(k), J(n),
+                                    J(0 if dtype is torch.bfloat16 else 1), V(torch.cuda.current_stream().cuda_stream))
     torch.cuda.synchronize()
     assert rc == 0
-    z = torch.nn.functional.layer_norm(x.double(), (k,), nw.double(), nb.double(), 1e-6) @ w[:, :n].double() + b[:n].double()
+    norm = torch.nn.functional.layer_norm(x.double(), (k,), nw.double(), nb.double(), 1e-6)
+    assert float((normed[:rows].double() - norm).norm() / norm.norm()) <= bound and bool((normed[rows] == 7.0).all())
+    z = norm @ w[:, :n].double() + b[:n].double()
     s = torch.sigmoid(z)
     ref = du.double() * s * (1 + z * (1 - s))
     assert float((out[:, :n].double() - ref).norm() / ref.norm()) <= bound
