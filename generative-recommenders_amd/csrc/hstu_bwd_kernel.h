@@ -663,10 +663,37 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
     const char* vbase = p.v + (W.seq_start * p.v_rs + (int64_t)W.h * p.v_hs) * 2;
     const int64_t k_rsb = p.k_rs * 2, v_rsb = p.v_rs * 2;
 
-    if (jt < jt_end) {
-        load_tile_u<BN, KROW, NT>(kbase, k_rsb, jt * BN, n - 1, smem, wave, lane);
-        load_tile_u<BN, VROW, NT>(vbase, v_rsb, jt * BN, n - 1, smem + KTILE, wave, lane);
+    // Per-lane byte offsets of this wave's copies inside a tile that lies wholly inside the sequence (32 bits, as in the key-stationary
+    // kernel): the rows clamped and multiplied out are some 15 vector instructions for every copy.
+    const bool fast_copy = k_rsb < (1 << 24) && v_rsb < (1 << 24);
+    constexpr int KINSTR = BN * (KROW / 16) / 64, VINSTR = BN * (VROW / 16) / 64, KCP = (KINSTR + NW - 1) / NW, VCP = (VINSTR + NW - 1) / NW;
+    unsigned koff[KCP], voff[VCP];
+#pragma unroll
+    for (int i = 0; i < KCP; ++i) {
+        const int pos = (wave + i * NW) * 64 + lane, row = pos / (KROW / 16);
+        koff[i] = (unsigned)(row * (int)k_rsb + (((pos % (KROW / 16)) ^ swz_u<KROW / 16>(row)) * 16));
     }
+#pragma unroll
+    for (int i = 0; i < VCP; ++i) {
+        const int pos = (wave + i * NW) * 64 + lane, row = pos / (VROW / 16);
+        voff[i] = (unsigned)(row * (int)v_rsb + (((pos % (VROW / 16)) ^ swz_u<VROW / 16>(row)) * 16));
+    }
+    auto copy_tile = [&](int t, char* stage_lds) __attribute__((always_inline)) {
+        if (fast_copy && (t + 1) * BN <= n) {
+            const char* kb = kbase + (int64_t)t * BN * k_rsb;
+            const char* vb = vbase + (int64_t)t * BN * v_rsb;
+#pragma unroll
+            for (int i = 0; i < KCP; ++i)
+                if (wave + i * NW < KINSTR) global_load_lds16_soff(kb, koff[i], stage_lds + (wave + i * NW) * 1024);
+#pragma unroll
+            for (int i = 0; i < VCP; ++i)
+                if (wave + i * NW < VINSTR) global_load_lds16_soff(vb, voff[i], stage_lds + KTILE + (wave + i * NW) * 1024);
+            return;
+        }
+        load_tile_u<BN, KROW, NT>(kbase, k_rsb, t * BN, n - 1, stage_lds, wave, lane);
+        load_tile_u<BN, VROW, NT>(vbase, v_rsb, t * BN, n - 1, stage_lds + KTILE, wave, lane);
+    };
+    if (jt < jt_end) copy_tile(jt, smem);
 
     vec8 qreg[KS], doreg[VS];
     load_q_operand<TT, KS>(qreg, p.q, W.seq_start, wq0 + l32, n, p.q_rs, p.q_hs, W.h, g, p.c1);
@@ -689,11 +716,7 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
         const int jn = next_tile(jt + 1);
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
-        if (jn < jt_end) {
-            char* nxt = smem + (stage ^ 1) * STAGE;
-            load_tile_u<BN, KROW, NT>(kbase, k_rsb, jn * BN, n - 1, nxt, wave, lane);
-            load_tile_u<BN, VROW, NT>(vbase, v_rsb, jn * BN, n - 1, nxt + KTILE, wave, lane);
-        }
+        if (jn < jt_end) copy_tile(jn, smem + (stage ^ 1) * STAGE);
         const char* kt = smem + stage * STAGE;
         const char* vt = kt + KTILE;
 #pragma unroll
@@ -705,10 +728,23 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
             f32x16_t s, dp;
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+            // The two chains alternating, operands requested four products ahead: with the chains one after the other 1409 us for 32
+            // sequences of 1024 .. 8192 rows, so 1372.
+            typedef TwoChains<KS, VS> Ops;
+            constexpr int PD = 4;
+            auto load_op = [&](int k) __attribute__((always_inline)) -> vec8 {
+                return Ops::first(k) ? *HSTU_LDS(const vec8, kt + sub * 32 * KROW + krow[Ops::index(k)])
+                                     : *HSTU_LDS(const vec8, vt + sub * 32 * VROW + vrow[Ops::index(k)]);
+            };
+            vec8 f[PD];
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) s = TT::mfma(*HSTU_LDS(const vec8, kt + sub * 32 * KROW + krow[ks]), qreg[ks], s);
+            for (int k = 0; k < PD && k < Ops::N; ++k) f[k] = load_op(k);
 #pragma unroll
-            for (int ks = 0; ks < VS; ++ks) dp = TT::mfma(*HSTU_LDS(const vec8, vt + sub * 32 * VROW + vrow[ks]), doreg[ks], dp);
+            for (int k = 0; k < Ops::N; ++k) {
+                if (Ops::first(k)) s = TT::mfma(f[k % PD], qreg[Ops::index(k)], s);
+                else dp = TT::mfma(f[k % PD], doreg[Ops::index(k)], dp);
+                if (k + PD < Ops::N) f[k % PD] = load_op(k + PD);
+            }
             vec8 dsb[2];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
