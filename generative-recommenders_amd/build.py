@@ -62,13 +62,14 @@ def build_library(verbose: bool = False) -> str:
 
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     common = [hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + ["-I", INCLUDE, "-I", CSRC]
-    objs = [os.path.join(CSRC, name) for name in ("hstu_api.o", "hstu_bwd_api.o", "hstu_fwd_fitted.o")]
+    objs = [os.path.join(CSRC, name) for name in ("hstu_api.o", "hstu_bwd_api.o", "hstu_fwd_fitted.o", "hstu_bwd_f32.o")]
     linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o"), os.path.join(CSRC, "hstu_uqvk.o"),
                    os.path.join(CSRC, "hstu_uqvk_bwd.o")]
     jobs = [
         common + ["-c", os.path.join(CSRC, "hstu_api.hip"), "-o", objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_bwd_api.hip"), "-o", objs[1]],
         common + ["-c", os.path.join(CSRC, "hstu_fwd_fitted.hip"), "-o", objs[2]],
+        common + ["-c", os.path.join(CSRC, "hstu_bwd_f32.hip"), "-o", objs[3]],
         common + ["-c", os.path.join(CSRC, "hstu_linear.hip"), "-o", linear_objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_linear_bwd.hip"), "-o", linear_objs[1]],
         # (matrix results in vector registers: see the file)

@@ -1,26 +1,14 @@
 // C ABI of the backward pass (hstu_hip_mha_bwd): validation and launch of the two kernels of hstu_bwd_kernel.h.
 // A translation unit of its own so that it compiles in parallel with the forward kernels.
-#include "hstu_hip.h"
+#include "hstu_bwd_launch.h"
 
-#include <hip/hip_runtime.h>
-
-#include <atomic>
 #include <cstdio>
 #include <cstring>
 
-#include "hstu_bwd_kernel.h"
-#include "hstu_bwd_pp_kernel.h"
-
-// defined with the forward entry points (hstu_api.hip); internal to the library
-extern "C" __attribute__((visibility("hidden"))) int hstu_hip_device_is_gfx950(void);
-extern "C" __attribute__((visibility("hidden"))) void hstu_hip_set_last_error(const char* what, int hip_error);
 extern "C" __attribute__((visibility("hidden"))) int hstu_hip_launch_rank(const void* offsets, int offsets_i64, int batch, int* order,
                                                                           void* stream);
 
 namespace {
-
-constexpr int kBwdWaves = 4, kBwdTile = 64, kBwdRows = kBwdWaves * 32;
-constexpr int kStoredWaves = 8, kStoredRows = kStoredWaves * 32;  // the dQ kernel that reads stored dS
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -30,94 +18,6 @@ size_t ds_bytes(const HstuFwdArgs* a) {
     return ((size_t)a->total_q + 32 * (size_t)a->batch) * (size_t)a->heads * pitch32 * 64;
 }
 
-template <class TT, int DQK, int DV, bool STORE>
-auto key_stationary_kernel(std::true_type) {
-    return hstu::hstu_bwd_dkdv_pp_kernel<TT, DQK, DV, STORE>;
-}
-template <class TT, int DQK, int DV, bool STORE>
-auto key_stationary_kernel(std::false_type) {
-    return hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, STORE>;
-}
-
-template <class TT, int DQK, int DV>
-int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
-    // three tile slots for the key-stationary kernel, two for the other; + 64: transposing reads of a 16-wide tile's unused half
-    constexpr int smem1 = 3 * kBwdTile * (DQK + DV) * 2 + 64;
-    constexpr int smem = 2 * kBwdTile * (DQK + DV) * 2 + 64;
-    constexpr int smem3 = 3 * kBwdTile * DQK * 2 + kStoredWaves * 3 * 4096;
-    // The key-stationary kernel: with two waves per SIMD where a tile copy gives every copying wave something to do and
-    // the byte offsets inside a tile of 64 rows fit its 32-bit arithmetic; the one-wave kernel otherwise.
-    constexpr bool kPairedDims = DQK >= 32 && DV >= 32;
-    auto k1p = key_stationary_kernel<TT, DQK, DV, false>(std::integral_constant<bool, kPairedDims>{});
-    auto k1ps = key_stationary_kernel<TT, DQK, DV, true>(std::integral_constant<bool, kPairedDims>{});
-    constexpr int smem1p = kPairedDims ? hstu::bwd_pp_lds_bytes<(DQK < 32 ? 32 : DQK), (DV < 32 ? 32 : DV)>() : 0;
-    const bool paired = kPairedDims && bp.f.q_rs < (1 << 22) && bp.do_rs < (1 << 22);
-    auto k1 = hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, false>;
-    auto k1s = hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, true>;
-    auto k2 = hstu::hstu_bwd_dq_kernel<TT, DQK, DV, kBwdWaves, kBwdTile>;
-    auto k3 = hstu::hstu_bwd_dq_stored_kernel<TT, DQK, kStoredWaves, kBwdTile>;
-    // (a function attribute belongs to the device it was set on: one flag per device)
-    static std::atomic<bool> attr_done[64];
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
-    if (dev < 0 || !attr_done[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void*)k1, hipFuncAttributeMaxDynamicSharedMemorySize, smem1);
-        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1s, hipFuncAttributeMaxDynamicSharedMemorySize, smem1);
-        if (kPairedDims) {
-            if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1p, hipFuncAttributeMaxDynamicSharedMemorySize, smem1p);
-            if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1ps, hipFuncAttributeMaxDynamicSharedMemorySize, smem1p);
-        }
-        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k3, hipFuncAttributeMaxDynamicSharedMemorySize, smem3);
-        if (e != hipSuccess) {
-            hstu_hip_set_last_error("hipFuncSetAttribute", (int)e);
-            return HSTU_ERR_LAUNCH;
-        }
-        if (dev >= 0) attr_done[dev] = true;
-    }
-    const unsigned grid = (unsigned)bp.f.slots_per_xcd * 8;
-    if (bp.ds) {
-        if (paired) hipLaunchKernelGGL(k1ps, dim3(grid), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
-        else hipLaunchKernelGGL(k1s, dim3(grid), dim3(kBwdWaves * 64), smem1, stream, bp);
-        hstu::BwdParams b3 = bp;  // the same items in blocks of 256 query rows
-        b3.f.num_mb = (bp.f.max_seq_len + kStoredRows - 1) / kStoredRows;
-        b3.f.slots_per_xcd = bp.f.pairs_per_xcd * b3.f.num_mb;
-        hipLaunchKernelGGL(k3, dim3((unsigned)b3.f.slots_per_xcd * 8), dim3(kStoredWaves * 64), smem3, stream, b3);
-    } else {
-        if (paired) hipLaunchKernelGGL(k1p, dim3(grid), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
-        else hipLaunchKernelGGL(k1, dim3(grid), dim3(kBwdWaves * 64), smem1, stream, bp);
-        hipLaunchKernelGGL(k2, dim3(grid), dim3(kBwdWaves * 64), smem, stream, bp);
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        hstu_hip_set_last_error("backward kernel launch", (int)e);
-        return HSTU_ERR_LAUNCH;
-    }
-    return HSTU_OK;
-}
-
-template <class TT, int DQK>
-int launch_bwd_dv(const hstu::BwdParams& bp, int dv, hipStream_t stream) {
-    switch (dv) {
-        case 16: return launch_bwd<TT, DQK, 16>(bp, stream);
-        case 32: return launch_bwd<TT, DQK, 32>(bp, stream);
-        case 64: return launch_bwd<TT, DQK, 64>(bp, stream);
-        case 128: return launch_bwd<TT, DQK, 128>(bp, stream);
-        default: return HSTU_ERR_BAD_HEAD_DIM;
-    }
-}
-
-template <class TT>
-int launch_bwd_dim(const hstu::BwdParams& bp, int dqk, int dv, hipStream_t stream) {
-    switch (dqk) {
-        case 16: return launch_bwd_dv<TT, 16>(bp, dv, stream);
-        case 32: return launch_bwd_dv<TT, 32>(bp, dv, stream);
-        case 64: return launch_bwd_dv<TT, 64>(bp, dv, stream);
-        case 128: return launch_bwd_dv<TT, 128>(bp, dv, stream);
-        default: return HSTU_ERR_BAD_HEAD_DIM;
-    }
-}
-
 }  // namespace
 
 extern "C" size_t hstu_hip_mha_bwd_workspace_bytes(const HstuFwdArgs* a) {
@@ -125,7 +25,9 @@ extern "C" size_t hstu_hip_mha_bwd_workspace_bytes(const HstuFwdArgs* a) {
     return align256((size_t)a->batch * sizeof(int)) + ds_bytes(a);
 }
 
-extern "C" int hstu_hip_mha_bwd(const HstuFwdArgs* a, const HstuBwdGrads* g, void* stream_) {
+__attribute__((visibility("hidden"))) int hstu_bwd_params(const HstuFwdArgs* a, const HstuBwdGrads* g, int64_t grad_mask, hstu::BwdParams& bp, bool& nothing,
+                                                          void* stream_) {
+    nothing = true;
     if (!a || !g) return HSTU_ERR_NULL_POINTER;
     HstuFwdArgs c = *a;  // the forward's own checks, with the unused output standing in as any aligned pointer
     c.out = const_cast<void*>(a->q);
@@ -147,11 +49,10 @@ extern "C" int hstu_hip_mha_bwd(const HstuFwdArgs* a, const HstuBwdGrads* g, voi
     const int64_t strides[8] = {g->do_row_stride, g->do_head_stride, g->dq_row_stride, g->dq_head_stride,
                                 g->dk_row_stride, g->dk_head_stride, g->dv_row_stride, g->dv_head_stride};
     for (int i = 0; i < 8; ++i)
-        if (strides[i] < 0 || (strides[i] & 7) != 0) return HSTU_ERR_MISALIGNED;
+        if (strides[i] < 0 || (strides[i] & (i < 2 ? 7 : grad_mask)) != 0) return HSTU_ERR_MISALIGNED;
     if (!hstu_hip_device_is_gfx950()) return HSTU_ERR_BAD_DEVICE;
-    hipStream_t stream = (hipStream_t)stream_;
+    nothing = false;
 
-    hstu::BwdParams bp;
     memset(&bp, 0, sizeof(bp));
     hstu::FwdParams& p = bp.f;
     p.q = (const char*)a->q;
@@ -202,6 +103,14 @@ extern "C" int hstu_hip_mha_bwd(const HstuFwdArgs* a, const HstuBwdGrads* g, voi
         bp.ds = (char*)a->workspace + align256((size_t)a->batch * sizeof(int));
         bp.ds_pitch32 = 4 * ((a->max_seq_len + 127) / 128);
     }
-    if (a->dtype == HSTU_BF16) return launch_bwd_dim<hstu::Bf16>(bp, a->dqk, a->dv, stream);
-    return launch_bwd_dim<hstu::Fp16>(bp, a->dqk, a->dv, stream);
+    return HSTU_OK;
+}
+
+extern "C" int hstu_hip_mha_bwd(const HstuFwdArgs* a, const HstuBwdGrads* g, void* stream) {
+    hstu::BwdParams bp;
+    bool nothing;
+    const int rc = hstu_bwd_params(a, g, 7, bp, nothing, stream);
+    if (rc != HSTU_OK || nothing) return rc;
+    if (a->dtype == HSTU_BF16) return launch_bwd_dim<hstu::Bf16>(bp, a->dqk, a->dv, (hipStream_t)stream);
+    return launch_bwd_dim<hstu::Fp16>(bp, a->dqk, a->dv, (hipStream_t)stream);
 }

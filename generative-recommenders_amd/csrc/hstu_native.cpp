@@ -157,7 +157,14 @@ void attention_backward(const Tensor& dout, const Tensor& q, const Tensor& k, co
     g.dk_row_stride = dk.stride(0), g.dk_head_stride = dk.stride(1);
     g.dv_row_stride = dv.stride(0), g.dv_head_stride = dv.stride(1);
     const c10::DeviceGuard guard(q.device());
-    const int rc = hstu_hip_mha_bwd(&a, &g, stream_of(q));
+    int rc;
+    if (q.scalar_type() == at::kFloat) {
+        const int64_t bytes = (int64_t)hstu_hip_mha_bwd_f32_copies_bytes(&a);
+        Tensor copies = at::empty({bytes}, q.options().dtype(at::kByte));
+        rc = hstu_hip_mha_bwd_f32(&a, &g, copies.data_ptr(), bytes, stream_of(q));
+    } else {
+        rc = hstu_hip_mha_bwd(&a, &g, stream_of(q));
+    }
     if (rc == HSTU_OK) return;
     // (the classes that the Python operators raise for a status)
     const std::string what = c10::str("hstu_hip: ", hstu_hip_status_string(rc), " (", hstu_hip_last_error(), ") [status ", rc, "]");
@@ -184,20 +191,15 @@ struct MhaFunction : torch::autograd::Function<MhaFunction> {
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const BackwardScope scope;
         const auto saved = ctx->get_saved_variables();
-        Tensor q = kernel_rows(saved[0]), k = kernel_rows(saved[1]), v = kernel_rows(saved[2]);
+        const Tensor q = kernel_rows(saved[0]), k = kernel_rows(saved[1]), v = kernel_rows(saved[2]);
         const OptTensor targets = saved[4].defined() ? OptTensor(saved[4].contiguous()) : OptTensor();
         const auto ws = ctx->saved_data.find("workspace");
         const OptTensor workspace = ws == ctx->saved_data.end() ? OptTensor() : OptTensor(ws->second.toTensor());
-        // fp32 inputs: the backward kernels take 16-bit operands, so they run on bf16 copies (fp32's range: dout can be tiny) and
-        // the gradients are widened again
-        const bool wide = q.scalar_type() == at::kFloat;
-        if (wide) q = q.to(at::kBFloat16), k = k.to(at::kBFloat16), v = v.to(at::kBFloat16);
         const Tensor dout = kernel_rows(grads[0].to(q.scalar_type()));
         Tensor dq = at::empty_like(q, at::MemoryFormat::Contiguous), dk = at::empty_like(k, at::MemoryFormat::Contiguous),
                dv = at::empty_like(v, at::MemoryFormat::Contiguous);
         attention_backward(dout, q, k, v, dq, dk, dv, saved[3].contiguous(), targets,
                            unpack(ctx->saved_data["call"].toIntVector(), ctx->saved_data["alpha"].toDouble()), workspace);
-        if (wide) dq = dq.to(at::kFloat), dk = dk.to(at::kFloat), dv = dv.to(at::kFloat);
         return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };

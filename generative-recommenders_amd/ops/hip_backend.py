@@ -108,6 +108,8 @@ EXPORTS = (
     "hstu_hip_mha_fwd_noalloc",
     "hstu_hip_check_contract",
     "hstu_hip_mha_bwd",
+    "hstu_hip_mha_bwd_f32",
+    "hstu_hip_mha_bwd_f32_copies_bytes",
     "hstu_hip_mha_bwd_workspace_bytes",
     "hstu_hip_workspace_bytes",
     "hstu_hip_plan",

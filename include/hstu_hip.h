@@ -221,6 +221,12 @@ typedef struct HstuBwdGrads {
 
 int hstu_hip_mha_bwd(const HstuFwdArgs* args, const HstuBwdGrads* grads, void* stream);
 
+/* The same with fp32 tensors (args->dtype HSTU_FP32; strides of all tensors multiples of 4, bases 16-byte aligned): q, k, v and dout are rounded to
+ * bf16 into `copies` (16-byte aligned, hstu_hip_mha_bwd_f32_copies_bytes(args) bytes), dq, dk, dv are the fp32 sums.  `args->workspace` means what it
+ * means there. */
+size_t hstu_hip_mha_bwd_f32_copies_bytes(const HstuFwdArgs* args);
+int hstu_hip_mha_bwd_f32(const HstuFwdArgs* args, const HstuBwdGrads* grads, void* copies, int64_t copies_bytes, void* stream);
+
 /*
  * ---- The data format either side of the path: per-batch concatenation of two jagged 2-D tensors ----
  *

@@ -436,6 +436,33 @@ def test_backward_of_fp32_inputs(pkg, dev, mi):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("store", [False, True])
+@pytest.mark.parametrize("dqk,dv", [(64, 32), (16, 128), (128, 16), (128, 128), (32, 64)])
+def test_backward_of_fp32_slices(pkg, dev, dqk, dv, store):
+    """q, k, v as column slices of one fp32 buffer and dout with padded rows: one launch rounds the four, the gradients are the fp32 sums
+    (not 16-bit values widened again)."""
+    from generative_recommenders_amd.ops import hip_backend
+
+    print(f"[case] bwd fp32 slices {dqk} {dv} {store}", flush=True)
+    lengths, H = [70, 0, 129, 1, 33], 3
+    q, k, v, dout, offsets = _inputs(77 + dqk, lengths, H, dqk, dv, torch.float32)
+    L = q.shape[0]
+    buffer = torch.cat([v.flatten(1), q.flatten(1), k.flatten(1)], dim=1).to(dev)
+    vs, qs, ks = torch.split(buffer, [H * dv, H * dqk, H * dqk], dim=1)
+    leaves = [t.view(L, H, -1).detach().requires_grad_(True) for t in (qs, ks, vs)]
+    ws = torch.empty(hip_backend.mha_bwd_workspace_bytes(L, len(lengths), H, 140), dtype=torch.uint8, device=dev) if store else None
+    out = pkg.hstu_mha(140, 0.125, *leaves, offsets.to(dev), contextual_seq_len=5, bwd_workspace=ws)
+    padded = torch.zeros(L, H, dv + 4, device=dev)
+    padded[:, :, :dv] = dout.to(dev)
+    grads = torch.autograd.grad(out, leaves, padded[:, :, :dv])
+    torch.cuda.synchronize()
+    refs = G.closed_form_grads(140, 0.125, q, k, v, offsets, dout, contextual_seq_len=5)
+    for name, got, ref in zip(("dq", "dk", "dv"), grads, refs):
+        assert got.dtype == torch.float32 and not torch.equal(got, got.bfloat16().float()), name
+        _close(got, ref, f"fp32 {name}")
+
+
+@pytest.mark.gpu
 def test_backward_rejections(pkg, dev):
     q, k, v, dout, offsets = _inputs(1, [40, 24], 2, 32, 32, torch.float32)
     with pytest.raises(NotImplementedError):  # fp8 inputs have no backward
