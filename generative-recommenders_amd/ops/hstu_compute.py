@@ -2,18 +2,19 @@
 signatures (``generative_recommenders/ops/hstu_compute.py:54-104``, ``:107-214``, ``:217-334``).
 
 ``hstu_compute_uqvk``: layer norm + uvqk projection + split + SiLU(u), in one hand-written gfx950 kernel for d_model 128,
-256, 384 and 512 (``csrc/hstu_uqvk_kernel.h``, ``csrc/hstu_uqvk_wide_kernel.h``); other shapes take a layer-norm kernel and hipBLASLt
+256, 384 and 512 (``csrc/hstu_uqvk_kernel.h``, ``csrc/hstu_uqvk_wide_kernel.h``, the choice in ``csrc/hstu_uqvk_launch.h``); other shapes take a layer-norm kernel and hipBLASLt
 with the bias and, for the u columns, the SiLU in its epilogue.  ``u, q, k, v`` come back as column slices of one
 ``[L, (2*hidden + 2*attn) * H]`` buffer, which ``hstu_mha`` / ``delta_hstu_mha`` read in place.
 
-``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  From 32768 rows on a hand-written GEMM reads u
-and attn where they are and ``act(u) * norm(attn)`` from a row-wise kernel; below, and for widths it does not take or with dropout, that
+``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  Up to 256 rows one kernel does it all
+(``csrc/hstu_output_rows_kernel.h``).  From 32768 rows on a hand-written GEMM reads u
+and attn where they are and ``act(u) * norm(attn)`` from a row-wise kernel; between them, and for widths it does not take or with dropout, that
 kernel writes the concatenated operand and hipBLASLt multiplies it with the residual as its C operand.
 (``csrc/hstu_linear.hip``, ``csrc/hstu_output_kernel.h``, ``include/hstu_linear.h``.)
 
 Device tensors only, bf16 or fp16; ``kernel`` is accepted and ignored.  The usual call, with or without gradients, goes through
-the native front (``csrc/hstu_native.cpp``): backward kernels for the row-wise parts (``csrc/hstu_linear_bwd.hip``), plain
-products around them.  What it leaves -- operands that need a copy first -- is handled here; its gradients come from a
+the native front (``csrc/hstu_native.cpp``): backward kernels for the row-wise parts (``csrc/hstu_linear_bwd.hip``), products on the
+producer's kernels (``csrc/hstu_uqvk_bwd.hip``) or the library's around them.  What it leaves -- operands that need a copy first -- is handled here; its gradients come from a
 recomputation with the framework's operators (see ``_grads_by_recomputation``).
 """
 
