@@ -63,13 +63,22 @@ struct UqvkFusedParams {
 
 constexpr int kUqvkStageRow = 64 * 2 + 16;  // staging row: 64 outputs + pad
 
-// N values as they are in fp32, rounded to E.  (fp16: left to itself the compiler makes one rounding of the last operation and this one, in
-// one kernel and not in the other.)
+// N values rounded to E by instructions of the compiler's: for sums as the matrix instructions leave them.
 template <class E, int N>
-__device__ __forceinline__ auto round_to(const float (&x)[N]) {
+__device__ __forceinline__ auto round_sums(const float (&x)[N]) {
     typedef __attribute__((ext_vector_type(N))) E vec;
     vec r;
+#pragma unroll
+    for (int j = 0; j < N; ++j) r[j] = (E)x[j];
+    return r;
+}
+// N values as they are in fp32, rounded to E.  (fp16: left to itself the compiler makes one rounding of the last operation and this one, in
+// one kernel and not in the other.)  Results of vector instructions only: the hardware does not interlock a matrix result against a
+// vector instruction's read, and the compiler does not count the wait states for reads inside an asm block.
+template <class E, int N>
+__device__ __forceinline__ auto round_to(const float (&x)[N]) {
     if constexpr (std::is_same<E, _Float16>::value) {
+        typedef __attribute__((ext_vector_type(N))) E vec;
         typedef __attribute__((ext_vector_type(N / 2))) unsigned words;
         words w;
 #pragma unroll
@@ -78,12 +87,10 @@ __device__ __forceinline__ auto round_to(const float (&x)[N]) {
             asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(o) : "v"(x[j]), "v"(x[j + 1]));
             w[j / 2] = o;
         }
-        r = __builtin_bit_cast(vec, w);
+        return __builtin_bit_cast(vec, w);
     } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) r[j] = (E)x[j];
+        return round_sums<E>(x);
     }
-    return r;
 }
 
 // The layer norm's arithmetic.  A row's bits must not depend on the batch, and the kernels for few and for many rows hold a row
@@ -375,7 +382,10 @@ __global__ __launch_bounds__(256, (UqvkRows<KT, RB, NB>::kPerCu)) void hstu_uqvk
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = v[j] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v[j]));
         }
-        *HSTU_LDS(elem4, stage + l32 * Geo::kStageRow + (dt * 32 + r4 * 8 + g * 4) * 2) = round_to<elem>(v);
+        elem4 o;
+        if constexpr (BIAS) o = round_to<elem>(v);
+        else o = round_sums<elem>(v);
+        *HSTU_LDS(elem4, stage + l32 * Geo::kStageRow + (dt * 32 + r4 * 8 + g * 4) * 2) = o;
     };
     auto read_rows = [&](int i) __attribute__((always_inline)) {
         rd[i % STORES] = *HSTU_LDS(const i32x4_t, stage + (i % STORES * RPS + rsub) * Geo::kStageRow + chunk * 16);

@@ -195,7 +195,10 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = v[j] * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v[j]));
             }
-            *HSTU_LDS(elem4, stage + rg * kWideStage + l32 * kUqvkStageRow + (dt * 32 + r4 * 8 + g * 4) * 2) = round_to<elem>(v);
+            elem4 o;
+            if constexpr (TRANS) o = round_sums<elem>(v);
+            else o = round_to<elem>(v);
+            *HSTU_LDS(elem4, stage + rg * kWideStage + l32 * kUqvkStageRow + (dt * 32 + r4 * 8 + g * 4) * 2) = o;
         };
         auto read_rows = [&](int i) __attribute__((always_inline)) {
             rd[i] = *HSTU_LDS(const i32x4_t, stage + (i >> 2) * kWideStage + ((i & 3) * 8 + rsub) * kUqvkStageRow + chunk * 16);

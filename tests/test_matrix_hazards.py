@@ -1,0 +1,107 @@
+"""Wait states between matrix instructions and the vector instructions that read their results, in the libraries as they are built.
+
+The hardware does not interlock such a read: the compiler counts the wait states and fills them up, but not for a read inside an asm block,
+and a kernel that reads too early rounds what the registers held before.  Needs no GPU: the code objects are listed with the toolchain's
+own disassembler.
+"""
+
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+_CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "generative-recommenders_amd", "csrc")
+_REGISTERS = re.compile(r"\b([av])(?:(\d+)\b|\[(\d+):(\d+)\])")
+_LINE = re.compile(r"^\s+(\S+)(?:\s+(.*?))?\s*// ([0-9A-F]+): ")
+
+
+def _registers(text):
+    out = set()
+    for bank, one, first, last in _REGISTERS.findall(text):
+        out.update((bank, i) for i in (range(int(one), int(one) + 1) if one else range(int(first), int(last) + 1)))
+    return out
+
+
+def _wait_states(name):
+    """Of a matrix instruction whose result a vector instruction reads: its passes + 3.  (The compiler leaves one more on this chip, except
+    where it counts a branch that is taken as two.)  8 passes for products of 32x32, 4 of 16x16; those of depth 64 have 16 and are followed
+    as far as the others: a path in the listing that no wave takes, through a scalar branch on a constant, has 13 states behind one."""
+    return (8 if "32x32" in name else 4) + 3
+
+
+def early_reads(listing):
+    """(matrix instructions, [(kernel, instruction, wait states left)]) of a listing of llvm-objdump -d."""
+    code, at, kernel = [], {}, None
+    for line in listing.splitlines():
+        m = _LINE.match(line)
+        if m:
+            at[int(m[3], 16)] = len(code)
+            code.append((m[1], m[2] or "", int(m[3], 16), kernel))
+        elif line.endswith(">:"):
+            kernel = line.split("<")[1][:-2]
+    products, early = 0, []
+    for i, (name, operands, _, kernel) in enumerate(code):
+        if not name.startswith("v_mfma"):
+            continue
+        products += 1
+        need = _wait_states(name)
+        todo, seen = [(i + 1, 0, frozenset(_registers(operands[: operands.index("]") + 1])))], {}
+        while todo:
+            j, waited, result = todo.pop()
+            if j >= len(code) or waited >= need or not result or seen.get(j, need) <= waited:
+                continue
+            seen[j] = waited
+            n, o, address, here = code[j]
+            if here != kernel or n == "s_endpgm":
+                continue
+            if not n.startswith(("s_", "v_mfma")):
+                first, _, rest = o.partition(",")
+                reads, writes = (_registers(o), set()) if "store" in n or "write" in n else (_registers(rest), _registers(first))
+                if reads & result:
+                    early.append((kernel, f"{n} {o}", waited))
+                    continue
+                result = result - writes
+            step = 1 + (int(o, 0) if n == "s_nop" else 0)
+            if n == "s_branch" or n.startswith("s_cbranch"):
+                offset = int(o.split()[0])
+                target = at.get(address + 4 + 4 * (offset - 65536 * (offset >= 32768)))
+                if target is not None:
+                    todo.append((target, waited + step, result))
+                if n == "s_branch":
+                    continue
+            todo.append((j + 1, waited + step, result))
+    return products, early
+
+
+def test_the_listing_reader_finds_an_early_read():
+    def listing(*lines):
+        return "0000 <k>:\n" + "\n".join(f"\t{text} // {4 * i:012X}: 00000000" for i, text in enumerate(lines))
+
+    product = "v_mfma_f32_32x32x16_f16 v[0:15], v[16:19], v[20:23], v[0:15]"
+    convert = "v_cvt_pk_f16_f32 v30, v2, v3"
+    assert early_reads(listing(product, "s_nop 9", convert))[1] == [("k", convert, 10)]
+    assert early_reads(listing(product, "s_nop 10", convert)) == (1, [])
+    assert early_reads(listing(product, "s_branch 1", "s_endpgm", "s_nop 8", convert))[1] == [("k", convert, 10)]
+    assert early_reads(listing(product, "v_mov_b32_e32 v2, v40", "v_mov_b32_e32 v3, v40", convert)) == (1, [])
+    assert early_reads(listing(product, "ds_write_b64 v50, v[2:3]"))[1] == [("k", "ds_write_b64 v50, v[2:3]", 0)]
+
+
+@pytest.mark.parametrize("library", ["libhstu_hip.so", "libhstu_linear.so"])
+def test_no_vector_instruction_reads_a_matrix_result_too_early(tmp_path, library):
+    objdump = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+    built = os.path.join(_CSRC, library)
+    if not os.path.exists(objdump) or not os.path.exists(built):
+        pytest.skip("needs llvm-objdump and the built library")
+    shutil.copy(built, tmp_path / library)
+    subprocess.run([objdump, "--offloading", library], cwd=tmp_path, check=True, capture_output=True)
+    objects = sorted(p for p in os.listdir(tmp_path) if p.endswith("gfx950"))
+    assert len(objects) == 4
+    total, early = 0, []
+    for name in objects:
+        text = subprocess.run([objdump, "-d", name], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+        products, found = early_reads(text)
+        total, early = total + products, early + found
+    assert total > 1000
+    assert not early, early[:10]
