@@ -158,8 +158,12 @@ __device__ __forceinline__ float ln_tree_lanes(float s) {
 }
 
 // Row r (rows past the end repeat the last one) through the layer norm, as the B operands of a lane: 8 consecutive k of every 16,
-// from 8 g on; the two half-waves share the row.
-template <class TT, int KS>
+// from 8 g on; the two half-waves share the row.  The chunks' sums are pinned in their order: left to itself the compiler moves a tree's leaves
+// so far apart that two loads wait until the others have been summed, and the operands end up in the register banks of W's.  LOADS_FIRST: no
+// arithmetic among the loads, as the kernel with 64 rows per wave wants it.  Left to itself / so, us: the kernel with 128 rows per workgroup,
+// d_model 512 into 256 columns, 100000 rows 66.5 / 65.1, into 512, 20000 rows 34.9 / 34.6; the one with 64 rows per wave, d_model 256 into
+// 1024, 100000 rows 99.9 / 96.2.
+template <class TT, int KS, bool LOADS_FIRST>
 __device__ __forceinline__ void uqvk_normalised_row(const UqvkFusedParams& p, int64_t r, int g, typename TT::vec8 (&xr)[KS]) {
     typedef typename TT::vec8 vec8;
     typedef typename TT::elem elem;
@@ -168,13 +172,22 @@ __device__ __forceinline__ void uqvk_normalised_row(const UqvkFusedParams& p, in
     const char* xp = p.x + (r * p.x_rs + 8 * g) * 2;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) xr[ks] = *(const vec8*)(xp + ks * 32);
-    asm volatile("" : : : "memory");  // (the loads before the arithmetic)
-    const float mean = ln_mean<K>(ln_tree<KS>([&](int ks) __attribute__((always_inline)) { return ln_chunk_sum(xr[ks]); }));
+    if constexpr (LOADS_FIRST) asm volatile("" : : : "memory");
+    const float mean = ln_mean<K>(ln_tree<KS>([&](int ks) __attribute__((always_inline)) {
+        float sum = ln_chunk_sum(xr[ks]);
+        asm volatile("" : "+v"(sum));
+        return sum;
+    }));
     // the rows stay packed between the passes: without this the compiler keeps all their fp32 conversions alive
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xr[ks]));
     const float rstd =
-        ln_rstd<K>(ln_tree<KS>([&](int ks) __attribute__((always_inline)) { return ln_chunk_squares(xr[ks], mean); }), p.eps);
+        ln_rstd<K>(ln_tree<KS>([&](int ks) __attribute__((always_inline)) {
+                       float sum = ln_chunk_squares(xr[ks], mean);
+                       asm volatile("" : "+v"(sum));
+                       return sum;
+                   }),
+                   p.eps);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(xr[ks]));
 #pragma unroll
@@ -579,7 +592,7 @@ __global__ __launch_bounds__(kUqvkWaves * 64, 2) void hstu_uqvk_fused_kernel(con
     // ---- this wave's rows: load, normalise, keep as B operands
     vec8 xreg[RG][KS];
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg) uqvk_normalised_row<TT, KS>(p, row0 + rg * 32 + l32, g, xreg[rg]);
+    for (int rg = 0; rg < RG; ++rg) uqvk_normalised_row<TT, KS, false>(p, row0 + rg * 32 + l32, g, xreg[rg]);
 
     // transposing reads of a W tile: lane supplies the address of 4 consecutive n of k row 8g + 4sec + j
     int waddr[2][4];

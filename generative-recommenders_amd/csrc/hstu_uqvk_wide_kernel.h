@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256, 1) void hstu_uqvk_wide_kernel(const UqvkFusedP
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) xreg[rg][ks] = *(const vec8*)(p.x + (r * p.x_rs + ks * 16 + 8 * g) * 2);
             } else {
-                uqvk_normalised_row<TT, KS>(p, row0 + rg * 32 + l32, g, xreg[rg]);
+                uqvk_normalised_row<TT, KS, true>(p, row0 + rg * 32 + l32, g, xreg[rg]);
             }
             // all of it here: the compiler would otherwise move the arithmetic of the second half into the first column block
 #pragma unroll
