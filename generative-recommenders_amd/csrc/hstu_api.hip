@@ -801,7 +801,7 @@ int common_vector_bytes(std::initializer_list<uint64_t> values) {
 }
 
 constexpr int kJaggedRows = 32, kTailRows = 16;  // rows per workgroup of the two kernels
-constexpr int64_t kShortRow = 1 << 26;           // bytes of a row up to which a block's accesses are counted in 32 bits
+constexpr int64_t kShortRow = 1 << 26;           // accesses of a row up to which a block's are counted in 32 bits
 
 int check_jagged_args(const HstuJaggedCopyArgs* a) {
     if (!a) return HSTU_ERR_NULL_POINTER;
@@ -845,17 +845,20 @@ int launch_jagged_copy(const HstuJaggedCopyArgs* a, hipStream_t stream) {
     const int vec = common_vector_bytes({(uint64_t)(uintptr_t)a->left, (uint64_t)(uintptr_t)a->right, (uint64_t)(uintptr_t)a->joined,
                                          (uint64_t)a->left_row_stride, (uint64_t)a->right_row_stride,
                                          (uint64_t)a->joined_row_stride, (uint64_t)a->row_bytes});
-#define HSTU_COPY_LAUNCH(V, INDEX) hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, V, kJaggedRows, INDEX>), grid, dim3(256), 0, stream, p)
-    if (a->row_bytes > kShortRow) {
-        HSTU_COPY_LAUNCH(1, uint64_t);
-    } else {
-        switch (vec) {
-            case 16: HSTU_COPY_LAUNCH(16, unsigned); break;
-            case 8: HSTU_COPY_LAUNCH(8, unsigned); break;
-            case 4: HSTU_COPY_LAUNCH(4, unsigned); break;
-            case 2: HSTU_COPY_LAUNCH(2, unsigned); break;
-            default: HSTU_COPY_LAUNCH(1, unsigned); break;
-        }
+    // (rows of more bytes than that, counted in 64 bits and copied byte by byte, took 17 times as long: 8 rows of 64 MB + 32 bytes 611 ms, so 35)
+#define HSTU_COPY_LAUNCH(V)                                                                                                      \
+    do {                                                                                                                         \
+        if (a->row_bytes / V > kShortRow)                                                                                        \
+            hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, V, kJaggedRows, uint64_t>), grid, dim3(256), 0, stream, p); \
+        else                                                                                                                     \
+            hipLaunchKernelGGL((hstu::hstu_jagged_copy_kernel<SPLIT, V, kJaggedRows, unsigned>), grid, dim3(256), 0, stream, p); \
+    } while (0)
+    switch (vec) {
+        case 16: HSTU_COPY_LAUNCH(16); break;
+        case 8: HSTU_COPY_LAUNCH(8); break;
+        case 4: HSTU_COPY_LAUNCH(4); break;
+        case 2: HSTU_COPY_LAUNCH(2); break;
+        default: HSTU_COPY_LAUNCH(1); break;
     }
 #undef HSTU_COPY_LAUNCH
     hipError_t e = hipGetLastError();
@@ -885,20 +888,22 @@ int hstu_hip_jagged_write_tail(void* joined, int64_t joined_row_stride, const vo
     hipStream_t stream = (hipStream_t)stream_;
     const int vec = common_vector_bytes({(uint64_t)(uintptr_t)joined, (uint64_t)(uintptr_t)tail, (uint64_t)joined_row_stride,
                                          (uint64_t)tail_row_stride, (uint64_t)row_bytes});
-#define HSTU_TAIL_LAUNCH(V, INDEX)                                                                                            \
+#define HSTU_TAIL_KERNEL(V, INDEX)                                                                                            \
     hipLaunchKernelGGL((hstu::hstu_jagged_write_tail_kernel<V, kTailRows, INDEX>), grid, dim3(256), 0, stream, (char*)joined,   \
                        joined_row_stride, offsets, offsets_i64, (const char*)tail, tail_row_stride, row_bytes, tail_len)
-    if (row_bytes > kShortRow) {
-        HSTU_TAIL_LAUNCH(1, uint64_t);
-    } else {
-        switch (vec) {
-            case 16: HSTU_TAIL_LAUNCH(16, unsigned); break;
-            case 8: HSTU_TAIL_LAUNCH(8, unsigned); break;
-            case 4: HSTU_TAIL_LAUNCH(4, unsigned); break;
-            case 2: HSTU_TAIL_LAUNCH(2, unsigned); break;
-            default: HSTU_TAIL_LAUNCH(1, unsigned); break;
-        }
+#define HSTU_TAIL_LAUNCH(V)                                           \
+    do {                                                              \
+        if (row_bytes / V > kShortRow) HSTU_TAIL_KERNEL(V, uint64_t); \
+        else HSTU_TAIL_KERNEL(V, unsigned);                           \
+    } while (0)
+    switch (vec) {
+        case 16: HSTU_TAIL_LAUNCH(16); break;
+        case 8: HSTU_TAIL_LAUNCH(8); break;
+        case 4: HSTU_TAIL_LAUNCH(4); break;
+        case 2: HSTU_TAIL_LAUNCH(2); break;
+        default: HSTU_TAIL_LAUNCH(1); break;
     }
+#undef HSTU_TAIL_KERNEL
 #undef HSTU_TAIL_LAUNCH
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

@@ -228,6 +228,38 @@ def test_write_kv_tail_blocks(pkg, dev, batch, tail, columns, dtype):
 
 
 @pytest.mark.gpu
+def test_rows_longer_than_64_megabytes_are_copied_as_wide(pkg, dev):
+    """A row just above 2^26 bytes takes what one of 2^26 takes: 16 bytes per access, whatever counts them (byte by byte it was 17 times as long;
+    the bound leaves a factor of 4 for the machine).  A row of more than 2^26 accesses, which are counted in 64 bits, on top."""
+    print("[case] jagged rows above 64 MB", flush=True)
+    offs = torch.tensor([0, 2], device=dev)
+
+    def run(columns):
+        a = torch.arange(2 * columns, device=dev).view(2, columns)
+        b = -a - 1
+        best = None
+        for _ in range(3):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            joined = pkg.concat_2D_jagged(4, a, b, 2, 2, offs, offs)
+            end.record()
+            end.synchronize()
+            ms = start.elapsed_time(end)
+            best = ms if best is None else min(best, ms)
+        assert torch.equal(joined, torch.cat([a, b]))
+        tail = joined.clone()
+        pkg.write_kv_tail(tail, torch.tensor([0, 4], device=dev), a)
+        assert torch.equal(tail, torch.cat([a, a]))
+        left, right = pkg.split_2D_jagged(4, joined, max_len_left=2, max_len_right=2, offsets_left=offs, offsets_right=offs)
+        assert torch.equal(left, a) and torch.equal(right, b)
+        return best
+
+    line = run(1 << 23)
+    assert run((1 << 23) + 2) < 4 * line
+    run((1 << 27) + 2)
+
+
+@pytest.mark.gpu
 def test_jagged_wrapper_rejections(pkg, dev):
     a = torch.zeros((4, 8), device=dev)
     with pytest.raises(AssertionError, match="values_left must be 2D"):
