@@ -800,7 +800,7 @@ int common_vector_bytes(std::initializer_list<uint64_t> values) {
     return vec;
 }
 
-constexpr int kJaggedRows = 32, kTailRows = 16;  // rows per workgroup of the two kernels
+constexpr int kJaggedRows = 32;  // rows per workgroup of the copy kernel
 constexpr int64_t kShortRow = 1 << 26;           // accesses of a row up to which a block's are counted in 32 bits
 
 int check_jagged_args(const HstuJaggedCopyArgs* a) {
@@ -884,13 +884,19 @@ int hstu_hip_jagged_write_tail(void* joined, int64_t joined_row_stride, const vo
     if (batch == 0 || tail_len == 0 || row_bytes == 0) return HSTU_OK;
     if (!joined || !offsets || !tail) return HSTU_ERR_NULL_POINTER;
     if (batch > 65535) return HSTU_ERR_BAD_SHAPE;
-    const dim3 grid((unsigned)((tail_len + kTailRows - 1) / kTailRows), (unsigned)batch);
     hipStream_t stream = (hipStream_t)stream_;
     const int vec = common_vector_bytes({(uint64_t)(uintptr_t)joined, (uint64_t)(uintptr_t)tail, (uint64_t)joined_row_stride,
                                          (uint64_t)tail_row_stride, (uint64_t)row_bytes});
+    // Rows per workgroup: 16 where they are two accesses or more of every thread (rows of 512 bytes), 32 of shorter rows, and the tail divided evenly:
+    // 20 rows as 16 and 4 took longer than one workgroup with all of them (1000 sequences of 20 rows of 1 KB 8.7 us, undivided 6.6, as 10 and 10
+    // 6.1; 256 sequences of 20 rows of 32 bytes, 16 per workgroup 2.06, 32 1.96).
+    const int most = row_bytes / vec >= 32 ? 16 : 32;
+    const int64_t blocks = ((int64_t)tail_len + most - 1) / most;
+    const int rows = (int)((tail_len + blocks - 1) / blocks);
+    const dim3 grid((unsigned)blocks, (unsigned)batch);
 #define HSTU_TAIL_KERNEL(V, INDEX)                                                                                            \
-    hipLaunchKernelGGL((hstu::hstu_jagged_write_tail_kernel<V, kTailRows, INDEX>), grid, dim3(256), 0, stream, (char*)joined,   \
-                       joined_row_stride, offsets, offsets_i64, (const char*)tail, tail_row_stride, row_bytes, tail_len)
+    hipLaunchKernelGGL((hstu::hstu_jagged_write_tail_kernel<V, INDEX>), grid, dim3(256), 0, stream, (char*)joined,   \
+                       joined_row_stride, offsets, offsets_i64, rows, (const char*)tail, tail_row_stride, row_bytes, tail_len)
 #define HSTU_TAIL_LAUNCH(V)                                           \
     do {                                                              \
         if (row_bytes / V > kShortRow) HSTU_TAIL_KERNEL(V, uint64_t); \

@@ -228,6 +228,32 @@ def test_write_kv_tail_blocks(pkg, dev, batch, tail, columns, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "tail,columns",
+    # tails that divide into equal blocks of 16 rows at most, into unequal ones, and of 32 rows (shorter rows); last rounds of one, two, three
+    # and four accesses of a thread, complete and not; widths of every access size
+    [(20, 512), (49, 512), (33, 512), (33, 248), (65, 128), (31, 64), (20, 8), (13, 352), (16, 384), (16, 392), (9, 900), (5, 1638), (100, 2), (37, 1), (21, 36)],
+)
+def test_write_kv_tail_and_copies_divide_rows_into_rounds(pkg, dev, tail, columns):
+    print(f"[case] write_kv_tail rounds {tail} {columns}", flush=True)
+    history = [0, 40, 7, 32]
+    ends = np.cumsum([h + tail for h in history])
+    offs = torch.tensor(np.concatenate([[0], ends]), dtype=torch.int64, device=dev)
+    old = torch.tensor(np.concatenate([[0], np.cumsum(history)]), dtype=torch.int64, device=dev)
+    full = torch.arange(int(ends[-1]) * columns, device=dev).remainder(30011).view(-1, columns).to(torch.int16)
+    new = (torch.arange(len(history) * tail * columns, device=dev).remainder(29989) - 30000).view(-1, columns).to(torch.int16)
+    want = full.clone()
+    for b, end in enumerate(ends):
+        want[int(end) - tail : int(end)] = new[b * tail : (b + 1) * tail]
+    pkg.write_kv_tail(full, offs, new)
+    left, right = pkg.split_2D_jagged(max(history) + tail, full, max_len_left=max(history), max_len_right=tail, offsets_left=old,
+                                      offsets_right=offs - old)
+    joined = pkg.concat_2D_jagged(max(history) + tail, left, right, max(history), tail, old, offs - old)
+    torch.cuda.synchronize()
+    assert torch.equal(full, want) and torch.equal(right, new) and torch.equal(joined, want)
+
+
+@pytest.mark.gpu
 def test_rows_longer_than_64_megabytes_are_copied_as_wide(pkg, dev):
     """A row just above 2^26 bytes takes what one of 2^26 takes: 16 bytes per access, whatever counts them (byte by byte it was 17 times as long;
     the bound leaves a factor of 4 for the machine).  A row of more than 2^26 accesses, which are counted in 64 bits, on top."""
