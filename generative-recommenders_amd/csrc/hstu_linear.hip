@@ -291,13 +291,16 @@ bool output_takes_fused(const HstuOutputArgs* a) {
     return a->path == 2 || (a->path == 0 && a->rows >= 32768 && a->dropout_ratio == 0.f && output_fused_shape(a));
 }
 
-// path = 0: the one kernel for a few rows, where a row's chunks are one per lane and the joined rows fit the LDS.  Up to 256 rows it is latency
-// for both (50 rows 7.8 us a pass, the two kernels of the library path 10.2; 256 rows 8.1 / 11.9); beyond, its workgroups of 32 x 32 would read W
-// once per 32 rows (1.5 MB of it for 3 x 512 into 512 columns) and need more than one round on the chip.
+// path = 0: the one kernel for up to 256 rows, where a row's chunks are one per lane, the joined rows fit the LDS, and all its workgroups of 32 rows x
+// 32 columns run at once: two per CU up to a depth of 512, beyond that (their LDS) one.  That far it is latency for both (us, against the two kernels
+// of the library path: 3 x 512 into 1024 columns, 50 rows 7.9 / 11.4, 256 rows 8.5 / 13.5; into 2048, 128 rows, the last that fit, 8.4 / 13.0).  A
+// second round takes as long again, with W read and the rows joined once more: 2 x 384 into 2048, 160 rows 12.8 / 11.1; into 8192, 64 rows 13.1 / 12.6,
+// 256 rows 51 / 19; 3 x 128 into 4096, 128 rows (one round) 8.3 / 12.2, 192 rows 12.5 / 11.5; 3 x 512 into 2048, 160 .. 256 rows 14.8 .. 15.3 / 15.3 .. 15.7.
 bool output_takes_rows(const HstuOutputArgs* a) {
-    const int64_t d = (int64_t)a->heads * a->linear_dim;
+    const int64_t d = (int64_t)a->heads * a->linear_dim, k = output_blocks(a) * d;
     if (a->path != 0 || a->rows > 256 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1)) return false;
-    if (a->d_out % 32 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512 || output_blocks(a) * d > hstu::kOutRowsMostK) return false;
+    if (a->d_out % 32 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512 || k > hstu::kOutRowsMostK) return false;
+    if ((a->rows + 31) / 32 * (a->d_out / 32) > (2 * hstu::out_rows_lds((int)k) <= 160 * 1024 ? 512 : 256)) return false;
     if (!a->group_norm) return true;
     const int lanes = a->linear_dim / 8;
     return a->linear_dim % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0;

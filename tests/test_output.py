@@ -271,6 +271,39 @@ def test_compute_output_of_a_few_rows(pkg, dev, N, H, ld, D, cu, cx, act, group_
     _close(got, lib.float().cpu(), "few rows vs library path")
 
 
+# (rows, blocks, heads, linear_dim, d_out) on both sides of the line: one round of workgroups of 32 rows x 32 columns, two per CU up to a depth of 512,
+# 256 rows, a depth of 1536
+ONE_ROUND = [(256, 3, 4, 128, 1024), (128, 3, 4, 128, 2048), (32, 3, 4, 128, 8192), (64, 2, 4, 128, 4096), (128, 1, 4, 128, 4096), (64, 1, 2, 64, 8192)]
+TWO_ROUNDS = [(256, 3, 4, 128, 1056), (129, 3, 4, 128, 2048), (33, 3, 4, 128, 8192), (65, 2, 4, 128, 4096), (129, 1, 4, 128, 4096), (65, 1, 2, 64, 8192),
+              (257, 1, 2, 64, 256)]
+
+
+@pytest.mark.parametrize("rows,blocks,H,ld,D", ONE_ROUND + TWO_ROUNDS)
+def test_output_of_a_few_rows_is_one_kernel_for_one_round_of_workgroups(rows, blocks, H, ld, D):
+    """The one kernel needs no workspace, the two of the library path do.  (By its rows alone the choice went to the one kernel in up to eight rounds: 256
+    rows of 2 x 384 into 8192 columns 51 us instead of 19.)  Needs no GPU."""
+    import ctypes
+
+    import __graft_entry__
+
+    __graft_entry__.load_package()
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    a = hc.HstuOutputArgs(rows=rows, d_out=D, heads=H, linear_dim=ld, concat_u=blocks > 1, concat_x=blocks > 2)
+    assert (hc.lib().hstu_output_workspace_bytes(ctypes.byref(a)) == 0) == ((rows, blocks, H, ld, D) in ONE_ROUND)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,blocks,H,ld,D", [c for c in ONE_ROUND + TWO_ROUNDS if c[4] in (1056, 2048, 8192)])
+def test_compute_output_on_both_sides_of_one_round(pkg, dev, N, blocks, H, ld, D):
+    print(f"[case] output of wide rows {N} {blocks} {H} {ld} {D}", flush=True)
+    cu, cx = blocks > 1, blocks > 2
+    attn, u, x, nw, nb, w = _inputs(N + D, N, H, ld, D, blocks, False, torch.bfloat16)
+    got = pkg.hstu_compute_output(*(t.to(dev) for t in (attn, u, x, nw, nb)), 1e-6, w.to(dev), H, ld, 0.0, False, cu, cx, "none", False, False)
+    torch.cuda.synchronize()
+    _close(got, O.compute_output(attn, u, x, nw, nb, w, 1e-6, concat_u=cu, concat_x=cx, num_heads=H, linear_dim=ld), "wide rows vs fp32 oracle")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N", [33000, 257])
 def test_compute_output_concat_gemm_on_views_of_wider_buffers(pkg, dev, N):
