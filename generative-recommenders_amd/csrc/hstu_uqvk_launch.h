@@ -59,15 +59,48 @@ int launch_rows(hstu::UqvkFusedParams p, int units_per_wave, hipStream_t stream)
                   dim3((unsigned)blocks, splits), p, stream);
 }
 
-constexpr long long kProductWide = 1024;  // units from which the product with a transposed matrix is kWide's
-
-enum class Kernel { kRows32, kRows64, kFused, kWide };
+enum class Kernel { kRows32, kRows64, kFused, kWide, kLibrary };
 struct Choice {
     Kernel kernel;
     int units_per_wave;
 };
 
-// The kernel of a call.  All sizes in us, this rule's choice against the kernel on the other side of the line.
+// The kernel of the product with a transposed matrix, or the library GEMM.  No norm to repeat, but only the products to gain from.  us, these kernels' / the
+// library's, whose time jumps by half between neighbouring sizes (depth 512 into 1024 columns: 10000 rows 17.6, 12000 33.3), so that no line suits all.
+//   * kRows32 while all column units can be waves of their own in one round, two workgroups per CU: depth 512, 1000 rows into 1536 columns 6.4 / 8.4,
+//     8000 into 256 6.8 / 9.4.
+//   * kWide at depth 256 from 6 units (row blocks of 256 x column blocks of 64) per CU on: 17000 rows into 2048 columns 27.6 / 50, kRows64 34.8; 8000 into
+//     6144 29.1 / 40, 46.8.  At depth 384 and 512 from more than 4 (depth 512, 17000 rows into 1024 34.5 / 42.1, 54000 into 1536 94 / 134; at 4 units 32768
+//     into 512 26.2 / 22.8), but for what kRows64 does in one round with up to 6 units per wave (12000 rows into 1536 32.0, kWide 34.6, the library 46).
+//   * At depth 384 and 512, W above the 4 MB of an XCD's L2: kRows32 with one workgroup per CU, kWide from 2.75 units on, the library between them
+//     (depth 512 into 6144 columns, 100 rows 4.8 / 7.2, 200 rows 10.0 / 8.2, 1000 rows 20.0 / 14.6, 2000 rows 21.0 / 28.4, 4000 rows 29.9 / 41).
+//   * Otherwise there into fewer than 1024 columns the library (5000 rows into 768 10.1 / 9.7), from there kRows64: with one unit per wave (1000 rows into
+//     3072 9.4 / 12.0), with several where they give seven tenths of the CUs a workgroup (2000 rows into 3072 13.8 / 14.2, 12000 into 1024 23.2 / 33.3;
+//     fewer: 3000 rows into 1536 13.2 / 11.9, 5000 into 2048 23.6 / 17.3).
+//   * Up to depth 256 kRows64, in one round with as many units per wave as that takes (54000 rows of depth 256 into 768 columns 30 / 50, 12000 of depth 128
+//     into 1536 13.5 / 26), and in several but for 256 columns of depth 256 in the second (54000 rows 17.3 / 15.2, 100000 29.5 / 34.9).
+Choice choose_product(int64_t rows, int n, int kt) {
+    const long long wide_units = (rows + 255) / 256 * (n / 64), blocks32 = (rows + 31) / 32, blocks64 = (rows + 63) / 64;
+    const int quarter32 = n / 128, quarter = kt <= 4 ? quarter32 : (quarter32 + 1) / 2;
+    const bool large = kt > 4 && (long long)n * kt * 128 > (4 << 20);
+    const bool wide = kt >= 4 && n >= 512 && wide_units >= (kt == 4 ? 1536 : large ? 704 : 1025) && wide_units <= 0x7fffffffLL;
+    if (blocks32 * quarter32 <= (large ? 256 : 512)) return {Kernel::kRows32, 1};
+    if (kt > 4 && (large || n < 1024)) return {wide ? Kernel::kWide : Kernel::kLibrary, 0};
+    if (kt == 4 && wide) return {Kernel::kWide, 0};
+    const int round = kt <= 4 ? 512 : 256;
+    for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2) {
+        const long long workgroups = blocks64 * ((quarter + per - 1) / per);
+        if (workgroups > round) continue;
+        if (wide && per == 8 && quarter > 6) break;
+        if (kt > 4 && per > 1 && workgroups * 10 < round * 7) return {Kernel::kLibrary, 0};
+        return {Kernel::kRows64, per};
+    }
+    if (wide) return {Kernel::kWide, 0};
+    if (kt == 4 && n == 256 && blocks64 <= 1024) return {Kernel::kLibrary, 0};
+    return {Kernel::kRows64, hstu::kUqvkMostUnits};
+}
+
+// The kernel of a call of the other products.  All sizes in us, this rule's choice against the kernel on the other side of the line.
 //   * kWide where its work, row blocks of 256 x column blocks of 64, gives each CU 16 units or more; below that the rows' preparation, 256
 //     at a time on one CU, outweighs the faster matrix phase.  Against kFused, d_model 512 into 2048 columns: 26000 rows 91 / 87, 32768
 //     85 / 100, 139264 329 / 408; into 4096: 12000 rows 87 / 83, 16384 88 / 98.  Against kRows64, d_model 256 into 2048: 24000 rows 52 / 48,
@@ -80,15 +113,12 @@ struct Choice {
 //     384 and 512 (into 512 columns, 24000 rows 35.1 / 33.4, 90000 rows 109 / 88; into 4096, 12000 rows 92 / 81) and kRows64's below
 //     (d_model 256 into 512 columns, 45000 rows 29.3 / 38.3).
 //   * the gradient of u: kRows32 and kRows64 by the same lines, kRows64 with as many units per wave as there are beyond them.
-//   * the product with a transposed matrix: no norm to repeat, so kWide from 4 units per CU on (depth 512 into 1536 columns, 17000 rows 42,
-//     kRows64 62; 54000 rows 94 / 134, 139264 rows 216 / 306).
 Choice choose(const hstu::UqvkFusedParams& p, int kt, int mode) {
-    const bool forward = mode == hstu::kUqvkForward || mode == hstu::kUqvkForward8;
+    if (mode == hstu::kProductT) return choose_product(p.rows, p.n_out, kt);
+    const bool forward = mode != hstu::kUqvkGradU;
     const long long wide_units = (p.rows + 255) / 256 * (p.n_out / 64);
     const bool whole64 = !forward || p.n_silu % 64 == 0;  // (SiLU per 64 columns)
-    const bool wide = mode != hstu::kUqvkGradU && kt >= 4 && p.n_out >= 512 && whole64 && wide_units >= (forward ? 4096 : kProductWide) &&
-                      wide_units <= 0x7fffffffLL;
-    if (forward && wide) return {Kernel::kWide, 0};
+    if (forward && kt >= 4 && p.n_out >= 512 && whole64 && wide_units >= 4096 && wide_units <= 0x7fffffffLL) return {Kernel::kWide, 0};
     const int quarter32 = p.n_out / 128;  // column units of a wave that walks a quarter of the columns
     const long long blocks32 = (p.rows + 31) / 32, blocks64 = (p.rows + 63) / 64;
     if (blocks32 * quarter32 <= 512) return {Kernel::kRows32, 1};
@@ -97,7 +127,6 @@ Choice choose(const hstu::UqvkFusedParams& p, int kt, int mode) {
     if (kt <= 4 || whole64) {
         for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2)
             if (blocks64 * ((quarter + per - 1) / per) <= round) return {Kernel::kRows64, per};
-        if (wide) return {Kernel::kWide, 0};
         if (kt <= 4 || !forward) return {Kernel::kRows64, hstu::kUqvkMostUnits};
     }
     return {Kernel::kFused, 0};

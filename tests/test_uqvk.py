@@ -323,6 +323,41 @@ def test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound):
     assert bool((out[:, n:] == 7.0).all())
 
 
+@pytest.mark.parametrize(
+    "rows,k,n,library",
+    # on both sides of the lines: units of their own for one round, and for W above 4 MB half of one; 64 rows with several units per wave, for seven tenths of
+    # the CUs and fewer; fewer columns; 64 rows per wave above 4 units per CU, and from 2.75 for W above 4 MB; 256 columns in the second round
+    [(1000, 512, 1536, False), (64, 512, 6144, False), (200, 512, 6144, True), (1000, 512, 6144, True), (2000, 512, 6144, False), (3000, 512, 1536, True),
+     (3000, 384, 1536, True), (5000, 512, 2048, True), (10000, 384, 1024, True), (4000, 512, 1536, False), (12000, 512, 1024, False), (17000, 384, 1024, False),
+     (32768, 512, 512, True), (32769, 512, 512, False), (10000, 512, 1536, True),
+     (24000, 512, 768, False), (54000, 256, 256, True), (32768, 256, 256, False), (100000, 256, 256, False), (54000, 128, 256, False)],
+)
+def test_which_products_with_a_transposed_weight_are_the_library_s(rows, k, n, library):
+    """Only the library's need a workspace.  (Into 1024 columns and more all of them were the kernels', up to 1.6 times as long on the GPU; the sizes
+    here were measured on both sides.)  Needs no GPU."""
+    import ctypes
+
+    import __graft_entry__
+
+    __graft_entry__.load_package()
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    hc.lib().hstu_linear_product_t_workspace_bytes.restype = ctypes.c_size_t
+    assert (hc.lib().hstu_linear_product_t_workspace_bytes(ctypes.c_int64(rows), ctypes.c_int32(k), ctypes.c_int32(n)) > 0) == library
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 3e-3), (torch.float16, 4e-4)])  # as above
+@pytest.mark.parametrize(
+    "rows,k,n",
+    # 64 rows per wave at depth 256 and with W above 4 MB, shares that differ; two, four and more units per wave of 64 rows; the library between them
+    [(33001, 256, 768), (2001, 512, 6144), (2817, 384, 6144), (4001, 512, 1536), (12001, 512, 1024), (17001, 384, 1024), (12001, 512, 1536), (10001, 512, 2048), (201, 512, 6144), (3001, 512, 1536),
+     (40001, 256, 256)],
+)
+def test_product_with_a_transposed_weight_in_the_middle(pkg, dev, rows, k, n, dtype, bound):
+    test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])  # the rounded norm, sums and result: 2.0e-3, 2.6e-4
 @pytest.mark.parametrize("rows,k,n", [(1, 512, 128), (33, 128, 384), (65, 256, 128), (4097, 512, 512), (2049, 384, 640), (20001, 512, 256), (40001, 256, 256)])
