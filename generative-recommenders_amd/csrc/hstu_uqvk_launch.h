@@ -100,7 +100,34 @@ Choice choose_product(int64_t rows, int n, int kt) {
     return {Kernel::kRows64, hstu::kUqvkMostUnits};
 }
 
-// The kernel of a call of the other products.  All sizes in us, this rule's choice against the kernel on the other side of the line.
+// The kernel of the gradient of u.  us, against what stood here before, layer norm + library GEMM + hstu_uqvk_silu_bwd.
+//   * kRows32 and kRows64 in one round as for the producer (choose), and up to depth 256 in more rounds too (depth 256, 90000 rows into 512 columns 83 / 126).
+//   * Several rounds at depth 384 and 512: kRows32, each workgroup all columns, two per CU, up to 384 columns (depth 384 into 128, 60000 rows 41.8 / 44.3, kRows64
+//     58.9: half its waves have no unit; depth 512 into 384, 20000 rows 32.1 / 36.0, kRows64 42.7), and into more while it has few rounds: depth 512 into 512,
+//     60000 rows 80.8 / 96.5, kRows64 87.3; 90000 rows 147.8, kRows64 140.5; depth 384 into 1024, 20000 rows 54.6 / 59.0, kRows64 65.9.
+//   * Beyond, kRows64 with the columns divided so that rounds x (the rows' preparation, about two units' time, + units) is smallest: depth 384 into 2048,
+//     24000 rows 4 units per wave 114, 8 125 / 129; 60000 rows 8 units 252, 4 280 / 312.  Just past one round it stays up to 8 % behind (depth 384 into 768,
+//     16500 rows 46.5 / 43.1).
+Choice choose_grad_u(int64_t rows, int n, int kt) {
+    const int quarter32 = n / 128, quarter = kt <= 4 ? quarter32 : (quarter32 + 1) / 2, round = kt <= 4 ? 512 : 256;
+    const long long blocks32 = (rows + 31) / 32, blocks64 = (rows + 63) / 64;
+    if (blocks32 * quarter32 <= 512) return {Kernel::kRows32, 1};
+    if (n <= 256 && kt > 4 && blocks32 <= 1024) return {Kernel::kRows32, quarter32};
+    for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2)
+        if (blocks64 * ((quarter + per - 1) / per) <= round) return {Kernel::kRows64, per};
+    if (kt <= 4) return {Kernel::kRows64, hstu::kUqvkMostUnits};
+    if (n <= 384 || (n <= 1024 && blocks32 * quarter32 <= 9216)) return {Kernel::kRows32, quarter32};
+    Choice best{Kernel::kRows64, 1};
+    double least = 1e300;
+    for (int per = 1; per <= hstu::kUqvkMostUnits; per *= 2) {
+        const int splits = (quarter + per - 1) / per;
+        const double cost = (double)((blocks64 * splits + 255) / 256) * (2 + (double)quarter / splits);
+        if (cost < least) least = cost, best.units_per_wave = per;
+    }
+    return best;
+}
+
+// The kernel of a call of the producer.  All sizes in us, this rule's choice against the kernel on the other side of the line.
 //   * kWide where its work, row blocks of 256 x column blocks of 64, gives each CU 16 units or more; below that the rows' preparation, 256
 //     at a time on one CU, outweighs the faster matrix phase.  Against kFused, d_model 512 into 2048 columns: 26000 rows 91 / 87, 32768
 //     85 / 100, 139264 329 / 408; into 4096: 12000 rows 87 / 83, 16384 88 / 98.  Against kRows64, d_model 256 into 2048: 24000 rows 52 / 48,
@@ -112,13 +139,12 @@ Choice choose_product(int64_t rows, int n, int kt) {
 //     4000 rows with 2 units per wave 21.3, with 1 29.0, with 4 27.5.  More rounds, and more than 8 units per wave, are kFused's at d_model
 //     384 and 512 (into 512 columns, 24000 rows 35.1 / 33.4, 90000 rows 109 / 88; into 4096, 12000 rows 92 / 81) and kRows64's below
 //     (d_model 256 into 512 columns, 45000 rows 29.3 / 38.3).
-//   * the gradient of u: kRows32 and kRows64 by the same lines, kRows64 with as many units per wave as there are beyond them.
 Choice choose(const hstu::UqvkFusedParams& p, int kt, int mode) {
     if (mode == hstu::kProductT) return choose_product(p.rows, p.n_out, kt);
-    const bool forward = mode != hstu::kUqvkGradU;
+    if (mode == hstu::kUqvkGradU) return choose_grad_u(p.rows, p.n_out, kt);
     const long long wide_units = (p.rows + 255) / 256 * (p.n_out / 64);
-    const bool whole64 = !forward || p.n_silu % 64 == 0;  // (SiLU per 64 columns)
-    if (forward && kt >= 4 && p.n_out >= 512 && whole64 && wide_units >= 4096 && wide_units <= 0x7fffffffLL) return {Kernel::kWide, 0};
+    const bool whole64 = p.n_silu % 64 == 0;  // (SiLU per 64 columns)
+    if (kt >= 4 && p.n_out >= 512 && whole64 && wide_units >= 4096 && wide_units <= 0x7fffffffLL) return {Kernel::kWide, 0};
     const int quarter32 = p.n_out / 128;  // column units of a wave that walks a quarter of the columns
     const long long blocks32 = (p.rows + 31) / 32, blocks64 = (p.rows + 63) / 64;
     if (blocks32 * quarter32 <= 512) return {Kernel::kRows32, 1};
@@ -127,7 +153,7 @@ Choice choose(const hstu::UqvkFusedParams& p, int kt, int mode) {
     if (kt <= 4 || whole64) {
         for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2)
             if (blocks64 * ((quarter + per - 1) / per) <= round) return {Kernel::kRows64, per};
-        if (kt <= 4 || !forward) return {Kernel::kRows64, hstu::kUqvkMostUnits};
+        if (kt <= 4) return {Kernel::kRows64, hstu::kUqvkMostUnits};
     }
     return {Kernel::kFused, 0};
 }

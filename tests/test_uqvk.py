@@ -358,6 +358,72 @@ def test_product_with_a_transposed_weight_in_the_middle(pkg, dev, rows, k, n, dt
     test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound)
 
 
+_CHOICE_HARNESS = """
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+namespace hstu {
+constexpr int kUqvkMostUnits = 16;
+enum { kUqvkForward, kUqvkForward8, kUqvkGradU, kProductT };
+struct UqvkFusedParams { int64_t rows; int n_out, n_silu; };
+}
+%s
+int main(int, char** a) {
+    const hstu::UqvkFusedParams p{atoll(a[2]), atoi(a[4]), atoi(a[4]) / 4};
+    const Choice c = choose(p, atoi(a[3]) / 64, atoi(a[1]));
+    const char* const names[] = {"rows32", "rows64", "fused", "wide", "library"};
+    printf("%%s %%d", names[(int)c.kernel], c.units_per_wave);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def choice(tmp_path_factory):
+    """The rule of csrc/hstu_uqvk_launch.h, compiled for the host: (mode, rows, depth, columns) -> kernel and units per wave."""
+    import shutil
+    import subprocess
+
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("no g++")
+    text = open(os.path.join(ROOT, "generative-recommenders_amd", "csrc", "hstu_uqvk_launch.h")).read()
+    rule = text[text.index("enum class Kernel") : text.index("template <class TT, int KT, int MODE>\nint launch_depth")]
+    src = tmp_path_factory.mktemp("choice") / "choice.cpp"
+    src.write_text(_CHOICE_HARNESS % rule)
+    exe = src.with_suffix("")
+    subprocess.run([gxx, "-O1", "-std=c++17", str(src), "-o", str(exe)], check=True)
+
+    def ask(mode, rows, depth, n):
+        name, units = subprocess.run([str(exe), str(mode), str(rows), str(depth), str(n)], check=True, capture_output=True, text=True).stdout.split()
+        return name, int(units)
+
+    return ask
+
+
+@pytest.mark.parametrize(
+    "rows,k,n,kernel,units",
+    # one round; several: few columns, more while the rounds are few, and beyond them the division that costs least; depths up to 256.  (With 64 rows
+    # and all columns per workgroup the second to the sixth took up to a third longer than layer norm, library GEMM and SiLU's derivative.)
+    [(16000, 512, 512, "rows64", 2), (60000, 384, 128, "rows32", 1), (45000, 512, 256, "rows32", 2), (200000, 384, 384, "rows32", 3), (60000, 512, 512, "rows32", 4),
+     (20000, 384, 1024, "rows32", 8), (90000, 512, 512, "rows64", 2), (24000, 384, 2048, "rows64", 4), (60000, 384, 2048, "rows64", 8),
+     (24000, 384, 4096, "rows64", 8), (90000, 256, 512, "rows64", 16), (200, 256, 4096, "rows32", 1)],
+)
+def test_which_kernel_takes_the_gradient_of_u(choice, rows, k, n, kernel, units):
+    assert choice(2, rows, k, n) == (kernel, units)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])  # as below
+@pytest.mark.parametrize(
+    "rows,k,n",
+    # several rounds at depth 384 and 512: 32 rows and one, three, four, eight units per wave; 64 rows with two, four and eight, columns divided
+    # over workgroups and not, a last unit that half of the waves have; all with remainders of the rows
+    [(33001, 384, 128), (20001, 512, 384), (57819, 512, 512), (20033, 384, 1024), (90001, 512, 512), (24001, 384, 2048), (17001, 512, 1408), (36001, 512, 3072)],
+)
+def test_gradient_of_u_in_several_rounds(pkg, dev, rows, k, n, dtype, bound):
+    test_gradient_of_u_in_front_of_silu(pkg, dev, rows, k, n, dtype, bound)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])  # the rounded norm, sums and result: 2.0e-3, 2.6e-4
 @pytest.mark.parametrize("rows,k,n", [(1, 512, 128), (33, 128, 384), (65, 256, 128), (4097, 512, 512), (2049, 384, 640), (20001, 512, 256), (40001, 256, 256)])
