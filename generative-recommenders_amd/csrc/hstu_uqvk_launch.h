@@ -134,11 +134,14 @@ Choice choose_grad_u(int64_t rows, int n, int kt) {
 //     45000 77 / 88; into 512: 90000 rows 61 / 52.  Columns: into 256 it is slower at every size (300000 rows of d_model 512: 197 / 177).
 //   * kRows32 while all column units can be waves of their own in one round of workgroups, two per CU: d_model 512 into 2048 columns, 1000
 //     rows 10.3, kRows64 12.4; 2000 rows (two rounds) 18.5 / 13.8.  Few columns, up to 256: up to two rounds of workgroups that hold all of
-//     them: d_model 512 into 128 columns, 24000 rows 14.5, kRows64 23.0, kFused 17.8; 90000 rows 45.5 / 72.1 / 41.1.
+//     them: d_model 512 into 128 columns, 24000 rows 14.5, kRows64 23.0, kFused 17.8; 90000 rows 45.5 / 72.1 / 41.1.  d_model 384: only where
+//     they are no slower than kFused there (into 128 columns, 24000 rows 13.6 / 13.5, 30000 15.6 / 14.1; into 256, 30000 22.9 / 22.8, 30700 23.1 / 21.6).
 //   * kRows64, dividing the columns over as many workgroups as one round holds (one per CU, two up to d_model 256): d_model 512 into 2048,
 //     4000 rows with 2 units per wave 21.3, with 1 29.0, with 4 27.5.  More rounds, and more than 8 units per wave, are kFused's at d_model
-//     384 and 512 (into 512 columns, 24000 rows 35.1 / 33.4, 90000 rows 109 / 88; into 4096, 12000 rows 92 / 81) and kRows64's below
-//     (d_model 256 into 512 columns, 45000 rows 29.3 / 38.3).
+//     384 and 512 (into 512 columns, 24000 rows 35.1 / 33.4, 90000 rows 109 / 88; into 4096, 12000 rows 92 / 81), more than 4 at d_model 384 (into
+//     2048, 8200 rows 40.7 / 34.1), 8 for fewer than 176 workgroups (d_model 512 into 4096, 5100 rows 44.8 / 41.1, 6000 45.4 / 48.2), and, where W exceeds an
+//     XCD's 4 MB of L2, more than 4 (d_model 512 into 6144, 5400 rows 67 / 60) or than 160 workgroups that each read it (into 8192, 2000 rows 49.0 / 35.7;
+//     into 5120, 2000 rows 31.3 / 32.7), and kRows64's below (d_model 256 into 512 columns, 45000 rows 29.3 / 38.3).
 Choice choose(const hstu::UqvkFusedParams& p, int kt, int mode) {
     if (mode == hstu::kProductT) return choose_product(p.rows, p.n_out, kt);
     if (mode == hstu::kUqvkGradU) return choose_grad_u(p.rows, p.n_out, kt);
@@ -148,11 +151,16 @@ Choice choose(const hstu::UqvkFusedParams& p, int kt, int mode) {
     const int quarter32 = p.n_out / 128;  // column units of a wave that walks a quarter of the columns
     const long long blocks32 = (p.rows + 31) / 32, blocks64 = (p.rows + 63) / 64;
     if (blocks32 * quarter32 <= 512) return {Kernel::kRows32, 1};
-    if (p.n_out <= 256 && kt > 4 && blocks32 <= 1024) return {Kernel::kRows32, quarter32};
+    if (p.n_out <= 256 && kt > 4 && blocks32 <= (kt == 8 ? 1024 : p.n_out == 128 ? 512 : 940)) return {Kernel::kRows32, quarter32};
     const int quarter = kt <= 4 ? quarter32 : (quarter32 + 1) / 2, round = kt <= 4 ? 512 : 256;
     if (kt <= 4 || whole64) {
-        for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2)
-            if (blocks64 * ((quarter + per - 1) / per) <= round) return {Kernel::kRows64, per};
+        const bool large = kt > 4 && (long long)p.n_out * kt * 128 > (4 << 20);
+        for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : kt == 8 && !large ? 8 : 4); per *= 2) {
+            const long long workgroups = blocks64 * ((quarter + per - 1) / per);
+            if (workgroups > round) continue;
+            if (kt > 4 && (large ? workgroups > 160 : per == 8 && workgroups < 176)) break;
+            return {Kernel::kRows64, per};
+        }
         if (kt <= 4) return {Kernel::kRows64, hstu::kUqvkMostUnits};
     }
     return {Kernel::kFused, 0};

@@ -412,6 +412,18 @@ def test_which_kernel_takes_the_gradient_of_u(choice, rows, k, n, kernel, units)
     assert choice(2, rows, k, n) == (kernel, units)
 
 
+@pytest.mark.parametrize(
+    "rows,k,n,kernel,units",
+    # both sides of the producer's lines: d_model 384 with few columns; 8 units per wave; W above 4 MB (on the other side of these the call took up to a third
+    # longer than with 128 rows per workgroup); 64 rows per wave
+    [(16384, 384, 128, "rows32", 1), (30000, 384, 128, "fused", 0), (30000, 384, 256, "rows32", 2), (30700, 384, 256, "fused", 0), (32768, 512, 128, "rows32", 1),
+     (8192, 384, 2048, "rows64", 4), (8200, 384, 2048, "fused", 0), (8200, 512, 2048, "fused", 0), (12000, 512, 2048, "rows64", 8), (5100, 512, 4096, "fused", 0), (6000, 512, 4096, "rows64", 8),
+     (2800, 512, 6144, "fused", 0), (1400, 512, 6144, "rows64", 4), (2000, 512, 5120, "rows64", 4), (2000, 512, 8192, "fused", 0), (500, 384, 8192, "fused", 0), (16384, 512, 4096, "wide", 0), (262144, 256, 512, "wide", 0), (262144, 256, 256, "rows64", 16), (300000, 128, 2048, "rows64", 16)],
+)
+def test_which_kernel_takes_the_producer(choice, rows, k, n, kernel, units):
+    assert choice(0, rows, k, n) == choice(1, rows, k, n) == (kernel, units)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,bound", [(torch.bfloat16, 4e-3), (torch.float16, 5e-4)])  # as below
 @pytest.mark.parametrize(
