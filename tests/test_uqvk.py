@@ -229,10 +229,11 @@ def test_uqvk_columns_divided_over_workgroups_give_the_same_bits(pkg, dev):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize(
     "L,d_model,H,attn,hidden",
-    # at least 16 row blocks of 256 x column blocks of 64 per CU (8 at d_model 256), with remainders 0, 1 and 255 of the rows; units that
-    # the 256 workgroups share evenly and not; the u columns a whole and an odd number of blocks; the fewest columns
+    # at least 16 row blocks of 256 x column blocks of 64 per CU (the two of d_model 256 with 2064 and 2056 units: several rounds of 64 rows per
+    # workgroup), with remainders 0, 1 and 255 of the rows; units that the 256 workgroups share evenly and not; the u columns a whole and an odd
+    # number of blocks; the fewest columns
     [(32768, 512, 4, 128, 128), (65537, 512, 2, 128, 128), (44031, 384, 3, 128, 128), (32769, 256, 4, 64, 64), (65791, 256, 2, 64, 64),
-     (131073, 512, 2, 64, 64), (52000, 384, 1, 512, 320)],
+     (131073, 512, 2, 64, 64), (52000, 384, 1, 512, 320), (65793, 256, 4, 64, 64), (131329, 256, 2, 64, 64), (66303, 256, 1, 320, 192)],
 )
 def test_uqvk_with_64_rows_per_wave_gives_the_bits_of_32(pkg, dev, L, d_model, H, attn, hidden, dtype):
     """The sums run in the same order, so every row is bit for bit what the kernel for few rows gives for it (which the tests
@@ -257,6 +258,7 @@ def test_uqvk_with_64_rows_per_wave_gives_the_bits_of_32(pkg, dev, L, d_model, H
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize(
     "d_model,H,attn,hidden,whole,parts",
     # several rounds of 128 rows per workgroup (d_model 384, 512) or of 64 (below), against: units of their own for 32 rows, up to the last
@@ -266,11 +268,11 @@ def test_uqvk_with_64_rows_per_wave_gives_the_bits_of_32(pkg, dev, L, d_model, H
      (384, 3, 96, 32, 24000, (1, 95, 5000, 16001)), (512, 1, 32, 32, 40001, (31, 16384, 32768)), (512, 1, 64, 64, 40000, (1, 8192, 8193, 32700)),
      (256, 4, 64, 64, 30001, (1, 2048, 2049, 4097, 8193, 16385)), (128, 3, 32, 96, 30000, (33, 5461, 5462, 20000))],
 )
-def test_uqvk_kernels_for_few_rows_give_the_same_bits(pkg, dev, d_model, H, attn, hidden, whole, parts):
+def test_uqvk_kernels_for_few_rows_give_the_same_bits(pkg, dev, d_model, H, attn, hidden, whole, parts, dtype):
     """All the fused kernels sum in the same order: a row's bits are the same in every batch.  The rows are compared from both ends of
     the large batch, whose last rows are held against the oracle."""
-    print(f"[case] uqvk few rows {d_model} {H} {attn} {hidden} {whole} {parts}", flush=True)
-    host = _inputs(whole, whole, d_model, H, attn, hidden, torch.bfloat16)
+    print(f"[case] uqvk few rows {d_model} {H} {attn} {hidden} {whole} {parts} {dtype}", flush=True)
+    host = _inputs(whole, whole, d_model, H, attn, hidden, dtype)
     x, nw, nb, w, b = [t.to(dev) for t in host]
     fp8 = hidden * H % 128 == 0
     ref = pkg.hstu_compute_uqvk(x, nw, nb, 1e-6, H, attn, hidden, w, b, path=2)
