@@ -151,6 +151,10 @@ def lib() -> ctypes.CDLL:
         L.hstu_hip_check_contract.argtypes = [ctypes.POINTER(HstuFwdArgs), ctypes.c_void_p, ctypes.c_void_p]
         L.hstu_hip_mha_bwd.restype = ctypes.c_int
         L.hstu_hip_mha_bwd.argtypes = [ctypes.POINTER(HstuFwdArgs), ctypes.POINTER(HstuBwdGrads), ctypes.c_void_p]
+        L.hstu_hip_mha_bwd_f32.restype = ctypes.c_int
+        L.hstu_hip_mha_bwd_f32.argtypes = [ctypes.POINTER(HstuFwdArgs), ctypes.POINTER(HstuBwdGrads), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+        L.hstu_hip_mha_bwd_f32_copies_bytes.restype = ctypes.c_size_t
+        L.hstu_hip_mha_bwd_f32_copies_bytes.argtypes = [ctypes.POINTER(HstuFwdArgs)]
         L.hstu_hip_mha_bwd_workspace_bytes.restype = ctypes.c_size_t
         L.hstu_hip_mha_bwd_workspace_bytes.argtypes = [ctypes.POINTER(HstuFwdArgs)]
         L.hstu_hip_plan.restype = ctypes.c_int
@@ -379,7 +383,8 @@ def mha_bwd(
     workspace: Optional[torch.Tensor] = None,
 ) -> None:
     """Fill ``dq``, ``dk``, ``dv`` on the current stream of ``q.device`` (full attention only).  ``sort_by_length``
-    starts the long sequences first; it never changes the result.
+    starts the long sequences first; it never changes the result.  All tensors are bf16, fp16 or fp32; of fp32 the operands
+    are rounded to bf16 by one launch and the gradients are the fp32 sums.
 
     Two forms, chosen by the caller and by nothing else (not by how much device memory happens to be free).  The
     default recomputes the scores for dq and needs no scratch beyond ``4 * batch`` bytes for the sort.  The stored
@@ -426,7 +431,11 @@ def mha_bwd(
     g.dv_row_stride, g.dv_head_stride = dv.stride(0), dv.stride(1)
     with torch.cuda.device(q.device):
         stream = torch.cuda.current_stream(q.device).cuda_stream
-        rc = lib().hstu_hip_mha_bwd(ctypes.byref(a), ctypes.byref(g), ctypes.c_void_p(stream))
+        if q.dtype == torch.float32:
+            copies = torch.empty(lib().hstu_hip_mha_bwd_f32_copies_bytes(ctypes.byref(a)), dtype=torch.uint8, device=q.device)
+            rc = lib().hstu_hip_mha_bwd_f32(ctypes.byref(a), ctypes.byref(g), copies.data_ptr(), copies.numel(), ctypes.c_void_p(stream))
+        else:
+            rc = lib().hstu_hip_mha_bwd(ctypes.byref(a), ctypes.byref(g), ctypes.c_void_p(stream))
     raise_for_status(rc)
 
 

@@ -78,12 +78,7 @@ class _HstuMhaFunction(torch.autograd.Function):
         q, k, v, seq_offsets = ctx.saved_tensors[:4]
         num_targets = ctx.saved_tensors[4] if ctx.has_targets else None
         max_seq_len, alpha, max_attn_len, contextual_seq_len, min_full_attn_seq_len = ctx.params
-        # fp32 inputs: the backward kernels take 16-bit operands, so they run on bf16 copies (fp32's range, 8 bits of
-        # mantissa; the products accumulate in fp32 as always) and the gradients are widened again -- the counterpart
-        # of the forward's fp16 copies, with the range of dout, which can be tiny, kept whole
-        wide = q.dtype == torch.float32
-        if wide:
-            q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+        q, k, v = _kernel_layout(q), _kernel_layout(k), _kernel_layout(v)  # (saved-tensor hooks give the values back in any layout)
         # the kernels write the gradient of every row of every sequence that keeps the contract; rows past max_seq_len of
         # a sequence that breaks it come back uninitialised, like the forward's (HSTU_HIP_CHECK_CONTRACT=1 raises instead)
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
@@ -98,8 +93,6 @@ class _HstuMhaFunction(torch.autograd.Function):
                 dout, q, k, v, dq, dk, dv, seq_offsets, num_targets, max_seq_len, alpha, max_attn_len, contextual_seq_len,
                 min_full_attn_seq_len, workspace=ctx.bwd_workspace,
             )
-        if wide:
-            dq, dk, dv = dq.float(), dk.float(), dv.float()
         return (dq, dk, dv) + (None,) * 12
 
 

@@ -463,6 +463,32 @@ def test_backward_of_fp32_slices(pkg, dev, dqk, dv, store):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scaled", [False, True])
+def test_backward_of_fp32_inputs_that_need_a_copy(pkg, dev, scaled):
+    """The Python operator's own route (operands that need a copy, an attn_scale): the same fp32 sums as the native front returns, bit for bit."""
+    print(f"[case] bwd fp32 through the Python operator, attn_scale {scaled}", flush=True)
+    lengths, H = [70, 0, 129, 1, 33], 2
+    q, k, v, dout, offsets = _inputs(99, lengths, H, 32, 64, torch.float32)
+    L = q.shape[0]
+    plain = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    want = torch.autograd.grad(pkg.hstu_mha(140, 0.125, *plain, offsets.to(dev), max_attn_len=20), plain, dout.to(dev))
+    if scaled:  # the plain call divides by max_seq_len: scaled by a power of two, so that the operands are the same bits again
+        scale = torch.full((L,), 2.0, device=dev)
+        out = pkg.hstu_mha(140, 0.125, *plain, offsets.to(dev), max_attn_len=20, attn_scale=scale / 140)
+        got = torch.autograd.grad(out, plain, dout.to(dev) / 2)
+    else:  # rows 4 bytes off the 16-byte boundaries
+        padded = [torch.zeros(t.numel() + 1, device=dev)[1:].view(t.shape).copy_(t).detach().requires_grad_(True) for t in plain]
+        got = torch.autograd.grad(pkg.hstu_mha(140, 0.125, *padded, offsets.to(dev), max_attn_len=20), padded, dout.to(dev))
+    torch.cuda.synchronize()
+    for name, g_, w_ in zip(("dq", "dk", "dv"), got, want):
+        assert g_.dtype == torch.float32 and not torch.equal(g_, g_.bfloat16().float()), name
+        if scaled:  # (2 / 140 * 140 is rounded: a unit in the last place of an operand)
+            assert float((g_ - w_).norm() / w_.norm()) < 2e-3, name
+        else:
+            assert torch.equal(g_, w_), name
+
+
+@pytest.mark.gpu
 def test_backward_rejections(pkg, dev):
     q, k, v, dout, offsets = _inputs(1, [40, 24], 2, 32, 32, torch.float32)
     with pytest.raises(NotImplementedError):  # fp8 inputs have no backward
