@@ -419,7 +419,7 @@ variable_list uqvk_backward(const AutogradContext* ctx, const Tensor& x, const T
     variable_list got(5);
     Tensor d_u = d.narrow(1, 0, n_u);
     Tensor normed;
-    if (du.defined() || weight_wanted) normed = at::empty({rows, dm}, x.options());
+    if (weight_wanted) normed = at::empty({rows, dm}, x.options());
     bool u_done = !du.defined(), normed_done = false;
     if (u_done) {
         d_u.zero_();
@@ -432,6 +432,7 @@ variable_list uqvk_backward(const AutogradContext* ctx, const Tensor& x, const T
         u_done = normed_done = rc == 0;
     }
     if (!normed_done && (!u_done || weight_wanted)) {
+        if (!normed.defined()) normed = at::empty({rows, dm}, x.options());
         check_linear(hstu_uqvk_layer_norm(x.const_data_ptr(), x.stride(0), norm_weight.const_data_ptr(), norm_bias.const_data_ptr(), (float)eps,
                                           normed.data_ptr(), dm, rows, (int32_t)dm, dense_dtype(x), stream));
     }
