@@ -683,7 +683,7 @@ extern "C" {
 
 const char* hstu_linear_last_error(void) { return g_last_error; }
 
-int hstu_linear_version(void) { return 101; }
+int hstu_linear_version(void) { return 102; }
 
 size_t hstu_uqvk_workspace_bytes(const HstuUqvkArgs* a) {
     if (!a || a->rows <= 0 || a->d_model <= 0) return 0;

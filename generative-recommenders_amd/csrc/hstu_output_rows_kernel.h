@@ -4,13 +4,12 @@
 // (hstu_compute_output of the reference, ops/hstu_compute.py:107-170).
 //
 // For many rows the step is the norm-multiply kernel and a GEMM of its own.  For a serving micro-batch that is two launches, a matrix
-// written and read, and a library call whose host time is more than either kernel's: 50 rows of 3 x 512 into 512 columns took 4.1 + 7.7 us on the
-// GPU and 15 us of the host.  Here a workgroup owns 32 rows x 32 columns (few enough that 50 rows are 32 workgroups, each reading 96 KB
+// written and read, and a library call whose host time is more than the kernels'.  Here a workgroup owns 32 rows x 32 columns (few enough that 50 rows are 32 workgroups, each reading 96 KB
 // of W).  Its four waves make the 32 rows of `joined` together (a row across the lanes, 8 rows per wave) and leave them in LDS,
 // rounded as the matrix would be; then each multiplies a quarter of the depth, with W's tiles in a ring of its own, so that the serial chain
 // is short and there is no barrier until the four partial sums are added, in a fixed order, with the residual.
-// 50 rows: 10.2 -> 7.8 us a pass on the GPU, 256 rows 11.9 -> 8.1, the host's call 14.5 -> less than that.  What is left is latency: the
-// launch, the rows from memory, their statistics (one row and a width of 256 take the same).
+// 3 x 512 into 512 columns, us on the GPU and of the host's call, the two kernels -> this one: 50 rows 10.4 and 13.5 -> 7.7 and 3.4, 256 rows 11.9 and
+// 13.7 -> 7.9 and 3.2.  What is left is latency: the launch, the rows from memory, their statistics (one row 7.6, 3 x 256 into 256 columns 7.0).
 #pragma once
 #include "hstu_common.h"
 #include "hstu_rows.h"

@@ -11,7 +11,7 @@
 // so that a lane ends up with one output row and, per 32-column block, four runs of four consecutive columns -- the
 // accumulator layout of the attention kernels.
 //
-// Three kernels, with the same order of all sums, so that a row's bits do not depend on which one takes it (the choice: hstu_uqvk.hip):
+// Three kernels, with the same order of all sums, so that a row's bits do not depend on which one takes it (the choice: hstu_uqvk_launch.h):
 //   * hstu_uqvk_rows_kernel, for the row counts that fill the chip once: there the time is latency, not products.  A workgroup's four
 //     waves share the normalisation of its 32 or 64 rows (a row lies across the lanes, so that loads are whole rows and a wave does a
 //     quarter of the arithmetic), hand the result over through LDS and then go their own ways: each walks column units of its own, with
@@ -21,7 +21,8 @@
 //
 // The first against the second (which had every size up to the third's), us, d_model 512 into 2048 columns: 50 rows 13.9 -> 6.5, 500 rows
 // 15.9 -> 7.7, 2000 rows 17.9 -> 13.8, 8192 rows 36.6 -> 30.4, 16000 rows 58.9 -> 51.9; d_model 256 into 1024: 1000 rows 11.1 -> 5.2,
-// 14200 rows 26.2 -> 18.1; d_model 128 into 2048: 24000 rows 49.2 -> 35.4.  What bounds it at 8192 rows of d_model 512 (256 workgroups, one
+// 14200 rows 26.2 -> 18.1; d_model 128, where it has every size, into 2048: 24000 rows 49.2 -> 35.4, 131072 rows 183 -> 138, 600000 rows 864 -> 652;
+// into 128: 131072 rows 22.8 -> 20.6, 600000 rows 85.5 -> 86.3.  What bounds it at 8192 rows of d_model 512 (256 workgroups, one
 // per CU): the matrix products take 6.8 us of the 28, the wait for the rows and their norm 6, copying W (1 MB per CU; a copy
 // instruction costs the wave some 25 cycles) 3 on top of the products, the epilogue, which nothing overlaps, 8.  A build with the epilogue under
 // the next unit's products took 34 us there: the products then share the issue with it piece by piece.
@@ -211,7 +212,7 @@ struct UqvkRows {
     static constexpr int K = KT * 64;
     static constexpr int kPerCu = KT * RB <= 8 ? 2 : 1;             // workgroups per CU: what the rows leave of the registers
     static constexpr int kTile = 32 * NB * 2;                       // a W tile: 32 k of a unit
-    static constexpr int kRing = kPerCu == 1 ? 8 : NB == 32 ? 8 : 4;  // tiles in a wave's ring
+    static constexpr int kRing = 8;                                 // tiles in a wave's ring
     static constexpr int kPanel = RB * 32 * K * 2;                  // the normalised rows
     static constexpr int kEarly = kRing - kPanel / (4 * kTile);     // ring slots beside them
     static constexpr int kStageRow = NB * 2 + 16;

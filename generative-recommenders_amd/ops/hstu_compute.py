@@ -134,8 +134,8 @@ def lib() -> ctypes.CDLL:
                                                ctypes.c_void_p, ctypes.c_void_p]
         L.hstu_linear_last_error.restype = ctypes.c_char_p
         L.hstu_linear_version.restype = ctypes.c_int
-        if L.hstu_linear_version() != 101:
-            raise RuntimeError(f"{LINEAR_LIB_PATH} is version {L.hstu_linear_version()}, this binding expects 101: rebuild it")
+        if L.hstu_linear_version() != 102:
+            raise RuntimeError(f"{LINEAR_LIB_PATH} is version {L.hstu_linear_version()}, this binding expects 102: rebuild it")
         _lib = L
     return _lib
 

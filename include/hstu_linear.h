@@ -185,19 +185,19 @@ int hstu_uqvk_layer_norm_bwd(const void* x, int64_t x_row_stride, const void* we
 int hstu_uqvk_silu_bwd(void* pre, int64_t pre_row_stride, const void* bias, const void* du, int64_t du_row_stride, int64_t rows, int64_t width,
                        int32_t dtype, void* stream);
 
-/* Gradient of a weight: out[m, n] = a^T @ b for a [rows, m] and b [rows, n] (strides in elements, rows 16-byte aligned; m and n
- * multiples of 8), fp32 sums rounded once; `b_sums`, if not NULL, gets the column sums of b [n] (the gradient of a bias).  The rows
- * are split over workgroups whose sums are added in a fixed order through `workspace` (16-byte aligned). */
-size_t hstu_linear_weight_grad_workspace_bytes(int32_t m, int32_t n, int64_t rows, int64_t a_row_stride, int64_t b_row_stride);
-int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, const void* b, int64_t b_row_stride, int32_t n, int64_t rows,
-                            int32_t dtype, void* out, void* b_sums, void* workspace, int64_t workspace_bytes, void* stream);
-
 /* The same gradient without that product in memory: out = du * (derivative of SiLU at LN(x) @ weight + bias) for a depth d_model of 128, 256,
  * 384 or 512 and a width that is a multiple of 128 (-6 otherwise).  weight [d_model, width] and the rows of x, du and out with strides in
  * elements, 16-byte aligned, below 2^22.  `normed`, if not NULL, gets LN(x) as hstu_uqvk_layer_norm writes it, [rows, d_model] dense. */
 int hstu_uqvk_u_grad(const void* x, int64_t x_row_stride, const void* norm_weight, const void* norm_bias, float eps, const void* weight,
                      int64_t weight_row_stride, const void* bias, const void* du, int64_t du_row_stride, void* out, int64_t out_row_stride,
                      void* normed, int64_t rows, int32_t d_model, int32_t width, int32_t dtype, void* stream);
+
+/* Gradient of a weight: out[m, n] = a^T @ b for a [rows, m] and b [rows, n] (strides in elements, rows 16-byte aligned; m and n
+ * multiples of 8), fp32 sums rounded once; `b_sums`, if not NULL, gets the column sums of b [n] (the gradient of a bias).  The rows
+ * are split over workgroups whose sums are added in a fixed order through `workspace` (16-byte aligned). */
+size_t hstu_linear_weight_grad_workspace_bytes(int32_t m, int32_t n, int64_t rows, int64_t a_row_stride, int64_t b_row_stride);
+int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, const void* b, int64_t b_row_stride, int32_t n, int64_t rows,
+                            int32_t dtype, void* out, void* b_sums, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* out [rows, n] = a [rows, k] @ weight [n, k]^T (strides in elements, rows 16-byte aligned, strides below 2^22; k and n multiples of 8), fp32
  * sums rounded once: d_joined = d_out @ output_weight^T and the like.  `workspace` (256-byte aligned) is for the shapes that the library's GEMM
@@ -210,7 +210,7 @@ const char* hstu_linear_last_error(void);
 
 /* Library version, major*10000 + minor*100 + patch.  101: HstuUqvkArgs gained qkv_fp8 / v_scale / q_scale / k_scale /
  * qkv_absmax and HstuOutputArgs gained dropout_ratio / dropout_seed / dropout_offset, all at the end of the structs: a
- * caller built against an older header passes shorter structs and must be rebuilt. */
+ * caller built against an older header passes shorter structs and must be rebuilt.  102: hstu_uqvk_u_grad, hstu_linear_product_t. */
 int hstu_linear_version(void);
 
 #ifdef __cplusplus
