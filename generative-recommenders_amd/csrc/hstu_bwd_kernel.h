@@ -111,7 +111,8 @@ struct KeyBlockWalk {
         end = q_hi / kQueryTile + 1;
         first = M.c > 0 ? 0 : S0 / kQueryTile;
         scan = M.w > 0 || M.c > 0 || has_targets;
-        full = full_rows(M, S0, kKeyBlock, kQueryTile);
+        full = {1, 0};  // (one or two tiles are sooner classified)
+        if (end - first > 2) full = full_rows(M, S0, kKeyBlock, kQueryTile);
     }
     __device__ __forceinline__ bool visits(const SeqMask& M, int jt, int S0, int n) const {
         if (jt < first || jt >= end) return false;
@@ -628,8 +629,9 @@ __global__ __launch_bounds__(NW * 64, 1) void hstu_bwd_dkdv_kernel(const BwdPara
 
 // ---- query-stationary kernel: dQ -----------------------------------------------------------------------------------
 
-template <class TT, int DQK, int DV, int NW, int BN>
-__global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams bp) {
+// TIGHT: four waves per SIMD for 32 and 64 columns of v and three for 128 (with 64 of q; what the LDS lets in), where the registers otherwise leave one fewer.
+template <class TT, int DQK, int DV, int NW, int BN, bool TIGHT>
+__global__ __launch_bounds__(NW * 64, TIGHT ? (DV == 128 ? 3 : 4) : 2) void hstu_bwd_dq_kernel(const BwdParams bp) {
     typedef typename TT::vec8 vec8;
     const FwdParams& p = bp.f;
     constexpr int BM = NW * 32;
@@ -654,7 +656,9 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
     const int wR1 = (wq0 + 32 < n ? wq0 + 32 : n) - 1;
 
     // key tiles and the wave's blocks of 32 keys that hold valid pairs only
-    const FullRange full_tile = full_keys(M, W.R0, W.R1, BN), full_block = full_keys(M, wR0, wR1, 32);
+    // (not for one or two tiles, which are sooner classified)
+    FullRange full_tile = {1, 0}, full_block = {1, 0};
+    if (W.jt_end - W.jt_begin > 2) full_tile = full_keys(M, W.R0, W.R1, BN), full_block = full_keys(M, wR0, wR1, 32);
     auto next_tile = [&](int t) { return t < W.jt_end && full_tile.has(t * BN) ? t : next_valid_tile<BN>(W, t); };
     int jt = next_tile(W.jt_begin);
     const int jt_end = W.jt_end;
@@ -667,27 +671,35 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
     // kernel): the rows clamped and multiplied out are some 15 vector instructions for every copy.
     const bool fast_copy = k_rsb < (1 << 24) && v_rsb < (1 << 24);
     constexpr int KINSTR = BN * (KROW / 16) / 64, VINSTR = BN * (VROW / 16) / 64, KCP = (KINSTR + NW - 1) / NW, VCP = (VINSTR + NW - 1) / NW;
-    unsigned koff[KCP], voff[VCP];
+    // TIGHT: only the first copy's, made for each tile anew (some six instructions); a wave's later copies are that one some multiple of 16 rows further
+    // on, where the swizzle is the same, so that the scalar base moves.
+    constexpr int KOFF = TIGHT ? 1 : KCP, VOFF = TIGHT ? 1 : VCP, KCR = NT / (KROW / 16), VCR = NT / (VROW / 16);
+    static_assert((KCP == 1 || KCR % 16 == 0) && (VCP == 1 || VCR % 16 == 0), "the swizzle has a period of 16 rows");
+    auto copy_offset = [&](int chunks, auto swizzle, int rsb, int i) __attribute__((always_inline)) {
+        int pos = threadIdx.x + i * NT;
+        if constexpr (TIGHT) asm volatile("" : "+v"(pos));
+        const int r = pos / chunks;
+        return (unsigned)(r * rsb + (((pos % chunks) ^ swizzle(r)) * 16));
+    };
+    unsigned koff[KOFF], voff[VOFF];
+    auto copy_offsets = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < KCP; ++i) {
-        const int pos = (wave + i * NW) * 64 + lane, row = pos / (KROW / 16);
-        koff[i] = (unsigned)(row * (int)k_rsb + (((pos % (KROW / 16)) ^ swz_u<KROW / 16>(row)) * 16));
-    }
+        for (int i = 0; i < KOFF; ++i) koff[i] = copy_offset(KROW / 16, swz_u<KROW / 16>, (int)k_rsb, i);
 #pragma unroll
-    for (int i = 0; i < VCP; ++i) {
-        const int pos = (wave + i * NW) * 64 + lane, row = pos / (VROW / 16);
-        voff[i] = (unsigned)(row * (int)v_rsb + (((pos % (VROW / 16)) ^ swz_u<VROW / 16>(row)) * 16));
-    }
+        for (int i = 0; i < VOFF; ++i) voff[i] = copy_offset(VROW / 16, swz_u<VROW / 16>, (int)v_rsb, i);
+    };
+    if constexpr (!TIGHT) copy_offsets();
     auto copy_tile = [&](int t, char* stage_lds) __attribute__((always_inline)) {
         if (fast_copy && (t + 1) * BN <= n) {
             const char* kb = kbase + (int64_t)t * BN * k_rsb;
             const char* vb = vbase + (int64_t)t * BN * v_rsb;
+            if constexpr (TIGHT) copy_offsets();
 #pragma unroll
             for (int i = 0; i < KCP; ++i)
-                if (wave + i * NW < KINSTR) global_load_lds16_soff(kb, koff[i], stage_lds + (wave + i * NW) * 1024);
+                if (wave + i * NW < KINSTR) global_load_lds16_soff(TIGHT ? kb + i * KCR * k_rsb : kb, koff[TIGHT ? 0 : i], stage_lds + (wave + i * NW) * 1024);
 #pragma unroll
             for (int i = 0; i < VCP; ++i)
-                if (wave + i * NW < VINSTR) global_load_lds16_soff(vb, voff[i], stage_lds + KTILE + (wave + i * NW) * 1024);
+                if (wave + i * NW < VINSTR) global_load_lds16_soff(TIGHT ? vb + i * VCR * v_rsb : vb, voff[TIGHT ? 0 : i], stage_lds + KTILE + (wave + i * NW) * 1024);
             return;
         }
         load_tile_u<BN, KROW, NT>(kbase, k_rsb, t * BN, n - 1, stage_lds, wave, lane);
@@ -733,8 +745,12 @@ __global__ __launch_bounds__(NW * 64, 2) void hstu_bwd_dq_kernel(const BwdParams
             typedef TwoChains<KS, VS> Ops;
             constexpr int PD = 4;
             auto load_op = [&](int k) __attribute__((always_inline)) -> vec8 {
-                return Ops::first(k) ? *HSTU_LDS(const vec8, kt + sub * 32 * KROW + krow[Ops::index(k)])
-                                     : *HSTU_LDS(const vec8, vt + sub * 32 * VROW + vrow[Ops::index(k)]);
+                const int i = Ops::index(k);
+                int off = Ops::first(k) ? krow[i] : vrow[i];
+                // (TIGHT, 64 or 128 columns of v: the upper half of a row from the lower one's offsets, for the registers as well)
+                if (TIGHT && VS == 8 && !Ops::first(k) && i >= 4) asm volatile("v_xor_b32 %0, 0x80, %1" : "=v"(off) : "v"(vrow[i - 4]));
+                if (TIGHT && VS == 4 && i >= 2) asm volatile("v_xor_b32 %0, 64, %1" : "=v"(off) : "v"(Ops::first(k) ? krow[i - 2] : vrow[i - 2]));
+                return *HSTU_LDS(const vec8, (Ops::first(k) ? kt + sub * 32 * KROW : vt + sub * 32 * VROW) + off);
             };
             vec8 f[PD];
 #pragma unroll

@@ -47,7 +47,11 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     const bool paired = kPairedDims && bp.f.q_rs < (1 << 22) && bp.do_rs < (1 << 22);
     auto k1 = hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, false>;
     auto k1s = hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, true>;
-    auto k2 = hstu::hstu_bwd_dq_kernel<TT, DQK, DV, kBwdWaves, kBwdTile>;
+    // dQ with 64 columns of q: one workgroup per CU more where that counts.  128 of v: always (512 sequences of 5 .. 120 rows, 8 heads 204 -> 189 us, 16 of 1024 ..
+    // 8192, 4 heads 1325 -> 1314).  32 and 64 of v: up to 256 rows, where it is latency (512 of 5 .. 64 rows, 2 heads 29.0 -> 27.8; 8 heads 87 -> 84); longer ones are
+    // faster without (64 of 200 .. 2048 rows, 2 heads 212, with it 232).
+    auto k2 = hstu::hstu_bwd_dq_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, DQK == 64 && DV == 128>;
+    auto k2short = hstu::hstu_bwd_dq_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, DQK == 64 && DV >= 32>;
     auto k3 = hstu::hstu_bwd_dq_stored_kernel<TT, DQK, kStoredWaves, kBwdTile>;
     // (a function attribute belongs to the device it was set on: one flag per device)
     static std::atomic<bool> attr_done[64];
@@ -61,6 +65,7 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
             if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1ps, hipFuncAttributeMaxDynamicSharedMemorySize, smem1p);
         }
         if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k2short, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k3, hipFuncAttributeMaxDynamicSharedMemorySize, smem3);
         if (e != hipSuccess) {
             hstu_hip_set_last_error("hipFuncSetAttribute", (int)e);
@@ -79,7 +84,7 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     } else {
         if (paired) hipLaunchKernelGGL(k1p, dim3(grid), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
         else hipLaunchKernelGGL(k1, dim3(grid), dim3(kBwdWaves * 64), smem1, stream, bp);
-        hipLaunchKernelGGL(k2, dim3(grid), dim3(kBwdWaves * 64), smem, stream, bp);
+        hipLaunchKernelGGL(bp.f.max_seq_len <= 256 ? k2short : k2, dim3(grid), dim3(kBwdWaves * 64), smem, stream, bp);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

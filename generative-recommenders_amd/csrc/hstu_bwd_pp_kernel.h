@@ -61,7 +61,8 @@ __global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(c
     walk.init(M, p.targets != nullptr, S0, n);
     const int jt_end = walk.end;
     auto next_tile = [&](int jt) { return walk.next(M, jt, S0, n); };
-    const FullRange full = full_rows(M, wS0, 32, 32);
+    FullRange full = {1, 0};
+    if (walk.end - walk.first > 2) full = full_rows(M, wS0, 32, 32);
     auto block_class = [&](int r0) { return full.has(r0) ? 2 : block_class32(M, !walk.scan, r0, wS0, n); };
 
     KeyMask key;

@@ -463,6 +463,23 @@ def test_backward_of_fp32_slices(pkg, dev, dqk, dv, store):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("dv", [32, 64, 128])
+@pytest.mark.parametrize("N", [256, 257])
+def test_backward_of_short_sequences_with_64_columns_of_q(pkg, dev, N, dv, dtype):
+    """The dQ kernel has another form up to 256 rows (64 columns of v) and for 128 of v, whose register-saving addresses must be the same ones: one to
+    three tiles, whole and partial, with and without the interval of full blocks, which starts at three."""
+    print(f"[case] bwd short {N} {dv} {dtype}", flush=True)
+    lengths = [256, 1, 64, 65, 0, 129, 190, 63]
+    q, k, v, dout, offsets = _inputs(N + dv, lengths, 3, 64, dv, dtype)
+    for mask in (dict(), dict(max_attn_len=70, contextual_seq_len=4)):
+        _, *got = _run_bwd(pkg, dev, N, 0.125, q, k, v, dout, offsets, **mask)
+        ref = G.closed_form_grads(N, 0.125, q.float(), k.float(), v.float(), offsets, dout.float(), **mask)
+        for name, g_, r_ in zip(("dq", "dk", "dv"), got, ref):
+            _close(g_, r_, name)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("scaled", [False, True])
 def test_backward_of_fp32_inputs_that_need_a_copy(pkg, dev, scaled):
     """The Python operator's own route (operands that need a copy, an attn_scale): the same fp32 sums as the native front returns, bit for bit."""

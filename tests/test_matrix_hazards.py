@@ -105,3 +105,24 @@ def test_no_vector_instruction_reads_a_matrix_result_too_early(tmp_path, library
         total, early = total + products, early + found
     assert total > 1000
     assert not early, early[:10]
+
+
+def test_the_dq_kernels_for_short_sequences_leave_their_waves_room(tmp_path):
+    """A SIMD has 512 vector registers per lane: four waves (three with 128 columns of v) in 128 (168) each, and none of them in memory.  (The general form of
+    the kernel needs 130 to 174, which cost calls with many short sequences up to 8 %.)"""
+    readelf, objdump = "/opt/rocm/llvm/bin/llvm-readelf", shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+    built = os.path.join(_CSRC, "libhstu_hip.so")
+    if not os.path.exists(readelf) or not os.path.exists(objdump) or not os.path.exists(built):
+        pytest.skip("needs llvm-readelf, llvm-objdump and the built library")
+    shutil.copy(built, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    seen = set()
+    for name in sorted(p for p in os.listdir(tmp_path) if p.endswith("gfx950")):
+        notes = subprocess.run([readelf, "--notes", name], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+        for kernel in notes.split("- .agpr_count")[1:]:
+            m = re.search(r"\.name:\s+\S*hstu_bwd_dq_kernelINS\S*?ELi64ELi(32|64|128)ELi4ELi64ELb1E", kernel)
+            if m:
+                count = {k: int(v) for k, v in re.findall(r"\.(vgpr_count|vgpr_spill_count):\s+(\d+)", kernel)}
+                assert count["vgpr_count"] <= (168 if m[1] == "128" else 128) and count["vgpr_spill_count"] == 0, kernel[:2000]
+                seen.add((name, m[0]))
+    assert len(seen) == 9  # three widths, three types
