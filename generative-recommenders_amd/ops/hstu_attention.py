@@ -8,7 +8,7 @@ messages and output shapes.  Differences, all explicit:
   the reference, a scheduling hint (long sequences are started first) that never changes the result;
 * ``hstu_mha`` is differentiable for bf16 / fp16 / fp32 inputs (``dq, dk, dv`` come from the backward kernels through
   an autograd function, as ``_AttentionFunction`` does in the reference, ``triton_hstu_attention.py:2978-3093``; for
-  fp32 inputs the backward runs on bf16 copies and widens its results); ``delta_hstu_mha`` and the fp8 form are
+  fp32 inputs the backward rounds its operands to bf16 and returns its fp32 sums); ``delta_hstu_mha`` and the fp8 form are
   forward only -- inputs that require grad under ``torch.enable_grad()`` raise ``NotImplementedError`` there;
 * tensors must live on a HIP device; there is no CPU or PyTorch fallback;
 * fp32 q/k/v are rounded to fp16 inside the library (11-bit significand; the reference's Triton path multiplies in
