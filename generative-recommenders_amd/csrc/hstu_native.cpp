@@ -382,16 +382,15 @@ constexpr int64_t kWeightGradColumns = 65536;
 
 void check_linear(int rc) { TORCH_CHECK(rc == 0, "hstu_linear: status ", rc, " (", hstu_linear_last_error(), ")"); }
 
-// a @ weight^T
+// a @ weight^T.  The shapes that are not the kernels' are the framework's product, which chooses for these rows: the library's plans are made for a size class
+// by the first rows that it sees, so that a gradient would depend on the batches before it, and asking for every batch costs the host 64 us.
 Tensor product_t(const Tensor& a, const Tensor& weight) {
     const int64_t rows = a.size(0), n = weight.size(0);
     const int32_t k = (int32_t)a.size(1);
-    Tensor out = at::empty({rows, n}, a.options()), scratch;
-    const size_t need = hstu_linear_product_t_workspace_bytes(rows, k, (int32_t)n);
-    void* workspace = nullptr;
-    if (need > 0) scratch = aligned_scratch(need, a, &workspace);
+    if (hstu_linear_product_t_workspace_bytes(rows, k, (int32_t)n) > 0) return at::mm(a, weight.t());
+    Tensor out = at::empty({rows, n}, a.options());
     check_linear(hstu_linear_product_t(a.const_data_ptr(), a.stride(0), weight.const_data_ptr(), weight.stride(0), rows, k, (int32_t)n, dense_dtype(a),
-                                       out.data_ptr(), n, workspace, (int64_t)need, stream_of(a)));
+                                       out.data_ptr(), n, nullptr, 0, stream_of(a)));
     return out;
 }
 

@@ -203,7 +203,7 @@ int hstu_linear_weight_grad(const void* a, int64_t a_row_stride, int32_t m, cons
 
 /* out [rows, n] = a [rows, k] @ weight [n, k]^T (strides in elements, rows 16-byte aligned, strides below 2^22; k and n multiples of 8), fp32
  * sums rounded once: d_joined = d_out @ output_weight^T and the like.  `workspace` (256-byte aligned) is for the shapes that the library's GEMM
- * takes; the others need none. */
+ * takes, by a plan that the first rows of a size class choose for the others; the others need none. */
 size_t hstu_linear_product_t_workspace_bytes(int64_t rows, int32_t k, int32_t n);
 int hstu_linear_product_t(const void* a, int64_t a_row_stride, const void* weight, int64_t weight_row_stride, int64_t rows, int32_t k, int32_t n,
                           int32_t dtype, void* out, int64_t out_row_stride, void* workspace, int64_t workspace_bytes, void* stream);

@@ -468,6 +468,38 @@ def test_gradient_of_u_in_front_of_silu(pkg, dev, rows, k, n, dtype, bound):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d_model,H,hidden", [(512, 4, 128), (320, 2, 64), (1024, 4, 64), (256, 3, 128), (768, 8, 96)])
+def test_gradient_of_x_does_not_depend_on_the_batches_before(pkg, dev, d_model, H, hidden):
+    """The product of the buffer's gradient with W^T is the framework's for these shapes, chosen for the batch's own rows: bit for bit that product through the
+    layer norm's backward, whichever row counts of a size class came first.  (With one plan per class of rows the first batch chose for the others:
+    other bits, and up to 1.9 times as long.)"""
+    import ctypes
+
+    print(f"[case] uqvk backward in changing batches {d_model} {H} {hidden}", flush=True)
+    V, I, J = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32
+    n_u, rows = hidden * H, (513, 639, 600, 520, 2561, 3071, 2800, 3055, 10241, 12287, 11000)
+    x, nw, nb, w, b = [t.to(dev) for t in _inputs(d_model, max(rows), d_model, H, hidden, hidden, torch.bfloat16)]
+    grad = torch.randn(max(rows), 4 * n_u, generator=torch.Generator(device=dev).manual_seed(1), device=dev).bfloat16()
+    grad[:, :n_u] = 0  # (u is not used)
+    lib = pkg.lib()
+    lib.hstu_uqvk_layer_norm_bwd_workspace_bytes.restype = ctypes.c_size_t
+    for n in rows:
+        xi = x[:n].clone().requires_grad_(True)
+        _, q, k, v = pkg.hstu_compute_uqvk(xi, nw, nb, 1e-6, H, hidden, hidden, w, b)
+        parts = [grad[:n, i * n_u : (i + 1) * n_u].reshape(n, H, hidden) for i in (2, 3, 1)]
+        (got,) = torch.autograd.grad((q, k, v), xi, parts)
+        dy = torch.mm(grad[:n].contiguous(), w.t())
+        want, dw, db = torch.empty_like(xi), torch.empty_like(nw), torch.empty_like(nb)
+        need = lib.hstu_uqvk_layer_norm_bwd_workspace_bytes(I(n), J(d_model))
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        rc = lib.hstu_uqvk_layer_norm_bwd(V(xi.data_ptr()), I(d_model), V(nw.data_ptr()), ctypes.c_float(1e-6), V(dy.data_ptr()), I(d_model), V(want.data_ptr()),
+                                          I(d_model), V(dw.data_ptr()), V(db.data_ptr()), I(n), J(d_model), J(0), V(ws.data_ptr()), I(need),
+                                          V(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert rc == 0 and torch.equal(got, want.detach()), n
+
+
+@pytest.mark.gpu
 def test_uqvk_with_a_total_length_that_changes_from_batch_to_batch(pkg, dev):
     """The hipBLASLt path keeps one plan per size class of the row count, not per row count: lengths of one class
     (1100, 1101, 1279), of others (640, 5000), and the first again, each against the oracle."""
