@@ -74,8 +74,10 @@ struct Choice {
 //     into 512 26.2 / 22.8), but for what kRows64 does in one round with up to 6 units per wave (12000 rows into 1536 32.0, kWide 34.6, the library 46).
 //   * At depth 384 and 512, W above the 4 MB of an XCD's L2: kRows32 with one workgroup per CU, kWide from 2.75 units on, the library between them
 //     (depth 512 into 6144 columns, 100 rows 4.8 / 7.2, 200 rows 10.0 / 8.2, 1000 rows 20.0 / 14.6, 2000 rows 21.0 / 28.4, 4000 rows 29.9 / 41).
-//   * Otherwise there into fewer than 1024 columns the library (5000 rows into 768 10.1 / 9.7), from there kRows64: with one unit per wave (1000 rows into
-//     3072 9.4 / 12.0), with several where they give seven tenths of the CUs a workgroup (2000 rows into 3072 13.8 / 14.2, 12000 into 1024 23.2 / 33.3;
+//     From 3 MB at depth 512 the library too between kRows32 (of 4 MB: with one workgroup per CU) and kWide (into 3072 columns, 1300 rows 11.9 / 10.0, 2315 16.7 /
+//     13.6, 4533 24.8 / 19.9, 5400 33.2 / 44.5; into 4096, 450 rows 8.4 / 7.0, 900 11.9 / 9.1, 2000 17.0 / 15.2, 3764 29.0 / 21.2, 4100 33.4 / 36.8).
+//   * Otherwise there into fewer than 1024 columns the library (5000 rows into 768 10.1 / 9.7), from there kRows64: with one unit per wave (1100 rows into
+//     2048 8.6 / 10.0), with several where they give seven tenths of the CUs a workgroup (2600 rows into 2560 14.9 / 19.0, 12000 into 1024 23.2 / 33.3;
 //     fewer: 3000 rows into 1536 13.2 / 11.9, 5000 into 2048 23.6 / 17.3).
 //   * Up to depth 256 kRows64, in one round with as many units per wave as that takes (54000 rows of depth 256 into 768 columns 30 / 50, 12000 of depth 128
 //     into 1536 13.5 / 26), and in several but for 256 columns of depth 256 in the second (54000 rows 17.3 / 15.2, 100000 29.5 / 34.9).
@@ -84,8 +86,8 @@ Choice choose_product(int64_t rows, int n, int kt) {
     const int quarter32 = n / 128, quarter = kt <= 4 ? quarter32 : (quarter32 + 1) / 2;
     const bool large = kt > 4 && (long long)n * kt * 128 > (4 << 20);
     const bool wide = kt >= 4 && n >= 512 && wide_units >= (kt == 4 ? 1536 : large ? 704 : 1025) && wide_units <= 0x7fffffffLL;
-    if (blocks32 * quarter32 <= (large ? 256 : 512)) return {Kernel::kRows32, 1};
-    if (kt > 4 && (large || n < 1024)) return {wide ? Kernel::kWide : Kernel::kLibrary, 0};
+    if (blocks32 * quarter32 <= (kt > 4 && (long long)n * kt * 128 >= (4 << 20) ? 256 : 512)) return {Kernel::kRows32, 1};
+    if (kt > 4 && (large || n < 1024 || (kt == 8 && n >= 3072))) return {wide ? Kernel::kWide : Kernel::kLibrary, 0};
     if (kt == 4 && wide) return {Kernel::kWide, 0};
     const int round = kt <= 4 ? 512 : 256;
     for (int per = 1; per <= (kt <= 4 ? hstu::kUqvkMostUnits : 8); per *= 2) {

@@ -328,11 +328,12 @@ def test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound):
 @pytest.mark.parametrize(
     "rows,k,n,library",
     # on both sides of the lines: units of their own for one round, and for W above 4 MB half of one; 64 rows with several units per wave, for seven tenths of
-    # the CUs and fewer; fewer columns; 64 rows per wave above 4 units per CU, and from 2.75 for W above 4 MB; 256 columns in the second round
+    # the CUs and fewer; fewer columns; 64 rows per wave above 4 units per CU, and from 2.75 for W above 4 MB; 256 columns in the second round; W of 3 and 4 MB
     [(1000, 512, 1536, False), (64, 512, 6144, False), (200, 512, 6144, True), (1000, 512, 6144, True), (2000, 512, 6144, False), (3000, 512, 1536, True),
      (3000, 384, 1536, True), (5000, 512, 2048, True), (10000, 384, 1024, True), (4000, 512, 1536, False), (12000, 512, 1024, False), (17000, 384, 1024, False),
      (32768, 512, 512, True), (32769, 512, 512, False), (10000, 512, 1536, True),
-     (24000, 512, 768, False), (54000, 256, 256, True), (32768, 256, 256, False), (100000, 256, 256, False), (54000, 128, 256, False)],
+     (24000, 512, 768, False), (672, 512, 3072, False), (700, 512, 3072, True), (4533, 512, 3072, True), (5400, 512, 3072, False), (256, 512, 4096, False), (450, 512, 4096, True),
+     (3764, 512, 4096, True), (4100, 512, 4096, False), (54000, 256, 256, True), (32768, 256, 256, False), (100000, 256, 256, False), (54000, 128, 256, False)],
 )
 def test_which_products_with_a_transposed_weight_are_the_library_s(rows, k, n, library):
     """Only the library's need a workspace.  (Into 1024 columns and more all of them were the kernels', up to 1.6 times as long on the GPU; the sizes
