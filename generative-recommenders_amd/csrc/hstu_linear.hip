@@ -18,12 +18,15 @@
 #include "hstu_uqvk_kernel.h"
 #include "hstu_output_kernel.h"
 #include "hstu_output_rows_kernel.h"
+#include "hstu_output_panel_kernel.h"
 
 // hstu_uqvk.hip, hstu_uqvk_bwd.hip
 int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
 int hstu_uqvk_grad_u_launch(const hstu::UqvkFusedParams& p, int depth, bool bf16, hipStream_t stream);
 bool hstu_product_t_takes(int64_t rows, int depth, int n);
 int hstu_product_t_launch(const hstu::UqvkFusedParams& p, int depth, bool bf16, hipStream_t stream);
+
+int hstu_output_panel_launch(const hstu::OutputPanelParams& p, int form, bool bf16, bool group, hipStream_t stream);
 
 namespace {
 
@@ -333,6 +336,30 @@ int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
         return -7;
     }
     return 0;
+}
+
+// path = 0: the one kernel for more rows, where u goes in as it is.  Returns its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are
+// this kernel's up to a width of 256 (3 x 256 into 512 columns, us: one row 7.0 -> 5.2, 256 rows 7.3 -> 5.5; 3 x 512: 7.7 against 8.2).  Past those it starts
+// at 320 rows; in front of that it would be faster as well (257 rows of 3 x 512 into 512 columns 12.2 -> 8.7), but there this path's results are the library's
+// bit for bit, which callers hold it to.
+int output_panel_form(const HstuOutputArgs* a) {
+    const int64_t d = (int64_t)a->heads * a->linear_dim;
+    if (a->path != 0 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return -1;
+    if (a->d_out % 128 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512) return -1;
+    if (a->group_norm) {
+        const int lanes = a->linear_dim / 8;
+        if (a->linear_dim % 8 != 0 || lanes > 64 || (lanes & (lanes - 1)) != 0) return -1;
+    }
+    if (a->rows < 320) return output_takes_rows(a) && d <= 256 ? hstu::kPanel32x128 : -1;
+    return hstu::output_panel_form(a->rows, (int)d, a->d_out, a->dtype == 0);
+}
+
+int launch_output_panel(const HstuOutputArgs* a, int form, hipStream_t stream) {
+    hstu::OutputPanelParams p;
+    const int rc = hstu::norm_mul_params(a, nullptr, (int64_t)output_blocks(a) * a->heads * a->linear_dim, false, p.nm);
+    if (rc != 0) return rc;
+    p.x = (const char*)a->x, p.x_rs = a->x_row_stride, p.w = (const char*)a->output_weight, p.out = (char*)a->out, p.n = a->d_out;
+    return hstu_output_panel_launch(p, form, a->dtype == 0, a->group_norm != 0, stream);
 }
 
 size_t output_fused_workspace(const HstuOutputArgs* a) {
@@ -820,7 +847,7 @@ int hstu_linear_product_t(const void* a, int64_t a_row_stride, const void* weigh
 
 size_t hstu_output_workspace_bytes(const HstuOutputArgs* a) {
     if (!a || a->rows <= 0 || a->heads <= 0 || a->linear_dim <= 0) return 0;
-    if (output_takes_rows(a)) return 0;
+    if (output_takes_rows(a) || output_panel_form(a) >= 0) return 0;
     if (output_takes_fused(a)) return output_fused_shape(a) ? output_fused_workspace(a) : 0;
     return joined_bytes(a) + kGemmScratch;
 }
@@ -870,6 +897,7 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
                  "elements: dropout runs on the library path (path 0 or 1)");
         return -6;
     }
+    if (const int form = output_panel_form(a); form >= 0) return launch_output_panel(a, form, stream);
     if (output_takes_rows(a)) {
         if (a->dtype == 0) return a->group_norm ? launch_output_rows<hstu::Bf16, true>(a, stream) : launch_output_rows<hstu::Bf16, false>(a, stream);
         return a->group_norm ? launch_output_rows<hstu::Fp16, true>(a, stream) : launch_output_rows<hstu::Fp16, false>(a, stream);

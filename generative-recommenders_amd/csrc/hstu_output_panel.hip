@@ -1,0 +1,59 @@
+// The one-kernel output step for more than a few rows (libhstu_linear.so).  Compiled with the matrix instructions' VGPR form: the sums are few.
+#include "hstu_output_panel_kernel.h"
+
+#include <atomic>
+#include <cstdio>
+
+// defined in hstu_linear.hip; internal to the library
+extern "C" __attribute__((visibility("hidden"))) void hstu_linear_set_last_error(const char* text);
+
+namespace {
+
+template <class TT, bool GROUP, int D, int RB, int NW>
+int launch_shape(const hstu::OutputPanelParams& p, hipStream_t stream) {
+    typedef hstu::OutputPanel<D, RB, NW> Geo;
+    auto kern = hstu::hstu_output_panel_kernel<TT, GROUP, D, RB, NW>;
+    static std::atomic<bool> attr_done[64];
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev >= 64) dev = -1;
+    hipError_t e = hipSuccess;
+    if (dev < 0 || !attr_done[dev]) {  // (a function attribute belongs to the device it was set on)
+        e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Geo::kLds);
+        if (e == hipSuccess && dev >= 0) attr_done[dev] = true;
+    }
+    if (e == hipSuccess) {
+        const long long octets = ((p.nm.rows + Geo::kRows - 1) / Geo::kRows + 7) / 8;
+        hipLaunchKernelGGL(kern, dim3((unsigned)(octets * 8 * (p.n / Geo::kCols))), dim3(NW * 64), Geo::kLds, stream, p);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) return 0;
+    char text[256];
+    snprintf(text, sizeof(text), "output panel kernel: %s", hipGetErrorString(e));
+    hstu_linear_set_last_error(text);
+    return -7;
+}
+
+template <class TT, bool GROUP, int D>
+int launch_form(const hstu::OutputPanelParams& p, int form, hipStream_t stream) {
+    if constexpr (D <= 256)
+        if (form == hstu::kPanel64x128) return launch_shape<TT, GROUP, D, 2, 4>(p, stream);
+    return form == hstu::kPanel32x128 ? launch_shape<TT, GROUP, D, 1, 4>(p, stream) : launch_shape<TT, GROUP, D, 2, 8>(p, stream);
+}
+
+template <class TT, bool GROUP>
+int launch_width(const hstu::OutputPanelParams& p, int form, hipStream_t stream) {
+    switch (p.nm.d) {
+        case 128: return launch_form<TT, GROUP, 128>(p, form, stream);
+        case 256: return launch_form<TT, GROUP, 256>(p, form, stream);
+        case 384: return launch_form<TT, GROUP, 384>(p, form, stream);
+        default: return launch_form<TT, GROUP, 512>(p, form, stream);
+    }
+}
+
+}  // namespace
+
+// p.nm.d: 128, 256, 384 or 512; form: one that output_panel_form gives for it
+int hstu_output_panel_launch(const hstu::OutputPanelParams& p, int form, bool bf16, bool group, hipStream_t stream) {
+    if (bf16) return group ? launch_width<hstu::Bf16, true>(p, form, stream) : launch_width<hstu::Bf16, false>(p, form, stream);
+    return group ? launch_width<hstu::Fp16, true>(p, form, stream) : launch_width<hstu::Fp16, false>(p, form, stream);
+}

@@ -6,10 +6,9 @@ signatures (``generative_recommenders/ops/hstu_compute.py:54-104``, ``:107-214``
 with the bias and, for the u columns, the SiLU in its epilogue.  ``u, q, k, v`` come back as column slices of one
 ``[L, (2*hidden + 2*attn) * H]`` buffer, which ``hstu_mha`` / ``delta_hstu_mha`` read in place.
 
-``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  Up to 256 rows, while its workgroups
-run at once, one kernel does it all (``csrc/hstu_output_rows_kernel.h``).  From 32768 rows on a hand-written GEMM reads u
-and attn where they are and ``act(u) * norm(attn)`` from a row-wise kernel; between them, and for widths it does not take or with dropout, that
-kernel writes the concatenated operand and hipBLASLt multiplies it with the residual as its C operand.
+``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  For few rows, and for more where u is not
+activated and the widths suit, one kernel does it all (``csrc/hstu_output_rows_kernel.h``, ``csrc/hstu_output_panel_kernel.h``).  From 32768 rows on a
+hand-written GEMM reads u and attn where they are and ``act(u) * norm(attn)`` from a row-wise kernel; otherwise, and with dropout, that kernel writes the concatenated operand and hipBLASLt multiplies it with the residual as its C operand.
 (``csrc/hstu_linear.hip``, ``csrc/hstu_output_kernel.h``, ``include/hstu_linear.h``.)
 
 Device tensors only, bf16 or fp16; ``kernel`` is accepted and ignored.  The usual call, with or without gradients, goes through

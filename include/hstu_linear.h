@@ -88,7 +88,7 @@ int hstu_uqvk_layer_norm(const void* x, int64_t x_row_stride, const void* weight
  *                           joined = u | attn | y only when concat_u AND concat_x, else y alone (as the reference)
  *              silu_u     : layer norm: the copied u block goes through SiLU; group norm: u does before both uses
  *     out = x + joined @ output_weight             [rows, d_out]
- * Two paths (see `path`).  Library path (any shape): the norm / multiply / concatenate step is one hand-written kernel
+ * Two paths (see `path`), and kernels that do the whole step for fewer rows.  Library path (any shape): the norm / multiply / concatenate step is one hand-written kernel
  * (one wave per row, HBM-bound) that writes `joined` in the inputs' type; the product with the residual as the GEMM's
  * C operand runs on hipBLASLt.  Concatenating path (d_out a multiple of 256): the same norm-multiply kernel writes y alone (and
  * SiLU(u) where that is a block of `joined`), and a hand-written GEMM kernel reads the blocks of `joined` where they
@@ -121,9 +121,11 @@ typedef struct HstuOutputArgs {
     int32_t path;              /* 1 = library path (norm-mul kernel + hipBLASLt); 2 = concatenating path (norm-mul kernel
                                   + hand-written GEMM over the blocks where they are): needs d_out a multiple of 256 and heads *
                                   linear_dim a multiple of 64 (and, with group norm, no SiLU on a copied u), else status
-                                  -6; 0 = one kernel for the whole step (no workspace) up to 256 rows where its workgroups
-                                  of 32 rows x 32 columns run at once, without dropout, heads * linear_dim a multiple of 128 up
-                                  to 512; the concatenating path where it applies and rows >= 32768; else the library */
+                                  -6; 0 = one kernel for the whole step (no workspace) where it is faster: without
+                                  dropout, heads * linear_dim a multiple of 128 up to 512, up to 256 rows where its
+                                  workgroups of 32 rows x 32 columns run at once, and from 320 rows on, u not activated,
+                                  d_out a multiple of 128, to a size that depends on both widths and the type; the
+                                  concatenating path where it applies and rows >= 32768; else the library */
     /* Dropout of `joined` (`F.dropout(y, p, training)` at the end of pytorch_norm_mul_dropout, pt_hstu_linear.py:80-84): the
      * whole concatenation goes through it, in fp32, before it is rounded; survivors are multiplied by 1 / (1 - ratio).
      * Element (r, c) of the [rows, blocks * heads * linear_dim] matrix is kept when word c % 4 of

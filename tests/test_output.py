@@ -304,6 +304,54 @@ def test_compute_output_on_both_sides_of_one_round(pkg, dev, N, blocks, H, ld, D
     _close(got, O.compute_output(attn, u, x, nw, nb, w, 1e-6, concat_u=cu, concat_x=cx, num_heads=H, linear_dim=ld), "wide rows vs fp32 oracle")
 
 
+# (rows, heads, linear_dim, d_out, copied blocks, group norm, dtype, whether the one kernel for more rows takes it): its first row count, both sides of the
+# line between its forms of 32 x 128 and 64 x 256 (64 x 128 where d_out is no multiple of 256), rows that fill no block, every width of a row (384: lanes
+# without a chunk), one to three blocks, heads of one and of all lanes of a row, and the sizes behind the last one it takes
+BF, FP = torch.bfloat16, torch.float16
+PANEL_CASES = [
+    (319, 4, 128, 512, 2, False, BF, False), (320, 4, 128, 512, 2, False, BF, True), (353, 16, 32, 128, 2, True, FP, True), (4096, 4, 128, 512, 2, False, FP, True),
+    (4097, 4, 128, 512, 2, False, FP, True), (8192, 8, 64, 512, 2, True, BF, True), (8193, 4, 128, 512, 2, False, FP, False),
+    (16385, 4, 128, 512, 2, False, BF, False), (1000, 3, 128, 384, 2, True, BF, True), (9000, 3, 128, 384, 2, False, FP, False), (5000, 3, 128, 768, 2, False, BF, True),
+    (8200, 8, 32, 256, 2, True, FP, True), (5600, 2, 128, 384, 2, False, BF, True), (20000, 1, 128, 640, 1, False, FP, True), (16385, 1, 128, 256, 0, True, BF, True),
+    (777, 4, 128, 1024, 0, False, FP, True), (2049, 2, 64, 512, 1, False, BF, True), (40000, 1, 128, 256, 2, False, BF, True), (600, 32, 8, 256, 2, True, FP, True),
+]
+
+
+@pytest.mark.parametrize("N,H,ld,D,copied,group_norm,dtype,taken", PANEL_CASES)
+def test_output_takes_one_kernel_where_it_is_faster(N, H, ld, D, copied, group_norm, dtype, taken):
+    """Which calls the one kernel for more than a few rows takes: those that need no workspace.  Needs no GPU."""
+    import ctypes
+
+    import __graft_entry__
+
+    __graft_entry__.load_package()
+    from generative_recommenders_amd.ops import hstu_compute as hc
+
+    def need(**more):
+        a = hc.HstuOutputArgs(rows=N, d_out=D, heads=H, linear_dim=ld, concat_u=copied > 0, concat_x=copied > 1, group_norm=group_norm, dtype=int(dtype == FP), **more)
+        return hc.lib().hstu_output_workspace_bytes(ctypes.byref(a))
+
+    assert (need() == 0) == taken
+    assert need(dropout_ratio=0.1) > 0 and need(silu_u=1) > 0 and need(path=1) > 0  # (what it does not do)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,ld,D,copied,group_norm,dtype,taken", [c for c in PANEL_CASES if c[-1]])
+def test_compute_output_of_more_rows_in_one_kernel(pkg, dev, N, H, ld, D, copied, group_norm, dtype, taken):
+    """On strided views, against the fp32 oracle and the library path (rounded once from fp32 sums, as both are)."""
+    print(f"[case] output in one kernel {N} {H} {ld} {D} copied {copied} group={group_norm} {dtype}", flush=True)
+    cu, cx = copied > 0, copied > 1
+    attn, u, x, nw, nb, w = _inputs(N + D, N, H, ld, D, _blocks(cu, cx, group_norm), group_norm, dtype)
+    wide = torch.cat([u, attn, x], dim=1).to(dev)
+    L = H * ld
+    args = (wide[:, L : 2 * L], wide[:, :L], wide[:, 2 * L :], nw.to(dev), nb.to(dev), 1e-6, w.to(dev), H, ld, 0.0, False, cu, cx, "none", group_norm, False)
+    got, lib = pkg.hstu_compute_output(*args), pkg.hstu_compute_output(*args, path=1)
+    torch.cuda.synchronize()
+    kw = dict(concat_u=cu, concat_x=cx, group_norm=group_norm, num_heads=H, linear_dim=ld)
+    _close(got, O.compute_output(attn, u, x, nw, nb, w, 1e-6, **kw), "one kernel vs fp32 oracle")
+    _close(got, lib.float().cpu(), "one kernel vs library path")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N", [33000, 257])
 def test_compute_output_concat_gemm_on_views_of_wider_buffers(pkg, dev, N):
