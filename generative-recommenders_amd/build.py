@@ -64,7 +64,7 @@ def build_library(verbose: bool = False) -> str:
     common = [hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + ["-I", INCLUDE, "-I", CSRC]
     objs = [os.path.join(CSRC, name) for name in ("hstu_api.o", "hstu_bwd_api.o", "hstu_fwd_fitted.o", "hstu_bwd_f32.o")]
     linear_objs = [os.path.join(CSRC, "hstu_linear.o"), os.path.join(CSRC, "hstu_linear_bwd.o"), os.path.join(CSRC, "hstu_uqvk.o"),
-                   os.path.join(CSRC, "hstu_uqvk_bwd.o"), os.path.join(CSRC, "hstu_output_panel.o")]
+                   os.path.join(CSRC, "hstu_uqvk_bwd.o")]
     jobs = [
         common + ["-c", os.path.join(CSRC, "hstu_api.hip"), "-o", objs[0]],
         common + ["-c", os.path.join(CSRC, "hstu_bwd_api.hip"), "-o", objs[1]],
@@ -75,7 +75,6 @@ def build_library(verbose: bool = False) -> str:
         # (matrix results in vector registers: see the file)
         common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_uqvk.hip"), "-o", linear_objs[2]],
         common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_uqvk_bwd.hip"), "-o", linear_objs[3]],
-        common + ["-mllvm", "-amdgpu-mfma-vgpr-form", "-c", os.path.join(CSRC, "hstu_output_panel.hip"), "-o", linear_objs[4]],
     ]
     native_compile, native_link, native_obj = _native_commands()
     jobs.append(native_compile)

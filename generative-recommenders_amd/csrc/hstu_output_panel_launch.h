@@ -1,4 +1,6 @@
-// The one-kernel output step for more than a few rows (libhstu_linear.so).  Compiled with the matrix instructions' VGPR form: the sums are few.
+// Launching the one-kernel output step for more than a few rows (hstu_output_panel_kernel.h); part of hstu_uqvk.hip, which is compiled with the matrix
+// instructions' VGPR form: the sums are few, and the vector instructions of the epilogue read them.
+#pragma once
 #include "hstu_output_panel_kernel.h"
 
 #include <atomic>
@@ -6,7 +8,6 @@
 
 // defined in hstu_linear.hip; internal to the library
 extern "C" __attribute__((visibility("hidden"))) void hstu_linear_set_last_error(const char* text);
-
 namespace {
 
 template <class TT, bool GROUP, int D, int RB, int NW>

@@ -1,5 +1,6 @@
-// The producer's kernels (libhstu_linear.so).  A translation unit of its own because of how it is compiled: see hstu_uqvk_launch.h.
+// The producer's kernels and the one-kernel output step (libhstu_linear.so).  A translation unit of its own because of how it is compiled: see hstu_uqvk_launch.h.
 #include "hstu_uqvk_launch.h"
+#include "hstu_output_panel_launch.h"
 
 // d_model: 128, 256, 384 or 512
 int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream) {
