@@ -75,6 +75,7 @@ __attribute__((visibility("hidden"))) int hstu_bwd_params(const HstuFwdArgs* a, 
     p.c1 = -a->alpha * 1.4426950408889634f;
     bp.gscale = a->alpha / (float)a->max_seq_len;
     bp.pscale = a->alpha == 0.0f ? 0.0f : -1.0f / ((float)a->max_seq_len * 1.4426950408889634f);
+    bp.total_q = a->total_q;
     bp.dout = (const char*)g->dout;
     bp.dq = (char*)g->dq, bp.dk = (char*)g->dk, bp.dv = (char*)g->dv;
     bp.do_rs = g->do_row_stride, bp.do_hs = g->do_head_stride;

@@ -44,6 +44,7 @@ struct BwdParams {
     // Stored-dS mode (both null / 0 otherwise): the key-stationary kernel writes every block of dS it forms, rounded
     // to the operand type, and hstu_bwd_dq_stored_kernel reads them back instead of forming S and dP again.
     char* ds;
+    int64_t total_q;  // rows of all sequences (the host's choice of launches)
     int ds_pitch32;  // blocks of 32 keys per row of blocks: 4 * ceil(max_seq_len / 128)
 };
 
@@ -630,8 +631,9 @@ __global__ __launch_bounds__(NW * 64, 1) void hstu_bwd_dkdv_kernel(const BwdPara
 // ---- query-stationary kernel: dQ -----------------------------------------------------------------------------------
 
 // TIGHT: four waves per SIMD for 32 and 64 columns of v and three for 128 (with 64 of q; what the LDS lets in), where the registers otherwise leave one fewer.
+// (`bid`: number of the item; threads from NW * 64 on have ended.)
 template <class TT, int DQK, int DV, int NW, int BN, bool TIGHT>
-__global__ __launch_bounds__(NW * 64, TIGHT ? (DV == 128 ? 3 : 4) : 2) void hstu_bwd_dq_kernel(const BwdParams bp) {
+__device__ __forceinline__ void bwd_dq_item(const BwdParams& bp, int bid) {
     typedef typename TT::vec8 vec8;
     const FwdParams& p = bp.f;
     constexpr int BM = NW * 32;
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(NW * 64, TIGHT ? (DV == 128 ? 3 : 4) : 2) void hstu
     const int g = lane >> 5, l32 = lane & 31;
 
     Work W;
-    if (!bwd_decode<BM>(p, W, blockIdx.x, false)) return;
+    if (!bwd_decode<BM>(p, W, bid, false)) return;
     const SeqMask& M = W.M;
     const int n = W.n;
     kv_tile_range(M, W.u, W.R0, W.R1, BN, W.jt_begin, W.jt_end);
@@ -802,6 +804,11 @@ __global__ __launch_bounds__(NW * 64, TIGHT ? (DV == 128 ? 3 : 4) : 2) void hstu
         stage ^= 1;
     }
     store_output<TT, DTK>(dqacc, 0, bp.dq, W.seq_start, wq0 + l32, n, bp.dq_rs, bp.dq_hs, W.h, g, bp.gscale, DQK);
+}
+
+template <class TT, int DQK, int DV, int NW, int BN, bool TIGHT>
+__global__ __launch_bounds__(NW * 64, TIGHT ? (DV == 128 ? 3 : 4) : 2) void hstu_bwd_dq_kernel(const BwdParams bp) {
+    bwd_dq_item<TT, DQK, DV, NW, BN, TIGHT>(bp, blockIdx.x);
 }
 
 // ---- dQ from stored dS --------------------------------------------------------------------------------------------

@@ -33,6 +33,15 @@ auto key_stationary_kernel(std::false_type) {
 }
 
 template <class TT, int DQK, int DV>
+auto both_kernel(std::true_type) {
+    return hstu::hstu_bwd_both_kernel<TT, DQK, DV>;
+}
+template <class TT, int DQK, int DV>
+auto both_kernel(std::false_type) {
+    return hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, false>;  // (not launched)
+}
+
+template <class TT, int DQK, int DV>
 int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     // three tile slots for the key-stationary kernel, two for the other; + 64: transposing reads of a 16-wide tile's unused half
     constexpr int smem1 = 3 * kBwdTile * (DQK + DV) * 2 + 64;
@@ -45,6 +54,7 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     auto k1ps = key_stationary_kernel<TT, DQK, DV, true>(std::integral_constant<bool, kPairedDims>{});
     constexpr int smem1p = kPairedDims ? hstu::bwd_pp_lds_bytes<(DQK < 32 ? 32 : DQK), (DV < 32 ? 32 : DV)>() : 0;
     const bool paired = kPairedDims && bp.f.q_rs < (1 << 22) && bp.do_rs < (1 << 22);
+    auto k12 = both_kernel<TT, DQK, DV>(std::integral_constant<bool, kPairedDims>{});
     auto k1 = hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, false>;
     auto k1s = hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, true>;
     // dQ with 64 columns of q: one workgroup per CU more where that counts.  128 of v: always (512 sequences of 5 .. 120 rows, 8 heads 204 -> 189 us, 16 of 1024 ..
@@ -62,6 +72,7 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
         if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1s, hipFuncAttributeMaxDynamicSharedMemorySize, smem1);
         if (kPairedDims) {
             if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1p, hipFuncAttributeMaxDynamicSharedMemorySize, smem1p);
+            if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k12, hipFuncAttributeMaxDynamicSharedMemorySize, smem1p);
             if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k1ps, hipFuncAttributeMaxDynamicSharedMemorySize, smem1p);
         }
         if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
@@ -74,6 +85,24 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
         if (dev >= 0) attr_done[dev] = true;
     }
     const unsigned grid = (unsigned)bp.f.slots_per_xcd * 8;
+    if constexpr (kPairedDims) {
+        // One launch for both kernels' items while few of them leave the chip idle: two latencies become one.  us, two launches / one: 8 sequences of 20 .. 150 rows, 2
+        // heads of 64 / 128 23.0 / 15.1; 4 of 500 .. 1500, 4 heads, 168 items each, 128 / 128 114 / 71; 16 of 100 .. 768, 64 / 32, fp32, 64.5 / 47.2.  An item of the one
+        // launch holds what the larger of the two kernels needs, with 128 columns a CU alone, so that more items than CUs pay where they differ in length: 32 of
+        // 100 .. 600, 4 heads, 420 items, 80 / 73; not the short (256 of 20 .. 250, 1 head, 384 items 54 / 64; 128 of 24 .. 60, 4 heads 31 / 35) nor the long (4 of
+        // 1000 .. 4000, 344 items 238 / 275).  Up to 64 columns two or three fit: 2 of 3000 .. 6000, 8 heads, 64 / 64, 632 items 318 / 278, 128 of 20 .. 250, 780
+        // items 52 / 57; 256 of 20 .. 250, 1 head, 32 / 32, 384 items 26 / 28.
+        const int64_t upper = (int64_t)bp.f.H * (bp.total_q / kBwdRows + bp.f.B);  // items at most, as the grid
+        const int64_t items = upper < (int64_t)grid ? upper : (int64_t)grid, len = bp.f.max_seq_len;
+        const int64_t most = DQK <= 64 && DV <= 64 ? (len <= 256 ? 384 : 768) : len <= 128 ? 128 : len <= 256 ? 256 : len <= 2048 ? 512 : 256;
+        if (!bp.ds && paired && items <= most) {
+            hipLaunchKernelGGL(k12, dim3(grid * 2), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
+            const hipError_t e = hipGetLastError();
+            if (e == hipSuccess) return HSTU_OK;
+            hstu_hip_set_last_error("backward kernel launch", (int)e);
+            return HSTU_ERR_LAUNCH;
+        }
+    }
     if (bp.ds) {
         if (paired) hipLaunchKernelGGL(k1ps, dim3(grid), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
         else hipLaunchKernelGGL(k1s, dim3(grid), dim3(kBwdWaves * 64), smem1, stream, bp);

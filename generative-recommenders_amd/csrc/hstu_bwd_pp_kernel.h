@@ -31,7 +31,7 @@ constexpr int bwd_pp_lds_bytes() {
 }
 
 template <class TT, int DQK, int DV, bool STORE>
-__global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(const BwdParams bp) {
+__device__ __forceinline__ void bwd_dkdv_pp_item(const BwdParams& bp, int bid) {
     typedef typename TT::vec8 vec8;
     static_assert(DQK >= 32 && DV >= 32 && DQK % 32 == 0 && DV % 32 == 0, "a tile copy is at least one instruction per copying wave");
     const FwdParams& p = bp.f;
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(c
     const int g = lane >> 5, l32 = lane & 31;
 
     Work W;
-    if (!bwd_decode<BM>(p, W, blockIdx.x, true)) return;
+    if (!bwd_decode<BM>(p, W, bid, true)) return;
     const SeqMask& M = W.M;
     const int n = W.n;
     const int S0 = W.R0;           // first key row of the workgroup
@@ -392,6 +392,24 @@ __global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(c
             run(tile, drain);
         }
         store_output<TT, DTK>(dkacc, 0, bp.dk, W.seq_start, wS0 + l32, n, bp.dk_rs, bp.dk_hs, W.h, g, bp.gscale, DQK);
+    }
+}
+
+template <class TT, int DQK, int DV, bool STORE>
+__global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(const BwdParams bp) {
+    bwd_dkdv_pp_item<TT, DQK, DV, STORE>(bp, blockIdx.x);
+}
+
+// Both gradients' items in one launch, in octets (one item per XCD) that alternate: the key-stationary items with eight waves, those of dQ with four.  For
+// few items: there a launch is the chain of its longest item (16 sequences of 100 .. 768 rows, 264 items each, fp32, dims 64 / 32: 28.7 and 27.6 us one
+// after the other, 37 together).
+template <class TT, int DQK, int DV>
+__global__ __launch_bounds__(kBwdPpWaves * 64, DQK == 128 ? 2 : DV == 128 ? 3 : 4) void hstu_bwd_both_kernel(const BwdParams bp) {
+    const int octet = blockIdx.x >> 3, item = (octet >> 1) * 8 + (blockIdx.x & 7);
+    if ((octet & 1) == 0) {
+        bwd_dkdv_pp_item<TT, DQK, DV, false>(bp, item);
+    } else if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) {
+        bwd_dq_item<TT, DQK, DV, 4, kQueryTile, DQK == 64>(bp, item);
     }
 }
 

@@ -548,3 +548,29 @@ def test_gradients_with_attn_scale(pkg, dev, per_row):
         rel = float((got - want).norm() / want.norm())
         assert rel <= 1e-2, f"{name}: relative error {rel:.3e}"
         assert float((got - want).abs().max()) <= 2e-2 * float(want.abs().max()), name
+
+
+# (dtype, dqk, dv, N, heads): the columns of q and v that decide what an item of the one launch holds, every line of its rule by N
+ONE_LAUNCH = [
+    (torch.bfloat16, 128, 128, 128, 2), (torch.float16, 64, 128, 256, 4), (torch.bfloat16, 128, 32, 700, 4), (torch.bfloat16, 128, 64, 2100, 2),
+    (torch.float16, 64, 64, 256, 4), (torch.bfloat16, 32, 32, 640, 8), (torch.bfloat16, 32, 64, 300, 3), (torch.float32, 64, 32, 520, 4), (torch.float32, 32, 128, 129, 2),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,dqk,dv,N,H", ONE_LAUNCH)
+def test_gradients_of_one_launch_are_those_of_two(dev, dtype, dqk, dv, N, H):
+    """A few sequences go through both kernels' items in one launch, with many more behind them they go through two: their gradients are the same bits (and
+    against the closed form both are checked above)."""
+    print(f"[case] one launch {dtype} {dqk}/{dv} N={N} H={H}", flush=True)
+    few = [N, 0, 1, min(N, 127), min(N, 129), 33]
+    many = few + [min(N, 130)] * (900 // H + 1)
+    q, k, v, dout, offsets = _inputs(N + dqk, many, H, dqk, dv, dtype)
+    rng = np.random.default_rng(N)
+    tg = torch.tensor([int(rng.integers(0, max(1, n - 2))) for n in many], dtype=torch.int64)
+    B, L = len(few), sum(few)
+    for mask in (dict(), dict(max_attn_len=70, contextual_seq_len=2)):
+        two = _direct(dev, N, 0.2, q, k, v, dout, offsets, dict(num_targets=tg, **mask))
+        one = _direct(dev, N, 0.2, q[:L], k[:L], v[:L], dout[:L], offsets[: B + 1], dict(num_targets=tg[:B], **mask))
+        for name, x, y in zip(("dq", "dk", "dv"), one, two):
+            assert torch.equal(x, y[:L]), (name, mask)
