@@ -338,20 +338,35 @@ int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
     return 0;
 }
 
-// path = 0: the one kernel for more rows, where u goes in as it is.  Returns its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are
+// path = 0: the one kernel for more rows, where u goes in as it is (output_panel_shape).  output_panel_form: its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are
 // this kernel's up to a width of 256 (3 x 256 into 512 columns, us: one row 7.0 -> 5.2, 256 rows 7.3 -> 5.5; 3 x 512: 7.7 against 8.2).  Past those it starts
 // at 320 rows; in front of that it would be faster as well (257 rows of 3 x 512 into 512 columns 12.2 -> 8.7), but there this path's results are the library's
 // bit for bit, which callers hold it to.
-int output_panel_form(const HstuOutputArgs* a) {
+bool output_panel_shape(const HstuOutputArgs* a) {
     const int64_t d = (int64_t)a->heads * a->linear_dim;
-    if (a->path != 0 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return -1;
-    if (a->d_out % 128 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512) return -1;
-    if (a->group_norm) {
-        const int lanes = a->linear_dim / 8;
-        if (a->linear_dim % 8 != 0 || lanes > 64 || (lanes & (lanes - 1)) != 0) return -1;
-    }
+    if (a->path != 0 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return false;
+    if (a->d_out % 128 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512) return false;
+    if (!a->group_norm) return true;
+    const int lanes = a->linear_dim / 8;
+    return a->linear_dim % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0;
+}
+
+int output_panel_form(const HstuOutputArgs* a) {
+    if (!output_panel_shape(a)) return -1;
+    const int d = a->heads * a->linear_dim;
     if (a->rows < 320) return output_takes_rows(a) && d <= 256 ? hstu::kPanel32x128 : -1;
-    return hstu::output_panel_form(a->rows, (int)d, a->d_out, a->dtype == 0);
+    return hstu::output_panel_form(a->rows, d, a->d_out, a->dtype == 0);
+}
+
+// Rows at the end of a concatenating call that the one kernel takes instead: those of the GEMM's last round of workgroups, one per CU, where they are one round
+// of the one kernel's.  (Its sums are the GEMM's, in order.)  us, without / with: 3 x 512 into 512 columns, 33000 rows (232 past a round) 109.5 / 94.2, 40960 rows 117.9 / 105.5,
+// 136226 rows 311.9 / 303.0; into 1024 columns, 36000 rows 158.0 / 149.4.  Two rounds of it cost as much as they save: 49152 rows into 512 columns 124.4 / 127.8.
+int64_t output_panel_tail(const HstuOutputArgs* a) {
+    const int64_t blocks = a->d_out / hstu::kOutWgCols, row_blocks = (a->rows + hstu::kOutRows - 1) / hstu::kOutRows;
+    if (!output_panel_shape(a) || 256 % blocks != 0) return 0;
+    const int64_t full = row_blocks * blocks / 256 * 256 / blocks;  // row blocks in full rounds
+    const int64_t tail = a->rows - full * hstu::kOutRows;
+    return full > 0 && tail > 0 && (tail + 63) / 64 * blocks <= 256 ? tail : 0;
 }
 
 int launch_output_panel(const HstuOutputArgs* a, int form, hipStream_t stream) {
@@ -905,7 +920,16 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
     if (output_takes_fused(a)) {
         if (!a->workspace) return -1;
         if ((size_t)a->workspace_bytes < output_fused_workspace(a) || ((uintptr_t)a->workspace & 255) != 0) return -4;
-        return launch_output_fused(a, stream);
+        const int64_t tail = output_panel_tail(a);
+        if (tail == 0) return launch_output_fused(a, stream);
+        HstuOutputArgs first = *a, last = *a;
+        const int64_t at = a->rows - tail;
+        first.rows = at, last.rows = tail;
+        last.attn = (const char*)a->attn + at * a->attn_row_stride * 2, last.u = (const char*)a->u + at * a->u_row_stride * 2;
+        last.x = (const char*)a->x + at * a->x_row_stride * 2, last.out = (char*)a->out + at * a->d_out * 2;
+        const int rc = launch_output_fused(&first, stream);
+        if (rc != 0) return rc;
+        return launch_output_panel(&last, hstu::output_panel_form(tail, a->heads * a->linear_dim, a->d_out, a->dtype == 0), stream);
     }
     if (!a->workspace) return -1;
     if ((size_t)a->workspace_bytes < joined_bytes(a) + kGemmScratch || ((uintptr_t)a->workspace & 255) != 0) return -4;

@@ -6,7 +6,8 @@
 // A workgroup of NW waves owns RB blocks of 32 rows and 32 NW columns.  Its waves read the rows of u and attn once (a row across D / 8 lanes) and
 // keep them in registers, y beside them; block after block of `joined` goes from there into LDS (the panel), rounded as the matrix would be, and every
 // wave multiplies it with its own 32 columns of W, whose tiles come through a private ring: barriers stand only where the panel changes.  The order of
-// all sums is that of the norm-multiply kernel and of the GEMM behind it (hstu_output_kernel.h): the results are theirs bit for bit.
+// all sums is that of the norm-multiply kernel and of the GEMM behind it (hstu_output_kernel.h): in bf16 the results are theirs bit for bit (in fp16 the
+// compiler rounds y's last product once here and twice there, or the other way round).
 //
 // Against the norm-multiply kernel and a GEMM (the library's), us on the GPU: 3 x 512 into 512 columns, 500 rows 13.1 -> 8.9, 2000 rows 19.9 -> 11.6,
 // 8192 rows 31.9 -> 20.8; 3 x 256 with group norm into 256, 14200 rows 27.1 -> 13.7; 3 x 128 into 256, 400000 rows 330 -> 161.  What bounds it (8192 rows
@@ -46,7 +47,7 @@ struct OutputPanel {
 //   width 128: to a d_out of 1152 at any rows: 400000 rows into 1024 columns 693 / 566
 //   width 256: into 512 columns at any rows (200000: 294 / 273), into 1024 16384 rows 51 / 48, 32768 rows 87 / 91; where d_out is no multiple of 256 the
 //     two kernels are slower: 60000 rows into 640 columns 167 / 108, into 1152 206 / 181
-//   width 384, 512: into 256 columns 65536 rows 95 / 90; else two rounds of the CUs (512 columns, 16384 rows 50 / 42, 24000 rows 65 / 61, 32000 rows 80 / 81;
+//   width 384, 512: two rounds of the CUs (256 columns, 32768 rows 62 / 51, 33000 rows 62 / 65; 512 columns, 16384 rows 50 / 42, 24000 rows 65 / 61, 32000 rows 80 / 81;
 //     1024 columns, 8192 rows 43 / 41, 12000 rows 57 / 61), in fp16, where the library is faster, one (512 columns, 9000 rows 34 / 38); where d_out is no multiple of 256 only
 //     the small form fits: into 384 columns 8000 rows 33 / 26, 12000 rows 38 / 38; into 640 4000 rows 32 / 25, 6000 rows 29 / 32
 enum { kPanel32x128 = 0, kPanel64x128 = 1, kPanel64x256 = 2 };
@@ -59,7 +60,7 @@ inline int output_panel_form(int64_t rows, int d, int n, bool bf16) {
         return whole ? kPanel64x256 : kPanel64x128;
     }
     if (!whole) return n <= 384 && small <= 768 ? kPanel32x128 : -1;
-    return large <= (n == 256 ? (bf16 ? 1024 : 512) : (bf16 ? 512 : 256)) ? kPanel64x256 : -1;
+    return large <= (bf16 || n == 256 ? 512 : 256) ? kPanel64x256 : -1;
 }
 
 template <class TT, bool GROUP, int D, int RB, int NW>

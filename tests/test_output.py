@@ -353,6 +353,25 @@ def test_compute_output_of_more_rows_in_one_kernel(pkg, dev, N, H, ld, D, copied
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,H,D,dtype,group_norm", [(32769, 3, 512, BF, False), (40960, 3, 512, FP, True), (40961, 3, 512, FP, True), (65600, 4, 256, BF, False), (36864, 4, 1024, BF, False)])
+def test_compute_output_past_a_round_of_the_concat_gemm(pkg, dev, N, H, D, dtype, group_norm):
+    """The rows of a last round with few workgroups go to the one kernel (one row, the last row count it takes, one more): in bf16 the bits of the GEMM; in fp16 the
+    compiler makes one rounding of y's product and its conversion in one of the two, half a unit of y, which the sum of 3 L such terms carries on."""
+    print(f"[case] output past a round {N} {H} {D} {dtype} group={group_norm}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(N)
+    L = H * 128
+    attn, u, x = (torch.randn((N, w), generator=g, device=dev).to(dtype) for w in (L, L, D))
+    nw, nb = (torch.rand(H if group_norm else L, generator=g, device=dev).to(dtype) for _ in range(2))
+    w = (torch.randn((3 * L, D), generator=g, device=dev) / 40).to(dtype)
+    args = (attn, u, x, nw, nb, 1e-6, w, H, 128, 0.0, False, True, True, "none", group_norm, False)
+    got, gemm = pkg.hstu_compute_output(*args), pkg.hstu_compute_output(*args, path=2)
+    if dtype == BF:
+        assert torch.equal(got, gemm)
+    else:  # y's error 2^-11 relative at most, of terms that add up at random; then the result's own rounding
+        assert float((got.float() - gemm.float()).norm()) <= 2**-10 * float(gemm.float().norm())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N", [33000, 257])
 def test_compute_output_concat_gemm_on_views_of_wider_buffers(pkg, dev, N):
     """u as the column slice of a [N, 4 * 512] buffer (what the producer leaves), attn as a slice of a padded one: the
