@@ -215,6 +215,7 @@ int launch_dim(const hstu::FwdParams& p, int d, int dv, int cfg, int grid_per_xc
 struct Plan {
     int cfg;               // tile configuration, 1-based
     int splits;            // workgroups per row block along kv (1 = no split)
+    bool one_each;         // a workgroup for every item there could be: no counters, no lists
     int chunk;             // kv tiles per run when split
     int fit_runs;          // runs fitted to the lengths (decode_fitted): workgroups per (head, row block), 0 = off; `splits` is then
                            // their average number per row block
@@ -322,8 +323,15 @@ Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX) {
     // Work lists for ragged batches (equal lengths are dealt arithmetically, a kv-split enumerates its runs
     // arithmetically too): 32 bytes per possible item; beyond 64 MB the arithmetic enumeration stays.
     const bool uniform = a->delta_size == 0 && a->total_kv == (int64_t)a->batch * a->max_seq_len;
+    // For few of the one-group kernel's items the list (for which the workspace still has room) costs more than it gives: the kernel that builds it takes 5 to 10 us
+    // (ranking the sequences another 10 at 256 of them), a workgroup that finds no rows leaves at once.  us, lists / a workgroup for every item there could be (4 heads of
+    // 64, ragged): 96 sequences of 20 .. 276 rows, 144 items per XCD, 24.2 / 17.6; 256 of 20 .. 128 27.2 / 17.2; 48 of 200 .. 700 31.2 / 28.6; 8 heads of 128, 20 of
+    // 300 .. 1300, 220 items 62.7 / 60.2.  More of them want the heaviest first: 64 of 200 .. 960, 4 heads of 128, 256 items 65.0 / 67.4; 100 of 300 .. 900, 400 items 81 / 86;
+    // 1024 items 190 / 203.  One row block per sequence: 1000 of 20 .. 128, 500 items, 81 / 75; 32 columns, where more than two workgroups fit a CU: 100 of 300 .. 900 53 / 48.
+    const long long num_mb = (rows_per_pair + bm - 1) / bm, slots = (a->batch * (long long)a->heads + 7) / 8 * num_mb;
+    pl.one_each = s == 1 && !uniform && pl.cfg == 3 && a->delta_size == 0 && slots <= (num_mb == 1 || a->dqk == 32 ? 512 : num_mb <= 4 ? 256 : 224);
     if (s == 1 && !uniform) {
-        const unsigned long long bytes = (unsigned long long)((a->batch * (long long)a->heads + 7) / 8) * (unsigned long long)((rows_per_pair + bm - 1) / bm) * 256ull;
+        const unsigned long long bytes = (unsigned long long)slots * 256ull;
         if (bytes <= (64ull << 20)) pl.items_bytes = (size_t)bytes + 32;  // 32: room to align the records
     }
     if (s > 1) {
@@ -660,6 +668,12 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
     fast_div_constants((unsigned)p.H, &p.h_magic, &p.h_shift);
     long long resident = (long long)current_device_cus() * (cfg == 2 ? 1 : 2) / 8;
     if (resident < 1) resident = 1;
+    if (plan.one_each) {
+        resident = slots;
+        // long sequences first only where there can be long ones, which repays the launch that ranks them (4 heads of 128, one in four of 32 sequences 1500 rows, the
+        // others 100: 65 us unranked, 45 ranked; 60 sequences of 100 .. 512, 8 heads 48 and 56)
+        if (p.num_mb <= 4) order = nullptr;
+    }
     const int grid_per_xcd = (int)(slots < resident ? slots : resident);
     if (cfg < 2 || slots <= grid_per_xcd) queue = nullptr;  // every workgroup has exactly one item
     int* items = nullptr;

@@ -28,3 +28,28 @@ def test_ranked_lists(pkg, dev, batch, heads, longest, i64):
     torch.cuda.synchronize()
     assert torch.equal(ranked, plain)
     assert_parity(ranked, O.hstu_mha_per_sequence(longest, 0.125, q.float(), k.float(), v.float(), offs.long(), num_targets=t.long()), "ranked lists")
+
+
+# (batch, heads, longest, columns): a workgroup for every item there could be, with one row block per sequence, up to four (unranked) and more (ranked); on the other
+# side of each line the lists, around the number of sequences that their kernel ranks itself; 32 columns have a line of their own
+@pytest.mark.parametrize("batch,heads,longest,d", [
+    (512, 8, 128, 64), (513, 8, 128, 64), (64, 8, 512, 128), (65, 8, 512, 64), (28, 8, 1000, 64), (29, 8, 1000, 64), (64, 8, 1000, 32), (65, 8, 1000, 32),
+    (255, 4, 384, 64), (256, 4, 384, 64), (257, 4, 384, 64)])
+def test_items_with_and_without_lists(pkg, dev, batch, heads, longest, d):
+    print(f"[case] items {batch} x {heads} heads up to {longest}, {d} columns", flush=True)
+    gen = torch.Generator().manual_seed(batch + longest)
+    lengths = torch.randint(0, longest + 1, (batch,), generator=gen).tolist()
+    lengths[0], lengths[1], lengths[-1] = longest, 0, longest
+    q, k, v, offs, t = make_case(batch, lengths, heads, d, targets=[min(3, n) for n in lengths])
+    args = [longest, 0.125] + [x.to(dev) for x in (q, k, v, offs)]
+    ranked = pkg.hstu_mha(*args, num_targets=t.to(dev), sort_by_length=True)
+    plain = pkg.hstu_mha(*args, num_targets=t.to(dev))
+    torch.cuda.synchronize()
+    assert torch.equal(ranked, plain)
+    some = [0, 1, 2, batch // 2, batch - 2, batch - 1]  # (the reference on the host takes the time)
+    for b in some:
+        lo, hi = int(offs[b]), int(offs[b + 1])
+        if hi == lo:
+            continue
+        one = O.hstu_mha_per_sequence(longest, 0.125, q[lo:hi].float(), k[lo:hi].float(), v[lo:hi].float(), torch.tensor([0, hi - lo]), num_targets=t[b : b + 1].long())
+        assert_parity(plain[lo:hi], one, f"items of sequence {b}")
