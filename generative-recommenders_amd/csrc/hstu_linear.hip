@@ -8,7 +8,6 @@
 
 #include <atomic>
 #include <cstdio>
-#include <cstdlib>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -19,6 +18,7 @@
 #include "hstu_output_kernel.h"
 #include "hstu_output_rows_kernel.h"
 #include "hstu_output_panel_kernel.h"
+#include "hstu_output_wide_kernel.h"
 
 // hstu_uqvk.hip, hstu_uqvk_bwd.hip
 int hstu_uqvk_launch(const hstu::UqvkFusedParams& p, int d_model, bool bf16, hipStream_t stream);
@@ -27,6 +27,7 @@ bool hstu_product_t_takes(int64_t rows, int depth, int n);
 int hstu_product_t_launch(const hstu::UqvkFusedParams& p, int depth, bool bf16, hipStream_t stream);
 
 int hstu_output_panel_launch(const hstu::OutputPanelParams& p, int form, bool bf16, bool group, hipStream_t stream);
+int hstu_output_wide_launch(const hstu::OutputPanelParams& p, bool bf16, bool group, hipStream_t stream);
 
 namespace {
 
@@ -338,14 +339,14 @@ int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
     return 0;
 }
 
-// path = 0: the one kernel for more rows, where u goes in as it is (output_panel_shape).  output_panel_form: its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are
+// path = 0: the panel kernel, one kernel for more rows, where u goes in as it is (output_panel_shape).  output_panel_form: its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are
 // this kernel's up to a width of 256 (3 x 256 into 512 columns, us: one row 7.0 -> 5.2, 256 rows 7.3 -> 5.5; 3 x 512: 7.7 against 8.2).  Past those it starts
 // at 320 rows; in front of that it would be faster as well (257 rows of 3 x 512 into 512 columns 12.2 -> 8.7), but there this path's results are the library's
 // bit for bit, which callers hold it to.
-bool output_panel_shape(const HstuOutputArgs* a) {
+bool output_panel_shape(const HstuOutputArgs* a, int most_d = 512, int path = 0) {
     const int64_t d = (int64_t)a->heads * a->linear_dim;
-    if (a->path != 0 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return false;
-    if (a->d_out % 128 != 0 || a->d_out > 8192 || d % 128 != 0 || d > 512) return false;
+    if ((a->path != 0 && a->path != path) || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return false;
+    if (a->d_out % 128 != 0 || a->d_out > 8192 || d % 128 != 0 || d > most_d) return false;
     if (!a->group_norm) return true;
     const int lanes = a->linear_dim / 8;
     return a->linear_dim % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0;
@@ -359,14 +360,57 @@ int output_panel_form(const HstuOutputArgs* a) {
 }
 
 // Rows at the end of a concatenating call that the one kernel takes instead: those of the GEMM's last round of workgroups, one per CU, where they are one round
-// of the one kernel's.  (Its sums are the GEMM's, in order.)  us, without / with: 3 x 512 into 512 columns, 33000 rows (232 past a round) 109.5 / 94.2, 40960 rows 117.9 / 105.5,
-// 136226 rows 311.9 / 303.0; into 1024 columns, 36000 rows 158.0 / 149.4.  Two rounds of it cost as much as they save: 49152 rows into 512 columns 124.4 / 127.8.
+// of the one kernel's.  (Its sums are the GEMM's, in order.)  us, without / with: 3 x 512 into 256 columns, 66000 rows (464 past a round) 131 / 111,
+// 73728 rows 138 / 117; 2 x 512 into 512, 33000 rows 83 / 74, 40960 rows 93 / 83.  Two rounds of it cost as much as they save.
 int64_t output_panel_tail(const HstuOutputArgs* a) {
     const int64_t blocks = a->d_out / hstu::kOutWgCols, row_blocks = (a->rows + hstu::kOutRows - 1) / hstu::kOutRows;
     if (!output_panel_shape(a) || 256 % blocks != 0) return 0;
     const int64_t full = row_blocks * blocks / 256 * 256 / blocks;  // row blocks in full rounds
     const int64_t tail = a->rows - full * hstu::kOutRows;
     return full > 0 && tail > 0 && (tail + 63) / 64 * blocks <= 256 ? tail : 0;
+}
+
+// path = 0 and 2: the one kernel whose workgroups own 128 rows and 512 columns, for all three blocks.  It takes calls that give more than half of the CUs an item -- up to there its time is
+// that of one item and the kernels above are faster: us, without / with it: 3 x 512 into 512 columns, 14000 rows (110 items) 38 / 39, 16500 50 / 39, 32768 77 / 61, 57819 133 / 106,
+// 136226 295 / 240; into 1024, 8192 rows 40 / 42, 9000 56 / 42, 57819 216 / 203; 3 x 256 into 512, 16384 rows 23.2 / 24.1, 17000 30.6 / 24.3, 136226 183 / 147; 3 x 384, 14000 rows
+// 31 / 34, 17000 41 / 35, 57819 112 / 89.  Where the panel kernel takes less (fp16, rows of 1024) from 100 items on: 3 x 512, fp16, 12000 rows 37 / 39, 14000 42 / 38; 3 x 1024, 10000
+// rows 61 / 65 (fp16), 14000 85 / 69 (both types), 57819 236 / 187.
+bool output_wide_shape(const HstuOutputArgs* a) {
+    const int d = a->heads * a->linear_dim;
+    if (!output_panel_shape(a, 1024, 2) || a->d_out % hstu::kOutWideCols != 0 || (d != 256 && d != 384 && d != 512 && d != 1024)) return false;
+    if (output_blocks(a) != 3 || (a->group_norm && a->heads > hstu::kOutWideHeads)) return false;
+    return a->attn_row_stride < (1 << 22) && a->u_row_stride < (1 << 22);  // 32-bit byte offsets within an item
+}
+bool output_takes_wide(const HstuOutputArgs* a) {
+    if (!output_wide_shape(a)) return false;
+    const int64_t items = (a->rows + hstu::kOutWideRows - 1) / hstu::kOutWideRows * (a->d_out / hstu::kOutWideCols);
+    const int d = a->heads * a->linear_dim;
+    return items > 128 || (items > 100 && (d > 512 || hstu::output_panel_form(a->rows, d, a->d_out, a->dtype == 0) < 0));
+}
+
+// Rows at the end of its last round, one item per CU, that the panel kernel takes instead: those that are one round of that kernel's (us, without / with: 3 x 512 into 512 columns, 33000
+// rows (232 past a round) 91 / 73, 40960 93 / 82, 136226 252 / 240; 45000, one and a half of the panel kernel's rounds, 95 / 98; into 1024, 20000 rows 88 / 77).
+int64_t output_wide_tail(const HstuOutputArgs* a) {
+    const int blocks = a->d_out / hstu::kOutWideCols;
+    if (!output_panel_shape(a, 512, 2) || 256 % blocks != 0) return 0;
+    const int64_t tail = a->rows % (256 / blocks * hstu::kOutWideRows);
+    return tail < a->rows && tail * blocks <= 8192 ? tail : 0;
+}
+
+int launch_output_wide(const HstuOutputArgs* a, hipStream_t stream) {
+    hstu::OutputPanelParams p;
+    const int rc = hstu::norm_mul_params(a, nullptr, (int64_t)output_blocks(a) * a->heads * a->linear_dim, false, p.nm);
+    if (rc != 0) return rc;
+    p.x = (const char*)a->x, p.x_rs = a->x_row_stride, p.w = (const char*)a->output_weight, p.out = (char*)a->out, p.n = a->d_out;
+    return hstu_output_wide_launch(p, a->dtype == 0, a->group_norm != 0, stream);
+}
+
+// A call's first `at` rows and the others.
+void output_split(const HstuOutputArgs* a, int64_t at, HstuOutputArgs& first, HstuOutputArgs& last) {
+    first = last = *a;
+    first.rows = at, last.rows = a->rows - at;
+    last.attn = (const char*)a->attn + at * a->attn_row_stride * 2, last.u = (const char*)a->u + at * a->u_row_stride * 2;
+    last.x = (const char*)a->x + at * a->x_row_stride * 2, last.out = (char*)a->out + at * a->d_out * 2;
 }
 
 int launch_output_panel(const HstuOutputArgs* a, int form, hipStream_t stream) {
@@ -862,7 +906,7 @@ int hstu_linear_product_t(const void* a, int64_t a_row_stride, const void* weigh
 
 size_t hstu_output_workspace_bytes(const HstuOutputArgs* a) {
     if (!a || a->rows <= 0 || a->heads <= 0 || a->linear_dim <= 0) return 0;
-    if (output_takes_rows(a) || output_panel_form(a) >= 0) return 0;
+    if (output_takes_wide(a) || output_takes_rows(a) || output_panel_form(a) >= 0) return 0;
     if (output_takes_fused(a)) return output_fused_shape(a) ? output_fused_workspace(a) : 0;
     return joined_bytes(a) + kGemmScratch;
 }
@@ -912,6 +956,15 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
                  "elements: dropout runs on the library path (path 0 or 1)");
         return -6;
     }
+    if (output_takes_wide(a)) {
+        const int64_t tail = output_wide_tail(a);
+        if (tail == 0) return launch_output_wide(a, stream);
+        HstuOutputArgs first, last;
+        output_split(a, a->rows - tail, first, last);
+        const int rc = launch_output_wide(&first, stream);
+        if (rc != 0) return rc;
+        return launch_output_panel(&last, hstu::output_panel_form(tail, a->heads * a->linear_dim, a->d_out, a->dtype == 0), stream);
+    }
     if (const int form = output_panel_form(a); form >= 0) return launch_output_panel(a, form, stream);
     if (output_takes_rows(a)) {
         if (a->dtype == 0) return a->group_norm ? launch_output_rows<hstu::Bf16, true>(a, stream) : launch_output_rows<hstu::Bf16, false>(a, stream);
@@ -922,11 +975,8 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
         if ((size_t)a->workspace_bytes < output_fused_workspace(a) || ((uintptr_t)a->workspace & 255) != 0) return -4;
         const int64_t tail = output_panel_tail(a);
         if (tail == 0) return launch_output_fused(a, stream);
-        HstuOutputArgs first = *a, last = *a;
-        const int64_t at = a->rows - tail;
-        first.rows = at, last.rows = tail;
-        last.attn = (const char*)a->attn + at * a->attn_row_stride * 2, last.u = (const char*)a->u + at * a->u_row_stride * 2;
-        last.x = (const char*)a->x + at * a->x_row_stride * 2, last.out = (char*)a->out + at * a->d_out * 2;
+        HstuOutputArgs first, last;
+        output_split(a, a->rows - tail, first, last);
         const int rc = launch_output_fused(&first, stream);
         if (rc != 0) return rc;
         return launch_output_panel(&last, hstu::output_panel_form(tail, a->heads * a->linear_dim, a->d_out, a->dtype == 0), stream);

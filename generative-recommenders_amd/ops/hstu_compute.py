@@ -7,7 +7,7 @@ with the bias and, for the u columns, the SiLU in its epilogue.  ``u, q, k, v`` 
 ``[L, (2*hidden + 2*attn) * H]`` buffer, which ``hstu_mha`` / ``delta_hstu_mha`` read in place.
 
 ``hstu_compute_output``: ``x + [u | attn | act(u) * norm(attn)] @ output_weight``.  For few rows, and for more where u is not
-activated and the widths suit, one kernel does it all (``csrc/hstu_output_rows_kernel.h``, ``csrc/hstu_output_panel_kernel.h``).  From 32768 rows on a
+activated and the widths suit, one kernel does it all (``csrc/hstu_output_rows_kernel.h``, ``csrc/hstu_output_panel_kernel.h``, ``csrc/hstu_output_wide_kernel.h``).  Else from 32768 rows on a
 hand-written GEMM reads u and attn where they are and ``act(u) * norm(attn)`` from a row-wise kernel; otherwise, and with dropout, that kernel writes the concatenated operand and hipBLASLt multiplies it with the residual as its C operand.
 (``csrc/hstu_linear.hip``, ``csrc/hstu_output_kernel.h``, ``include/hstu_linear.h``.)
 
@@ -557,7 +557,7 @@ def hstu_compute_output(
     writes ``joined`` and hipBLASLt multiplies it; 2 = the norm-mul kernel writes ``y`` alone and a hand-written GEMM
     reads ``u`` and ``attn`` where they are (``NotImplementedError`` if the shape does not fit: d_model a multiple of 256,
     heads * linear_dim a multiple of 64 -- or with dropout, whose mask covers the copied blocks too); 0 = whichever is
-    faster for the shape (2 where it fits, rows >= 32768 and nothing is dropped).  Dropout as in ``norm_mul_dropout``."""
+    faster for the shape (one kernel for the whole step; 2 where that does not take it, 2 fits, rows >= 32768 and nothing is dropped).  Dropout as in ``norm_mul_dropout``."""
     state = None
     if training and dropout_ratio > 0.0:
         _check_output(attn, u, x, norm_weight, norm_bias, output_weight, mul_u_activation_type)  # before the generator moves on

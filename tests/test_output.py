@@ -306,14 +306,18 @@ def test_compute_output_on_both_sides_of_one_round(pkg, dev, N, blocks, H, ld, D
 
 # (rows, heads, linear_dim, d_out, copied blocks, group norm, dtype, whether the one kernel for more rows takes it): its first row count, both sides of the
 # line between its forms of 32 x 128 and 64 x 256 (64 x 128 where d_out is no multiple of 256), rows that fill no block, every width of a row (384: lanes
-# without a chunk), one to three blocks, heads of one and of all lanes of a row, and the sizes behind the last one it takes
+# without a chunk), one to three blocks, heads of one and of all lanes of a row, and the sizes behind the last one it takes; in the last lines the form of
+# 128 x 512, from its first size on (128 or 100 items), with one row in its last block, a second round, a last round that goes to the others, and too many heads for it
 BF, FP = torch.bfloat16, torch.float16
 PANEL_CASES = [
     (319, 4, 128, 512, 2, False, BF, False), (320, 4, 128, 512, 2, False, BF, True), (353, 16, 32, 128, 2, True, FP, True), (4096, 4, 128, 512, 2, False, FP, True),
     (4097, 4, 128, 512, 2, False, FP, True), (8192, 8, 64, 512, 2, True, BF, True), (8193, 4, 128, 512, 2, False, FP, False),
-    (16385, 4, 128, 512, 2, False, BF, False), (1000, 3, 128, 384, 2, True, BF, True), (9000, 3, 128, 384, 2, False, FP, False), (5000, 3, 128, 768, 2, False, BF, True),
+    (1000, 3, 128, 384, 2, True, BF, True), (9000, 3, 128, 384, 2, False, FP, False), (5000, 3, 128, 768, 2, False, BF, True),
     (8200, 8, 32, 256, 2, True, FP, True), (5600, 2, 128, 384, 2, False, BF, True), (20000, 1, 128, 640, 1, False, FP, True), (16385, 1, 128, 256, 0, True, BF, True),
     (777, 4, 128, 1024, 0, False, FP, True), (2049, 2, 64, 512, 1, False, BF, True), (40000, 1, 128, 256, 2, False, BF, True), (600, 32, 8, 256, 2, True, FP, True),
+    (16385, 4, 128, 512, 2, False, BF, True), (16513, 8, 32, 512, 2, True, FP, True), (16600, 3, 128, 512, 2, False, FP, True), (12800, 4, 128, 512, 2, False, FP, False),
+    (12801, 4, 128, 512, 2, True, FP, True), (6400, 8, 128, 1024, 2, False, BF, False), (6401, 8, 128, 1024, 2, True, BF, True), (45000, 2, 128, 512, 2, False, BF, True),
+    (33001, 4, 128, 512, 2, True, BF, True), (20000, 16, 32, 512, 2, True, BF, False), (16385, 4, 128, 512, 1, False, BF, False),
 ]
 
 
@@ -353,7 +357,7 @@ def test_compute_output_of_more_rows_in_one_kernel(pkg, dev, N, H, ld, D, copied
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,H,D,dtype,group_norm", [(32769, 3, 512, BF, False), (40960, 3, 512, FP, True), (40961, 3, 512, FP, True), (65600, 4, 256, BF, False), (36864, 4, 1024, BF, False)])
+@pytest.mark.parametrize("N,H,D,dtype,group_norm", [(65537, 3, 256, BF, False), (81920, 3, 256, FP, True), (81921, 3, 256, FP, True), (65600, 4, 256, BF, False)])
 def test_compute_output_past_a_round_of_the_concat_gemm(pkg, dev, N, H, D, dtype, group_norm):
     """The rows of a last round with few workgroups go to the one kernel (one row, the last row count it takes, one more): in bf16 the bits of the GEMM; in fp16 the
     compiler makes one rounding of y's product and its conversion in one of the two, half a unit of y, which the sum of 3 L such terms carries on."""
