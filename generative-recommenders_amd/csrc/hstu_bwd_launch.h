@@ -92,9 +92,18 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
         // 100 .. 600, 4 heads, 420 items, 80 / 73; not the short (256 of 20 .. 250, 1 head, 384 items 54 / 64; 128 of 24 .. 60, 4 heads 31 / 35) nor the long (4 of
         // 1000 .. 4000, 344 items 238 / 275).  Up to 64 columns two or three fit: 2 of 3000 .. 6000, 8 heads, 64 / 64, 632 items 318 / 278, 128 of 20 .. 250, 780
         // items 52 / 57; 256 of 20 .. 250, 1 head, 32 / 32, 384 items 26 / 28.
+        // Long ones with 128 columns pay while both halves have a CU per item (forward and backward: 5 of 2100 .. 4200, 1 head, 112 items 329 / 249; 1 of 5700, 4 heads, 176
+        // items 468 / 438; 4 of 1600 .. 6400, 2 heads, 206 items 446 / 455).  Contextual rows make dQ's first block of a sequence the longest chain by far, and behind an item
+        // of the other kind it is longer still: 4 of 1600 .. 6400, 2 heads 598 / 745, 112 items 403 / 464; 8 of 1000 .. 1200, 304 items 168 / 183; but 8 of 300 .. 1500, 122 items
+        // 149 / 128 and 16 of 100 .. 768, 240 items 100 / 81.
         const int64_t upper = (int64_t)bp.f.H * (bp.total_q / kBwdRows + bp.f.B);  // items at most, as the grid
         const int64_t items = upper < (int64_t)grid ? upper : (int64_t)grid, len = bp.f.max_seq_len;
-        const int64_t most = DQK <= 64 && DV <= 64 ? (len <= 256 ? 384 : 768) : len <= 128 ? 128 : len <= 256 ? 256 : len <= 2048 ? 512 : 256;
+        const bool ctx = bp.f.c > 0;
+        const int64_t most = DQK <= 64 && DV <= 64 ? (len <= 256 ? 384 : 768)
+                             : len <= 128          ? 128
+                             : len <= 256          ? 256
+                             : len <= 2048         ? (ctx && len > 768 ? 256 : 512)
+                                                   : (ctx ? 0 : 192);
         if (!bp.ds && paired && items <= most) {
             hipLaunchKernelGGL(k12, dim3(grid * 2), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
             const hipError_t e = hipGetLastError();
