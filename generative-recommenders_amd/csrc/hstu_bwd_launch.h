@@ -34,7 +34,7 @@ auto key_stationary_kernel(std::false_type) {
 
 template <class TT, int DQK, int DV>
 auto both_kernel(std::true_type) {
-    return hstu::hstu_bwd_both_kernel<TT, DQK, DV>;
+    return hstu::hstu_bwd_dkdv_pp_kernel<TT, DQK, DV, false, true>;
 }
 template <class TT, int DQK, int DV>
 auto both_kernel(std::false_type) {

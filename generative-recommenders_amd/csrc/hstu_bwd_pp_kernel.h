@@ -30,8 +30,12 @@ constexpr int bwd_pp_lds_bytes() {
     return 3 * kQueryTile * (DQK + DV) * 2 + 2 * 4 * 2048;
 }
 
-template <class TT, int DQK, int DV, bool STORE>
-__device__ __forceinline__ void bwd_dkdv_pp_item(const BwdParams& bp, int bid) {
+// BOTH: both gradients' items in one launch, in octets (one item per XCD) that alternate: the key-stationary items with eight waves, those of dQ with four.
+// For few items: there a launch is the chain of its longest item (16 sequences of 100 .. 768 rows, 264 items each, fp32, dims 64 / 32: 28.7 and 27.6 us one
+// after the other, 37 together).  (The body is a kernel's and not a function's that two kernels call: as such it held 8 more scalars in vector registers and
+// was 2 to 3 % slower with 32 columns and stored dS.)
+template <class TT, int DQK, int DV, bool STORE, bool BOTH = false>
+__global__ __launch_bounds__(kBwdPpWaves * 64, !BOTH ? 1 : DQK == 128 ? 2 : DV == 128 ? 3 : 4) void hstu_bwd_dkdv_pp_kernel(const BwdParams bp) {
     typedef typename TT::vec8 vec8;
     static_assert(DQK >= 32 && DV >= 32 && DQK % 32 == 0 && DV % 32 == 0, "a tile copy is at least one instruction per copying wave");
     const FwdParams& p = bp.f;
@@ -51,7 +55,16 @@ __device__ __forceinline__ void bwd_dkdv_pp_item(const BwdParams& bp, int bid) {
     const int g = lane >> 5, l32 = lane & 31;
 
     Work W;
-    if (!bwd_decode<BM>(p, W, bid, true)) return;
+    if constexpr (BOTH) {
+        const int octet = blockIdx.x >> 3, item = (octet >> 1) * 8 + (blockIdx.x & 7);
+        if (octet & 1) {
+            if (wave < 4) bwd_dq_item<TT, DQK, DV, 4, kQueryTile, DQK == 64>(bp, item);
+            return;
+        }
+        if (!bwd_decode<BM>(p, W, item, true)) return;
+    } else {
+        if (!bwd_decode<BM>(p, W, blockIdx.x, true)) return;
+    }
     const SeqMask& M = W.M;
     const int n = W.n;
     const int S0 = W.R0;           // first key row of the workgroup
@@ -392,24 +405,6 @@ __device__ __forceinline__ void bwd_dkdv_pp_item(const BwdParams& bp, int bid) {
             run(tile, drain);
         }
         store_output<TT, DTK>(dkacc, 0, bp.dk, W.seq_start, wS0 + l32, n, bp.dk_rs, bp.dk_hs, W.h, g, bp.gscale, DQK);
-    }
-}
-
-template <class TT, int DQK, int DV, bool STORE>
-__global__ __launch_bounds__(kBwdPpWaves * 64, 1) void hstu_bwd_dkdv_pp_kernel(const BwdParams bp) {
-    bwd_dkdv_pp_item<TT, DQK, DV, STORE>(bp, blockIdx.x);
-}
-
-// Both gradients' items in one launch, in octets (one item per XCD) that alternate: the key-stationary items with eight waves, those of dQ with four.  For
-// few items: there a launch is the chain of its longest item (16 sequences of 100 .. 768 rows, 264 items each, fp32, dims 64 / 32: 28.7 and 27.6 us one
-// after the other, 37 together).
-template <class TT, int DQK, int DV>
-__global__ __launch_bounds__(kBwdPpWaves * 64, DQK == 128 ? 2 : DV == 128 ? 3 : 4) void hstu_bwd_both_kernel(const BwdParams bp) {
-    const int octet = blockIdx.x >> 3, item = (octet >> 1) * 8 + (blockIdx.x & 7);
-    if ((octet & 1) == 0) {
-        bwd_dkdv_pp_item<TT, DQK, DV, false>(bp, item);
-    } else if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 4) {
-        bwd_dq_item<TT, DQK, DV, 4, kQueryTile, DQK == 64>(bp, item);
     }
 }
 
