@@ -219,6 +219,7 @@ struct Plan {
     int chunk;             // kv tiles per run when split
     int fit_runs;          // runs fitted to the lengths (decode_fitted): workgroups per (head, row block), 0 = off; `splits` is then
                            // their average number per row block
+    int line_weight;       // > 0: those workgroups share the plane's tiles as one line instead (decode_line)
     // the workspace, in this order:
     size_t queue_bytes;    // work-item counters and list lengths of the persistent kernels
     size_t order_bytes;    // sequence ranking
@@ -243,8 +244,8 @@ bool rows_fit_buffer_offsets(const HstuFwdArgs* a) {
     return (int64_t)a->max_seq_len * rs * es < (1LL << 32);
 }
 
-// `scratch`: bytes of workspace at hand; an automatic kv-split is one that fits.
-Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX) {
+// `scratch`: bytes of workspace at hand; an automatic kv-split is one that fits.  `line`: whether a plane's tiles may be cut as one line.
+Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX, bool line = true) {
     Plan pl{};
     pl.splits = 1;
     // The streaming two-group kernel (256-row blocks, one workgroup per CU) wins when the average sequence is long;
@@ -298,27 +299,42 @@ Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX) {
         // (30 x 7300 .. 14600 x 91: 173 and 150).  Short runs still pay: 50 candidates x 400 rows, 16.7 us unsplit, 12.4 us in
         // runs of one tile.  Below 6 tiles saved the extra kernel and the partial sums cost more than the shorter runs save;
         // with fewer than four workgroups per sequence there is little to fit (32 x 1024 .. 4096 x 256: 76 us, equal counts 73).
-        if (a->max_attn_len == 0 && a->contextual_seq_len == 0 && a->batch <= 64 && max_tiles <= (1 << 20)) {
-            const long long chip = pl.cfg == 2 ? 256 : blocks * 4 <= 256 ? 256 : 512;
-            const long long num_mb = (rows_per_pair + bm - 1) / bm, planes = a->heads * num_mb;
-            const long long tiles = a->total_kv / kTileRows + a->batch;  // of a plane, at most
-            long long runs = chip / 8 / num_mb * 8 / a->heads;
-            if (runs > tiles) runs = tiles;
-            if (runs >= 4 * a->batch && max_tiles - (tiles + runs - 1) / runs >= 6) {
-                pl.fit_runs = (int)runs;
-                pl.splits = (int)(runs / a->batch);
-                pl.counts_bytes = split_counts_bytes;
-                pl.partial_bytes = (size_t)planes * runs * (rows_per_pair < bm ? rows_per_pair : bm) * a->dv * sizeof(float);
-                if (pl.total() <= scratch) return pl;
-                pl.fit_runs = 0, pl.splits = 1;  // their partial sums take more than those of equal counts can
-                pl.counts_bytes = pl.partial_bytes = 0;
-            }
+        const bool fits = a->max_attn_len == 0 && a->contextual_seq_len == 0 && a->batch <= 64 && max_tiles <= (1 << 20);
+        const long long chip = pl.cfg == 2 ? 256 : blocks * 4 <= 256 ? 256 : 512;
+        const long long num_mb = (rows_per_pair + bm - 1) / bm, planes = a->heads * num_mb;
+        const long long tiles = a->total_kv / kTileRows + a->batch;  // of a plane, at most
+        const size_t run_bytes = (size_t)planes * (rows_per_pair < bm ? rows_per_pair : bm) * a->dv * sizeof(float);
+        long long runs = chip / 8 / num_mb * 8 / a->heads;
+        if (runs > tiles) runs = tiles;
+        if (fits && runs >= 4 * a->batch && max_tiles - (tiles + runs - 1) / runs >= 6) {
+            pl.fit_runs = (int)runs;
+            pl.splits = (int)(runs / a->batch);
+            pl.counts_bytes = split_counts_bytes;
+            pl.partial_bytes = runs * run_bytes;
+            if (pl.total() <= scratch) return pl;
+            pl.fit_runs = 0, pl.splits = 1;  // their partial sums take more than those of equal counts can
+            pl.counts_bytes = pl.partial_bytes = 0;
         }
         long long want = resident / blocks;
         if (want > max_tiles / 16) want = max_tiles / 16;
         if (want > kMaxSplits) want = kMaxSplits;
         while (want >= 2 && pl.total() + split_counts_bytes + want * split_bytes + 256 > scratch) --want;
         if (want >= 2) s = (int)want;
+        // Fewer workgroups than that per sequence: the plane's tiles as one line (decode_line), where the longest run is at least 8 tiles longer than a workgroup's part of
+        // it.  us without / with (bf16, lengths of the histories x candidates): 34 of 2400 .. 2550 x 19, 8 heads of 32 67 / 45; 18 of 250 .. 4200 x 3, 8 of 128 57 / 35; 46 of 400 .. 1600 x 3,
+        // 4 of 128 40 / 28; 39 of 650 .. 10800 x 212, 4 of 128 243 / 157; 16 of 500 .. 8000 x 512 105 / 89; 32 of 1024 .. 4096 x 256 74 / 74.  Not for shorter ones (36 of 550 x 278 38 / 52; 40 of
+        // 100 .. 400 x 30 16 / 21) nor for many row blocks (46 of 4500 .. 9000 x 389, 8 heads 798 / 877; 64 of 500 .. 4000 x 500 214 / 221).  What an item costs besides its steps, in tiles (2, 5, 9: the
+        // first 45 / 47 / 50, the last but one of the gains 91 / 89 / 87):
+        const int weight = pl.cfg == 2 ? 8 : 4;
+        if (line && fits && runs > 0 && (max_tiles + s - 1) / s - (tiles + a->batch * weight + runs - 1) / runs >= 8 &&
+            (tiles + a->batch * weight) * runs < (1ll << 31)) {
+            pl.fit_runs = (int)runs, pl.line_weight = weight, pl.splits = 2;
+            pl.counts_bytes = split_counts_bytes;
+            pl.partial_bytes = (runs + a->batch) * run_bytes;
+            if (pl.total() <= scratch) return pl;
+            pl.fit_runs = pl.line_weight = 0, pl.splits = 1;
+            pl.counts_bytes = pl.partial_bytes = 0;
+        }
     }
     // Work lists for ragged batches (equal lengths are dealt arithmetically, a kv-split enumerates its runs
     // arithmetically too): 32 bytes per possible item; beyond 64 MB the arithmetic enumeration stays.
@@ -382,6 +398,8 @@ void fill_decode_params(hstu::FwdParams& p) {
     d.w = p.w;
     d.f = p.f;
     d.fit_runs = p.fit_runs;
+    d.line_weight = p.line_weight;
+    d.line_wgs = p.line_wgs;
     d.mb_magic = p.mb_magic;
     d.mb_shift = p.mb_shift;
     d.h_magic = p.h_magic;
@@ -646,7 +664,10 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
         p.partial = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(base + plan.counts_bytes) + 255) & ~(uintptr_t)255);
         p.partial_stride = (int64_t)a->total_q * a->heads * a->dv;
         p.kv_chunk = plan.chunk;
-        if (plan.fit_runs > 0) p.fit_runs = plan.fit_runs, plan.splits = 1;  // (an item is one run: decode_fitted)
+        if (plan.fit_runs > 0) {
+            p.fit_runs = plan.fit_runs, plan.splits = 1;  // (an item is one run: decode_fitted, decode_line)
+            p.line_weight = plan.line_weight, p.fit_slots = plan.fit_runs + (plan.line_weight > 0 ? a->batch : 0);
+        }
     }
     p.kv_splits = plan.splits;
 
@@ -658,7 +679,9 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
     const int bm = cfg == 2 ? 256 : 128;
     p.num_mb = (rows_per_pair + bm - 1) / bm;
     const long long pairs_per_xcd = (num_pairs + 7) / 8;
-    const long long slots = p.fit_runs > 0 ? (((long long)p.fit_runs * a->heads + 7) / 8) * p.num_mb : pairs_per_xcd * p.num_mb * plan.splits;
+    const long long wgs = (((long long)p.fit_runs * a->heads + 7) / 8) * p.num_mb;  // per XCD, of fitted runs
+    const long long slots = p.fit_runs > 0 ? wgs * (p.line_weight > 0 ? a->batch : 1) : pairs_per_xcd * p.num_mb * plan.splits;
+    p.line_wgs = (int)wgs;
     p.fit_rows = rows_per_pair < bm ? rows_per_pair : bm;
     if (slots <= 0) return HSTU_OK;
     if (slots * 8 > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
@@ -674,8 +697,9 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
         // others 100: 65 us unranked, 45 ranked; 60 sequences of 100 .. 512, 8 heads 48 and 56)
         if (p.num_mb <= 4) order = nullptr;
     }
+    if (p.line_weight > 0) resident = wgs;
     const int grid_per_xcd = (int)(slots < resident ? slots : resident);
-    if (cfg < 2 || slots <= grid_per_xcd) queue = nullptr;  // every workgroup has exactly one item
+    if (cfg < 2 || slots <= grid_per_xcd || p.line_weight > 0) queue = nullptr;  // every workgroup has exactly one item (or its part of a line)
     int* items = nullptr;
     if (queue && plan.items_bytes > 0 && ws_bytes >= plan.total()) items = (int*)(ws + plan.total() - plan.cast_bytes - plan.items_bytes);
     // Equal-length sequences (every one as long as max_seq_len allows): dealing the items with a fixed stride is
@@ -769,7 +793,7 @@ int hstu_hip_mha_fwd_noalloc(const HstuFwdArgs* a, void* stream_) {
     if (rc != HSTU_OK) return rc;
     if (a->total_q == 0 || a->batch == 0) return HSTU_OK;
     if (!current_device_is_gfx950()) return HSTU_ERR_BAD_DEVICE;
-    const size_t need = make_plan(a).total();
+    const size_t need = make_plan(a, SIZE_MAX, false).total();  // (a line's partial sums may take more: it is cut where they fit)
     if (need > (size_t)HSTU_NOALLOC_SCRATCH_BYTES) {
         snprintf(g_last_error, sizeof(g_last_error), "this call would use %zu bytes of scratch memory; the fixed area holds %zu", need,
                  (size_t)HSTU_NOALLOC_SCRATCH_BYTES);

@@ -62,7 +62,7 @@ struct DecodeParams {
     int items_cap, kv_splits, kv_chunk, c, pairs_per_xcd, num_mb, B, H;
     int uniform, max_seq_len, offsets_i64, targets_i64, delta, w, f, fit_runs;
     unsigned mb_magic, mb_shift, h_magic, h_shift;
-    int pad1[2];
+    int line_weight, line_wgs;
 };
 static_assert(sizeof(DecodeParams) == 128, "two loads of 16 dwords");
 
@@ -114,6 +114,9 @@ struct FwdParams {
     // Delta form with few row blocks: runs fitted to the lengths (see decode_fitted).  fit_runs: workgroups per plane (0 = off);
     // `partial` then holds [plane][workgroup][fit_rows][dv], and split_counts the first workgroup << 16 | number of runs.
     int fit_runs, fit_rows;
+    // The same with the tiles of a plane as one line that is cut into equal parts (see decode_line).  line_weight: tiles that a sequence counts for besides its own (0 = runs of
+    // one workgroup each, as above); line_wgs: workgroups per XCD; fit_slots: partial sums per plane.
+    int line_weight, line_wgs, fit_slots;
     alignas(64) DecodeParams dec;  // copies of the fields above that decode_work reads
 };
 
@@ -471,6 +474,8 @@ __device__ __forceinline__ int fast_div(int x, unsigned magic, unsigned shift) {
 // The row blocks of a head, which read the same keys, share an XCD.
 template <int BM, int BN>
 __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, int slot, int xcd, int64_t& seq_start, int64_t& seq_end, int& mb);
+template <int BM, int BN>
+__device__ __forceinline__ bool decode_line(Work& w, const DecodeParams& p, int slot, int xcd, int64_t& seq_start, int64_t& seq_end, int& mb);
 
 // Decode work item `bid` (the workgroup id in a one-item-per-workgroup launch) of the launch whose FwdParams are the
 // kernel's first argument.  Workgroup ids go round-robin
@@ -505,7 +510,8 @@ __device__ __forceinline__ bool decode_work(Work& w, int bid) {
     int64_t seq_start, seq_end;
     int t = 0;
     if constexpr (FIT) {
-        if (!decode_fitted<BM, BN>(w, p, slot, xcd, seq_start, seq_end, mb)) return false;
+        if (!(p.line_weight > 0 ? decode_line<BM, BN>(w, p, slot, xcd, seq_start, seq_end, mb) : decode_fitted<BM, BN>(w, p, slot, xcd, seq_start, seq_end, mb)))
+            return false;
         if (p.targets) t = p.targets_i64 ? (int)HSTU_CONST(int64_t, p.targets)[w.b] : HSTU_CONST(int, p.targets)[w.b];
     } else if (p.items) {
         // everything straight from the list: one load
@@ -606,6 +612,27 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
     return v;
 }
 
+// kv tiles of sequence `lane` for row block mb: its last row ends at n - delta + the block's end
+template <int BM, int BN>
+__device__ __forceinline__ int tiles_of_lane(const DecodeParams& p, int lane, int mb) {
+    if (lane >= p.B) return 0;
+    const int64_t n64 = p.offsets_i64 ? ((const int64_t*)p.offsets)[lane + 1] - ((const int64_t*)p.offsets)[lane]
+                                      : (int64_t)(((const int*)p.offsets)[lane + 1] - ((const int*)p.offsets)[lane]);
+    const int n = n64 > p.max_seq_len ? p.max_seq_len : (int)n64;
+    const int end = (mb + 1) * BM < p.delta ? (mb + 1) * BM : p.delta;
+    return n > 0 && n >= p.delta ? (n - p.delta + end + BN - 1) / BN : 0;
+}
+
+__device__ __forceinline__ void sequence_bounds(const DecodeParams& p, int b, int64_t& seq_start, int64_t& seq_end) {
+    if (p.offsets_i64) {
+        seq_start = HSTU_CONST(int64_t, p.offsets)[b];
+        seq_end = HSTU_CONST(int64_t, p.offsets)[b + 1];
+    } else {
+        seq_start = HSTU_CONST(int, p.offsets)[b];
+        seq_end = HSTU_CONST(int, p.offsets)[b + 1];
+    }
+}
+
 template <int BM, int BN>
 __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, int slot, int xcd, int64_t& seq_start, int64_t& seq_end, int& mb) {
     const int lane = threadIdx.x & 63;
@@ -614,14 +641,7 @@ __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, in
     const int k = g0 * 8 + xcd;  // (head, workgroup of the plane)
     const int h = k / p.fit_runs, i = k - h * p.fit_runs;
     if (h >= p.H) return false;
-    int tiles = 0;  // of sequence `lane`, for this row block: its last row ends at n - delta + the block's end
-    if (lane < p.B) {
-        const int64_t n64 = p.offsets_i64 ? ((const int64_t*)p.offsets)[lane + 1] - ((const int64_t*)p.offsets)[lane]
-                                          : (int64_t)(((const int*)p.offsets)[lane + 1] - ((const int*)p.offsets)[lane]);
-        const int n = n64 > p.max_seq_len ? p.max_seq_len : (int)n64;
-        const int end = (mb + 1) * BM < p.delta ? (mb + 1) * BM : p.delta;
-        if (n > 0 && n >= p.delta) tiles = (n - p.delta + end + BN - 1) / BN;
-    }
+    const int tiles = tiles_of_lane<BM, BN>(p, lane, mb);
     const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(tiles), 63);
     const int mean = (int)(((unsigned)total + (unsigned)p.fit_runs - 1) / (unsigned)p.fit_runs);
     // (An approximate quotient serves as well as the exact one: every workgroup computes the same.  But a sequence of one tile has
@@ -650,13 +670,49 @@ __device__ __forceinline__ bool decode_fitted(Work& w, const DecodeParams& p, in
     w.jt_begin = (int)((unsigned)(w.split * t) / (unsigned)r);
     w.jt_end = (int)((unsigned)((w.split + 1) * t) / (unsigned)r);
     if (r > 1) w.fit_slot = (h * p.num_mb + mb) * p.fit_runs + i;
-    if (p.offsets_i64) {
-        seq_start = HSTU_CONST(int64_t, p.offsets)[b];
-        seq_end = HSTU_CONST(int64_t, p.offsets)[b + 1];
-    } else {
-        seq_start = HSTU_CONST(int, p.offsets)[b];
-        seq_end = HSTU_CONST(int, p.offsets)[b + 1];
-    }
+    sequence_bounds(p, b, seq_start, seq_end);
+    return true;
+}
+
+// The kv tiles of a plane's sequences one after the other, cut into equal parts, one per workgroup: where there are few workgroups per sequence, whole runs leave
+// those of the longest history alone at the end.  A part may reach into several sequences, which are an item each (the first in round 0 and so on, so that
+// a workgroup whose round finds nothing is done); `line_weight` tiles in front of each stand for what such an item costs besides its steps.  The partial sums of workgroup i
+// and sequence b are number i + b of the plane (going along the line, one of the two grows from item to item), so that a sequence's are neighbours.
+template <int BM, int BN>
+__device__ __forceinline__ bool decode_line(Work& w, const DecodeParams& p, int slot, int xcd, int64_t& seq_start, int64_t& seq_end, int& mb) {
+    const int lane = threadIdx.x & 63;
+    const int round = slot / p.line_wgs, pos = slot - round * p.line_wgs;
+    const int lw = (round & 1) ? p.line_wgs - 1 - pos : pos;  // (the deal's direction alternates)
+    const int g0 = fast_div(lw, p.mb_magic, p.mb_shift);
+    mb = lw - g0 * p.num_mb;
+    const int k = g0 * 8 + xcd;  // (head, workgroup of the plane)
+    const int h = k / p.fit_runs, i = k - h * p.fit_runs;
+    if (h >= p.H) return false;
+    const int tiles = tiles_of_lane<BM, BN>(p, lane, mb);
+    const int weight = tiles > 0 ? tiles + p.line_weight : 0;
+    const int upto = wave_inclusive_scan(weight);
+    const unsigned total = (unsigned)__builtin_amdgcn_readlane(upto, 63);
+    const unsigned parts = total < (unsigned)p.fit_runs ? total : (unsigned)p.fit_runs;  // (no part is empty)
+    if ((unsigned)i >= parts) return false;
+    // (the host keeps total * parts below 2^31)
+    const int at = upto - tiles;  // of the sequence's first tile
+    int lo = (int)((unsigned)i * total / parts) - at, hi = (int)((unsigned)(i + 1) * total / parts) - at;
+    lo = lo > 0 ? lo : 0;
+    hi = hi < tiles ? hi : tiles;
+    uint64_t mine = __ballot(hi > lo);
+    for (int r = 0; r < round; ++r) mine &= mine - 1;
+    if (mine == 0) return false;
+    const int b = __builtin_ctzll(mine);
+    const unsigned t = (unsigned)__builtin_amdgcn_readlane(tiles, b), a = (unsigned)__builtin_amdgcn_readlane(at, b);
+    // tile x of the line is part ((x + 1) parts - 1) / total's
+    const int first = (int)(((a + 1) * parts - 1) / total), last = (int)(((a + t) * parts - 1) / total);
+    w.b = b, w.h = h;
+    w.split = i - first;
+    w.nsplit = (last - first + 1) | (first + b) << 16;
+    w.jt_begin = __builtin_amdgcn_readlane(lo, b);
+    w.jt_end = __builtin_amdgcn_readlane(hi, b);
+    if (last > first) w.fit_slot = (h * p.num_mb + mb) * (p.fit_runs + p.B) + i + b;
+    sequence_bounds(p, b, seq_start, seq_end);
     return true;
 }
 
@@ -1159,7 +1215,7 @@ __global__ __launch_bounds__(256) void hstu_reduce_splits_kernel(const FwdParams
     int64_t pitch = p.partial_stride;
     if (p.fit_runs > 0) {
         pitch = (int64_t)p.fit_rows * dv;
-        src = p.partial + ((int64_t)(h * p.num_mb + mb) * p.fit_runs + (runs >> 16)) * pitch + (int64_t)(r - mb * bm) * dv + c * 4;
+        src = p.partial + ((int64_t)(h * p.num_mb + mb) * p.fit_slots + (runs >> 16)) * pitch + (int64_t)(r - mb * bm) * dv + c * 4;
         runs &= 0xffff;
         if (runs == 1) return;  // stored by its one workgroup
     }

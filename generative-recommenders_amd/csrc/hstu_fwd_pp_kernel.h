@@ -136,6 +136,7 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
     int* const queue = p_arg.queue;
     int round = 0;
     int bid = lw < slots_per_xcd ? lw * 8 + xcd : -1;
+    bool over = false;
     auto process_item = [&]() __attribute__((always_inline)) {
     // Per-lane values that depend on the lane number only are recomputed for every item (a few dozen VALU
     // instructions): hoisted out of the item loop they would be spilled.  The empty asm hides from the compiler
@@ -150,7 +151,10 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
     asm volatile("" : "+s"(pk));
     const FwdParams& p = *(const FwdParams*)pk;
     Work W;
-    if (!decode_work<BM, BN, FIT>(W, bid)) return;
+    if (!decode_work<BM, BN, FIT>(W, bid)) {
+        over = FIT;  // (neither have its later rounds anything: decode_fitted, decode_line)
+        return;
+    }
     const SeqMask& M = W.M;
     const int n = W.n;
     const int nq = W.m1;  // one past the last row of this item: rows from here on are never loaded or stored
@@ -486,6 +490,7 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
             if (ns < slots_per_xcd) next = ns * 8 + xcd;
         }
         process_item();
+        if (FIT && over) break;
         if (queue) {
             if (threadIdx.x == 0) {
                 int nb = -1;

@@ -18,6 +18,11 @@ CASES = [
     ([6000, 40, 3513] + [65] * 61, 33, 1, 64),           # 64 sequences (every lane), most of them one or two tiles
     # one tile among long histories, whose longest runs are 41 tiles (41 * (1 / 41) is below 1 in fp32): not a run more than workgroups
     ([204 * 64 - 5, 164 * 64 - 3] * 3 + [204 * 64, 40], 16, 8, 32),
+    # fewer than four workgroups per sequence: the tiles as one line (decode_line)
+    ([2000 + 37 * i for i in range(18)], 3, 8, 128),     # parts that end inside sequences
+    ([7000] + [65] * 63, 33, 4, 64),                     # 64 sequences; parts that hold many of them, a sequence in many parts
+    ([300, 8000] + [364] * 30 + [4096, 301], 300, 2, 32),  # row blocks with a part over, sequences without history, whole tiles
+    ([500 + 331 * i for i in range(20)], 129, 8, 128),   # more sequences than workgroups per plane, two row blocks
 ]
 
 
