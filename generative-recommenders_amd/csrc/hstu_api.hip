@@ -136,6 +136,19 @@ int launch(const hstu::FwdParams& p, hipStream_t stream) {
     return HSTU_OK;
 }
 
+// Constants for fast_div (device side): x / d == (x * magic) >> (32 + shift) for 0 <= x < 2^31; magic 0 means d == 1.
+void fast_div_constants(unsigned d, unsigned* magic, unsigned* shift) {
+    if (d <= 1) {
+        *magic = 0;
+        *shift = 0;
+        return;
+    }
+    unsigned l = 0;
+    while ((1ull << l) < d) ++l;  // ceil(log2 d) >= 1
+    *magic = (unsigned)((1ull << (31 + l)) / d + 1);
+    *shift = l - 1;
+}
+
 template <class TT, int DQK, int DV, int BN, int NG>
 int launch_pp(const hstu::FwdParams& p, int grid_per_xcd, int64_t total_q, hipStream_t stream) {
     if (p.fit_runs > 0) {
@@ -152,11 +165,19 @@ int launch_pp(const hstu::FwdParams& p, int grid_per_xcd, int64_t total_q, hipSt
         return HSTU_ERR_LAUNCH;
     }
     if (p.kv_splits > 1 || p.fit_runs > 0) {
-        const long long threads = (long long)total_q * p.H * (DV / 4);
-        const long long blocks = (threads + 255) / 256;
-        if (blocks > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
-        hipLaunchKernelGGL(hstu::hstu_reduce_splits_kernel<typename TT::out_elem>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                           p, total_q, DV, NG == 1 ? 128 : 256);
+        constexpr int LG = DV == 32 ? 3 : DV == 64 ? 4 : 5;
+        static_assert(DV == 4 << LG, "the reduce kernel's threads per row and head");
+        const long long rows = (long long)total_q * p.H, blocks = (rows + (256 >> LG) - 1) / (256 >> LG);
+        if (rows > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
+        hstu::ReduceParams rp;
+        rp.offsets = p.offsets, rp.offsets_i64 = p.offsets_i64, rp.partial = p.partial, rp.counts = p.split_counts;
+        rp.o = p.o, rp.o_rs = p.o_rs, rp.o_hs = p.o_hs;
+        rp.attn_scale = p.attn_scale, rp.attn_scale_per_row = p.attn_scale_per_row, rp.oscale = p.oscale, rp.oscale_unit = p.oscale_unit;
+        rp.B = p.B, rp.H = p.H, rp.num_mb = p.num_mb, rp.max_seq_len = p.max_seq_len, rp.delta = p.delta, rp.rows = (unsigned)rows;
+        rp.fit_slots = p.fit_runs > 0 ? p.fit_slots : 0, rp.pitch = p.fit_runs > 0 ? (int64_t)p.fit_rows * DV : p.partial_stride;
+        rp.h_magic = p.h_magic, rp.h_shift = p.h_shift;
+        fast_div_constants((unsigned)(p.delta > 0 ? p.delta : 1), &rp.delta_magic, &rp.delta_shift);
+        hipLaunchKernelGGL((hstu::hstu_reduce_splits_kernel<typename TT::out_elem, LG, NG == 1 ? 128 : 256>), dim3((unsigned)blocks), dim3(256), 0, stream, rp);
         e = hipGetLastError();
         if (e != hipSuccess) {
             set_last_error("reduce kernel launch", e);
@@ -360,19 +381,6 @@ Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX, bool line = true
 }
 
 size_t scratch_bytes(const HstuFwdArgs* a) { return a->workspace ? (size_t)a->workspace_bytes : 0; }
-
-// Constants for fast_div (device side): x / d == (x * magic) >> (32 + shift) for 0 <= x < 2^31; magic 0 means d == 1.
-void fast_div_constants(unsigned d, unsigned* magic, unsigned* shift) {
-    if (d <= 1) {
-        *magic = 0;
-        *shift = 0;
-        return;
-    }
-    unsigned l = 0;
-    while ((1ull << l) < d) ++l;  // ceil(log2 d) >= 1
-    *magic = (unsigned)((1ull << (31 + l)) / d + 1);
-    *shift = l - 1;
-}
 
 void fill_decode_params(hstu::FwdParams& p) {
     hstu::DecodeParams& d = p.dec;

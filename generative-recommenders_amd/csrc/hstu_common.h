@@ -1172,28 +1172,47 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&oacc)[DT][QT], in
         }
 }
 
+// What the kernel below needs: one stretch of kernel arguments, fetched at once.
+struct ReduceParams {
+    const void* offsets;
+    const float* partial;
+    const int* counts;
+    char* o;
+    const float* attn_scale;
+    int64_t o_rs, o_hs;
+    int64_t pitch;                  // floats from one run's sums of a row to the next one's
+    int offsets_i64, attn_scale_per_row, B, H, num_mb, max_seq_len, delta;
+    int fit_slots;                  // fitted runs: partial sums per plane; 0 = equal runs, whose sums are [run][row][head][dv]
+    unsigned rows;                  // total_q * H, below 2^31
+    unsigned h_magic, h_shift, delta_magic, delta_shift;  // division by H and by delta (fast_div)
+    float oscale, oscale_unit;
+};
+
 // out = oscale * (sum of the runs of the row's row block), rounded once; one thread per 4 consecutive dv.
 // The thread finds its sequence (delta mode: row / delta; otherwise a binary search of the offsets), skips
 // rows the forward kernel does not produce (past max_seq_len, or a sequence shorter than delta) and reads the
 // number of runs that run 0 of its row block recorded.
-template <class ELEM>
-__global__ __launch_bounds__(256) void hstu_reduce_splits_kernel(const FwdParams p, int64_t total_q, int dv, int bm) {
+// A few rows are the chain of the kernel's own latencies: arguments, count and offsets, sums.  So the divisions are multiplications by the host's constants (64-bit
+// ones were most of the kernel), the count is asked for beside the offsets, and up to seven runs' sums together.  LG: dv / 4 = 2^LG; BM: rows of a block.
+template <class ELEM, int LG, int BM>
+__global__ __launch_bounds__(256) void hstu_reduce_splits_kernel(const ReduceParams p) {
     typedef __attribute__((ext_vector_type(4))) ELEM elem4;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over total_q * H * dv / 4
-    const int dv4 = dv >> 2;
-    if (idx >= total_q * p.H * dv4) return;
-    const int c = (int)(idx % dv4);
-    const int64_t rh = idx / dv4;
-    const int h = (int)(rh % p.H);
-    const int64_t row = rh / p.H;
+    constexpr int DV = 4 << LG;
+    const unsigned rh = blockIdx.x * (256u >> LG) + (threadIdx.x >> LG);  // (row, head)
+    const int c = threadIdx.x & ((1 << LG) - 1);
+    if (rh >= p.rows) return;
+    const int row = fast_div((int)rh, p.h_magic, p.h_shift), h = (int)rh - row * p.H;
     auto offset = [&](int j) -> int64_t {
         return p.offsets_i64 ? ((const int64_t*)p.offsets)[j] : (int64_t)((const int*)p.offsets)[j];
     };
-    int b, r;
+    int r, runs;
     if (p.delta > 0) {
-        b = (int)(row / p.delta);
-        r = (int)(row - (int64_t)b * p.delta);
-        int64_t n = offset(b + 1) - offset(b);
+        const int b = fast_div(row, p.delta_magic, p.delta_shift);
+        r = row - b * p.delta;
+        runs = p.counts[(b * p.H + h) * p.num_mb + r / BM];  // (of a block that nobody made it is not looked at)
+        int64_t n;
+        if (p.offsets_i64) n = ((const int64_t*)p.offsets)[b + 1] - ((const int64_t*)p.offsets)[b];
+        else n = (int64_t)(((const int*)p.offsets)[b + 1] - ((const int*)p.offsets)[b]);
         if (n > p.max_seq_len) n = p.max_seq_len;
         if (n <= 0 || n < p.delta) return;
     } else {
@@ -1202,38 +1221,42 @@ __global__ __launch_bounds__(256) void hstu_reduce_splits_kernel(const FwdParams
             const int mid = (lo + hi) >> 1;
             if (offset(mid) <= row) lo = mid; else hi = mid;
         }
-        b = lo;
-        const int64_t start = offset(b);
-        int64_t n = offset(b + 1) - start;
+        const int64_t start = offset(lo);
+        int64_t n = offset(lo + 1) - start;
         if (n > p.max_seq_len) n = p.max_seq_len;
         if (row - start >= n) return;
         r = (int)(row - start);
+        runs = p.counts[(lo * p.H + h) * p.num_mb + r / BM];
     }
-    const int mb = r / bm;
-    int runs = p.split_counts[(b * p.H + h) * p.num_mb + mb];
-    const float* src = p.partial + idx * 4;
-    int64_t pitch = p.partial_stride;
-    if (p.fit_runs > 0) {
-        pitch = (int64_t)p.fit_rows * dv;
-        src = p.partial + ((int64_t)(h * p.num_mb + mb) * p.fit_slots + (runs >> 16)) * pitch + (int64_t)(r - mb * bm) * dv + c * 4;
+    const float* src = p.partial + (int64_t)rh * DV + c * 4;
+    if (p.fit_slots > 0) {
+        const int mb = r / BM;
+        src = p.partial + ((int64_t)(h * p.num_mb + mb) * p.fit_slots + (runs >> 16)) * p.pitch + (r - mb * BM) * DV + c * 4;
         runs &= 0xffff;
         if (runs == 1) return;  // stored by its one workgroup
     }
+    // N loads in flight, added in order; past the last run that one's again, not added
     f32x4_t acc = *(const f32x4_t*)src;
-    int s = 1;
-    for (; s + 4 <= runs; s += 4) {  // four loads in flight, added in order
-        f32x4_t x[4];
+    auto add = [&](int s, auto Count) __attribute__((always_inline)) {
+        constexpr int N = decltype(Count)::value;
+        f32x4_t x[N];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = *(const f32x4_t*)(src + (s + j) * pitch);
+        for (int j = 0; j < N; ++j) x[j] = *(const f32x4_t*)(src + (s + j < runs ? s + j : runs - 1) * p.pitch);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc += x[j];
+        for (int j = 0; j < N; ++j) acc = s + j < runs ? acc + x[j] : acc;
+    };
+    if (runs <= 2) {
+        if (runs == 2) add(1, std::integral_constant<int, 1>{});
+    } else if (runs <= 4) {
+        add(1, std::integral_constant<int, 3>{});
+    } else {
+        for (int s = 1; s < runs; s += 7) add(s, std::integral_constant<int, 7>{});
     }
-    for (; s < runs; ++s) acc += *(const f32x4_t*)(src + s * pitch);
+    const float osc = !p.attn_scale ? p.oscale : p.oscale_unit * p.attn_scale[p.attn_scale_per_row ? row : 0];
     elem4 o4;
-    const float osc = output_scale(p, row);
 #pragma unroll
     for (int i = 0; i < 4; ++i) o4[i] = (ELEM)(acc[i] * osc);
-    *(elem4*)(p.o + (row * p.o_rs + (int64_t)h * p.o_hs) * 2 + c * 8) = o4;
+    *(elem4*)(p.o + ((int64_t)row * p.o_rs + (int64_t)h * p.o_hs) * 2 + c * 8) = o4;
 }
 
 // The same copy through a buffer descriptor: 16 bytes per lane from descriptor base + soffset (wave-uniform) + voffset
