@@ -300,7 +300,9 @@ def test_uqvk_kernels_for_few_rows_give_the_same_bits(pkg, dev, d_model, H, attn
     # one row; remainders of 32 and 64 rows; units of their own, several per wave, 64 rows per wave with shares that differ (depths 256, 384,
     # 512); more columns than the waves of a workgroup have units for; the library's shapes (depths 64 and 1152, few columns)
     [(1, 512, 1536), (33, 128, 128), (65, 256, 384), (4097, 512, 1024), (2049, 384, 1152), (8193, 128, 640), (20001, 512, 1536), (30001, 256, 768),
-     (33333, 384, 512), (70, 64, 64), (300, 1152, 256), (20000, 512, 128)],
+     (33333, 384, 512), (70, 64, 64), (300, 1152, 256), (20000, 512, 128),
+     # the depth shared by four waves: fewer blocks of 64 than waves, shares that differ, one row in the last block of 32, one whole round of workgroups
+     (1, 64, 64), (32, 192, 128), (33, 640, 384), (2048, 768, 256), (500, 4096, 512)],
 )
 def test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound):
     """hstu_linear_product_t on rows that are slices of wider buffers, against the product in 64 bits."""
@@ -333,7 +335,9 @@ def test_product_with_a_transposed_weight(pkg, dev, rows, k, n, dtype, bound):
      (3000, 384, 1536, True), (5000, 512, 2048, True), (10000, 384, 1024, True), (4000, 512, 1536, False), (12000, 512, 1024, False), (17000, 384, 1024, False),
      (32768, 512, 512, True), (32769, 512, 512, False), (10000, 512, 1536, True),
      (24000, 512, 768, False), (672, 512, 3072, False), (700, 512, 3072, True), (4533, 512, 3072, True), (5400, 512, 3072, False), (256, 512, 4096, False), (450, 512, 4096, True),
-     (3764, 512, 4096, True), (4100, 512, 4096, False), (54000, 256, 256, True), (32768, 256, 256, False), (100000, 256, 256, False), (54000, 128, 256, False)],
+     (3764, 512, 4096, True), (4100, 512, 4096, False), (54000, 256, 256, True), (32768, 256, 256, False), (100000, 256, 256, False), (54000, 128, 256, False),
+     # other depths: one round of workgroups of 32 rows x 64 columns
+     (2048, 768, 256, False), (2049, 768, 256, True), (1, 2048, 16384, False), (33, 2048, 16384, True), (512, 2048, 512, False), (513, 2048, 512, True), (70, 72, 64, True), (70, 640, 72, True)],
 )
 def test_which_products_with_a_transposed_weight_are_the_library_s(rows, k, n, library):
     """Only the library's need a workspace.  (Into 1024 columns and more all of them were the kernels', up to 1.6 times as long on the GPU; the sizes
