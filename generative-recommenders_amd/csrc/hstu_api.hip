@@ -697,7 +697,10 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
     p.slots_per_xcd = (int)slots;
     fast_div_constants((unsigned)p.num_mb, &p.mb_magic, &p.mb_shift);
     fast_div_constants((unsigned)p.H, &p.h_magic, &p.h_shift);
-    long long resident = (long long)current_device_cus() * (cfg == 2 ? 1 : 2) / 8;
+    // workgroups of a CU: of the one-group kernel two, with 32 columns (161 registers) the three that fit (us, two / three: 256 sequences of 64 .. 1024, 4 heads 112 / 104; 256 of 256
+    // 31 / 26; 200 of 512 56 / 52; 100 of 300 .. 900 50 / 50); 64 columns fit as often and are faster without (256 of 64 .. 1024 138 / 149; 200 of 512 73 / 86)
+    const int per_cu = cfg == 2 ? 1 : a->dqk == 32 && a->dtype != HSTU_FP8_E4M3 ? 3 : 2;
+    long long resident = (long long)current_device_cus() * per_cu / 8;
     if (resident < 1) resident = 1;
     if (plan.one_each) {
         resident = slots;
