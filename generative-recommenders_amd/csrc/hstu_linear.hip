@@ -310,14 +310,14 @@ bool output_takes_rows(const HstuOutputArgs* a) {
     return a->linear_dim % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0;
 }
 
-template <class TT, bool GROUP>
-int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
+template <class TT, bool GROUP, bool ACT>
+int launch_output_rows_act(const HstuOutputArgs* a, hipStream_t stream) {
     hstu::OutputRowsParams p;
     const int rc = hstu::norm_mul_params(a, nullptr, (int64_t)output_blocks(a) * a->heads * a->linear_dim, false, p.nm);
     if (rc != 0) return rc;
     p.x = (const char*)a->x, p.x_rs = a->x_row_stride, p.w = (const char*)a->output_weight, p.out = (char*)a->out;
     p.n = a->d_out, p.k = output_blocks(a) * p.nm.d;
-    auto kern = hstu::hstu_output_rows_kernel<TT, GROUP>;
+    auto kern = hstu::hstu_output_rows_kernel<TT, GROUP, ACT>;
     // (a function attribute belongs to the device it was set on: one flag per device)
     static std::atomic<bool> attr_done[64];
     int dev = -1;
@@ -337,6 +337,12 @@ int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
         return -7;
     }
     return 0;
+}
+
+template <class TT, bool GROUP>
+int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
+    if (a->silu_u || (!GROUP && a->mul_u_activation != HSTU_MUL_U_NONE)) return launch_output_rows_act<TT, GROUP, true>(a, stream);
+    return launch_output_rows_act<TT, GROUP, false>(a, stream);
 }
 
 // path = 0: the panel kernel, one kernel for more rows, where u goes in as it is (output_panel_shape).  output_panel_form: its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are

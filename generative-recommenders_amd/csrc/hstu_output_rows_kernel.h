@@ -9,7 +9,8 @@
 // rounded as the matrix would be; then each multiplies a quarter of the depth, with W's tiles in a ring of its own, so that the serial chain
 // is short and there is no barrier until the four partial sums are added, in a fixed order, with the residual.
 // 3 x 512 into 512 columns, us on the GPU and of the host's call, the two kernels -> this one: 50 rows 10.4 and 13.5 -> 7.7 and 3.4, 256 rows 11.9 and
-// 13.7 -> 7.9 and 3.2.  What is left is latency: the launch, the rows from memory, their statistics (one row 7.6, 3 x 256 into 256 columns 7.0).
+// 13.7 -> 7.9 and 3.2.  What is left is latency: the launch, its instructions (ACT: u goes through an activation; without those of that 7.7 -> 7.5, one row 7.6 -> 7.25, 384 columns of u 7.4 -> 7.0), the
+// rows from memory, their statistics.  (All of W that the LDS holds asked for at once, and the residual at the start, gained nothing: 7.9.)
 #pragma once
 #include "hstu_common.h"
 #include "hstu_rows.h"
@@ -32,7 +33,7 @@ constexpr int kOutRowsSumRow = 32 * 4 + 16; // a row of partial sums
 constexpr int out_rows_lds(int k) { return 4 * kOutRowsRing * kOutRowsTile + 32 * k * 2; }
 static_assert(4 * 32 * kOutRowsSumRow <= 4 * kOutRowsRing * kOutRowsTile, "the partial sums take the place of the rings");
 
-template <class TT, bool GROUP>
+template <class TT, bool GROUP, bool ACT>
 __global__ __launch_bounds__(256, 1) void hstu_output_rows_kernel(const OutputRowsParams p) {
     typedef typename TT::vec8 vec8;
     typedef typename TT::elem elem;
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(256, 1) void hstu_output_rows_kernel(const OutputRo
         for (int j = 0; j < 8; ++j) {
             const float uf = (float)uv[i][j];
             float mul = uf;
-            if (nm.silu_u || (!GROUP && nm.mul_act != HSTU_MUL_U_NONE)) {
+            if constexpr (ACT) {
                 const float sg = sigmoid_f(uf), us = uf * sg;
                 if constexpr (GROUP) {
                     if (nm.silu_u) mul = us;
