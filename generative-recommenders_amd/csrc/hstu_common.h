@@ -755,69 +755,109 @@ static __global__ __launch_bounds__(HSTU_PLAN_THREADS) void hstu_plan_kernel(con
         }
         __syncthreads();
     }
-    for (int c = 0; c < NC; ++c) cnt[c][tid] = 0;
     const int num_mb = p.num_mb;
     const int total = p.pairs_per_xcd * num_mb;  // candidates: every row block a pair could have
+    int b = 0, h = 0, n = 0, nq = 0, rbase = 0, u = 0, t = 0;
+    int64_t seq_start = 0;
+    bool live = false;
+    SeqMask M;
+    auto look_up = [&](int pl) {  // pair number pl of this XCD
+        const int pair = pair_of(pl, xcd);
+        live = pair < p.B * p.H;
+        if (!live) return;
+        const int rseq = fast_div(pair, p.h_magic, p.h_shift);
+        b = rank ? order[rseq] : p.order ? p.order[rseq] : rseq;
+        h = pair - rseq * p.H;
+        seq_start = p.offsets_i64 ? ((const int64_t*)p.offsets)[b] : (int64_t)((const int*)p.offsets)[b];
+        const int64_t len = (p.offsets_i64 ? ((const int64_t*)p.offsets)[b + 1] : (int64_t)((const int*)p.offsets)[b + 1]) - seq_start;
+        t = 0;
+        if (p.targets) t = p.targets_i64 ? (int)((const int64_t*)p.targets)[b] : ((const int*)p.targets)[b];
+        n = len > p.max_seq_len ? p.max_seq_len : (int)len;
+        nq = p.delta > 0 ? p.delta : n;
+        rbase = p.delta > 0 ? n - p.delta : 0;
+        live = n > 0 && rbase >= 0;
+        M.n = n;
+        M.w = p.w;
+        M.c = p.c;
+        M.f = p.f;
+        M.shift = p.c > 0 ? p.c - 1 : 0;
+        u = n - t;
+        M.max_id = u - M.shift;
+        M.idclamp = p.targets ? M.max_id : 0x7fffffff;
+    };
+    auto class_of = [&](int mb) -> int {  // -1: no such row block
+        int m0, m1;
+        if (!live || !row_block_rows(nq, mb, bm, row_blocks_end_aligned(p), m0, m1)) return -1;
+        int jb, je;
+        kv_tile_range(M, u, rbase + m0, rbase + m1 - 1, bn, jb, je);
+        const int tiles = je - jb;
+        if (tiles <= 0) return -1;
+        const int c = 31 - __builtin_clz((unsigned)tiles);
+        return c > NC - 1 ? NC - 1 : c;
+    };
+    auto put = [&](int pos, int mb) {  // record `pos` of this XCD's list
+        if (pos < p.items_cap) {
+            typedef __attribute__((ext_vector_type(4))) int i32x4;
+            i32x4* rec = (i32x4*)(items + 8 * ((int64_t)xcd * p.items_cap + pos));
+            rec[0] = (i32x4){b, h, mb, n};
+            rec[1] = (i32x4){(int)(unsigned)(uint64_t)seq_start, (int)(unsigned)((uint64_t)seq_start >> 32), t, 0};
+        }
+    };
+    if (total <= NT) {
+        // A candidate each: looked up once, counted by ballot, placed from registers.  (The kernel is latency, on the way of every ragged batch: as two walks 7.5 us at 32
+        // sequences of up to 8192 rows, 5.3 so; 256 of up to 1024, which it ranks too, 8.4 and 5.8.)
+        const int pl = fast_div(tid, p.mb_magic, p.mb_shift), mb = num_mb - 1 - (tid - pl * num_mb);  // heaviest block of a pair first
+        int c = -1;
+        if (tid < total) {
+            look_up(pl);
+            c = class_of(mb);
+        }
+        int before = 0;  // of this class in this wave
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            const uint64_t those = __ballot(c == k);
+            if (c == k) before = __popcll(those & ((1ull << lane) - 1));
+            if (lane == 0) wave_sum[k][wave] = __popcll(those);
+        }
+        __syncthreads();
+        if (wave == 0) {  // exclusive prefix over (class, heaviest first, wave)
+            constexpr int PER = NC * NW / 64;
+            static_assert(NC * NW % 64 == 0, "whole entries per lane");
+            int mine[PER], sum = 0;
+#pragma unroll
+            for (int k = 0; k < PER; ++k) {
+                const int e = lane * PER + k;
+                mine[k] = sum;
+                sum += wave_sum[NC - 1 - e / NW][e % NW];
+            }
+            const int upto = wave_inclusive_scan(sum);
+#pragma unroll
+            for (int k = 0; k < PER; ++k) {
+                const int e = lane * PER + k;
+                wave_sum[NC - 1 - e / NW][e % NW] = upto - sum + mine[k];
+            }
+            if (lane == 63) nitems[xcd] = upto < p.items_cap ? upto : p.items_cap;
+        }
+        __syncthreads();
+        if (c >= 0) put(wave_sum[c][wave] + before, mb);
+        return;
+    }
+    for (int c = 0; c < NC; ++c) cnt[c][tid] = 0;
     const int run = (total + NT - 1) / NT;
     const int k_end = (tid + 1) * run < total ? (tid + 1) * run : total;
     auto walk = [&](bool place) {
-        int cur_pl = -1, b = 0, h = 0, n = 0, nq = 0, rbase = 0, u = 0, t = 0;
-        int64_t seq_start = 0;
-        bool live = false;
-        SeqMask M;
-        auto put = [&](int pos, int mb) {  // record `pos` of this XCD's list
-            if (pos < p.items_cap) {
-                typedef __attribute__((ext_vector_type(4))) int i32x4;
-                i32x4* rec = (i32x4*)(items + 8 * ((int64_t)xcd * p.items_cap + pos));
-                rec[0] = (i32x4){b, h, mb, n};
-                rec[1] = (i32x4){(int)(unsigned)(uint64_t)seq_start, (int)(unsigned)((uint64_t)seq_start >> 32), t, 0};
-            }
-        };
+        int cur_pl = -1;
         for (int k = tid * run; k < k_end; ++k) {
             const int pl = k / num_mb;
             const int mb = num_mb - 1 - (k - pl * num_mb);  // heaviest block of a pair first
             if (place && k < CACHE && cls[k] < 0) continue;  // second walk: known not to exist
-            if (!place && k < CACHE) cls[k] = -1;
             if (pl != cur_pl) {
                 cur_pl = pl;
-                const int pair = pair_of(pl, xcd);
-                live = pair < p.B * p.H;
-                if (live) {
-                    const int rseq = pair / p.H;
-                    b = rank ? order[rseq] : p.order ? p.order[rseq] : rseq;
-                    h = pair - rseq * p.H;
-                    seq_start = p.offsets_i64 ? ((const int64_t*)p.offsets)[b] : (int64_t)((const int*)p.offsets)[b];
-                    const int64_t len = (p.offsets_i64 ? ((const int64_t*)p.offsets)[b + 1] : (int64_t)((const int*)p.offsets)[b + 1]) - seq_start;
-                    n = len > p.max_seq_len ? p.max_seq_len : (int)len;
-                    nq = p.delta > 0 ? p.delta : n;
-                    rbase = p.delta > 0 ? n - p.delta : 0;
-                    live = n > 0 && rbase >= 0;
-                    t = 0;
-                    if (p.targets) t = p.targets_i64 ? (int)((const int64_t*)p.targets)[b] : ((const int*)p.targets)[b];
-                    M.n = n;
-                    M.w = p.w;
-                    M.c = p.c;
-                    M.f = p.f;
-                    M.shift = p.c > 0 ? p.c - 1 : 0;
-                    u = n - t;
-                    M.max_id = u - M.shift;
-                    M.idclamp = p.targets ? M.max_id : 0x7fffffff;
-                }
+                look_up(pl);
             }
-            int c;
-            if (place && k < CACHE) {
-                c = cls[k];  // the class is remembered from the first walk
-            } else {
-                int m0, m1;
-                if (!live || !row_block_rows(nq, mb, bm, row_blocks_end_aligned(p), m0, m1)) continue;
-                int jb, je;
-                kv_tile_range(M, u, rbase + m0, rbase + m1 - 1, bn, jb, je);
-                const int tiles = je - jb;
-                if (tiles <= 0) continue;
-                c = 31 - __builtin_clz((unsigned)tiles);
-                c = c > NC - 1 ? NC - 1 : c;
-                if (!place && k < CACHE) cls[k] = (signed char)c;
-            }
+            const int c = place && k < CACHE ? cls[k] : class_of(mb);  // (remembered from the first walk)
+            if (!place && k < CACHE) cls[k] = (signed char)c;
+            if (c < 0) continue;
             if (place) put(cbase[c] + cnt[c][tid], mb);
             cnt[c][tid] += 1;
         }
