@@ -360,11 +360,12 @@ Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX, bool line = true
     // Work lists for ragged batches (equal lengths are dealt arithmetically, a kv-split enumerates its runs
     // arithmetically too): 32 bytes per possible item; beyond 64 MB the arithmetic enumeration stays.
     const bool uniform = a->delta_size == 0 && a->total_kv == (int64_t)a->batch * a->max_seq_len;
-    // For few of the one-group kernel's items the list (for which the workspace still has room) costs more than it gives: the kernel that builds it takes 5 to 10 us
+    // For few of the one-group kernel's items the list (for which the workspace still has room) costs more than it gives: the kernel that builds it takes 5 to 6 us
     // (ranking the sequences another 10 at 256 of them), a workgroup that finds no rows leaves at once.  us, lists / a workgroup for every item there could be (4 heads of
-    // 64, ragged): 96 sequences of 20 .. 276 rows, 144 items per XCD, 24.2 / 17.6; 256 of 20 .. 128 27.2 / 17.2; 48 of 200 .. 700 31.2 / 28.6; 8 heads of 128, 20 of
-    // 300 .. 1300, 220 items 62.7 / 60.2.  More of them want the heaviest first: 64 of 200 .. 960, 4 heads of 128, 256 items 65.0 / 67.4; 100 of 300 .. 900, 400 items 81 / 86;
-    // 1024 items 190 / 203.  One row block per sequence: 1000 of 20 .. 128, 500 items, 81 / 75; 32 columns, where more than two workgroups fit a CU: 100 of 300 .. 900 53 / 48.
+    // 64, ragged, ranked): 96 sequences of 20 .. 276 rows, 144 items per XCD, 23.3 / 16.4; 256 of 20 .. 128 33.9 / 14.9; 48 of 200 .. 700 27.5 / 24.2; 8 heads, 28 of 64 .. 1000,
+    // 224 items, 31.5 / 29.5, 64 of 100 .. 512, 256 items, 35.7 / 34.0; 8 heads of 128, 20 of 300 .. 1300, 220 items 67.1 / 63.0.  More of them want the heaviest first (with a list
+    // that took 2 us longer): 64 of 200 .. 960, 4 heads of 128, 256 items 65.0 / 67.4; 100 of 300 .. 900, 400 items 81 / 86; 1024 items 190 / 203.  One row block per sequence:
+    // 500 of 20 .. 128, 8 heads, 500 items, 56.7 / 44.3; 32 columns, where more than two workgroups fit a CU: 100 of 300 .. 900 47.0 / 44.7.
     const long long num_mb = (rows_per_pair + bm - 1) / bm, slots = (a->batch * (long long)a->heads + 7) / 8 * num_mb;
     pl.one_each = s == 1 && !uniform && pl.cfg == 3 && a->delta_size == 0 && slots <= (num_mb == 1 || a->dqk == 32 ? 512 : num_mb <= 4 ? 256 : 224);
     if (s == 1 && !uniform) {

@@ -31,10 +31,11 @@ def test_ranked_lists(pkg, dev, batch, heads, longest, i64):
 
 
 # (batch, heads, longest, columns): a workgroup for every item there could be, with one row block per sequence, up to four (unranked) and more (ranked); on the other
-# side of each line the lists, around the number of sequences that their kernel ranks itself; 32 columns have a line of their own
+# side of each line the lists, around the number of sequences that their kernel ranks itself and the 1024 candidates of an XCD that it looks up one to a thread;
+# 32 columns have a line of their own
 @pytest.mark.parametrize("batch,heads,longest,d", [
     (512, 8, 128, 64), (513, 8, 128, 64), (64, 8, 512, 128), (65, 8, 512, 64), (28, 8, 1000, 64), (29, 8, 1000, 64), (64, 8, 1000, 32), (65, 8, 1000, 32),
-    (255, 4, 384, 64), (256, 4, 384, 64), (257, 4, 384, 64)])
+    (255, 4, 384, 64), (256, 4, 384, 64), (257, 4, 384, 64), (256, 8, 512, 64), (257, 8, 512, 64), (205, 8, 640, 32)])
 def test_items_with_and_without_lists(pkg, dev, batch, heads, longest, d):
     print(f"[case] items {batch} x {heads} heads up to {longest}, {d} columns", flush=True)
     gen = torch.Generator().manual_seed(batch + longest)
