@@ -383,6 +383,37 @@ Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX, bool line = true
 
 size_t scratch_bytes(const HstuFwdArgs* a) { return a->workspace ? (size_t)a->workspace_bytes : 0; }
 
+// The launch of a plan on a device of `cus` CUs: work items per XCD, and for the persistent kernels the workgroups that stay resident
+// (the same number on every XCD).
+struct Grid {
+    int num_mb;
+    long long pairs_per_xcd;
+    long long fit_wgs;  // per XCD: workgroups of fitted runs, 0 without
+    long long slots;    // per XCD: items
+    int per_xcd;        // per XCD: workgroups
+};
+
+Grid make_grid(const HstuFwdArgs* a, const Plan& plan, int cus) {
+    const int rows_per_pair = a->delta_size > 0 ? a->delta_size : a->max_seq_len;
+    const int bm = plan.cfg == 2 ? 256 : 128;
+    Grid g;
+    g.num_mb = (rows_per_pair + bm - 1) / bm;
+    g.pairs_per_xcd = ((long long)a->batch * a->heads + 7) / 8;
+    g.fit_wgs = (((long long)plan.fit_runs * a->heads + 7) / 8) * g.num_mb;
+    g.slots = plan.fit_runs > 0 ? g.fit_wgs * (plan.line_weight > 0 ? a->batch : 1) : g.pairs_per_xcd * g.num_mb * plan.splits;
+    // workgroups of a CU: of the one-group kernel two, with 32 columns (161 registers) the three that fit (us, two / three: 256 sequences of 64 .. 1024, 4 heads 112 / 104; 256 of 256
+    // 31 / 26; 200 of 512 56 / 52; 100 of 300 .. 900 50 / 50); 64 columns fit as often and are faster without (256 of 64 .. 1024 138 / 149; 200 of 512 73 / 86)
+    const int per_cu = plan.cfg == 2 ? 1 : a->dqk == 32 && a->dtype != HSTU_FP8_E4M3 ? 3 : 2;
+    long long resident = (long long)cus * per_cu / 8;
+    if (resident < 1) resident = 1;
+    if (plan.one_each) resident = g.slots;
+    // Fitted runs: a workgroup each, also where the device has fewer CUs than make_plan sized them for (a partition of it): the kernel's
+    // workgroups end at the first item that decodes to nothing, as those behind the last run of a head do.
+    if (plan.fit_runs > 0) resident = g.fit_wgs;
+    g.per_xcd = (int)(g.slots < resident ? g.slots : resident);
+    return g;
+}
+
 void fill_decode_params(hstu::FwdParams& p) {
     hstu::DecodeParams& d = p.dec;
     memset(&d, 0, sizeof(d));
@@ -502,6 +533,19 @@ int hstu_hip_plan(const HstuFwdArgs* a, int32_t* tile_config, int32_t* kv_splits
     const Plan pl = make_plan(a, scratch_bytes(a));
     if (tile_config) *tile_config = pl.cfg;
     if (kv_splits) *kv_splits = pl.splits;
+    return HSTU_OK;
+}
+
+int hstu_hip_plan_grid(const HstuFwdArgs* a, int32_t cus, int32_t* form, int32_t* items, int32_t* workgroups) {
+    const int rc = hstu_hip_check_args(a);
+    if (rc != HSTU_OK) return rc;
+    if (cus <= 0) return HSTU_ERR_BAD_SHAPE;
+    const Plan pl = make_plan(a, scratch_bytes(a));
+    const Grid g = make_grid(a, pl, cus);
+    if (g.slots * 8 > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
+    if (form) *form = pl.line_weight > 0 ? HSTU_PLAN_LINE : pl.fit_runs > 0 ? HSTU_PLAN_FITTED : pl.splits > 1 ? HSTU_PLAN_EQUAL_RUNS : HSTU_PLAN_WHOLE;
+    if (items) *items = (int32_t)g.slots;
+    if (workgroups) *workgroups = pl.cfg < 2 ? (int32_t)g.slots : g.per_xcd;
     return HSTU_OK;
 }
 
@@ -680,37 +724,24 @@ int hstu_hip_mha_fwd(const HstuFwdArgs* a, void* stream_) {
     }
     p.kv_splits = plan.splits;
 
-    // the grid: work items per XCD, and for the persistent kernels the workgroups that stay resident (one 8-wave
-    // or two 4-wave workgroups per CU; the same number on every XCD)
     const int cfg = plan.cfg;
     const int rows_per_pair = a->delta_size > 0 ? a->delta_size : a->max_seq_len;
-    const long long num_pairs = (long long)a->batch * a->heads;
     const int bm = cfg == 2 ? 256 : 128;
-    p.num_mb = (rows_per_pair + bm - 1) / bm;
-    const long long pairs_per_xcd = (num_pairs + 7) / 8;
-    const long long wgs = (((long long)p.fit_runs * a->heads + 7) / 8) * p.num_mb;  // per XCD, of fitted runs
-    const long long slots = p.fit_runs > 0 ? wgs * (p.line_weight > 0 ? a->batch : 1) : pairs_per_xcd * p.num_mb * plan.splits;
-    p.line_wgs = (int)wgs;
+    const Grid grid = make_grid(a, plan, current_device_cus());
+    p.num_mb = grid.num_mb;
+    p.line_wgs = (int)grid.fit_wgs;
     p.fit_rows = rows_per_pair < bm ? rows_per_pair : bm;
+    const long long slots = grid.slots;
     if (slots <= 0) return HSTU_OK;
     if (slots * 8 > 0x7fffffffLL) return HSTU_ERR_BAD_SHAPE;
-    p.pairs_per_xcd = (int)pairs_per_xcd;
+    p.pairs_per_xcd = (int)grid.pairs_per_xcd;
     p.slots_per_xcd = (int)slots;
     fast_div_constants((unsigned)p.num_mb, &p.mb_magic, &p.mb_shift);
     fast_div_constants((unsigned)p.H, &p.h_magic, &p.h_shift);
-    // workgroups of a CU: of the one-group kernel two, with 32 columns (161 registers) the three that fit (us, two / three: 256 sequences of 64 .. 1024, 4 heads 112 / 104; 256 of 256
-    // 31 / 26; 200 of 512 56 / 52; 100 of 300 .. 900 50 / 50); 64 columns fit as often and are faster without (256 of 64 .. 1024 138 / 149; 200 of 512 73 / 86)
-    const int per_cu = cfg == 2 ? 1 : a->dqk == 32 && a->dtype != HSTU_FP8_E4M3 ? 3 : 2;
-    long long resident = (long long)current_device_cus() * per_cu / 8;
-    if (resident < 1) resident = 1;
-    if (plan.one_each) {
-        resident = slots;
-        // long sequences first only where there can be long ones, which repays the launch that ranks them (4 heads of 128, one in four of 32 sequences 1500 rows, the
-        // others 100: 65 us unranked, 45 ranked; 60 sequences of 100 .. 512, 8 heads 48 and 56)
-        if (p.num_mb <= 4) order = nullptr;
-    }
-    if (p.line_weight > 0) resident = wgs;
-    const int grid_per_xcd = (int)(slots < resident ? slots : resident);
+    // a workgroup each, few row blocks: long sequences first only where there can be long ones, which repays the launch that ranks them (4 heads of 128,
+    // one in four of 32 sequences 1500 rows, the others 100: 65 us unranked, 45 ranked; 60 sequences of 100 .. 512, 8 heads 48 and 56)
+    if (plan.one_each && p.num_mb <= 4) order = nullptr;
+    const int grid_per_xcd = grid.per_xcd;
     if (cfg < 2 || slots <= grid_per_xcd || p.line_weight > 0) queue = nullptr;  // every workgroup has exactly one item (or its part of a line)
     int* items = nullptr;
     if (queue && plan.items_bytes > 0 && ws_bytes >= plan.total()) items = (int*)(ws + plan.total() - plan.cast_bytes - plan.items_bytes);

@@ -152,7 +152,7 @@ __global__ __launch_bounds__(NG * 256, 2) void hstu_fwd_pp_kernel(const FwdParam
     const FwdParams& p = *(const FwdParams*)pk;
     Work W;
     if (!decode_work<BM, BN, FIT>(W, bid)) {
-        over = FIT;  // (neither have its later rounds anything: decode_fitted, decode_line)
+        over = FIT;  // (decode_fitted: its only item; decode_line: its rounds behind an empty one are empty)
         return;
     }
     const SeqMask& M = W.M;

@@ -390,7 +390,7 @@ __global__ __launch_bounds__(512, 2) void hstu_fwd_stream_kernel(const FwdParams
         for (;;) {
             if (next_bid < 0) return false;
             if (decode_work<BM, BN, FIT>(W, next_bid) && W.jt_end > W.jt_begin) return true;
-            if constexpr (FIT) return false;  // (neither have its later rounds anything: decode_fitted, decode_line)
+            if constexpr (FIT) return false;  // (decode_fitted: its only item; decode_line: its rounds behind an empty one are empty)
             if (queue) {
                 if (drawer) publish_next(resolve_ticket(draw_ticket()));
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)

@@ -113,6 +113,7 @@ EXPORTS = (
     "hstu_hip_mha_bwd_workspace_bytes",
     "hstu_hip_workspace_bytes",
     "hstu_hip_plan",
+    "hstu_hip_plan_grid",
     "hstu_hip_tile_configs",
     "hstu_hip_tile_config_name",
     "hstu_hip_concat_2d_jagged",
@@ -159,6 +160,8 @@ def lib() -> ctypes.CDLL:
         L.hstu_hip_mha_bwd_workspace_bytes.argtypes = [ctypes.POINTER(HstuFwdArgs)]
         L.hstu_hip_plan.restype = ctypes.c_int
         L.hstu_hip_plan.argtypes = [ctypes.POINTER(HstuFwdArgs), ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
+        L.hstu_hip_plan_grid.restype = ctypes.c_int
+        L.hstu_hip_plan_grid.argtypes = [ctypes.POINTER(HstuFwdArgs), ctypes.c_int32] + [ctypes.POINTER(ctypes.c_int32)] * 3
         L.hstu_hip_workspace_bytes.restype = ctypes.c_size_t
         L.hstu_hip_workspace_bytes.argtypes = [ctypes.POINTER(HstuFwdArgs)]
         L.hstu_hip_tile_configs.restype = ctypes.c_int
@@ -207,10 +210,8 @@ def tile_config_names() -> list:
     return [L.hstu_hip_tile_config_name(i + 1).decode() for i in range(L.hstu_hip_tile_configs())]
 
 
-def plan_for(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size=0, tile_config=0, kv_splits=0,
-             sort_by_length=False, dtype=HSTU_BF16):
-    """(tile configuration, kv runs) the library would choose for a call of these sizes when given the workspace it
-    asks for.  Touches no device memory."""
+def _plan_args(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size, tile_config, kv_splits, sort_by_length, dtype, workspace_bytes):
+    """Arguments of a call of these sizes for the plan queries, with the workspace it asks for or with ``workspace_bytes``."""
     a = HstuFwdArgs()
     a.batch, a.heads, a.dqk, a.dv = batch, heads, dqk, dv
     a.total_q, a.total_kv, a.max_seq_len, a.delta_size = total_q, total_kv, max_seq_len, delta_size
@@ -221,11 +222,32 @@ def plan_for(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size=0
     a.v_row_stride = a.o_row_stride = heads * dv
     a.q_head_stride = a.k_head_stride = dqk
     a.v_head_stride = a.o_head_stride = dv
-    need = lib().hstu_hip_workspace_bytes(ctypes.byref(a))
+    need = lib().hstu_hip_workspace_bytes(ctypes.byref(a)) if workspace_bytes is None else workspace_bytes
     a.workspace, a.workspace_bytes = (256, need) if need else (None, 0)
+    return a
+
+
+def plan_for(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size=0, tile_config=0, kv_splits=0,
+             sort_by_length=False, dtype=HSTU_BF16):
+    """(tile configuration, kv runs) the library would choose for a call of these sizes when given the workspace it
+    asks for.  Touches no device memory."""
+    a = _plan_args(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size, tile_config, kv_splits, sort_by_length, dtype, None)
     cfg, splits = ctypes.c_int32(0), ctypes.c_int32(0)
     raise_for_status(lib().hstu_hip_plan(ctypes.byref(a), ctypes.byref(cfg), ctypes.byref(splits)))
     return cfg.value, splits.value
+
+
+PLAN_FORMS = ("whole", "equal runs", "fitted", "line")
+
+
+def plan_grid_for(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size=0, tile_config=0, kv_splits=0,
+                  sort_by_length=False, dtype=HSTU_BF16, workspace_bytes=None, cus=256):
+    """(form, items per XCD, workgroups per XCD) of the launch that plan makes on a device of ``cus`` CUs; ``form``, one of ``PLAN_FORMS``, is how
+    the kv range of a row block is cut.  ``workspace_bytes``: the workspace at hand (default: what the call asks for).  Touches no device memory."""
+    a = _plan_args(batch, heads, dqk, dv, total_q, total_kv, max_seq_len, delta_size, tile_config, kv_splits, sort_by_length, dtype, workspace_bytes)
+    form, items, wgs = ctypes.c_int32(0), ctypes.c_int32(0), ctypes.c_int32(0)
+    raise_for_status(lib().hstu_hip_plan_grid(ctypes.byref(a), cus, ctypes.byref(form), ctypes.byref(items), ctypes.byref(wgs)))
+    return PLAN_FORMS[form.value], items.value, wgs.value
 
 
 def contract_checks_enabled() -> bool:

@@ -179,6 +179,16 @@ size_t hstu_hip_workspace_bytes(const HstuFwdArgs* args);
  */
 int hstu_hip_plan(const HstuFwdArgs* args, int32_t* tile_config, int32_t* kv_splits);
 
+/*
+ * How that plan cuts the kv range of a row block, and the launch it makes on a device of `cus` CUs: items and workgroups of each of the eight
+ * XCDs (any pointer may be NULL).  Returns what hstu_hip_check_args returns.  Diagnostic only; touches no device.
+ */
+#define HSTU_PLAN_WHOLE 0      /* not at all */
+#define HSTU_PLAN_EQUAL_RUNS 1 /* in runs of as many tiles */
+#define HSTU_PLAN_FITTED 2     /* in runs fitted to the lengths, one per workgroup */
+#define HSTU_PLAN_LINE 3       /* the tiles of a head's sequences are one line, a part of it per workgroup, an item per sequence in it (at most `batch`) */
+int hstu_hip_plan_grid(const HstuFwdArgs* args, int32_t cus, int32_t* form, int32_t* items, int32_t* workgroups);
+
 /* Number of selectable tile configurations and a short name for each (1-based ids). */
 int hstu_hip_tile_configs(void);
 const char* hstu_hip_tile_config_name(int id);

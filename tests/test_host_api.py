@@ -329,3 +329,19 @@ def test_a_kv_split_is_cut_to_the_workspace_at_hand(backend):
     assert runs(2 * run + other) == 2 and runs(2 * run + other - 1) == 1 and runs(0) == 1
     a.kv_splits = 4
     assert runs(2 * run) == 4  # asked for: the call itself refuses a workspace that is too small
+
+
+@pytest.mark.parametrize("cus", [256, 128, 64, 32, 8])
+def test_fitted_runs_have_a_workgroup_each_on_any_device(backend, cus):
+    """The kernel's workgroups end at the first item that decodes to nothing, which only the last of a workgroup's items may: fitted runs need a workgroup each, a
+    line its own number of them, also on a partition of the device with fewer CUs than the runs are sized for.  (With as many workgroups as such a device holds, those that
+    drew an unused run of one head left the runs of the next one undone.)"""
+    shapes = [  # batch, heads, dim, rows, delta, longest, tile configuration
+        (5, 4, 128, 12000, 100, 16100, 0), (3, 3, 128, 2000, 64, 7007, 3), (2, 1, 128, 2650, 300, 5007, 0), (64, 1, 64, 210, 33, 6007, 2), (2, 2, 64, 1300, 129, 2507, 3),
+        (18, 8, 128, 2300, 3, 2636, 0), (64, 4, 64, 174, 33, 7007, 0), (20, 8, 128, 3700, 129, 6796, 2)]
+    forms = set()
+    for B, H, D, rows, delta, N, cfg in shapes:
+        form, items, wgs = backend.plan_grid_for(B, H, D, D, B * delta, B * rows, N, delta_size=delta, tile_config=cfg, cus=cus)
+        forms.add(form)
+        assert form in ("fitted", "line") and items == wgs * (B if form == "line" else 1), (B, H, D, rows, delta, N, cfg)
+    assert forms == {"fitted", "line"}
