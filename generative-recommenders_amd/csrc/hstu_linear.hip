@@ -349,9 +349,9 @@ int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
 // this kernel's up to a width of 256 (3 x 256 into 512 columns, us: one row 7.0 -> 5.2, 256 rows 7.3 -> 5.5; 3 x 512: 7.7 against 8.2).  Past those it starts
 // at 320 rows; in front of that it would be faster as well (257 rows of 3 x 512 into 512 columns 12.2 -> 8.7), but there this path's results are the library's
 // bit for bit, which callers hold it to.
-bool output_panel_shape(const HstuOutputArgs* a, int most_d = 512, int path = 0) {
+bool output_panel_shape(const HstuOutputArgs* a, int most_d = 512) {
     const int64_t d = (int64_t)a->heads * a->linear_dim;
-    if ((a->path != 0 && a->path != path) || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return false;
+    if (a->path != 0 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return false;
     if (a->d_out % 128 != 0 || a->d_out > 8192 || d % 128 != 0 || d > most_d) return false;
     if (!a->group_norm) return true;
     const int lanes = a->linear_dim / 8;
@@ -376,14 +376,14 @@ int64_t output_panel_tail(const HstuOutputArgs* a) {
     return full > 0 && tail > 0 && (tail + 63) / 64 * blocks <= 256 ? tail : 0;
 }
 
-// path = 0 and 2: the one kernel whose workgroups own 128 rows and 512 columns, for all three blocks.  It takes calls that give more than half of the CUs an item -- up to there its time is
+// path = 0: the one kernel whose workgroups own 128 rows and 512 columns, for all three blocks.  It takes calls that give more than half of the CUs an item -- up to there its time is
 // that of one item and the kernels above are faster: us, without / with it: 3 x 512 into 512 columns, 14000 rows (110 items) 38 / 39, 16500 50 / 39, 32768 77 / 61, 57819 133 / 106,
 // 136226 295 / 240; into 1024, 8192 rows 40 / 42, 9000 56 / 42, 57819 216 / 203; 3 x 256 into 512, 16384 rows 23.2 / 24.1, 17000 30.6 / 24.3, 136226 183 / 147; 3 x 384, 14000 rows
 // 31 / 34, 17000 41 / 35, 57819 112 / 89.  Where the panel kernel takes less (fp16, rows of 1024) from 100 items on: 3 x 512, fp16, 12000 rows 37 / 39, 14000 42 / 38; 3 x 1024, 10000
 // rows 61 / 65 (fp16), 14000 85 / 69 (both types), 57819 236 / 187.
 bool output_wide_shape(const HstuOutputArgs* a) {
     const int d = a->heads * a->linear_dim;
-    if (!output_panel_shape(a, 1024, 2) || a->d_out % hstu::kOutWideCols != 0 || (d != 256 && d != 384 && d != 512 && d != 1024)) return false;
+    if (!output_panel_shape(a, 1024) || a->d_out % hstu::kOutWideCols != 0 || (d != 256 && d != 384 && d != 512 && d != 1024)) return false;
     if (output_blocks(a) != 3 || (a->group_norm && a->heads > hstu::kOutWideHeads)) return false;
     return a->attn_row_stride < (1 << 22) && a->u_row_stride < (1 << 22);  // 32-bit byte offsets within an item
 }
@@ -398,7 +398,7 @@ bool output_takes_wide(const HstuOutputArgs* a) {
 // rows (232 past a round) 91 / 73, 40960 93 / 82, 136226 252 / 240; 45000, one and a half of the panel kernel's rounds, 95 / 98; into 1024, 20000 rows 88 / 77).
 int64_t output_wide_tail(const HstuOutputArgs* a) {
     const int blocks = a->d_out / hstu::kOutWideCols;
-    if (!output_panel_shape(a, 512, 2) || 256 % blocks != 0) return 0;
+    if (!output_panel_shape(a) || 256 % blocks != 0) return 0;
     const int64_t tail = a->rows % (256 / blocks * hstu::kOutWideRows);
     return tail < a->rows && tail * blocks <= 8192 ? tail : 0;
 }

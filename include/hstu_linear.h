@@ -121,7 +121,7 @@ typedef struct HstuOutputArgs {
     int32_t path;              /* 1 = library path (norm-mul kernel + hipBLASLt); 2 = concatenating path (norm-mul kernel
                                   + hand-written GEMM over the blocks where they are): needs d_out a multiple of 256 and heads *
                                   linear_dim a multiple of 64 (and, with group norm, no SiLU on a copied u), else status
-                                  -6 (a call that the kernel of d_out a multiple of 512 below takes goes there); 0 = one kernel for the whole step (no workspace) where it is faster: without
+                                  -6; 0 = one kernel for the whole step (no workspace) where it is faster: without
                                   dropout, heads * linear_dim a multiple of 128 up to 512, up to 256 rows where its
                                   workgroups of 32 rows x 32 columns run at once, and from 320 rows on, u not activated,
                                   d_out a multiple of 128, to a size that depends on both widths and the type, past it where d_out is a

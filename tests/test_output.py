@@ -337,6 +337,7 @@ def test_output_takes_one_kernel_where_it_is_faster(N, H, ld, D, copied, group_n
 
     assert (need() == 0) == taken
     assert need(dropout_ratio=0.1) > 0 and need(silu_u=1) > 0 and need(path=1) > 0  # (what it does not do)
+    assert D % 256 != 0 or need(path=2) > 0  # (asked for: the norm-multiply kernel and the GEMM)
 
 
 @pytest.mark.gpu
@@ -379,7 +380,8 @@ def test_compute_output_past_a_round_of_the_concat_gemm(pkg, dev, N, H, D, dtype
 @pytest.mark.parametrize("N", [33000, 257])
 def test_compute_output_concat_gemm_on_views_of_wider_buffers(pkg, dev, N):
     """u as the column slice of a [N, 4 * 512] buffer (what the producer leaves), attn as a slice of a padded one: the
-    GEMM kernel reads them through their row strides.  N = 33000 also takes this path when none is asked for."""
+    GEMM kernel reads them through their row strides, in the same order of sums whatever the row count.  When no path is asked for, 33000 rows go to the
+    kernel of 128 rows x 512 columns per workgroup, whose sums are in another order, and 257 to the library."""
     print(f"[case] concat-gemm output on strided views N={N}", flush=True)
     H, ld, D = 4, 128, 512
     attn, u, x, nw, nb, w = _inputs(77 + N, N, H, ld, D, 3, False, torch.bfloat16)
@@ -395,7 +397,14 @@ def test_compute_output_concat_gemm_on_views_of_wider_buffers(pkg, dev, N):
     torch.cuda.synchronize()
     _close(got, O.compute_output(attn, u, x, nw, nb, w, 1e-6, concat_u=True, concat_x=True), "views: out vs fp32 oracle")
     _close(got, lib.float().cpu(), "views: out vs library path")
-    assert torch.equal(auto, got if N >= 32768 else lib)
+    if N == 257:
+        assert torch.equal(auto, lib)
+        return
+    _close(auto, O.compute_output(attn, u, x, nw, nb, w, 1e-6, concat_u=True, concat_x=True), "views: automatic choice vs fp32 oracle")
+    _close(auto, got.float().cpu(), "views: automatic choice vs GEMM")  # (the same rounded operands, sums in fp32, rounded once)
+    few = 8000
+    first = pkg.hstu_compute_output(attn_view[:few], u_view[:few], args[2][:few], *args[3:], path=2)
+    assert torch.equal(got[:few], first) and not torch.equal(auto, got)
 
 
 @pytest.mark.gpu
@@ -416,8 +425,8 @@ def test_compute_output_concat_gemm_other_widths(pkg, dev, D):
 
 @pytest.mark.gpu
 def test_compute_output_at_the_benchmark_size(pkg, dev):
-    """524288 rows, 3 x 512 -> 512 (the size of `bench.py --workload output`): the automatic choice is the concatenating
-    GEMM and it agrees with the library path everywhere; a zero weight returns the residual bit for bit (every row block
+    """524288 rows, 3 x 512 -> 512 (the size of `bench.py --workload output`): the automatic choice (the kernel of 128 rows x 512 columns per
+    workgroup) and the concatenating GEMM agree with the library path everywhere; a zero weight returns the residual bit for bit (every row block
     and both column halves are stored, none twice with different values); rows picked across the whole range, the last
     one included, against the fp32 oracle."""
     print("[case] output at 524288 rows", flush=True)
@@ -432,14 +441,16 @@ def test_compute_output_at_the_benchmark_size(pkg, dev):
     auto = pkg.hstu_compute_output(*args)
     got = pkg.hstu_compute_output(*args, path=2)
     lib = pkg.hstu_compute_output(*args, path=1)
-    zero = pkg.hstu_compute_output(attn, u, x, nw, nb, 1e-6, torch.zeros_like(w), H, ld, 0.0, False, True, True, "none", False, False, path=2)
     torch.cuda.synchronize()
-    assert torch.equal(auto, got) and torch.equal(zero, x)
-    diff = (got.float() - lib.float())
-    assert float(diff.norm() / lib.float().norm()) <= 1e-2 and float(diff.abs().max()) <= 2e-2 * float(lib.float().abs().max())
     rows = torch.tensor([0, 1, 255, 256, 257, 70001, 262143, 262144, 400000, N - 257, N - 2, N - 1], device=dev)
     ref = O.compute_output(attn[rows].cpu(), u[rows].cpu(), x[rows].cpu(), nw.cpu(), nb.cpu(), w.cpu(), 1e-6, concat_u=True, concat_x=True)
-    _close(got[rows], ref, "benchmark size: sampled rows vs fp32 oracle")
+    for path, out in ((0, auto), (2, got)):
+        zero = pkg.hstu_compute_output(attn, u, x, nw, nb, 1e-6, torch.zeros_like(w), H, ld, 0.0, False, True, True, "none", False, False, path=path)
+        assert torch.equal(zero, x), path
+        diff = out.float() - lib.float()
+        assert float(diff.norm() / lib.float().norm()) <= 1e-2 and float(diff.abs().max()) <= 2e-2 * float(lib.float().abs().max()), path
+        _close(out[rows], ref, f"benchmark size: sampled rows vs fp32 oracle, path {path}")
+    assert not torch.equal(auto, got)  # (two kernels)
 
 
 @pytest.mark.gpu
