@@ -969,7 +969,7 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
         output_split(a, a->rows - tail, first, last);
         const int rc = launch_output_wide(&first, stream);
         if (rc != 0) return rc;
-        return launch_output_panel(&last, hstu::output_panel_form(tail, a->heads * a->linear_dim, a->d_out, a->dtype == 0), stream);
+        return launch_output_panel(&last, hstu::output_panel_tail_form(tail, a->d_out), stream);
     }
     if (const int form = output_panel_form(a); form >= 0) return launch_output_panel(a, form, stream);
     if (output_takes_rows(a)) {
@@ -985,7 +985,7 @@ int hstu_output_forward(const HstuOutputArgs* a, void* stream_) {
         output_split(a, a->rows - tail, first, last);
         const int rc = launch_output_fused(&first, stream);
         if (rc != 0) return rc;
-        return launch_output_panel(&last, hstu::output_panel_form(tail, a->heads * a->linear_dim, a->d_out, a->dtype == 0), stream);
+        return launch_output_panel(&last, hstu::output_panel_tail_form(tail, a->d_out), stream);
     }
     if (!a->workspace) return -1;
     if ((size_t)a->workspace_bytes < joined_bytes(a) + kGemmScratch || ((uintptr_t)a->workspace & 255) != 0) return -4;

@@ -63,6 +63,9 @@ inline int output_panel_form(int64_t rows, int d, int n, bool bf16) {
     return large <= (bf16 || n == 256 ? 512 : 256) ? kPanel64x256 : -1;
 }
 
+// The form for the rows at the end of another kernel's call, at most a round of the 64 x 256 workgroups (n a multiple of 256).
+inline int output_panel_tail_form(int64_t rows, int n) { return (rows + 31) / 32 * (n / 128) <= 512 ? kPanel32x128 : kPanel64x256; }
+
 template <class TT, bool GROUP, int D, int RB, int NW>
 __global__ __launch_bounds__(NW * 64, 2) void hstu_output_panel_kernel(const OutputPanelParams p) {
     typedef typename TT::vec8 vec8;

@@ -39,7 +39,10 @@ template <class TT, bool GROUP, int D>
 int launch_form(const hstu::OutputPanelParams& p, int form, hipStream_t stream) {
     if constexpr (D <= 256)
         if (form == hstu::kPanel64x128) return launch_shape<TT, GROUP, D, 2, 4>(p, stream);
-    return form == hstu::kPanel32x128 ? launch_shape<TT, GROUP, D, 1, 4>(p, stream) : launch_shape<TT, GROUP, D, 2, 8>(p, stream);
+    if (form == hstu::kPanel32x128) return launch_shape<TT, GROUP, D, 1, 4>(p, stream);
+    if (form == hstu::kPanel64x256 && p.n % 256 == 0) return launch_shape<TT, GROUP, D, 2, 8>(p, stream);
+    hstu_linear_set_last_error("output panel kernel: no such form for this shape");
+    return -6;
 }
 
 template <class TT, bool GROUP>
@@ -97,7 +100,7 @@ int hstu_output_wide_launch(const hstu::OutputPanelParams& p, bool bf16, bool gr
     return group ? launch_wide_width<hstu::Fp16, true>(p, stream) : launch_wide_width<hstu::Fp16, false>(p, stream);
 }
 
-// p.nm.d: 128, 256, 384 or 512; form: one that output_panel_form gives for it
+// p.nm.d: 128, 256, 384 or 512; form: one that output_panel_form or output_panel_tail_form gives for it
 int hstu_output_panel_launch(const hstu::OutputPanelParams& p, int form, bool bf16, bool group, hipStream_t stream) {
     if (bf16) return group ? launch_width<hstu::Bf16, true>(p, form, stream) : launch_width<hstu::Bf16, false>(p, form, stream);
     return group ? launch_width<hstu::Fp16, true>(p, form, stream) : launch_width<hstu::Fp16, false>(p, form, stream);
