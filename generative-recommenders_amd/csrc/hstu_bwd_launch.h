@@ -41,6 +41,34 @@ auto both_kernel(std::false_type) {
     return hstu::hstu_bwd_dkdv_kernel<TT, DQK, DV, kBwdWaves, kBwdTile, false>;  // (not launched)
 }
 
+// One launch for both kernels' items while few of them leave the chip idle: two latencies become one.  An item of the one launch holds what the larger of the two
+// kernels needs: with 128 columns a CU alone, up to 64 columns two or three fit.  `items` is counted from the sizes the host knows (rows / 128 and one more per
+// sequence, no more than the grid), as if every XCD had as many as the busiest, since fewer than 8 pairs of sequence and head lie on as many XCDs; `len` is at most twice the
+// mean length.  us, two launches / one (a count in front: items):
+//   128 columns, len to 128    128 19.5 / 12.4, 332 21.4 / 21.9 (128 of 24 .. 60 rows, 4 heads, 31 / 35)
+//                to 256        196 32.3 / 24.6 (256 of 20 .. 250, 1 head, 54 / 64)
+//                to 2048       296 94.6 / 84.9, 410 139 / 137; contextual rows, which make dQ's first block of a sequence the longest chain, past 768 rows only while each has a
+//                              CU: 116 111 / 107 (8 of 1000 .. 1200, 2 heads, 168 / 183)
+//                beyond        256 220 / 146, 312 264 / 227, 396 365 / 361, 504 442 / 497, 616 647 / 776; contextual: 4 of 1600 .. 6400, 1 head, 403 / 464
+//                windows that make the chains as long as one another, of short and of long sequences: 144 62.9 / 44.0, 176 31.5 / 33.5, 192 62.8 / 67.4, 268 162 / 168
+//   64 columns, len to 256     384 36.3 / 28.2, 432 28.4 / 30.8 (128 of 20 .. 250, 4 heads, 52 / 57)
+//                beyond        576 409 / 320, 752 205 / 190, 824 689 / 651, 936 1218 / 1363
+// Workgroups that find no rows (max_seq_len far above the lengths) cost more than those of the two kernels do.  128 columns: a grid of 960 32.9 / 30.4, 1304 61 / 86, 1760 66 / 92,
+// 2160 73 / 93; 64 columns: 3744 81 / 58, 5600 31 / 40, 60144 137 / 211.
+inline bool one_launch(int dqk, int dv, int64_t batch, int64_t heads, int64_t rows, int64_t max_seq_len, int64_t window, bool contextual, int64_t grid) {
+    if (batch <= 0 || heads <= 0) return false;
+    const int64_t pairs = batch * heads, upper = heads * (rows / 128 + batch);
+    int64_t items = upper < grid ? upper : grid;
+    if (pairs < 8) items = items * 8 / pairs;
+    const int64_t len = max_seq_len < 2 * rows / batch ? max_seq_len : 2 * rows / batch;
+    if (dqk <= 64 && dv <= 64) return grid <= 4096 && items <= (len <= 256 ? 384 : 768);
+    if (grid > 1024) return false;
+    if (window > 0 && window < len / 2 && (len <= 256 || len > 1400)) return items <= 144;
+    if (contextual && max_seq_len > 768) return max_seq_len <= 2048 && items <= 256;
+    if (len <= 256) return items <= (len <= 128 ? 128 : 256);
+    return items <= (len <= 2048 ? 512 : 384);
+}
+
 template <class TT, int DQK, int DV>
 int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     // three tile slots for the key-stationary kernel, two for the other; + 64: transposing reads of a 16-wide tile's unused half
@@ -86,25 +114,8 @@ int launch_bwd(const hstu::BwdParams& bp, hipStream_t stream) {
     }
     const unsigned grid = (unsigned)bp.f.slots_per_xcd * 8;
     if constexpr (kPairedDims) {
-        // One launch for both kernels' items while few of them leave the chip idle: two latencies become one.  us, two launches / one: 8 sequences of 20 .. 150 rows, 2
-        // heads of 64 / 128 23.0 / 15.1; 4 of 500 .. 1500, 4 heads, 168 items each, 128 / 128 114 / 71; 16 of 100 .. 768, 64 / 32, fp32, 64.5 / 47.2.  An item of the one
-        // launch holds what the larger of the two kernels needs, with 128 columns a CU alone, so that more items than CUs pay where they differ in length: 32 of
-        // 100 .. 600, 4 heads, 420 items, 80 / 73; not the short (256 of 20 .. 250, 1 head, 384 items 54 / 64; 128 of 24 .. 60, 4 heads 31 / 35) nor the long (4 of
-        // 1000 .. 4000, 344 items 238 / 275).  Up to 64 columns two or three fit: 2 of 3000 .. 6000, 8 heads, 64 / 64, 632 items 318 / 278, 128 of 20 .. 250, 780
-        // items 52 / 57; 256 of 20 .. 250, 1 head, 32 / 32, 384 items 26 / 28.
-        // Long ones with 128 columns pay while both halves have a CU per item (forward and backward: 5 of 2100 .. 4200, 1 head, 112 items 329 / 249; 1 of 5700, 4 heads, 176
-        // items 468 / 438; 4 of 1600 .. 6400, 2 heads, 206 items 446 / 455).  Contextual rows make dQ's first block of a sequence the longest chain by far, and behind an item
-        // of the other kind it is longer still: 4 of 1600 .. 6400, 2 heads 598 / 745, 112 items 403 / 464; 8 of 1000 .. 1200, 304 items 168 / 183; but 8 of 300 .. 1500, 122 items
-        // 149 / 128 and 16 of 100 .. 768, 240 items 100 / 81.
-        const int64_t upper = (int64_t)bp.f.H * (bp.total_q / kBwdRows + bp.f.B);  // items at most, as the grid
-        const int64_t items = upper < (int64_t)grid ? upper : (int64_t)grid, len = bp.f.max_seq_len;
-        const bool ctx = bp.f.c > 0;
-        const int64_t most = DQK <= 64 && DV <= 64 ? (len <= 256 ? 384 : 768)
-                             : len <= 128          ? 128
-                             : len <= 256          ? 256
-                             : len <= 2048         ? (ctx && len > 768 ? 256 : 512)
-                                                   : (ctx ? 0 : 192);
-        if (!bp.ds && paired && items <= most) {
+        const bool one = one_launch(DQK, DV, bp.f.B, bp.f.H, bp.total_q, bp.f.max_seq_len, bp.f.w, bp.f.c > 0, grid);
+        if (!bp.ds && paired && one) {
             hipLaunchKernelGGL(k12, dim3(grid * 2), dim3(hstu::kBwdPpWaves * 64), smem1p, stream, bp);
             const hipError_t e = hipGetLastError();
             if (e == hipSuccess) return HSTU_OK;

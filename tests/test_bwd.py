@@ -574,3 +574,33 @@ def test_gradients_of_one_launch_are_those_of_two(dev, dtype, dqk, dv, N, H):
         one = _direct(dev, N, 0.2, q[:L], k[:L], v[:L], dout[:L], offsets[: B + 1], dict(num_targets=tg[:B], **mask))
         for name, x, y in zip(("dq", "dk", "dv"), one, two):
             assert torch.equal(x, y[:L]), (name, mask)
+
+
+@pytest.mark.parametrize(
+    "dqk,dv,lengths,heads,longest,window,contextual,one",
+    # the sides of every line of the rule: short and long sequences, 64 and 128 columns, a window, contextual rows; fewer pairs than XCDs; a max_seq_len far above
+    # the lengths (up to 1.6 times as long in one launch), and one whose grid a launch could not hold twice
+    [(64, 128, [85] * 8, 2, 150, 0, 0, True), (128, 128, [50] * 32, 4, 100, 0, 0, True), (128, 128, [50] * 33, 4, 100, 0, 0, False), (64, 128, [140] * 32, 4, 250, 0, 0, True),
+     (64, 128, [140] * 33, 4, 250, 0, 0, False), (128, 32, [1200] * 12, 4, 2000, 0, 0, True), (128, 32, [1200] * 13, 4, 2000, 0, 0, False), (128, 128, [1379] * 5, 2, 1379, 0, 6, True),
+     (128, 128, [1379] * 13, 2, 1379, 0, 6, False), (128, 64, [4000] * 2, 1, 4000, 0, 0, True), (128, 64, [4000] * 2, 1, 4000, 0, 6, False), (128, 32, [7981], 2, 7981, 0, 0, False),
+     (64, 128, [2988], 1, 2988, 747, 0, False), (64, 128, [2071], 1, 2071, 517, 0, True), (64, 64, [140] * 48, 4, 250, 0, 0, True), (64, 64, [140] * 49, 4, 250, 0, 0, False),
+     (32, 64, [5469], 1, 5469, 0, 0, True), (32, 64, [14000], 1, 14000, 0, 0, False), (32, 64, [310] * 14, 8, 310, 0, 0, True), (32, 64, [310] * 14, 8, 68627, 0, 0, False),
+     (64, 128, [60], 2, 1024, 0, 0, True), (64, 128, [60], 2, 63355, 0, 0, False), (32, 32, [60], 8, 100_000_000, 0, 0, False)],
+)
+def test_which_backward_is_one_launch(tmp_path, dqk, dv, lengths, heads, longest, window, contextual, one):
+    """The rule of csrc/hstu_bwd_launch.h, compiled for the host."""
+    import os
+    import shutil
+    import subprocess
+
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("needs g++")
+    text = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "generative-recommenders_amd", "csrc", "hstu_bwd_launch.h")).read()
+    rule = text[text.index("// One launch for both kernels' items") : text.index("template <class TT, int DQK, int DV>\nint launch_bwd(")]
+    batch = len(lengths)
+    grid = (batch * heads + 7) // 8 * ((longest + 127) // 128) * 8
+    src = tmp_path / "rule.cpp"
+    src.write_text("#include <cstdint>\n" + rule + f"int main() {{ return one_launch({dqk}, {dv}, {batch}, {heads}, {sum(lengths)}, {longest}, {window}, {int(contextual > 0)}, {grid}) ? 1 : 0; }}\n")
+    subprocess.run([gxx, "-std=c++17", str(src), "-o", str(tmp_path / "rule")], check=True)
+    assert subprocess.run([str(tmp_path / "rule")]).returncode == int(one)
