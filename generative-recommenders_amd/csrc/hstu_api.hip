@@ -342,13 +342,19 @@ Plan make_plan(const HstuFwdArgs* a, size_t scratch = SIZE_MAX, bool line = true
         while (want >= 2 && pl.total() + split_counts_bytes + want * split_bytes + 256 > scratch) --want;
         if (want >= 2) s = (int)want;
         // Fewer workgroups than that per sequence: the plane's tiles as one line (decode_line), where the longest run is at least 8 tiles longer than a workgroup's part of
-        // it.  us without / with (bf16, lengths of the histories x candidates): 34 of 2400 .. 2550 x 19, 8 heads of 32 67 / 45; 18 of 250 .. 4200 x 3, 8 of 128 57 / 35; 46 of 400 .. 1600 x 3,
-        // 4 of 128 40 / 28; 39 of 650 .. 10800 x 212, 4 of 128 243 / 157; 16 of 500 .. 8000 x 512 105 / 89; 32 of 1024 .. 4096 x 256 74 / 74.  Not for shorter ones (36 of 550 x 278 38 / 52; 40 of
-        // 100 .. 400 x 30 16 / 21) nor for many row blocks (46 of 4500 .. 9000 x 389, 8 heads 798 / 877; 64 of 500 .. 4000 x 500 214 / 221).  What an item costs besides its steps, in tiles (2, 5, 9: the
-        // first 45 / 47 / 50, the last but one of the gains 91 / 89 / 87):
+        // it (14 without equal runs and with several row blocks, whose rows all go through partial sums).  us without / with (bf16, lengths of the histories x candidates): 34 of 2400 .. 2550 x 19, 8
+        // heads of 32 67 / 45; 18 of 250 .. 4200 x 3, 8 of 128 57 / 35; 46 of 400 .. 1600 x 3, 4 of 128 40 / 28; 39 of 650 .. 10800 x 212, 4 of 128 243 / 157; 16 of 500 .. 8000 x 512 105 / 89; 32 of
+        // 1024 .. 4096 x 256 74 / 74.  Not for shorter ones (36 of 550 x 278 38 / 52; 40 of 100 .. 400 x 30 16 / 21) nor for many row blocks (46 of 4500 .. 9000 x 389, 8 heads 798 / 877; 64 of
+        // 500 .. 4000 x 500 214 / 221).  Where max_seq_len is more than 2.5 times the mean length it says little about the longest: then the mean has to be that much longer (51 of 38 .. 64 x 132,
+        // max_seq_len 5666, 4 of 128 15.3 / 28.2; 49 of 2112 x 72, 45342, 8 of 128 95 / 118; 37 of 668 .. 13378 x 23, 33629, 8 of 32 213 / 102), or, beside equal runs, which such a
+        // max_seq_len makes too long, at least 8 tiles (17 of 258 .. 431 x 103, 12971, 8 of 64 17.3 / 19.9; 32 of 212 .. 4247 x 5, 9300, 8 of 32 88 / 36).
+        // What an item costs besides its steps, in tiles (2, 5, 9: the first 45 / 47 / 50, the last but one of the gains 91 / 89 / 87):
         const int weight = pl.cfg == 2 ? 8 : 4;
-        if (line && fits && runs > 0 && (max_tiles + s - 1) / s - (tiles + a->batch * weight + runs - 1) / runs >= 8 &&
-            (tiles + a->batch * weight) * runs < (1ll << 31)) {
+        const bool near_mean = 2ll * a->max_seq_len * a->batch <= 5ll * a->total_kv;
+        const long long part = runs > 0 ? (tiles + a->batch * weight + runs - 1) / runs : 0;
+        const bool pays = s > 1 ? avg_tiles >= 8 && (max_tiles + s - 1) / s - part >= 8
+                                : (near_mean ? max_tiles : avg_tiles) - part >= (num_mb > 1 ? 14 : 8);
+        if (line && fits && runs > 0 && pays && (tiles + a->batch * weight) * runs < (1ll << 31)) {
             pl.fit_runs = (int)runs, pl.line_weight = weight, pl.splits = 2;
             pl.counts_bytes = split_counts_bytes;
             pl.partial_bytes = (runs + a->batch) * run_bytes;

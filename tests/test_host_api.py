@@ -338,10 +338,23 @@ def test_fitted_runs_have_a_workgroup_each_on_any_device(backend, cus):
     drew an unused run of one head left the runs of the next one undone.)"""
     shapes = [  # batch, heads, dim, rows, delta, longest, tile configuration
         (5, 4, 128, 12000, 100, 16100, 0), (3, 3, 128, 2000, 64, 7007, 3), (2, 1, 128, 2650, 300, 5007, 0), (64, 1, 64, 210, 33, 6007, 2), (2, 2, 64, 1300, 129, 2507, 3),
-        (18, 8, 128, 2300, 3, 2636, 0), (64, 4, 64, 174, 33, 7007, 0), (20, 8, 128, 3700, 129, 6796, 2)]
+        (18, 8, 128, 2300, 3, 2636, 0), (64, 4, 64, 616, 33, 9007, 0), (20, 8, 128, 3700, 129, 6796, 2)]
     forms = set()
     for B, H, D, rows, delta, N, cfg in shapes:
         form, items, wgs = backend.plan_grid_for(B, H, D, D, B * delta, B * rows, N, delta_size=delta, tile_config=cfg, cus=cus)
         forms.add(form)
         assert form in ("fitted", "line") and items == wgs * (B if form == "line" else 1), (B, H, D, rows, delta, N, cfg)
     assert forms == {"fitted", "line"}
+
+
+@pytest.mark.parametrize(
+    "batch,heads,dim,rows,delta,longest,form",
+    # the lengths' mean and max_seq_len: both sides of 2.5 between them, with and without equal runs, one row block and several.  (With the longest that max_seq_len
+    # allows taken for granted, the calls that are not a line here and have a long max_seq_len took up to 1.8 times as long.)
+    [(18, 8, 128, 2300, 3, 2636, "line"), (51, 4, 128, 183, 132, 5666, "whole"), (49, 8, 128, 2184, 72, 45342, "whole"), (37, 8, 32, 7046, 23, 33629, "line"),
+     (32, 8, 32, 2235, 5, 9300, "line"), (17, 8, 64, 447, 103, 12971, "equal runs"), (34, 4, 128, 700, 130, 1400, "whole"), (34, 4, 128, 700, 130, 1440, "line"),
+     (3, 4, 64, 128, 22, 1113, "whole"), (40, 8, 64, 1000, 20, 2500, "line"), (40, 8, 64, 1000, 20, 2501, "whole")],
+)
+def test_which_deltas_cut_their_tiles_as_a_line(backend, batch, heads, dim, rows, delta, longest, form):
+    got = backend.plan_grid_for(batch, heads, dim, dim, batch * delta, batch * rows, longest, delta_size=delta)[0]
+    assert got == form
