@@ -380,7 +380,9 @@ int64_t output_panel_tail(const HstuOutputArgs* a) {
 // that of one item and the kernels above are faster: us, without / with it: 3 x 512 into 512 columns, 14000 rows (110 items) 38 / 39, 16500 50 / 39, 32768 77 / 61, 57819 133 / 106,
 // 136226 295 / 240; into 1024, 8192 rows 40 / 42, 9000 56 / 42, 57819 216 / 203; 3 x 256 into 512, 16384 rows 23.2 / 24.1, 17000 30.6 / 24.3, 136226 183 / 147; 3 x 384, 14000 rows
 // 31 / 34, 17000 41 / 35, 57819 112 / 89.  Where the panel kernel takes less (fp16, rows of 1024) from 100 items on: 3 x 512, fp16, 12000 rows 37 / 39, 14000 42 / 38; 3 x 1024, 10000
-// rows 61 / 65 (fp16), 14000 85 / 69 (both types), 57819 236 / 187.
+// rows 61 / 65 (fp16), 14000 85 / 69 (both types), 57819 236 / 187.  The two kernels' last round is fuller where there are more column blocks: 3 x 1024 into 1024 columns 6656 rows (104 items)
+// 61.6 / 68.5, 8957 rows (140) 114 / 71; into 1536 5504 rows (129) 67 / 69, 6778 (159) 83 / 76; into 2048 3323 rows (104) 59 / 67, 4096 (128) 63 / 68, 4477 (140) 83 / 74 (fp16); 3 x 512, fp16, into 1024
+// 7036 rows (110) 38.1 / 39.1.
 bool output_wide_shape(const HstuOutputArgs* a) {
     const int d = a->heads * a->linear_dim;
     if (!output_panel_shape(a, 1024) || a->d_out % hstu::kOutWideCols != 0 || (d != 256 && d != 384 && d != 512 && d != 1024)) return false;
@@ -391,7 +393,8 @@ bool output_takes_wide(const HstuOutputArgs* a) {
     if (!output_wide_shape(a)) return false;
     const int64_t items = (a->rows + hstu::kOutWideRows - 1) / hstu::kOutWideRows * (a->d_out / hstu::kOutWideCols);
     const int d = a->heads * a->linear_dim;
-    return items > 128 || (items > 100 && (d > 512 || hstu::output_panel_form(a->rows, d, a->d_out, a->dtype == 0) < 0));
+    if (items > (a->d_out <= 1024 ? 128 : 136)) return true;
+    return items > 100 && a->d_out == 512 && (d > 512 || hstu::output_panel_form(a->rows, d, a->d_out, a->dtype == 0) < 0);
 }
 
 // Rows at the end of its last round, one item per CU, that the panel kernel takes instead: those that are one round of that kernel's (us, without / with: 3 x 512 into 512 columns, 33000

@@ -41,26 +41,29 @@ struct OutputPanel {
     static constexpr int kLds = kPanel + NW * kRing * kTile > kRows * kSumRow ? kPanel + NW * kRing * kTile : kRows * kSumRow;
 };
 
-// Which form takes a call, -1: none.  32 x 128 while two of its workgroups per CU hold all of it (us, against 64 x 256: 3 x 512 into 512 columns, 4000
-// rows 15.7 / 17.6, 6000 rows 23.1 / 18.5; 3 x 256 into 256, 8192 rows 10.5 / 11.6, 10000 rows 12.9 / 12.3), then the larger ones, whose W is read by fewer.
+// Which form takes a call, -1: none.  What counts is the XCD that gets most workgroups: row blocks go to the eight in turn, each with all its column blocks (3 x 512 into 1536 columns,
+// 1341 rows, 504 workgroups of 32 x 128, 72 of them on one XCD: 27.7 us, as two rounds, where 64 are one; the library 23.0).  32 x 128 while two of its workgroups per CU hold all of it (us, against
+// 64 x 256: 3 x 512 into 512 columns, 4000 rows 15.7 / 17.6, 6000 rows 23.1 / 18.5; 3 x 256 into 256, 8192 rows 10.5 / 11.6, 10000 rows 12.9 / 12.3), then the larger ones, whose W is read by fewer.
 // They pay as long as the norm, made once per column block, costs less than a matrix written and read (us, the two kernels / this one):
 //   width 128: to a d_out of 1152 at any rows: 400000 rows into 1024 columns 693 / 566
 //   width 256: into 512 columns at any rows (200000: 294 / 273), into 1024 16384 rows 51 / 48, 32768 rows 87 / 91; where d_out is no multiple of 256 the
 //     two kernels are slower: 60000 rows into 640 columns 167 / 108, into 1152 206 / 181
-//   width 384, 512: two rounds of the CUs (256 columns, 32768 rows 62 / 51, 33000 rows 62 / 65; 512 columns, 16384 rows 50 / 42, 24000 rows 65 / 61, 32000 rows 80 / 81;
-//     1024 columns, 8192 rows 43 / 41, 12000 rows 57 / 61), in fp16, where the library is faster, one (512 columns, 9000 rows 34 / 38); where d_out is no multiple of 256 only
-//     the small form fits: into 384 columns 8000 rows 33 / 26, 12000 rows 38 / 38; into 640 4000 rows 32 / 25, 6000 rows 29 / 32
+//   width 384, 512: a round of the CUs, and up to 768 columns the most of a second one, half of it into 1024 (256 columns, 32768 rows 62 / 51, 33000 rows 62 / 65; 512 columns, 16384 rows 50 / 42, 24000 rows 65 / 61, 32000
+//     rows 80 / 81; 768 columns, 5440 rows, 33 workgroups on an XCD, 32.2 / 34.7, 6140 rows 48 / 35, 10877 rows, 66 of them, 42 / 51; 1024 columns, 6143 rows 47 / 36, 7040 rows, 56 of them, 36.5 / 41.0, 12000 rows 57 / 61; 1536 columns,
+//     2690 rows, 36 on an XCD, 28.4 / 35.9, 4670 rows 35.9 / 37.3; 2048 columns, 3072 rows 31.7 / 37.5), in fp16, where the library is faster, the first round (512 columns, 9000 rows 34 / 38); where
+//     d_out is no multiple of 256 only the small form fits: into 384 columns 8000 rows 33 / 26, 12000 rows 38 / 38; into 640 4000 rows 32 / 25, 6000 rows 29 / 32
 enum { kPanel32x128 = 0, kPanel64x128 = 1, kPanel64x256 = 2 };
 inline int output_panel_form(int64_t rows, int d, int n, bool bf16) {
-    const int64_t small = (rows + 31) / 32 * (n / 128), large = (rows + 63) / 64 * (n / 256);
-    if (small <= 512) return kPanel32x128;
+    const int64_t small = ((rows + 31) / 32 + 7) / 8 * (n / 128), large = ((rows + 63) / 64 + 7) / 8 * (n / 256);  // on one XCD of 32 CUs
+    if (small <= 64) return kPanel32x128;
     const bool whole = n % 256 == 0;
     if (d <= 256) {
         if (n > 1152 || (d == 256 && whole && n > 512 && rows * n > (16 << 20))) return -1;
         return whole ? kPanel64x256 : kPanel64x128;
     }
-    if (!whole) return n <= 384 && small <= 768 ? kPanel32x128 : -1;
-    return large <= (bf16 || n == 256 ? 512 : 256) ? kPanel64x256 : -1;
+    if (!whole) return n <= 384 && small <= 96 ? kPanel32x128 : -1;
+    const bool second = (bf16 || n == 256) && n <= 1024;
+    return large <= 32 || (second && large >= 36 && large <= (n > 768 ? 48 : 64)) ? kPanel64x256 : -1;
 }
 
 // The form for the rows at the end of another kernel's call, at most a round of the 64 x 256 workgroups (n a multiple of 256).

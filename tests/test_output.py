@@ -307,7 +307,7 @@ def test_compute_output_on_both_sides_of_one_round(pkg, dev, N, blocks, H, ld, D
 # (rows, heads, linear_dim, d_out, copied blocks, group norm, dtype, whether the one kernel for more rows takes it): its first row count, both sides of the
 # line between its forms of 32 x 128 and 64 x 256 (64 x 128 where d_out is no multiple of 256), rows that fill no block, every width of a row (384: lanes
 # without a chunk), one to three blocks, heads of one and of all lanes of a row, and the sizes behind the last one it takes; in the last lines the form of
-# 128 x 512, from its first size on (128 or 100 items), with one row in its last block, a second round, a last round that goes to the others (into 2048 columns more rows of it
+# 128 x 512, from its first size on (128, 136 or 100 items), with one row in its last block, a second round, a last round that goes to the others (into 2048 columns more rows of it
 # than those take by themselves), and too many heads for it
 BF, FP = torch.bfloat16, torch.float16
 PANEL_CASES = [
@@ -317,8 +317,11 @@ PANEL_CASES = [
     (8200, 8, 32, 256, 2, True, FP, True), (5600, 2, 128, 384, 2, False, BF, True), (20000, 1, 128, 640, 1, False, FP, True), (16385, 1, 128, 256, 0, True, BF, True),
     (777, 4, 128, 1024, 0, False, FP, True), (2049, 2, 64, 512, 1, False, BF, True), (40000, 1, 128, 256, 2, False, BF, True), (600, 32, 8, 256, 2, True, FP, True),
     (16385, 4, 128, 512, 2, False, BF, True), (16513, 8, 32, 512, 2, True, FP, True), (16600, 3, 128, 512, 2, False, FP, True), (12800, 4, 128, 512, 2, False, FP, False),
-    (12801, 4, 128, 512, 2, True, FP, True), (6400, 8, 128, 1024, 2, False, BF, False), (6401, 8, 128, 1024, 2, True, BF, True), (45000, 2, 128, 512, 2, False, BF, True),
+    (12801, 4, 128, 512, 2, True, FP, True), (8192, 8, 128, 1024, 2, False, BF, False), (8193, 8, 128, 1024, 2, True, BF, True), (45000, 2, 128, 512, 2, False, BF, True),
     (33001, 4, 128, 512, 2, True, BF, True), (9692, 2, 128, 2048, 2, False, BF, True), (20000, 16, 32, 512, 2, True, BF, False), (16385, 4, 128, 512, 1, False, BF, False),
+    # column blocks whose row blocks do not divide by the eight XCDs: what counts is the one that gets most
+    (1341, 4, 128, 1536, 2, False, BF, True), (2690, 4, 128, 1536, 2, False, BF, False), (5440, 4, 128, 768, 2, False, BF, False), (6140, 4, 128, 768, 2, True, BF, True),
+    (10877, 4, 128, 768, 2, False, BF, False), (6144, 4, 128, 1024, 2, False, BF, True), (6145, 4, 128, 1024, 2, False, BF, False), (3072, 4, 128, 2048, 2, False, BF, False), (4224, 8, 128, 2048, 2, False, FP, False), (4477, 8, 128, 2048, 2, False, FP, True),
 ]
 
 
