@@ -66,3 +66,43 @@ def test_runs_at_scratch_limits(pkg, dev):
         hb.mha_fwd(q, k, v, out, offs, None, N, alpha, delta, 0, 0, 0, workspace_bytes=limit)
         torch.cuda.synchronize()
         assert_parity(out, want, f"{limit} bytes")
+
+
+def test_a_line_at_scratch_limits(pkg, dev):
+    """Workspaces that hold a line's partial sums, one byte less, none: the plan falls back and the result stays."""
+    from generative_recommenders_amd.ops import hip_backend as hb
+
+    lengths, delta, heads, dim = [500 + 331 * i for i in range(20)], 129, 4, 64
+    B, N, alpha = len(lengths), max(lengths) + 7, dim**-0.5
+    q, k, v, offs, _ = make_case(13, lengths, heads, dim, delta_size=delta)
+    want = O.cached_hstu_mha_per_sequence(N, alpha, q.float(), k.float(), v.float(), offs, None)
+    sizes = (B, heads, dim, dim, B * delta, int(offs[-1]), N)
+    need = hb._plan_args(*sizes, delta, 0, 0, False, hb.HSTU_BF16, None).workspace_bytes
+    q, k, v, offs = (x.to(dev) for x in (q, k, v, offs))
+    forms = []
+    for limit in (need, need - 1, need // 4, 600, 0):
+        forms.append(hb.plan_grid_for(*sizes, delta_size=delta, workspace_bytes=limit)[0])
+        print(f"[case] a line with {limit} bytes of scratch memory: {forms[-1]}", flush=True)
+        out = torch.full((B * delta, heads, dim), float("nan"), dtype=q.dtype, device=dev)
+        hb.mha_fwd(q, k, v, out, offs, None, N, alpha, delta, 0, 0, 0, workspace_bytes=limit)
+        torch.cuda.synchronize()
+        assert_parity(out, want, f"{limit} bytes")
+    assert forms[0] == "line" and "line" not in forms[1:]
+
+
+def test_a_line_past_sequences_shorter_than_the_candidates(pkg, dev):
+    """They have no result (the caller's contract is broken for them): their rows stay as they were, the others' are what they are without the line."""
+    from generative_recommenders_amd.ops import hip_backend as hb
+
+    lengths, delta, heads, dim = [2000, 30, 2600, 0] + [2000 + 37 * i for i in range(14)] + [1], 64, 8, 128
+    B, N, alpha = len(lengths), 2700, dim**-0.5
+    assert hb.plan_grid_for(B, heads, dim, dim, B * delta, sum(lengths), N, delta_size=delta)[0] == "line"
+    print("[case] a line past short sequences", flush=True)
+    q, k, v, offs = (x.to(dev) for x in make_case(14, lengths, heads, dim, delta_size=delta)[:4])
+    got, whole = (torch.full((B, delta, heads, dim), 7.0, dtype=q.dtype, device=dev) for _ in range(2))
+    hb.mha_fwd(q, k, v, got.view(B * delta, heads, dim), offs, None, N, alpha, delta, 0, 0, 0)
+    hb.mha_fwd(q, k, v, whole.view(B * delta, heads, dim), offs, None, N, alpha, delta, 0, 0, 0, kv_splits=1)
+    torch.cuda.synchronize()
+    short = torch.tensor([n < delta for n in lengths], device=dev)
+    assert bool((got[short] == 7.0).all()) and bool((whole[short] == 7.0).all())
+    assert float((got[~short].float() - whole[~short].float()).norm() / whole[~short].float().norm()) <= 2.0**-8

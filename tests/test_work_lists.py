@@ -54,3 +54,29 @@ def test_items_with_and_without_lists(pkg, dev, batch, heads, longest, d):
             continue
         one = O.hstu_mha_per_sequence(longest, 0.125, q[lo:hi].float(), k[lo:hi].float(), v[lo:hi].float(), torch.tensor([0, hi - lo]), num_targets=t[b : b + 1].long())
         assert_parity(plain[lo:hi], one, f"items of sequence {b}")
+
+
+@pytest.mark.parametrize("batch,heads,longest,window,contextual", [(520, 8, 128, 0, 10), (70, 8, 512, 100, 6), (300, 4, 640, 0, 130), (33, 8, 1000, 200, 3)])
+def test_lists_with_contextual_rows(pkg, dev, batch, heads, longest, window, contextual):
+    """The one-group kernel through lists where a sequence's first row block is its longest: against the same call without scratch memory, which deals the row blocks
+    arithmetically, and some sequences against the oracle."""
+    from generative_recommenders_amd.ops import hip_backend as hb
+
+    print(f"[case] lists with {contextual} contextual rows {batch} x {heads} heads up to {longest}, window {window}", flush=True)
+    gen = torch.Generator().manual_seed(batch + contextual)
+    lengths = torch.randint(contextual + 3, longest + 1, (batch,), generator=gen).tolist()
+    lengths[0], lengths[1], lengths[-1] = longest, 0, contextual + 3
+    q, k, v, offs, t = make_case(batch, lengths, heads, 64, targets=[min(3, n) for n in lengths])
+    form, items, wgs = hb.plan_grid_for(batch, heads, 64, 64, q.shape[0], q.shape[0], longest, tile_config=3)
+    assert form == "whole" and items > wgs  # (counters and lists, not a workgroup for every item there could be)
+    dq, dk, dv, do, dt = (x.to(dev) for x in (q, k, v, offs, t))
+    got, plain = (torch.full_like(dv, float("nan")) for _ in range(2))
+    for out, limit in ((got, None), (plain, 0)):
+        hb.mha_fwd(dq, dk, dv, out, do, dt, longest, 0.125, 0, window, contextual, 0, tile_config=3, workspace_bytes=limit)
+    torch.cuda.synchronize()
+    assert torch.equal(got, plain) and bool(torch.isfinite(got).all())
+    for b in (0, 2, batch // 2, batch - 1):
+        lo, hi = int(offs[b]), int(offs[b + 1])
+        one = O.hstu_mha_per_sequence(longest, 0.125, q[lo:hi].float(), k[lo:hi].float(), v[lo:hi].float(), torch.tensor([0, hi - lo]), num_targets=t[b : b + 1].long(),
+                                      max_attn_len=window, contextual_seq_len=contextual)
+        assert_parity(got[lo:hi], one, f"contextual items of sequence {b}")
