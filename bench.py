@@ -313,7 +313,7 @@ def run_linear(name, args, pkg, torch):
         attn_flops = workloads.algorithmic_flops(wl)
         flops = 2.0 * L * d_model * n_out + attn_flops + 2.0 * L * 3 * H * D * d_model
         nbytes = 2.0 * (L * d_model * 3 + d_model * n_out + 3 * H * D * d_model)  # x in (twice: the residual), out
-        kernel = "hstu_uqvk_wide_kernel + hstu_fwd_stream_kernel + hstu_norm_mul_kernel + hstu_output_gemm_kernel"
+        kernel = "hstu_uqvk_wide_kernel + hstu_fwd_stream_kernel + hstu_output_wide_kernel"
         metric = "STU layer fwd TFLOP/s (uqvk, attention, output; 64 x 8192 tokens, d_model 512, H4 d128)"
     elif name in ("uqvk", "layernorm"):
         nw, nb = rnd(d_model, scale=0.1, shift=1.0), rnd(d_model, scale=0.1)
@@ -338,8 +338,8 @@ def run_linear(name, args, pkg, torch):
             step = lambda: hstu_compute.hstu_compute_output(attn, u, x, nw, nb, 1e-6, w, H, D, 0.0, False, True, True, "none", False, False, path=args.output_path)  # noqa: E731
             cpu = lambda r: output_oracle.compute_output(attn[:r].float().cpu(), u[:r].float().cpu(), x[:r].float().cpu(), nw.float().cpu(), nb.float().cpu(), w.float().cpu(), 1e-6, concat_u=True, concat_x=True)  # noqa: E731
             flops, nbytes = 2.0 * L * 3 * H * D * d_model, 2.0 * (2 * L * H * D + 2 * L * d_model + 3 * H * D * d_model)
-            kernel = ("hstu_norm_mul_kernel + hipBLASLt GEMM (residual as C operand)" if args.output_path == 1
-                      else "hstu_norm_mul_kernel (y alone) + hstu_output_gemm_kernel")
+            kernel = {1: "hstu_norm_mul_kernel + hipBLASLt GEMM (residual as C operand)",
+                      2: "hstu_norm_mul_kernel (y alone) + hstu_output_gemm_kernel"}.get(args.output_path, "hstu_output_wide_kernel")
             metric = "hstu_compute_output fwd TFLOP/s (524288 tokens, 3 x 512 -> 512)"
         else:
             step = lambda: hstu_compute.norm_mul_dropout(attn, u, nw, nb, 1e-6, 0.0, False, False, True, True, "none")  # noqa: E731
@@ -360,7 +360,8 @@ def run_linear(name, args, pkg, torch):
     else:
         roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": round(gbs / PEAK_HBM_GBS, 4)}
         value, unit = round(gbs, 1), "GB/s"
-    traffic = traffic_fields(name + "_library" if (name == "uqvk" and args.uqvk_path == 1) or (name == "output" and args.output_path == 1) else name)
+    traffic = traffic_fields(name + "_library" if (name == "uqvk" and args.uqvk_path == 1) or (name == "output" and args.output_path == 1)
+                             else name + "_gemm" if name == "output" and args.output_path == 2 else name)
     if name == "cfg5_e2e":
         roof["note"] = "both kernels' flops over their summed time, against the bf16 peak (the attention's own peak is fp8's: see workload cfg5)"
     roof.update({**traffic, "kernel": kernel, **timing_fields(st),
@@ -475,7 +476,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=5)
     ap.add_argument("--workload", default="headline")
     ap.add_argument("--tile-config", type=int, default=0)
-    ap.add_argument("--output-path", type=int, default=0, help="workload output: 0 / 2 = norm-multiply kernel + concatenating GEMM kernel, 1 = norm-multiply kernel + hipBLASLt")
+    ap.add_argument("--output-path", type=int, default=0, help="workload output: 0 = one kernel for the whole step, 1 = norm-multiply kernel + hipBLASLt, 2 = norm-multiply kernel + concatenating GEMM kernel")
     ap.add_argument("--uqvk-path", type=int, default=0, help="workload uqvk: 0 / 2 = fused kernel, 1 = layer-norm kernel + hipBLASLt")
     ap.add_argument("--bwd-form", choices=["stored", "recompute"], default="stored",
                     help="workloads bwd, bwd_cfg3: dS stored in scratch memory and dq streamed from it, or the scores recomputed for dq")
