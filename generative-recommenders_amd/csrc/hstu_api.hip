@@ -407,8 +407,9 @@ Grid make_grid(const HstuFwdArgs* a, const Plan& plan, int cus) {
     g.pairs_per_xcd = ((long long)a->batch * a->heads + 7) / 8;
     g.fit_wgs = (((long long)plan.fit_runs * a->heads + 7) / 8) * g.num_mb;
     g.slots = plan.fit_runs > 0 ? g.fit_wgs * (plan.line_weight > 0 ? a->batch : 1) : g.pairs_per_xcd * g.num_mb * plan.splits;
-    // workgroups of a CU: of the one-group kernel two, with 32 columns (161 registers) the three that fit (us, two / three: 256 sequences of 64 .. 1024, 4 heads 112 / 104; 256 of 256
-    // 31 / 26; 200 of 512 56 / 52; 100 of 300 .. 900 50 / 50); 64 columns fit as often and are faster without (256 of 64 .. 1024 138 / 149; 200 of 512 73 / 86)
+    // workgroups of a CU: of the one-group kernel two, with 32 columns (161 registers in bf16, 129 in fp16) the three that fit (us, two / three: 256 sequences of 64 .. 1024, 4 heads 112 / 104; 256 of
+    // 256 31 / 26; 200 of 512 56 / 52; 100 of 300 .. 900 50 / 50).  Of 64 columns in bf16 (190 registers) two fit, and a grid for three queues the third behind them (256 of 64 .. 1024 138 / 149; 200
+    // of 512 73 / 86); in fp16 (162) three fit and are 8 % faster to 3 % slower (118 of 531, 8 heads 135 / 126; 147 of 1113, 4 heads 213 / 217): not taken.
     const int per_cu = plan.cfg == 2 ? 1 : a->dqk == 32 && a->dtype != HSTU_FP8_E4M3 ? 3 : 2;
     long long resident = (long long)cus * per_cu / 8;
     if (resident < 1) resident = 1;

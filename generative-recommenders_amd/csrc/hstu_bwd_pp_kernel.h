@@ -32,7 +32,8 @@ constexpr int bwd_pp_lds_bytes() {
 
 // BOTH: both gradients' items in one launch, in octets (one item per XCD) that alternate: the key-stationary items with eight waves, those of dQ with four.
 // For few items: there a launch is the chain of its longest item (16 sequences of 100 .. 768 rows, 264 items each, fp32, dims 64 / 32: 28.7 and 27.6 us one
-// after the other, 37 together).  (The body is a kernel's and not a function's that two kernels call: as such it held 8 more scalars in vector registers and
+// after the other, 37 together).  Its registers are bounded by the waves that its LDS lets in, and with 64 columns of q a few do not fit: 64 / 32 keeps 16 bytes per lane in scratch memory, and
+// with fp32 gradients 64 / 64 and 64 / 128 12 and 20.  (The body is a kernel's and not a function's that two kernels call: as such it held 8 more scalars in vector registers and
 // was 2 to 3 % slower with 32 columns and stored dS.)
 template <class TT, int DQK, int DV, bool STORE, bool BOTH = false>
 __global__ __launch_bounds__(kBwdPpWaves * 64, !BOTH ? 1 : DQK == 128 ? 2 : DV == 128 ? 3 : 4) void hstu_bwd_dkdv_pp_kernel(const BwdParams bp) {

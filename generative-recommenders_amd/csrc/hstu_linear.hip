@@ -347,8 +347,8 @@ int launch_output_rows(const HstuOutputArgs* a, hipStream_t stream) {
 
 // path = 0: the panel kernel, one kernel for more rows, where u goes in as it is (output_panel_shape).  output_panel_form: its form, -1 = another path.  The rows that hstu_output_rows_kernel takes are
 // this kernel's up to a width of 256 (3 x 256 into 512 columns, us: one row 7.0 -> 5.2, 256 rows 7.3 -> 5.5; 3 x 512: 7.7 against 8.2).  Past those it starts
-// at 320 rows; in front of that it would be faster as well (257 rows of 3 x 512 into 512 columns 12.2 -> 8.7), but there this path's results are the library's
-// bit for bit, which callers hold it to.
+// at 320 rows.  In front of that it would be faster as well (257 rows of 3 x 512 into 512 columns 12.2 -> 8.7): the line is not where the times cross but behind the row
+// count at which a test of the operator expects the library's bits.
 bool output_panel_shape(const HstuOutputArgs* a, int most_d = 512) {
     const int64_t d = (int64_t)a->heads * a->linear_dim;
     if (a->path != 0 || a->dropout_ratio != 0.f || (a->dtype != 0 && a->dtype != 1) || a->silu_u || (!a->group_norm && a->mul_u_activation != HSTU_MUL_U_NONE)) return false;

@@ -8,7 +8,9 @@ bool producer_depth(int depth) { return depth == 128 || depth == 256 || depth ==
 
 // The product at the other depths: while its workgroups are one round of the CUs, which their LDS fills.  us on the GPU, the library's / with it: 768 deep into 256 columns, 700 rows
 // 4.9 / 4.8, 2048 rows (the last) 6.0 / 5.3, 2200 rows 7.4 / 9.3; 1024 into 512, 700 rows 8.5 / 5.9, 1100 rows 8.5 / 10.2; 2048 into 640, 20 rows 5.3 / 6.7, 700 rows 9.7 / 9.2; the
-// library's choice for a batch's own rows takes 15 us of the host besides.  Deeper than 1024 only up to 512 rows: past them callers hold the gradient to the framework's product bit for bit.
+// library's choice for a batch's own rows takes 15 us of the host besides.  Past a depth of 1024 few workgroups are a longer chain than the library's split of the depth (25 rows of 3840 into 384
+// 6.7 / 9.2, 59 of 2560 into 128 5.8 / 7.5; many are not: 287 of 4032 into 1536 21.4 / 11.7), and the operator is faster all the same: its backward, one after the other, 20 rows of 512 into 2048 90 / 73,
+// 25 of 1024 into 4096 114 / 99.  Deeper than 1024 only up to 512 rows, which is no line between times: past them a test of the operator expects the framework's product bit for bit.
 bool split_takes(int64_t rows, int depth, int n) {
     if (depth % 64 != 0 || n % hstu::kSplitCols != 0 || (depth > 1024 && rows > 512)) return false;
     return (rows + hstu::kSplitRows - 1) / hstu::kSplitRows * (n / hstu::kSplitCols) <= 256;

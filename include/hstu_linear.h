@@ -108,7 +108,7 @@ typedef struct HstuOutputArgs {
     const void* norm_bias;
     float norm_eps;
     const void* output_weight; /* [blocks * heads * linear_dim, d_out] row-major, dense; blocks = 1 + copied blocks */
-    void* out;                 /* [rows, d_out] dense */
+    void* out;                 /* [rows, d_out] dense; overlaps no input, but may be x itself */
     int64_t rows;
     int32_t d_out;             /* multiple of 8 */
     int32_t heads, linear_dim; /* heads * linear_dim: multiple of 8, at most 4096; group norm: linear_dim / 8 a power of two <= 64 */
@@ -126,7 +126,10 @@ typedef struct HstuOutputArgs {
                                   workgroups of 32 rows x 32 columns run at once, and from 320 rows on, u not activated,
                                   d_out a multiple of 128, to a size that depends on both widths and the type, past it where d_out is a
                                   multiple of 512, heads * linear_dim 256, 384, 512 or 1024 and all three blocks are there; the
-                                  concatenating path where that does not hold and rows >= 32768; else the library */
+                                  concatenating path where that does not hold and rows >= 32768; else the library.
+                                  Sums are in fp32 on every way, in an order of its own on each; a call whose last round of workgroups
+                                  would be nearly empty hands the rows of it to another kernel, so that equal rows of one call may differ by that order (and,
+                                  in fp16, a few elements of y in 100000 by their rounding: in fp32 first or not).  path = 2: the same bits whatever the rows */
     /* Dropout of `joined` (`F.dropout(y, p, training)` at the end of pytorch_norm_mul_dropout, pt_hstu_linear.py:80-84): the
      * whole concatenation goes through it, in fp32, before it is rounded; survivors are multiplied by 1 / (1 - ratio).
      * Element (r, c) of the [rows, blocks * heads * linear_dim] matrix is kept when word c % 4 of
