@@ -47,14 +47,15 @@ auto both_kernel(std::false_type) {
 // mean length.  us, two launches / one (a count in front: items):
 //   128 columns, len to 128    128 19.5 / 12.4, 332 21.4 / 21.9 (128 of 24 .. 60 rows, 4 heads, 31 / 35)
 //                to 256        196 32.3 / 24.6 (256 of 20 .. 250, 1 head, 54 / 64)
-//                to 2048       296 94.6 / 84.9, 410 139 / 137; contextual rows, which make dQ's first block of a sequence the longest chain, past 768 rows only while each has a
-//                              CU: 116 111 / 107 (8 of 1000 .. 1200, 2 heads, 168 / 183)
-//                beyond        256 220 / 146, 312 264 / 227, 396 365 / 361, 504 442 / 497, 616 647 / 776; contextual: 4 of 1600 .. 6400, 1 head, 403 / 464
-//                windows that make the chains as long as one another, of short and of long sequences: 144 62.9 / 44.0, 176 31.5 / 33.5, 192 62.8 / 67.4, 268 162 / 168
+//                to 2048       296 94.6 / 84.9, 410 139 / 137; contextual rows, which make dQ's first block of a sequence the longest chain, only while each has a CU, past
+//                              1024 rows half of one: 116 111 / 107, 160 139 / 155 (8 of 1000 .. 1200, 2 heads, 168 / 183), 161 (33 of 230 .. 769) 58.1 / 53.4
+//                beyond        256 220 / 146, 312 264 / 227, 396 365 / 361, 504 442 / 497, 616 647 / 776; contextual: 4 of 1600 .. 6400, 1 head, 403 / 464, also with a window: 2 of 1557 .. 2595, 648, 146 / 184
+//                windows that make the chains as long as one another, of short, of long and of equal sequences: 144 62.9 / 44.0, 176 31.5 / 33.5, 192 62.8 / 67.4, 196 (7 of 749)
+//                              31.9 / 34.9, 268 162 / 168; others 269 (58 of 350 .. 584) 50.5 / 43.5
 //   64 columns, len to 256     384 36.3 / 28.2, 432 28.4 / 30.8 (128 of 20 .. 250, 4 heads, 52 / 57)
 //                beyond        576 409 / 320, 752 205 / 190, 824 689 / 651, 936 1218 / 1363
 // Workgroups that find no rows (max_seq_len far above the lengths) cost more than those of the two kernels do.  128 columns: a grid of 960 32.9 / 30.4, 1304 61 / 86, 1760 66 / 92,
-// 2160 73 / 93; 64 columns: 3744 81 / 58, 5600 31 / 40, 60144 137 / 211.
+// 2160 73 / 93, with such a window 560 63.9 / 68.4, 904 54 / 63; 64 columns: 3744 81 / 58, 5600 31 / 40, 60144 137 / 211.
 inline bool one_launch(int dqk, int dv, int64_t batch, int64_t heads, int64_t rows, int64_t max_seq_len, int64_t window, bool contextual, int64_t grid) {
     if (batch <= 0 || heads <= 0) return false;
     const int64_t pairs = batch * heads, upper = heads * (rows / 128 + batch);
@@ -62,9 +63,9 @@ inline bool one_launch(int dqk, int dv, int64_t batch, int64_t heads, int64_t ro
     if (pairs < 8) items = items * 8 / pairs;
     const int64_t len = max_seq_len < 2 * rows / batch ? max_seq_len : 2 * rows / batch;
     if (dqk <= 64 && dv <= 64) return grid <= 4096 && items <= (len <= 256 ? 384 : 768);
-    if (grid > 1024) return false;
-    if (window > 0 && window < len / 2 && (len <= 256 || len > 1400)) return items <= 144;
-    if (contextual && max_seq_len > 768) return max_seq_len <= 2048 && items <= 256;
+    if (grid > 1024 || (contextual && max_seq_len > 2048)) return false;
+    if (window > 0 && window < len / 2 && (len <= 256 || len > 1400 || 8 * batch * max_seq_len <= 9 * rows)) return items <= 144 && grid <= 512;
+    if (contextual && max_seq_len > 768) return items <= (len > 1024 ? 128 : 256);
     if (len <= 256) return items <= (len <= 128 ? 128 : 256);
     return items <= (len <= 2048 ? 512 : 384);
 }

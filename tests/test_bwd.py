@@ -582,8 +582,9 @@ def test_gradients_of_one_launch_are_those_of_two(dev, dtype, dqk, dv, N, H):
     # the lengths (up to 1.6 times as long in one launch), and one whose grid a launch could not hold twice
     [(64, 128, [85] * 8, 2, 150, 0, 0, True), (128, 128, [50] * 32, 4, 100, 0, 0, True), (128, 128, [50] * 33, 4, 100, 0, 0, False), (64, 128, [140] * 32, 4, 250, 0, 0, True),
      (64, 128, [140] * 33, 4, 250, 0, 0, False), (128, 32, [1200] * 12, 4, 2000, 0, 0, True), (128, 32, [1200] * 13, 4, 2000, 0, 0, False), (128, 128, [1379] * 5, 2, 1379, 0, 6, True),
-     (128, 128, [1379] * 13, 2, 1379, 0, 6, False), (128, 64, [4000] * 2, 1, 4000, 0, 0, True), (128, 64, [4000] * 2, 1, 4000, 0, 6, False), (128, 32, [7981], 2, 7981, 0, 0, False),
-     (64, 128, [2988], 1, 2988, 747, 0, False), (64, 128, [2071], 1, 2071, 517, 0, True), (64, 64, [140] * 48, 4, 250, 0, 0, True), (64, 64, [140] * 49, 4, 250, 0, 0, False),
+     (128, 128, [1379] * 6, 2, 1379, 0, 6, False), (128, 32, [500] * 33, 1, 769, 0, 6, True), (128, 64, [4000] * 2, 1, 4000, 0, 0, True), (128, 64, [4000] * 2, 1, 4000, 0, 6, False), (128, 32, [7981], 2, 7981, 0, 0, False),
+     (64, 128, [2988], 1, 2988, 747, 0, False), (64, 128, [2071], 1, 2071, 517, 0, True), (64, 128, [2076] * 2, 1, 2600, 648, 6, False), (128, 32, [2232], 1, 14364, 558, 0, False),
+     (32, 128, [749] * 7, 4, 749, 187, 0, False), (32, 128, [467] * 58, 1, 584, 146, 6, True), (64, 64, [140] * 48, 4, 250, 0, 0, True), (64, 64, [140] * 49, 4, 250, 0, 0, False),
      (32, 64, [5469], 1, 5469, 0, 0, True), (32, 64, [14000], 1, 14000, 0, 0, False), (32, 64, [310] * 14, 8, 310, 0, 0, True), (32, 64, [310] * 14, 8, 68627, 0, 0, False),
      (64, 128, [60], 2, 1024, 0, 0, True), (64, 128, [60], 2, 63355, 0, 0, False), (32, 32, [60], 8, 100_000_000, 0, 0, False)],
 )
